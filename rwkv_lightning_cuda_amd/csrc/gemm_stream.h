@@ -1,0 +1,96 @@
+// What the two files of the packed-weight GEMM share: the launch arguments and the exact expansion of int8 / int4 codes
+// to fp16 (gemm_stream.hip: packing, dispatch, split-K reduce and the register-staged tiles; gemm_ring.hip: the
+// LDS-ring tiles).
+#pragma once
+
+#include "ops.h"
+
+namespace rwkv {
+
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+struct StreamProblem {
+  const half_t* x;
+  const uint4_t* wp;
+  const half_t* scale;
+  const uint8_t* zp;
+  void* y;
+  float* partial;  // [splits][M][N] fp32, only with splits > 1
+  int N;
+  int fmt;
+  int group_n, group_k;  // int4: scale and zero point of (column n, 128-group k) at n * group_n + k * group_k
+};
+
+// Up to kMaxProblems products that share M, K and the split (each with its own weights, format, x and y) in one
+// launch: grid.y runs over the column blocks of all problems, block_end[] are the prefix sums.
+struct StreamArgs {
+  StreamProblem p[kMaxProblems];
+  int block_end[kMaxProblems];
+  int n_problems;
+  int M, K;
+  int splits, k_per_split;
+  int row_tiles, col_blocks;
+  int epilogue, out_f32;
+  RowCopy copy;  // rides on the launch: its first blocks move these rows (they are no operand of the product)
+};
+
+// shared out between the first blocks of the launch (those with y == z == 0), so that no single block carries it on its
+// critical path; in a launch whose other wavefronts are busy, called by the last `threads` of the block
+__device__ __forceinline__ void ride_along_copy(const RowCopy& cp, unsigned threads = 0) {
+  constexpr unsigned kCopyBlocks = 8;
+  const unsigned nb = gridDim.x < kCopyBlocks ? gridDim.x : kCopyBlocks;
+  if (threads == 0) threads = blockDim.x;
+  if (blockIdx.x < nb && blockIdx.y == 0 && blockIdx.z == 0 && cp.n > 0) {
+    const unsigned t = threadIdx.x - (blockDim.x - threads);
+    for (int i = (blockIdx.x * threads + t) * 8; i < cp.n; i += nb * threads * 8)
+      *reinterpret_cast<uint4_t*>(cp.dst + i) = *reinterpret_cast<const uint4_t*>(cp.src + i);
+  }
+}
+
+__device__ __forceinline__ half8_t make_half8(half2_t a, half2_t b, half2_t c, half2_t d) {
+  half8_t r;
+  r[0] = a[0]; r[1] = a[1]; r[2] = b[0]; r[3] = b[1];
+  r[4] = c[0]; r[5] = c[1]; r[6] = d[0]; r[7] = d[1];
+  return r;
+}
+
+// 8 int8 codes (two dwords) -> 8 fp16, exact: byte^0x80 under exponent 0x64 is 1024 + (code + 128).
+__device__ __forceinline__ half8_t expand_w8(uint32_t d0, uint32_t d1) {
+  const half2_t bias = {static_cast<half_t>(1152.0f), static_cast<half_t>(1152.0f)};
+  d0 ^= 0x80808080u;
+  d1 ^= 0x80808080u;
+  return make_half8(as_half2(__builtin_amdgcn_perm(0x64646464u, d0, 0x04010400u)) - bias,
+                    as_half2(__builtin_amdgcn_perm(0x64646464u, d0, 0x04030402u)) - bias,
+                    as_half2(__builtin_amdgcn_perm(0x64646464u, d1, 0x04010400u)) - bias,
+                    as_half2(__builtin_amdgcn_perm(0x64646464u, d1, 0x04030402u)) - bias);
+}
+
+// 8 int4 codes (one dword, element 2i in the low nibble of byte i) minus the zero point -> 8 fp16, exact.
+__device__ __forceinline__ half8_t expand_w4(uint32_t d, half2_t bias) {
+  const uint32_t even = d & 0x0f0f0f0fu;
+  const uint32_t odd = (d >> 4) & 0x0f0f0f0fu;
+  return make_half8(as_half2(__builtin_amdgcn_perm(odd, even, 0x0c040c00u) | 0x64006400u) - bias,
+                    as_half2(__builtin_amdgcn_perm(odd, even, 0x0c050c01u) | 0x64006400u) - bias,
+                    as_half2(__builtin_amdgcn_perm(odd, even, 0x0c060c02u) | 0x64006400u) - bias,
+                    as_half2(__builtin_amdgcn_perm(odd, even, 0x0c070c03u) | 0x64006400u) - bias);
+}
+
+__device__ __forceinline__ float finish_value(float v, int epilogue) {
+  v = round_h(v);
+  if (epilogue == RWKV_EPI_RELU_SQUARE) {
+    v = fmaxf(v, 0.0f);
+    v = round_h(v * v);
+  }
+  return v;
+}
+
+// gemm_ring.hip: the tile shapes of the LDS-ring kernel: 32 * mt rows, nb * wp bands of 32 columns, kc k per stage.
+struct RingShape {
+  int mt, nb, wp, kc;
+};
+constexpr RingShape kRingShapes[] = {{1, 1, 2, 128}, {1, 1, 2, 256}, {2, 1, 2, 256}, {2, 2, 2, 128}, {1, 1, 4, 128}, {2, 1, 4, 128}, {4, 1, 2, 128}, {4, 1, 4, 128}};
+// fmt: the format of the launch's problems; mixed: fp16 problems among them, with half as many columns per block
+bool gemm_ring_has(const RingShape& shape, int fmt, bool mixed);
+int gemm_ring_launch(hipStream_t st, const RingShape& shape, int fmt, bool mixed, const StreamArgs& g);
+
+}  // namespace rwkv

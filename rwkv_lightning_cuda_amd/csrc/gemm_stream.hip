@@ -14,22 +14,17 @@
 // to the matrix core after an exact in-register expansion of the codes, without any transpose or LDS
 // traffic for the weights; every weight byte leaves HBM once per 32*MT rows of X.
 //
-// Work split.  A block covers 32*MT rows x 128 output columns x one K slice with one or two groups of four
-// wavefronts: each wavefront streams one band, the groups take alternate chunks of KC = 128 k and meet in LDS at
-// the end.  The X rows of a chunk are staged in LDS and shared by the four wavefronts of the group.  Chunks
-// are software-pipelined: weight pieces are requested three chunks ahead into a ring of register sets, X two
-// chunks ahead, the X fragments of the next MFMA step are read from LDS while the current one runs; one barrier
-// per chunk.  With more than one K split each block writes an fp32 partial tile and a second small kernel
-// sums the partials in split order (a fixed order: results do not depend on scheduling) and applies scale and
-// epilogue.
+// Two kernels stream that order.  gemm_ring.hip: up to a few hundred rows (all rows for int4 codes), where the product is
+// bound by the weights' and X's way into the CUs.  Here: the wide tiles for more rows, bound by the matrix core.  With more
+// than one K split each block writes an fp32 partial tile and a second small kernel sums the partials in split order (a
+// fixed order: results do not depend on scheduling) and applies scale and epilogue - or the LayerNorm kernel that consumes
+// the result does (DeferredReduce).
 #include <algorithm>
-#include <cstdlib>
+#include <climits>
 
-#include "ops.h"
+#include "gemm_stream.h"
 
 namespace rwkv {
-
-typedef float float16_t __attribute__((ext_vector_type(16)));
 
 template <int FMT>
 struct PackTraits;
@@ -86,99 +81,25 @@ int pack_weights_launch(hipStream_t st, int fmt, int N, int K, const void* w, vo
 
 // ---- the GEMM ---------------------------------------------------------------------------------------------------------
 
-struct StreamProblem {
-  const half_t* x;
-  const uint4_t* wp;
-  const half_t* scale;
-  const uint8_t* zp;
-  void* y;
-  float* partial;  // [splits][M][N] fp32, only with splits > 1
-  int N;
-  int fmt;
-};
-
-// Up to kMaxProblems products that share M, K and the split (each with its own weights, format, x and y) in one
-// launch: grid.y runs over the column blocks of all problems, block_end[] are the prefix sums.
-struct StreamArgs {
-  StreamProblem p[kMaxProblems];
-  int block_end[kMaxProblems];
-  int n_problems;
-  int M, K;
-  int splits, k_per_split;
-  int row_tiles, col_blocks;
-  int epilogue, out_f32;
-  RowCopy copy;  // rides on the launch: its first blocks move these rows (they are no operand of the product)
-};
-
-// shared out between the first blocks of the launch, so that no single block carries it on its critical path
-__device__ __forceinline__ void ride_along_copy(const RowCopy& cp) {
-  constexpr unsigned kCopyBlocks = 8;
-  const unsigned nb = gridDim.x < kCopyBlocks ? gridDim.x : kCopyBlocks;
-  if (blockIdx.x < nb && blockIdx.y == 0 && blockIdx.z == 0 && cp.n > 0) {
-    for (int i = (blockIdx.x * blockDim.x + threadIdx.x) * 8; i < cp.n; i += nb * blockDim.x * 8)
-      *reinterpret_cast<uint4_t*>(cp.dst + i) = *reinterpret_cast<const uint4_t*>(cp.src + i);
-  }
-}
-
-__device__ __forceinline__ half8_t make_half8(half2_t a, half2_t b, half2_t c, half2_t d) {
-  half8_t r;
-  r[0] = a[0]; r[1] = a[1]; r[2] = b[0]; r[3] = b[1];
-  r[4] = c[0]; r[5] = c[1]; r[6] = d[0]; r[7] = d[1];
-  return r;
-}
-
-// 8 int8 codes (two dwords) -> 8 fp16, exact: byte^0x80 under exponent 0x64 is 1024 + (code + 128).
-__device__ __forceinline__ half8_t expand_w8(uint32_t d0, uint32_t d1) {
-  const half2_t bias = {static_cast<half_t>(1152.0f), static_cast<half_t>(1152.0f)};
-  d0 ^= 0x80808080u;
-  d1 ^= 0x80808080u;
-  return make_half8(as_half2(__builtin_amdgcn_perm(0x64646464u, d0, 0x04010400u)) - bias,
-                    as_half2(__builtin_amdgcn_perm(0x64646464u, d0, 0x04030402u)) - bias,
-                    as_half2(__builtin_amdgcn_perm(0x64646464u, d1, 0x04010400u)) - bias,
-                    as_half2(__builtin_amdgcn_perm(0x64646464u, d1, 0x04030402u)) - bias);
-}
-
-// 8 int4 codes (one dword, element 2i in the low nibble of byte i) minus the zero point -> 8 fp16, exact.
-__device__ __forceinline__ half8_t expand_w4(uint32_t d, half2_t bias) {
-  const uint32_t even = d & 0x0f0f0f0fu;
-  const uint32_t odd = (d >> 4) & 0x0f0f0f0fu;
-  return make_half8(as_half2(__builtin_amdgcn_perm(odd, even, 0x0c040c00u) | 0x64006400u) - bias,
-                    as_half2(__builtin_amdgcn_perm(odd, even, 0x0c050c01u) | 0x64006400u) - bias,
-                    as_half2(__builtin_amdgcn_perm(odd, even, 0x0c060c02u) | 0x64006400u) - bias,
-                    as_half2(__builtin_amdgcn_perm(odd, even, 0x0c070c03u) | 0x64006400u) - bias);
-}
-
-template <int FMT, int MT, int KC, int WG = 4>
+// The wide tile: 32 * MT rows, chunks of KC k, four wavefronts.
+template <int FMT, int MT, int KC>
 struct Tile {
   using P = PackTraits<FMT>;
   static constexpr int BM = 32 * MT;
   static constexpr int G = 2 * P::KR;
   static constexpr int GROUPS = KC / G;
-  static constexpr int NW = GROUPS * P::PIECES;     // weight pieces per lane per chunk
+  static constexpr int NW = GROUPS * P::PIECES;     // weight pieces per lane per chunk and band
   static constexpr int STEPS = P::KR / 8;
   static constexpr int XSTRIDE = KC + 8;            // fp16 per staged row: 16-byte pad keeps b128 reads conflict-free
-  static constexpr int GT = 64 * WG;                // threads of a wavefront group
+  static constexpr int GT = 256;                    // threads of the block
   static constexpr int XV = BM * (KC / 8) / GT;     // 16-byte vectors of X per thread per chunk
-  static constexpr int QG = KC / 128;               // int4 scale groups per chunk
-  static constexpr int NACC = MT == 1 ? 2 : 1;      // independent accumulation chains per row tile
-  static constexpr int DEPTH = (NW * 4 <= 16) ? 4 : (NW * 4 <= 32 ? 3 : 2);  // weight register sets in the ring
   static constexpr int kTileHalfs = BM * XSTRIDE;   // one staged X tile
-  static_assert(KC % 128 == 0 && XV >= 1, "chunk must hold whole int4 groups and at least one vector per thread");
 };
 
-__device__ __forceinline__ float finish_value(float v, int epilogue) {
-  v = round_h(v);
-  if (epilogue == RWKV_EPI_RELU_SQUARE) {
-    v = fmaxf(v, 0.0f);
-    v = round_h(v * v);
-  }
-  return v;
-}
-
 // One chunk's slice of X held by a thread between request and its store to LDS.
-template <int FMT, int MT, int KC, int WG>
+template <int FMT, int MT, int KC>
 struct XRegs {
-  using T = Tile<FMT, MT, KC, WG>;
+  using T = Tile<FMT, MT, KC>;
   uint4_t xv[T::XV];
 
   // vector i of the thread's slice
@@ -209,295 +130,21 @@ struct XRegs {
   }
 };
 
-// One chunk's weight pieces (and int4 group scales) held by a lane between request and use.
+// One chunk's weight pieces held by a lane between request and use.
 template <int FMT, int MT, int KC>
 struct WRegs {
   using T = Tile<FMT, MT, KC>;
   uint4_t w[T::NW];
-  // int4 group scale and zero point as loaded: converted at their use in multiply().  Converted beside the loads,
-  // they would make every request wait for all the weights in flight.
-  half_t sc[T::QG];
-  uint32_t zb[T::QG];
 
-  // piece i of the chunk at kc (fp16 and int8 codes: no group scales)
+  // piece i of the chunk at kc
   __device__ __forceinline__ void request_piece(int i, int kc, const uint4_t* wband) {
-    using P = typename T::P;
-    w[i] = wband[static_cast<int64_t>(kc / T::G) * (P::PIECES * 64) + i * 64];
+    w[i] = wband[static_cast<int64_t>(kc / T::G) * (T::P::PIECES * 64) + i * 64];
   }
-
-  __device__ __forceinline__ void request(const StreamArgs& g, const StreamProblem& pr, int kc, const uint4_t* wband,
-                                          int n) {
-    using P = typename T::P;
-    const uint4_t* wp = wband + static_cast<int64_t>(kc / T::G) * (P::PIECES * 64);
+  __device__ __forceinline__ void request(int kc, const uint4_t* wband) {
 #pragma unroll
-    for (int i = 0; i < T::NW; ++i) w[i] = wp[i * 64];
-    if constexpr (FMT == RWKV_FMT_W4) {
-      const int64_t q0 = static_cast<int64_t>(n) * (g.K >> 7) + (kc >> 7);
-#pragma unroll
-      for (int q = 0; q < T::QG; ++q) {
-        sc[q] = pr.scale[q0 + q];
-        zb[q] = pr.zp[q0 + q];
-      }
-    }
-  }
-
-  // The X fragments of MFMA step ks+1 are read from LDS while step ks runs (the compiler on its own issues each
-  // read right before its use, which leaves the matrix core idle for the LDS latency on every step);
-  // __builtin_amdgcn_sched_barrier(0) keeps the reads where they are written.
-  __device__ __forceinline__ void multiply(const half_t* xs, int j, int h, float16_t (&acc)[MT][T::NACC],
-                                           float16_t (&part)[MT][T::NACC]) const {
-    using P = typename T::P;
-    constexpr int NK = T::GROUPS * T::STEPS;
-    float scf[T::QG], zbf[T::QG];
-    if constexpr (FMT == RWKV_FMT_W4) {
-#pragma unroll
-      for (int q = 0; q < T::QG; ++q) {
-        uint32_t sr = __builtin_bit_cast(unsigned short, sc[q]), zr = zb[q];
-        asm volatile("" : "+v"(sr), "+v"(zr));  // the conversions stay here, below the requests of this chunk
-        scf[q] = h2f(__builtin_bit_cast(half_t, static_cast<unsigned short>(sr)));
-        zbf[q] = 1024.0f + static_cast<float>(zr);
-      }
-    }
-    const half_t* xlane = xs + j * T::XSTRIDE + h * P::KR;
-    half8_t a[2][MT];
-    auto load_a = [&](int ks, half8_t (&dst)[MT]) {
-      const half_t* xa = xlane + (ks / T::STEPS) * T::G + 8 * (ks % T::STEPS);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) dst[mt] = *reinterpret_cast<const half8_t*>(xa + mt * 32 * T::XSTRIDE);
-    };
-    load_a(0, a[0]);
-#pragma unroll
-    for (int ks = 0; ks < NK; ++ks) {
-      const int gi = ks / T::STEPS;
-      const int s = ks % T::STEPS;
-      if (ks + 1 < NK) load_a(ks + 1, a[(ks + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
-      half8_t b;
-      if constexpr (FMT == RWKV_FMT_F16) {
-        const uint4_t piece = w[gi * 2 + s];
-        b = __builtin_bit_cast(half8_t, piece);
-      } else if constexpr (FMT == RWKV_FMT_W8) {
-        const uint4_t piece = w[gi];
-        b = s == 0 ? expand_w8(piece[0], piece[1]) : expand_w8(piece[2], piece[3]);
-      } else {
-        const uint4_t piece = w[gi];
-        const half_t zf = static_cast<half_t>(zbf[(gi * T::G) >> 7]);
-        const half2_t bias = {zf, zf};
-        b = expand_w4(piece[s], bias);
-      }
-      constexpr int kChainMask = T::NACC - 1;
-      const int chain = ks & kChainMask;
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        if constexpr (FMT == RWKV_FMT_W4) {
-          part[mt][chain] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks & 1][mt], b, part[mt][chain], 0, 0, 0);
-        } else {
-          acc[mt][chain] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks & 1][mt], b, acc[mt][chain], 0, 0, 0);
-        }
-      }
-      if constexpr (FMT == RWKV_FMT_W4) {
-        if (s == T::STEPS - 1 && ((gi + 1) * T::G) % 128 == 0) {  // end of a 128-group: fold with its scale
-          const float s128 = scf[(gi * T::G) >> 7];
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int c = 0; c < T::NACC; ++c)
-#pragma unroll
-              for (int v = 0; v < 16; ++v) {
-                acc[mt][c][v] = fmaf(part[mt][c][v], s128, acc[mt][c][v]);
-                part[mt][c][v] = 0.0f;
-              }
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int i = 0; i < T::NW; ++i) request_piece(i, kc, wband);
   }
 };
-
-// One block of one problem: 32 * WG columns x the block's K slice.  The block has KG groups of WG wavefronts (one
-// 32-column band of the weights per wavefront); group kg takes chunks kg, kg + KG, ... of the slice with its own
-// pair of X tiles in LDS, and the groups' sums meet in LDS at the end (in group order), so that a CU holds two
-// wavefronts per SIMD - one's code expansion overlaps the other's matrix-core time - without more fp32 partial
-// tiles in HBM.
-//
-// Per group and chunk c: the X slice of chunk c+2 is requested into registers, the weight pieces of chunk
-// c+D-1 into a ring of D register sets, the matrix core runs chunk c out of LDS tile c&1, then the X slice of
-// chunk c+1 (requested one iteration earlier) is stored to the other tile; one barrier per chunk.  Every load
-// of the loop is issued unconditionally - past the end of the slice it re-reads the current chunk, which is in
-// cache - because a load under a branch makes the compiler's s_waitcnt accounting assume the shorter path
-// and wait for everything in flight.  Within an iteration X is requested before the weights, so that waiting
-// for X does not wait for the younger weight loads.
-template <int FMT, int MT, int KC, int KG, int WG>
-__device__ __forceinline__ void stream_block(const StreamArgs& g, const StreamProblem& pr, int row_tile, int col_block,
-                                             int split, half_t* xs_all) {
-  using T = Tile<FMT, MT, KC, WG>;
-  using P = typename T::P;
-  constexpr int BM = T::BM;
-  constexpr int GT = T::GT;
-
-  const int tid = threadIdx.x % GT;  // thread within its k-group
-  const int kg = threadIdx.x / GT;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
-  const int j = lane & 31;
-  const int h = lane >> 5;
-  const int m0 = row_tile * BM;
-  const int band_here = col_block * WG + wave;  // 32-row band of W = 32 output columns
-  const bool active = band_here * 32 < pr.N;
-  const int band = active ? band_here : pr.N / 32 - 1;  // a wavefront past the last band repeats it and stores nothing
-  const int n = band * 32 + j;
-  constexpr int KSTRIDE = KC * KG;  // between consecutive chunks of one group
-  const int kbeg = split * g.k_per_split + kg * KC;
-  const int nchunks = g.k_per_split / KSTRIDE;
-  half_t* xs = xs_all + kg * 2 * T::kTileHalfs;
-
-  float16_t acc[MT][T::NACC], part[MT][T::NACC];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int c = 0; c < T::NACC; ++c)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        acc[mt][c][v] = 0.0f;
-        part[mt][c][v] = 0.0f;
-      }
-
-  // this lane's first piece of the band; consecutive pieces are 64 uint4 apart
-  const uint4_t* wband = pr.wp + (static_cast<int64_t>(band) * (g.K / T::G)) * (P::PIECES * 64) + lane;
-  // the column's int8 scale now: read in the epilogue it costs every block a trip to memory (1.2 us per launch)
-  half_t scale_h = static_cast<half_t>(1.0f);
-  if constexpr (FMT == RWKV_FMT_W8) scale_h = pr.scale[n];
-
-  constexpr int D = T::DEPTH;
-  WRegs<FMT, MT, KC> wr[D];
-  XRegs<FMT, MT, KC, WG> xr[2];
-  const int last = nchunks - 1;
-  xr[0].request(g, pr, tid, m0, kbeg);
-  xr[1].request(g, pr, tid, m0, kbeg + min(1, last) * KSTRIDE);
-#pragma unroll
-  for (int i = 0; i < D - 1; ++i) wr[i].request(g, pr, kbeg + min(i, last) * KSTRIDE, wband, n);
-  xr[0].store_x(tid, xs);
-  __syncthreads();
-  constexpr int U = (D % 2 == 0) ? D : 2 * D;  // unroll: register sets and LDS tiles are indexed statically
-  // Whole rounds of U chunks run as one basic block: with an exit between the chunks the compiler waits for every
-  // load in flight at the head of each round (the weight ring then drains once per round).  The chunks left over
-  // (K slices that are not a multiple of U chunks) take the same steps with the exits.
-  const int whole = nchunks - nchunks % U;
-  int c0 = 0;
-  for (; c0 < whole; c0 += U) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int c = c0 + u;
-      xr[u & 1].request(g, pr, tid, m0, kbeg + (c + 2 <= last ? c + 2 : c) * KSTRIDE);
-      wr[(u + D - 1) % D].request(g, pr, kbeg + (c + D - 1 <= last ? c + D - 1 : c) * KSTRIDE, wband, n);
-      wr[u % D].multiply(xs + (u & 1) * T::kTileHalfs, j, h, acc, part);
-      xr[(u + 1) & 1].store_x(tid, xs + ((u + 1) & 1) * T::kTileHalfs);
-      __syncthreads();
-    }
-  }
-  if (c0 < nchunks) {
-#pragma unroll
-    for (int u = 0; u < U - 1; ++u) {
-      const int c = c0 + u;
-      if (c >= nchunks) break;
-      xr[u & 1].request(g, pr, tid, m0, kbeg + (c + 2 <= last ? c + 2 : c) * KSTRIDE);
-      wr[(u + D - 1) % D].request(g, pr, kbeg + (c + D - 1 <= last ? c + D - 1 : c) * KSTRIDE, wband, n);
-      wr[u % D].multiply(xs + (u & 1) * T::kTileHalfs, j, h, acc, part);
-      xr[(u + 1) & 1].store_x(tid, xs + ((u + 1) & 1) * T::kTileHalfs);
-      __syncthreads();
-    }
-  }
-
-  if constexpr (T::NACC == 2) {
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mt][0][v] += acc[mt][1][v];
-  }
-  // The X tiles are free after the last barrier.  The other groups hand their sums to group 0 through them; group 0
-  // then lays the finished 32*MT x 32*WG tile out in LDS (rows padded by 8 floats) and all threads write it to
-  // memory in 16/32-byte pieces along the rows - the accumulator layout itself would give 2-byte stores 64 bytes
-  // apart.
-  constexpr int kCols = 32 * WG;         // columns of the block
-  constexpr int kStageLd = kCols + 8;
-  constexpr int kRedFloats = (KG - 1) * MT * 16 * GT;
-  float* stage = reinterpret_cast<float*>(xs_all) + kRedFloats;
-  static_assert(kRedFloats * 4 + BM * kStageLd * 4 <= KG * 2 * T::kTileHalfs * 2, "epilogue tile exceeds the LDS tiles");
-  if constexpr (KG > 1) {
-    float* red = reinterpret_cast<float*>(xs_all);
-    if (kg > 0) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) red[((kg - 1) * MT * 16 + mt * 16 + v) * GT + tid] = acc[mt][0][v];
-    }
-    __syncthreads();
-  }
-  const bool partial_out = g.splits > 1;
-  if (kg == 0) {
-    const float scl = partial_out ? 1.0f : h2f(scale_h);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        float sum = acc[mt][0][v];
-#pragma unroll
-        for (int q = 1; q < KG; ++q) sum += reinterpret_cast<const float*>(xs_all)[((q - 1) * MT * 16 + mt * 16 + v) * GT + tid];
-        const int row = mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-        stage[row * kStageLd + wave * 32 + j] = partial_out ? sum : finish_value(mul_f32(sum, scl), g.epilogue);
-      }
-  }
-  __syncthreads();
-  float* part_out = partial_out ? pr.partial + static_cast<int64_t>(split) * g.M * pr.N : nullptr;
-  const int col0 = col_block * kCols;
-  constexpr int kPieces = kCols / 8;  // 8-column pieces per row
-  for (int idx = threadIdx.x; idx < BM * kPieces; idx += GT * KG) {
-    const int row = idx / kPieces;
-    const int piece = idx % kPieces;
-    const int col = col0 + piece * 8;
-    if (m0 + row >= g.M || col >= pr.N) continue;
-    const float4_t lo = *reinterpret_cast<const float4_t*>(stage + row * kStageLd + piece * 8);
-    const float4_t hi = *reinterpret_cast<const float4_t*>(stage + row * kStageLd + piece * 8 + 4);
-    const int64_t o = static_cast<int64_t>(m0 + row) * pr.N + col;
-    if (partial_out || g.out_f32) {
-      float* dst = partial_out ? part_out + o : static_cast<float*>(pr.y) + o;
-      *reinterpret_cast<float4_t*>(dst) = lo;
-      *reinterpret_cast<float4_t*>(dst + 4) = hi;
-    } else {
-      half8_t hv;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        hv[e] = f2h(lo[e]);
-        hv[4 + e] = f2h(hi[e]);
-      }
-      *reinterpret_cast<half8_t*>(static_cast<half_t*>(pr.y) + o) = hv;
-    }
-  }
-}
-
-// grid = row tiles x roundup(column blocks over all problems x splits, 8), one-dimensional; block = 64 * WG * KG.
-// Workgroups go to the eight XCDs round-robin by linear id, each XCD with its own L2: the id is decoded so that
-// the row tiles of one (column block, split) pair - which stream the same weights - land on the same XCD.
-template <int MT, int KC, int KG, int WG>
-__global__ __launch_bounds__(64 * WG * KG) void gemm_stream_kernel(StreamArgs g) {
-  __shared__ __align__(16) half_t xs[KG * 2 * 32 * MT * (KC + 8)];
-  ride_along_copy(g.copy);
-  const int id = blockIdx.x;
-  const int row_tile = (id >> 3) % g.row_tiles;
-  const int pair = (id / (8 * g.row_tiles)) * 8 + (id & 7);
-  if (pair >= g.col_blocks * g.splits) return;
-  const int col_all = pair % g.col_blocks;
-  const int split = pair / g.col_blocks;
-  int pi = 0;
-  while (pi + 1 < g.n_problems && col_all >= g.block_end[pi]) ++pi;
-  const int col_block = col_all - (pi > 0 ? g.block_end[pi - 1] : 0);
-  const StreamProblem& pr = g.p[pi];
-  switch (pr.fmt) {
-    case RWKV_FMT_W8: stream_block<RWKV_FMT_W8, MT, KC, KG, WG>(g, pr, row_tile, col_block, split, xs); break;
-    case RWKV_FMT_W4: stream_block<RWKV_FMT_W4, MT, KC, KG, WG>(g, pr, row_tile, col_block, split, xs); break;
-    default: stream_block<RWKV_FMT_F16, MT, KC, KG, WG>(g, pr, row_tile, col_block, split, xs); break;
-  }
-}
 
 // ---- many rows: 128 rows x 256 columns per block, two bands per wavefront -------------------------------------------
 // From a few hundred rows on the product is bound by the matrix core and by LDS, not by the weights: with one band
@@ -519,7 +166,7 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
                                                   int split, half_t* xs) {
   static_assert(!ROLL || FMT == RWKV_FMT_W8, "the rolling weight set is laid out for int8 pieces (two MFMA steps each)");
   constexpr int KC = 128, NB = 2;
-  using T = Tile<FMT, MT, KC, 4>;
+  using T = Tile<FMT, MT, KC>;
   using P = typename T::P;
   constexpr int BM = T::BM;
   static_assert(FMT != RWKV_FMT_W4, "the wide tile takes int8 and fp16 weights");
@@ -562,11 +209,11 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
   constexpr int NK = T::GROUPS * T::STEPS;        // MFMA steps of a chunk
   if constexpr (ROLL) {
     WRegs<FMT, MT, KC> w[NB];
-    XRegs<FMT, MT, KC, 4> xq;
+    XRegs<FMT, MT, KC> xq;
     const int last = nchunks - 1;
     xq.request(g, pr, tid, m0, kbeg);
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) w[nb].request(g, pr, kbeg, wband[nb], n[nb]);
+    for (int nb = 0; nb < NB; ++nb) w[nb].request(kbeg, wband[nb]);
     xq.store_x(tid, xs);
     __syncthreads();
     static_assert(T::XV % (NK / 2) == 0 && T::STEPS == 2 && T::NW == T::GROUPS,
@@ -626,14 +273,14 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
   static_assert(T::XV == NK && NB * T::NW % NK == 0, "one X vector and a whole number of weight pieces per MFMA step");
   static_assert(MT == 4, "the ring variant is the 128-row tile");
   WRegs<FMT, MT, KC> wr[D][NB];
-  XRegs<FMT, MT, KC, 4> xr[2];
+  XRegs<FMT, MT, KC> xr[2];
   const int last = nchunks - 1;
   xr[0].request(g, pr, tid, m0, kbeg);
   xr[1].request(g, pr, tid, m0, kbeg + min(1, last) * KC);
 #pragma unroll
   for (int i = 0; i < D - 1; ++i)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) wr[i][nb].request(g, pr, kbeg + min(i, last) * KC, wband[nb], n[nb]);
+    for (int nb = 0; nb < NB; ++nb) wr[i][nb].request(kbeg + min(i, last) * KC, wband[nb]);
   xr[0].store_x(tid, xs);
   __syncthreads();
 
@@ -773,6 +420,29 @@ __global__ __launch_bounds__(256, MIXED ? 1 : 2) void gemm_stream_wide_kernel(St
   }
 }
 
+// int4 scales and zero points by group: the 32 columns of a band then lie in one piece of 64 (32) bytes, where the rows of
+// [N][K/128] put every column in a cache line of its own (K = 16384, 17 / 64 / 256 rows: 19.4 / 25.8 / 57.9 -> 16.2 / 23.1 /
+// 53.9 us per 4096-column product).  Load time only.
+__global__ __launch_bounds__(256) void transpose_groups_kernel(int N, int groups, const half_t* __restrict__ scale,
+                                                               const uint8_t* __restrict__ zp, half_t* __restrict__ scale_t,
+                                                               uint8_t* __restrict__ zp_t) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= static_cast<int64_t>(N) * groups) return;
+  const int n = static_cast<int>(i % N);
+  const int q = static_cast<int>(i / N);
+  scale_t[i] = scale[static_cast<int64_t>(n) * groups + q];
+  zp_t[i] = zp[static_cast<int64_t>(n) * groups + q];
+}
+
+int transpose_groups_launch(hipStream_t st, int N, int groups, const half_t* scale, const uint8_t* zp, half_t* scale_t,
+                            uint8_t* zp_t) {
+  RWKV_REQUIRE(N > 0 && groups > 0 && scale && zp && scale_t && zp_t, "transpose_groups: bad arguments");
+  const unsigned blocks = static_cast<unsigned>((static_cast<int64_t>(N) * groups + 255) / 256);
+  hipLaunchKernelGGL(transpose_groups_kernel, dim3(blocks), dim3(256), 0, st, N, groups, scale, zp, scale_t, zp_t);
+  RWKV_LAUNCH_CHECK();
+  return RWKV_OK;
+}
+
 struct ReduceProblem {
   const float4_t* partial;
   const half_t* scale;  // NULL unless the problem's weights are int8 codes
@@ -827,129 +497,170 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(ReduceArgs g) {
   }
 }
 
-// RWKV_GEMM_BLOCKS (tuning hook) = blocks wanted per launch before K is split.  200 of the 256 CUs: a grid of
-// 206 blocks (the r/k/v + LoRA rank-in launch at two row tiles) is 25-30 % faster unsplit than split in two.
-static int env_int(const char* name, int fallback) {
-  const char* e = getenv(name);
-  const int v = e ? atoi(e) : 0;
-  return v > 0 ? v : fallback;
-}
-static int target_blocks() {
-  static const int v = env_int("RWKV_GEMM_BLOCKS", 200);
-  return v;
-}
-
-// Tile per row count (measured on 4096x4096, 16384x4096 and 4096x16384 int8 weights): up to 64 rows one 32-row
-// tile per block, so that two or more row tiles share the weights through their XCD's L2 and the split stays
-// small; up to 512 rows 64-row tiles; both with two wavefront groups per block.  Above that 128-row tiles with
-// one group (128 accumulator registers per lane leave no room for a second wavefront per SIMD).
-// 33..64 rows against enough column blocks to occupy the CUs without a K split (the head): one 64-row tile, so that
-// no weight is requested by two blocks (268 MB of int8 codes at 64 rows: 95 -> 75 us).
-// Up to 32 rows, where 128-column blocks would need a K split: blocks of 64 columns with four groups of two
-// wavefronts - twice the blocks per matrix, so half the split (less partial-sum traffic) or none (no reduce
-// launch): 16 rows x 16384 columns 23.4 -> 19.6 us; decode steps of 8 / 16 / 32 rows 7 / 5 / 3 % faster.  At 64
-// rows the narrow blocks lose (24.5 -> 30 us): every block reads all of X.
-// From 385 rows on, int8 and fp16 weights, when 128 x 256 tiles alone give 128 blocks or more: the wide tile, whose
-// wavefronts feed two MFMAs from every X fragment they read from LDS and whose blocks request half the X bytes per
-// flop (int8 codes, 2048 rows: 16384x4096 436 -> 345 us, 4096x16384 400 -> 317 us; 512 rows x 16384 columns
-// 138 -> 104 us).  With fewer blocks it would need a K split where the 64-row tiles need none (512 rows x 4096
-// columns: 35 us against 42).  Its registers have no room for the int4 codes' zero points.
-constexpr int kWideMinRows = 384, kWideMinBlocks = 128;
 struct StreamConfig {
-  int mt, kc, kg, wg;
-  int nb = 1;  // bands per wavefront
-  int cols() const { return 32 * wg * nb; }
+  RingShape ring = {0, 0, 0, 0};  // mt == 0: the wide tile
+  int wide_mt = 0;                // wide tile: 2 (64 x 256, int8 only) or 4 (128 x 256)
+  int fmt = RWKV_FMT_F16;         // ring: the launch's format
+  bool mixed = false;             // ring: fp16 problems beside it
+  int splits = 1;
+  bool is_ring() const { return ring.mt > 0; }
+  int rows() const { return 32 * (is_ring() ? ring.mt : wide_mt); }
+  int cols(int problem_fmt) const {
+    if (!is_ring()) return 256;
+    const int bn = 32 * ring.nb * ring.wp;
+    return mixed && problem_fmt == RWKV_FMT_F16 ? bn / 2 : bn;
+  }
+  int k_step() const { return is_ring() ? ring.kc : 128; }
 };
-// (narrow matrices, K up to 2048, take it from 257 rows: at 256 rows x 6656 / 8192 x 2048 the 64 x 128 tiles need
-// 19.0 / 19.8 us against 24.5 / 24.9; at 384 rows it is ahead again, 30.2 / 33.4 against 33.9 / 35.1)
-bool linear_packed_int8_tile(int M, int K) {
-  return M > (K <= 2048 ? 256 : 128) && M <= 1024 && (K <= 4096 || M <= 384);
-}
-
-static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, const int* fmts) {
-  int cb128 = 0;
-  for (int i = 0; i < n_problems; ++i) cb128 += ceil_div(Ns[i], 128);
-  if (M <= 32 && K % (128 * 4) == 0 && cb128 < target_blocks()) {
-    // Narrow matrices (K up to 2048) whose 64-column blocks would not fill the chip without a K split: 32-column
-    // blocks of one wavefront per K group instead - twice the blocks, half the split or none, and with no split no
-    // reduce launch (us with the reduce, 64- / 32-column blocks, 8 rows: 6656 x 2048 11.1 / 9.4, 8192 x 2048
-    // 11.4 / 9.9, 2048 x 2048 8.6 / 8.4; at K = 4096 the 64-column blocks win, 4096 x 4096 11.5 / 12.2).
-    int cb64 = 0;
-    for (int i = 0; i < n_problems; ++i) cb64 += ceil_div(Ns[i], 64);
-    if (K <= 2048 && cb64 < target_blocks()) return StreamConfig{1, 128, 4, 1};
-    return StreamConfig{1, 128, 4, 2};
-  }
-  if (M > 32 && M <= 64 && cb128 >= target_blocks()) return StreamConfig{2, 128, 2, 4};
-  // 33..64 rows of narrow matrices (K up to 2048): the 64-column blocks again, which here need no K split where the
-  // 128-column blocks do, and X is short (us with the reduce, 128- / 64-column blocks, 64 rows: 6656 x 2048
-  // 14.0 / 11.5, 8192 x 2048 15.5 / 12.1, 2048 x 2048 10.7 / 9.6)
-  if (M > 32 && M <= 64 && K <= 2048 && K % (128 * 4) == 0 && 2 * cb128 < target_blocks()) return StreamConfig{1, 128, 4, 2};
-  if (M <= 64) return StreamConfig{1, 128, 2, 4};
-  // 65..128 rows against few column blocks (4096 columns and fewer) and a short K: 32-row tiles need half the K
-  // split of 64-row tiles for the same number of blocks (128 rows x 4096 x 4096: 19.8 -> 16.6 us; with K = 16384
-  // the 64-row tiles win, 35.5 us against 38.1)
-  // ... and where the 32-row tiles alone fill the chip and the 64-row tiles do not (128 rows x 6656 x 2048:
-  // 19.5 -> 13.4 us, 8192 x 2048: 21.7 -> 14.0; at 96 rows both would split and the 64-row tiles stay ahead)
-  if (M <= 128 && K <= 4096 && ceil_div(M, 64) * cb128 < target_blocks() &&
-      (ceil_div(M, 64) * cb128 * 2 <= target_blocks() || ceil_div(M, 32) * cb128 >= target_blocks()))
-    return StreamConfig{1, 128, 2, 4};
-  // 129..1024 rows, int8 weights only, and K up to 4096 or up to 384 rows: the 64 x 256 tile of two bands per
-  // wavefront that fits three wavefronts per SIMD (us, 64 x 256 / 128 x 256 / 64 x 128 tiles; * = with a K split:
-  // 256 rows x 16384 x 4096 51 / 59* / 64, 384 x 16384 x 4096 74 / 100* / 105, 384 x 4096 x 16384 85* / 96* / 112*,
-  // 768 x 12288 x 4096 115 / 139 / 160, 1024 x 4096 x 4096 47 / 56* / 66; against it 512 x 4096 x 16384
-  // 108* / 102* / 119 and 1024 x 4096 x 16384 193 / 177* / 223).  Launches with fp16 problems among them keep the
-  // tiles below.
-  bool all_w8 = true;
-  for (int i = 0; i < n_problems; ++i) all_w8 = all_w8 && fmts[i] == RWKV_FMT_W8;
-  if (all_w8 && linear_packed_int8_tile(M, K)) return StreamConfig{2, 128, 1, 4, 2};
-  // 129..256 rows against enough column blocks: 128-row tiles give one round of blocks where 64-row tiles give
-  // two (256 rows x 16384 x 4096: 62.5 -> 56 us)
-  if (M > 128 && M <= 256 && 2 * cb128 >= target_blocks() && 2 * cb128 <= 256) return StreamConfig{4, 128, 1, 4};
-  bool any_w4 = false;
-  int cb256 = 0;
-  for (int i = 0; i < n_problems; ++i) {
-    any_w4 = any_w4 || fmts[i] == RWKV_FMT_W4;
-    cb256 += ceil_div(Ns[i], 256);
-  }
-  if (M > kWideMinRows && !any_w4 && ceil_div(M, 128) * cb256 >= kWideMinBlocks) return StreamConfig{4, 128, 1, 4, 2};
-  if (M <= 512) return StreamConfig{2, 128, 2, 4};
-  return StreamConfig{4, 128, 1, 4};
-}
-static int count_col_blocks(const StreamConfig& c, int n_problems, const int* Ns) {
+static int count_col_blocks(const StreamConfig& c, int n_problems, const int* Ns, const int* fmts) {
   int col_blocks = 0;
-  for (int i = 0; i < n_problems; ++i) col_blocks += ceil_div(Ns[i], c.cols());
+  for (int i = 0; i < n_problems; ++i) col_blocks += ceil_div(Ns[i], c.cols(fmts[i]));
   return col_blocks;
 }
 
-// Split count: a power of two that gives enough blocks to occupy the CUs, K slices whole chunks of every group.
-static int choose_splits(const StreamConfig& c, int M, int col_blocks, int K) {
-  const int tiles = ceil_div(M, 32 * c.mt) * col_blocks;
-  int splits = 1;
-  while (tiles * splits < target_blocks() && K % (splits * 2 * c.kc * c.kg) == 0 && splits < 32) splits *= 2;
-  return splits;
+// Estimated microseconds of a launch: what the choice between tiles and K splits goes by.  Fitted to sweeps of every tile over
+// 17 .. 2048 rows x the matrices of the presets (2048 .. 65536 columns, 768 .. 16384 k, three formats); the tile it picks is
+// within a few percent of the best one of the sweep.
+//   ring: a fixed part (launch, first stage, epilogue); the bytes of the busiest CU at what a CU takes in while all of them
+//   stream (94 GB/s; 130 while half of the chip idles); what of the HBM stream of the weights does not hide behind that; the
+//   products; per further round of blocks its start and end, which a second block hides where two fit a CU.
+//   wide: bound by the matrix core (1 PFLOP/s with the shader clock these products run at).
+//   K splits: their fp32 planes and, where no consumer sums them, the reduce launch.
+static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred) {
+  constexpr int kCus = 256;
+  const int bm = c.rows();
+  int blocks = 0, bn_max = 0;
+  float block_bytes = 0.0f, w_bytes = 0.0f, n_total = 0.0f;
+  for (int i = 0; i < n_problems; ++i) {
+    const int bn = c.cols(fmts[i]);
+    const float per = fmts[i] == RWKV_FMT_F16 ? 2.0f : (fmts[i] == RWKV_FMT_W8 ? 1.0f : 0.55f);
+    blocks += ceil_div(Ns[i], bn);
+    block_bytes = std::max(block_bytes, bn * per + bm * 2.0f);
+    bn_max = std::max(bn_max, bn);
+    w_bytes += per * Ns[i];
+    n_total += Ns[i];
+  }
+  const float k_block = static_cast<float>(K) / c.splits;
+  blocks *= ceil_div(M, bm) * c.splits;
+  block_bytes *= k_block;
+  w_bytes *= static_cast<float>(K);
+  const int full = blocks / kCus, rest = blocks % kCus;
+  const int rounds = full + (rest > 0 ? 1 : 0);
+  float us;
+  if (c.is_ring()) {
+    us = 6.0f + 0.42f * w_bytes / 6.5e6f;
+    us += full * block_bytes / 94e3f;
+    if (rest > 0) us += block_bytes / (130e3f - 36e3f * std::max(0, rest - 128) / 128.0f);
+    const float gflop = 2e-9f * bm * bn_max * k_block * kCus;
+    const bool two_per_cu = c.ring.mt == 1 && c.ring.kc == 128;
+    const bool wide_ring = c.ring.mt == 4 || c.ring.wp == 4;
+    us += rounds * gflop * (c.fmt == RWKV_FMT_W4 ? (wide_ring ? 0.73f : 0.57f) : (c.ring.mt == 4 && c.fmt == RWKV_FMT_W8 ? 0.55f : (c.ring.nb == 2 ? 0.38f : 0.28f)));
+    us += (two_per_cu ? 1.5f : 4.5f) * (rounds - 1);
+  } else if (c.wide_mt == 2) {
+    us = 7.0f + 34.0f * std::max(1.0f, blocks * 1.05f / kCus) * k_block / 4096.0f;
+  } else {
+    us = 6.0f + (full + (rest > 0 ? (full > 0 ? 0.75f + 0.25f * rest / kCus : 1.0f) : 0.0f)) * (11.0f + 58.0f * k_block / 4096.0f);
+  }
+  if (c.splits > 1) us += (deferred ? 0.5f : 2.6f) + c.splits * M * n_total * (deferred ? 6.0f : 8.0f) / 5e6f;
+  return us;
 }
 
-// The formats are not known here: the larger of what the tiles with and without int4 weights would need.
+// Whether the planes of a K split may be left to the launch's consumer.  The choice of tile and split goes by this alone and
+// not by whether this call leaves them: a product has the same sums either way.
+static bool sums_at_consumer(int n_problems, int epilogue, int out_f32) {
+  return n_problems == 1 && epilogue == RWKV_EPI_NONE && !out_f32;
+}
+
+// Rows from which the wide tiles, whose wavefronts feed two MFMAs from every X fragment they read from LDS, are looked at.
+constexpr int kWideMinRows = 160;
+// Launches of int8 problems only have a wide tile of their own at these sizes (three blocks per CU).
+bool linear_packed_int8_tile(int M, int K) { return M > 512 && M <= 1024 && K <= 4096 && K > 2048; }
+
+static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, int max_splits) {
+  bool any[3] = {false, false, false};
+  for (int i = 0; i < n_problems; ++i) any[fmts[i]] = true;
+  StreamConfig best;
+  float best_us = 1e30f;
+  auto consider = [&](StreamConfig c) {
+    for (c.splits = 1; c.splits == 1 || (c.splits <= max_splits && K % (c.splits * c.k_step()) == 0); c.splits *= 2) {
+      const float us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred);
+      if (us < best_us) {
+        best_us = us;
+        best = c;
+      }
+    }
+  };
+  StreamConfig c;
+  c.fmt = any[RWKV_FMT_W8] ? RWKV_FMT_W8 : (any[RWKV_FMT_W4] ? RWKV_FMT_W4 : RWKV_FMT_F16);
+  c.mixed = c.fmt != RWKV_FMT_F16 && any[RWKV_FMT_F16];
+  for (const RingShape& shape : kRingShapes) {
+    if (!gemm_ring_has(shape, c.fmt, c.mixed)) continue;
+    c.ring = shape;
+    consider(c);
+  }
+  if (M >= kWideMinRows && !any[RWKV_FMT_W4]) {
+    c.ring = RingShape{0, 0, 0, 0};
+    c.wide_mt = 4;
+    // (from 1025 rows on, with most of the chip busy, the wide tile is the faster one whatever the estimates' last percent)
+    if (M > 1024 && ceil_div(M, 128) * count_col_blocks(c, n_problems, Ns, fmts) >= 200) best_us = 1e30f;
+    consider(c);
+    if (!any[RWKV_FMT_F16] && K <= 4096 && M <= 1024) {
+      c.wide_mt = 2;
+      consider(c);
+    }
+  }
+  return best;
+}
+
+// The formats are not known here, nor whether a consumer sums the planes: the largest that any of the choices would need.
 size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const int* Ns) {
   int64_t n_total = 0;
   for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
   int fmts[kMaxProblems];
-  size_t need = 0;
-  for (int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16}) {  // all int8, some int4, neither (fp16 among them)
-    for (int i = 0; i < n_problems && i < kMaxProblems; ++i) fmts[i] = fmt;
-    const StreamConfig c = choose_config(M, K, n_problems, Ns, fmts);
-    const int splits = choose_splits(c, M, count_col_blocks(c, n_problems, Ns), K);
-    if (splits > 1) need = std::max(need, static_cast<size_t>(splits) * M * n_total * sizeof(float));
+  int splits = 1;
+  for (int mix = 0; mix < 5; ++mix) {  // one format, or int8 / int4 problems with fp16 ones behind them
+    const int first = mix == 0 || mix == 3 ? RWKV_FMT_W8 : (mix == 1 || mix == 4 ? RWKV_FMT_W4 : RWKV_FMT_F16);
+    for (int i = 0; i < n_problems && i < kMaxProblems; ++i) fmts[i] = mix >= 3 && i >= std::min(3, n_problems - 1) ? RWKV_FMT_F16 : first;
+    for (const bool deferred : {false, true})
+      splits = std::max(splits, choose_config(M, K, n_problems, Ns, fmts, deferred, 32).splits);
   }
-  return need;
+  return splits > 1 ? static_cast<size_t>(splits) * M * n_total * sizeof(float) : 0;
 }
 
 size_t linear_packed_workspace_bytes(int M, int N, int K) { return linear_packed_multi_workspace_bytes(M, K, 1, &N); }
+
+static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
+                         void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy, bool fit_splits);
 
 int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue,
                         int out_f32, void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy) {
   RWKV_REQUIRE(n_problems >= 1 && n_problems <= kMaxProblems, "linear_packed: %d problems (1..%d allowed)", n_problems,
                kMaxProblems);
+  bool any[3] = {false, false, false};
+  for (int i = 0; i < n_problems; ++i) {
+    RWKV_REQUIRE(linear_packed_supported(problems[i].fmt, M, problems[i].N, K), "linear_packed: unsupported shape M=%d N=%d K=%d fmt=%d",
+                 M, problems[i].N, K, problems[i].fmt);
+    any[problems[i].fmt] = true;
+  }
+  if (!(any[RWKV_FMT_W8] && any[RWKV_FMT_W4]))
+    return packed_launch(st, M, K, n_problems, problems, epilogue, out_f32, workspace, workspace_bytes, defer, copy, n_problems > 1);
+  // int8 and int4 matrices side by side have no launch in common: one per format.  (fit_splits: formats may come in any mix, the
+  // workspace was sized without knowing it: no more K splits than fit)
+  for (const int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16}) {
+    PackedProblem part[kMaxProblems];
+    int n = 0;
+    for (int i = 0; i < n_problems; ++i)
+      if (problems[i].fmt == fmt) part[n++] = problems[i];
+    if (n == 0) continue;
+    const int rc = packed_launch(st, M, K, n, part, epilogue, out_f32, workspace, workspace_bytes, nullptr, copy, true);
+    if (rc != RWKV_OK) return rc;
+    copy = nullptr;
+  }
+  return RWKV_OK;
+}
+
+static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
+                         void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy, bool fit_splits) {
   StreamArgs g;
   ReduceArgs r;
   if (copy) {
@@ -966,24 +677,28 @@ int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const Pack
     Ns[i] = problems[i].N;
     fmts[i] = problems[i].fmt;
   }
-  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts);
+  int64_t n_total = 0;
+  for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
+  const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
+  const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace ? workspace_bytes / plane : 0)) : 32;
+  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, sums_at_consumer(n_problems, epilogue, out_f32), max_splits);
   int col_blocks = 0;
   for (int i = 0; i < n_problems; ++i) {
     const PackedProblem& q = problems[i];
-    RWKV_REQUIRE(linear_packed_supported(q.fmt, M, q.N, K), "linear_packed: unsupported shape M=%d N=%d K=%d fmt=%d", M,
-                 q.N, K, q.fmt);
     RWKV_REQUIRE(q.x && q.packed && q.y, "linear_packed: NULL tensor");
     RWKV_REQUIRE(q.fmt == RWKV_FMT_F16 || q.scale, "linear_packed: quantised weights need a scale tensor");
     RWKV_REQUIRE(q.fmt != RWKV_FMT_W4 || q.zp, "linear_packed: W4 weights need a zero-point tensor");
-    col_blocks += ceil_div(q.N, cfg.cols());
+    col_blocks += ceil_div(q.N, cfg.cols(q.fmt));
     g.block_end[i] = col_blocks;
-    g.p[i] = StreamProblem{q.x, static_cast<const uint4_t*>(q.packed), q.scale, q.zp, q.y, nullptr, q.N, q.fmt};
+    const int groups = K / 128;
+    const bool by_group = q.groups_first;
+    g.p[i] = StreamProblem{q.x, static_cast<const uint4_t*>(q.packed), q.scale, q.zp, q.y, nullptr, q.N, q.fmt,
+                           by_group ? 1 : groups, by_group ? q.N : 1};
   }
-  g.splits = r.splits = choose_splits(cfg, M, col_blocks, K);
+  g.splits = r.splits = cfg.splits;
   g.k_per_split = K / g.splits;
   if (g.splits > 1) {
-    size_t need = 0;
-    for (int i = 0; i < n_problems; ++i) need += static_cast<size_t>(g.splits) * M * problems[i].N * sizeof(float);
+    const size_t need = g.splits * plane;
     RWKV_REQUIRE(workspace && workspace_bytes >= need, "linear_packed: workspace of %zu bytes needed, got %zu", need,
                  workspace_bytes);
     float* at = static_cast<float*>(workspace);
@@ -998,29 +713,24 @@ int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const Pack
       at += static_cast<size_t>(g.splits) * M * problems[i].N;
     }
   }
-  RWKV_REQUIRE(g.k_per_split % (cfg.kc * cfg.kg) == 0, "linear_packed: K slice %d is not a whole number of %d-chunks",
-               g.k_per_split, cfg.kc * cfg.kg);
-  g.row_tiles = ceil_div(M, 32 * cfg.mt);
+  RWKV_REQUIRE(g.k_per_split % cfg.k_step() == 0, "linear_packed: K slice %d is not a whole number of %d-chunks", g.k_per_split,
+               cfg.k_step());
+  for (int i = n_problems - 1; i < kMaxProblems; ++i) g.block_end[i] = INT_MAX;
+  g.row_tiles = ceil_div(M, cfg.rows());
   g.col_blocks = col_blocks;
-  const int pairs8 = ceil_div(col_blocks * g.splits, 8) * 8;
-  const dim3 grid(g.row_tiles * pairs8);
-  const dim3 block(64 * cfg.wg * cfg.kg);
-  bool all_w8 = true;
-  for (int i = 0; i < n_problems; ++i) all_w8 = all_w8 && problems[i].fmt == RWKV_FMT_W8;
-  if (cfg.nb == 2 && cfg.mt == 2) {
-    RWKV_REQUIRE(all_w8, "linear_packed: the 64 x 256 tile takes int8 weights only");
-    hipLaunchKernelGGL((gemm_stream_wide_kernel<false, 2>), grid, block, 0, st, g);
-  } else if (cfg.nb == 2) hipLaunchKernelGGL((gemm_stream_wide_kernel<true, 4>), grid, block, 0, st, g);
-  else if (cfg.wg == 1) hipLaunchKernelGGL((gemm_stream_kernel<1, 128, 4, 1>), grid, block, 0, st, g);
-  else if (cfg.wg == 2) hipLaunchKernelGGL((gemm_stream_kernel<1, 128, 4, 2>), grid, block, 0, st, g);
-  else if (cfg.mt == 1) hipLaunchKernelGGL((gemm_stream_kernel<1, 128, 2, 4>), grid, block, 0, st, g);
-  else if (cfg.mt == 2) hipLaunchKernelGGL((gemm_stream_kernel<2, 128, 2, 4>), grid, block, 0, st, g);
-  else hipLaunchKernelGGL((gemm_stream_kernel<4, 128, 1, 4>), grid, block, 0, st, g);
-  RWKV_LAUNCH_CHECK();
+  if (cfg.is_ring()) {
+    const int rc = gemm_ring_launch(st, cfg.ring, cfg.fmt, cfg.mixed, g);
+    if (rc != RWKV_OK) return rc;
+  } else {
+    const dim3 grid(g.row_tiles * ceil_div(col_blocks * g.splits, 8) * 8);
+    if (cfg.wide_mt == 2) hipLaunchKernelGGL((gemm_stream_wide_kernel<false, 2>), grid, dim3(256), 0, st, g);
+    else hipLaunchKernelGGL((gemm_stream_wide_kernel<true, 4>), grid, dim3(256), 0, st, g);
+    RWKV_LAUNCH_CHECK();
+  }
   if (defer) *defer = DeferredReduce{};
   if (g.splits == 1) return RWKV_OK;
   if (defer) {
-    RWKV_REQUIRE(n_problems == 1 && epilogue == RWKV_EPI_NONE && !out_f32,
+    RWKV_REQUIRE(sums_at_consumer(n_problems, epilogue, out_f32),
                  "linear_packed: a deferred reduce takes one problem, fp16 output and no epilogue");
     defer->partial = g.p[0].partial;
     defer->scale = problems[0].fmt == RWKV_FMT_W8 ? problems[0].scale : nullptr;

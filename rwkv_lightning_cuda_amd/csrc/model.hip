@@ -26,6 +26,24 @@ struct Matrix {
   const half_t* scale = nullptr;
   const uint8_t* zp = nullptr;
   void* packed = nullptr;  // owned: the same codes in the MFMA-native order, for calls with >= 16 rows
+  half_t* scale_by_group = nullptr;  // int4, in the same block behind the codes: scale and zero point as [K/128][N]
+  uint8_t* zp_by_group = nullptr;
+  void free_copies() {
+    if (packed) (void)hipFree(packed);
+    if (sparse_t) (void)hipFree(sparse_t);
+    packed = sparse_t = nullptr;
+    scale_by_group = nullptr;
+    zp_by_group = nullptr;
+  }
+  PackedProblem packed_problem(int N, const half_t* x, void* y) const {
+    PackedProblem p = {packed, scale, zp, x, y, N, fmt};
+    if (fmt == RWKV_FMT_W4) {
+      p.scale = scale_by_group;
+      p.zp = zp_by_group;
+      p.groups_first = true;
+    }
+    return p;
+  }
   void* sparse_t = nullptr;  // owned, ffn.value only: the [F,C] copy for the one-token row-skipping product
 };
 
@@ -45,12 +63,9 @@ struct rwkv_hip_model {
   std::vector<Layer> layers;
 
   ~rwkv_hip_model() {
-    if (head.packed) (void)hipFree(head.packed);
+    head.free_copies();
     for (Layer& l : layers) {
-      for (Matrix& mat : l.m) {
-        if (mat.packed) (void)hipFree(mat.packed);
-        if (mat.sparse_t) (void)hipFree(mat.sparse_t);
-      }
+      for (Matrix& mat : l.m) mat.free_copies();
       for (void* q : l.lora_in_packed)
         if (q) (void)hipFree(q);
       for (half_t* q : l.lora_out_packed)
@@ -313,8 +328,8 @@ int apply_matrix(const rwkv_hip_session* s, const Matrix& mat, int M, int N, int
   if (defer) *defer = DeferredReduce{};
   // (rows longer than the few-row GEMV keeps in registers go to the packed product from its smallest row count on)
   if (mat.packed && (M >= packed_min_rows(s->model) || (M >= kPackedMinRows && K > 4096))) {
-    return linear_packed(s->stream, mat.fmt, M, N, K, x, mat.packed, mat.scale, mat.zp, epilogue, out_f32, y, s->gemm_ws,
-                         s->gemm_ws_bytes, defer, copy);
+    const PackedProblem q = mat.packed_problem(N, x, y);
+    return linear_packed_multi(s->stream, M, K, 1, &q, epilogue, out_f32, s->gemm_ws, s->gemm_ws_bytes, defer, copy);
   }
   if (copy && copy->n > 0) {
     RWKV_HIP_TRY(hipMemcpyAsync(copy->dst, copy->src, sizeof(half_t) * copy->n, hipMemcpyDeviceToDevice, s->stream));
@@ -563,7 +578,7 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
           // one streaming-GEMM launch (+ one split-K reduce) for the three projections and the rank-ins
           PackedProblem p[7];
           for (int i = 0; i < 3; ++i)
-            p[i] = PackedProblem{w.m[mids[i]].packed, w.m[mids[i]].scale, w.m[mids[i]].zp, xs[i], ys[i], C, w.m[mids[i]].fmt};
+            p[i] = w.m[mids[i]].packed_problem(C, xs[i], ys[i]);
           for (int i = 0; i < n_lora; ++i)
             p[3 + i] = PackedProblem{w.lora_in_packed[i], nullptr, nullptr, lx[i], lh[i], ranks[i], RWKV_FMT_F16};
           // Where a launch of int8 problems only has a tile of its own (several wavefronts per SIMD), three int8
@@ -981,19 +996,22 @@ int rwkv_hip_model_set_matrix(rwkv_hip_model* m, int layer, int id, int fmt, con
   Matrix& slot = id == RWKV_M_HEAD ? m->head : m->layers[layer].m[id];
   if (slot.packed || slot.sparse_t) {
     RWKV_HIP_TRY(hipDeviceSynchronize());
-    if (slot.packed) RWKV_HIP_TRY(hipFree(slot.packed));
-    if (slot.sparse_t) RWKV_HIP_TRY(hipFree(slot.sparse_t));
-    slot.packed = nullptr;
-    slot.sparse_t = nullptr;
+    slot.free_copies();
   }
   if (linear_packed_supported(fmt, kPackedMinRows, N, K)) {
     // second copy of the codes in the order the MFMA path streams (batched decode and prefill)
     const size_t bytes = fmt == RWKV_FMT_F16 ? static_cast<size_t>(N) * K * 2
                                              : (fmt == RWKV_FMT_W8 ? static_cast<size_t>(N) * K : static_cast<size_t>(N) * K / 2);
-    RWKV_HIP_TRY(hipMalloc(&mat.packed, bytes));
-    const int rc = pack_weights_launch(nullptr, fmt, N, K, data, mat.packed);
+    const size_t groups = fmt == RWKV_FMT_W4 ? static_cast<size_t>(N) * (K / 128) : 0;
+    RWKV_HIP_TRY(hipMalloc(&mat.packed, bytes + groups * 3));
+    int rc = pack_weights_launch(nullptr, fmt, N, K, data, mat.packed);
+    if (rc == RWKV_OK && fmt == RWKV_FMT_W4) {
+      mat.scale_by_group = reinterpret_cast<half_t*>(static_cast<unsigned char*>(mat.packed) + bytes);
+      mat.zp_by_group = reinterpret_cast<uint8_t*>(mat.scale_by_group + groups);
+      rc = transpose_groups_launch(nullptr, N, K / 128, mat.scale, mat.zp, mat.scale_by_group, mat.zp_by_group);
+    }
     if (rc != RWKV_OK) {
-      (void)hipFree(mat.packed);
+      mat.free_copies();
       return rc;
     }
     RWKV_HIP_TRY(hipStreamSynchronize(nullptr));
@@ -1004,8 +1022,7 @@ int rwkv_hip_model_set_matrix(rwkv_hip_model* m, int layer, int id, int fmt, con
     const int rc = fmt == RWKV_FMT_W4 ? ffn_sparse_pack_w4_launch(nullptr, N, K, data, mat.scale, mat.zp, mat.sparse_t)
                                       : ffn_sparse_pack_launch(nullptr, fmt, N, K, data, mat.sparse_t);
     if (rc != RWKV_OK) {
-      (void)hipFree(mat.sparse_t);
-      if (mat.packed) (void)hipFree(mat.packed);
+      mat.free_copies();
       return rc;
     }
     RWKV_HIP_TRY(hipStreamSynchronize(nullptr));

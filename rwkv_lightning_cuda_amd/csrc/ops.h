@@ -90,6 +90,8 @@ struct DeferredReduce {
   int splits = 0;
 };
 int pack_weights_launch(hipStream_t st, int fmt, int N, int K, const void* w, void* packed);
+// int4 scales and zero points [N][groups] -> [groups][N]
+int transpose_groups_launch(hipStream_t st, int N, int groups, const half_t* scale, const uint8_t* zp, half_t* scale_t, uint8_t* zp_t);
 // Workspace for one call: fp32 split-K partials (0 when the shape needs no split).
 size_t linear_packed_workspace_bytes(int M, int N, int K);
 // defer (single problem, fp16 output, no epilogue): the consumer sums the partials instead of a reduce launch.
@@ -105,6 +107,7 @@ struct PackedProblem {
   void* y;
   int N;
   int fmt;
+  bool groups_first = false;  // int4: scale and zp are [K/128][N] (one 64-byte piece per 32 columns) instead of [N][K/128]
 };
 // Row counts and K at which a launch of int8 problems only gets a tile of its own (several wavefronts per SIMD):
 // callers with int8 and fp16 problems for one launch do better with two launches there.

@@ -915,6 +915,34 @@ def test_linear_packed_matches_oracle(gpu, orc, fmt_name, M, N, K):
     assert err <= 2 * F16_TOL
 
 
+@pytest.mark.parametrize("fmt_name", ["f16", "w8", "w4"])
+@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (31, 64, 256), (32, 96, 768), (33, 4128, 512), (63, 2080, 1280), (65, 8256, 256),
+                                   (97, 16416, 256), (128, 64, 3840), (129, 8224, 768), (255, 16416, 256), (257, 352, 1792)])
+def test_linear_packed_tile_edges(gpu, orc, fmt_name, M, N, K):
+    """The LDS-ring tiles where they can go wrong: one row, rows on both sides of a tile's edge, one band of columns and a
+    block that is cut, as few stages as there are (K = 256) and stage counts that are no multiple of the rings."""
+    hip = gpu
+    rng = np.random.default_rng(M + N + K)
+    fmt = {"f16": hip.FMT_F16, "w8": hip.FMT_W8, "w4": hip.FMT_W4}[fmt_name]
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float16)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    parts = _quant_parts(orc, hip, fmt, w)
+    dparts = [dev(hip, p) if p is not None else None for p in parts]
+    packed = hip.DeviceArray(parts[0].shape, parts[0].dtype)
+    hip.pack_weights(fmt, N, K, dparts[0], packed)
+    ws = hip.DeviceArray((max(hip.linear_packed_workspace(M, N, K), 16),), np.uint8)
+    y = hip.DeviceArray((M + 1, N), np.float16)   # one row more: nothing may be stored past the last row
+    y.fill0()
+    hip.linear_packed(fmt, M, N, K, dev(hip, x), packed, dparts[1], dparts[2], y, ws)
+    hip.device_sync()
+    got = y.numpy()
+    want = orc.gemv(fmt, x, parts[0], parts[1], parts[2])
+    err = rel_err(got[:M].astype(np.float32), want.astype(np.float32))
+    assert err <= F16_TOL
+    untouched = not got[M].any()
+    assert untouched
+
+
 def test_pack_weights_is_the_documented_permutation(gpu):
     """Tile (band nt, k group kg) holds, for lane j + 32h, the KR consecutive k of row 32 nt + j starting at
     kg*G + h*KR, as 64 x 16-byte pieces (two pieces for fp16)."""

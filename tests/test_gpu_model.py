@@ -136,6 +136,32 @@ def test_many_row_prefill_chunk_on_the_wide_gemm_tile(gpu, orc, fmt):
     sess.close()
 
 
+def test_matrices_of_different_formats_side_by_side(gpu):
+    """int8, int4 and fp16 projections of one layer: the packed launches (24 tokens in one call) against the GEMV (token by
+    token), which takes any mix of formats in one launch."""
+    from rwkv_lightning_cuda_amd.model import DeviceMatrix, HipModel, Session, State, synth_weights
+    hip = gpu
+    dims = small_dims()
+    weights = synth_weights(dims, 31)
+    model = HipModel.from_host_weights(dims, weights, hip.FMT_W8)
+    for layer, (name, mid, fmt) in enumerate([("att_k", hip.M_ATT_K, hip.FMT_W4), ("att_v", hip.M_ATT_V, hip.FMT_F16),
+                                              ("att_r", hip.M_ATT_R, hip.FMT_W4)]):
+        N, K = dims.mat_shape(name)
+        model.set_matrix(layer, mid, DeviceMatrix.from_f16_device(fmt, N, K, hip.DeviceArray.from_numpy(weights["layers"][layer][name])))
+    tokens = np.random.default_rng(9).integers(0, dims.V, (2, 24))
+    logits = []
+    for step in (24, 1):
+        sess = Session(model)
+        st = State(dims, 2)
+        lg = hip.DeviceArray((2, dims.V), np.float32)
+        for t in range(0, 24, step):
+            sess.forward(tokens[:, t:t + step], st, lg)
+        logits.append(lg.numpy())
+        sess.close()
+    cos = cosine(logits[0], logits[1])
+    assert cos >= 0.9995
+
+
 @pytest.mark.parametrize("H", [3, 5])
 def test_odd_head_count_on_the_row_tiled_rank_out(gpu, orc, H):
     """C = 64 H with H odd leaves the last 128-channel block of the LoRA rank-out half empty: the packed copy of the
