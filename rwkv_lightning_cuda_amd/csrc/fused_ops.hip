@@ -12,6 +12,8 @@
 // 1024 threads by row length - decode steps have few rows, so the wavefronts of a row are the only parallelism the
 // launch has: 512 threads instead of 256 with two slices each make a 4096-wide row 15-25 % faster), so a row is
 // read from HBM once for the two-pass mean/variance and the normalise+lerp epilogue.
+#include <type_traits>
+
 #include "ops.h"
 
 namespace rwkv {
@@ -66,29 +68,34 @@ __global__ __launch_bounds__(NT) void ln_fused_kernel(LnArgs a) {
           const float* pp = a.res_partial + src + c;
           float4_t s0 = *reinterpret_cast<const float4_t*>(pp);
           float4_t s1 = *reinterpret_cast<const float4_t*>(pp + 4);
-          // The other partials four at a time, all requested before the first is added (in split order, as
-          // always); past the last split the last one is read again and left out.  A plain loop over the splits
-          // would wait for each partial before it asks for the next: one trip to memory per split.
-          for (int base = 1; base < a.res_splits; base += 4) {
-            float4_t q0[4], q1[4];
+          // The other partials seven (up to four splits: three) at a time, all requested before the first is added (in
+          // split order, as always); past the last split the last one is read again and left out.  A plain loop over the
+          // splits would wait for each partial before it asks for the next: one trip to memory per split.
+          auto add_planes = [&](auto batch_c) {
+            constexpr int kBatch = decltype(batch_c)::value;
+            for (int base = 1; base < a.res_splits; base += kBatch) {
+              float4_t q0[kBatch], q1[kBatch];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int sp = base + u < a.res_splits ? base + u : a.res_splits - 1;
-              q0[u] = *reinterpret_cast<const float4_t*>(pp + sp * a.res_plane);
-              q1[u] = *reinterpret_cast<const float4_t*>(pp + sp * a.res_plane + 4);
-            }
-            // (keeps the four requests together: their only uses sit under the conditions below, and the compiler
-            // would move each load down into its condition)
+              for (int u = 0; u < kBatch; ++u) {
+                const int sp = base + u < a.res_splits ? base + u : a.res_splits - 1;
+                q0[u] = *reinterpret_cast<const float4_t*>(pp + sp * a.res_plane);
+                q1[u] = *reinterpret_cast<const float4_t*>(pp + sp * a.res_plane + 4);
+              }
+              // (keeps the requests together: their only uses sit under the conditions below, and the compiler
+              // would move each load down into its condition)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) asm volatile("" : "+v"(q0[u]), "+v"(q1[u]));
+              for (int u = 0; u < kBatch; ++u) asm volatile("" : "+v"(q0[u]), "+v"(q1[u]));
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              if (base + u < a.res_splits) {
-                s0 = s0 + q0[u];
-                s1 = s1 + q1[u];
+              for (int u = 0; u < kBatch; ++u) {
+                if (base + u < a.res_splits) {
+                  s0 = s0 + q0[u];
+                  s1 = s1 + q1[u];
+                }
               }
             }
-          }
+          };
+          if (a.res_splits <= 4) add_planes(std::integral_constant<int, 3>{});
+          else add_planes(std::integral_constant<int, 7>{});
           float scl[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) scl[e] = a.res_scale ? h2f(sv8[e]) : 1.0f;

@@ -525,7 +525,8 @@ static int count_col_blocks(const StreamConfig& c, int n_problems, const int* Ns
 //   stream (94 GB/s; 130 while half of the chip idles); what of the HBM stream of the weights does not hide behind that; the
 //   products; per further round of blocks its start and end, which a second block hides where two fit a CU.
 //   wide: bound by the matrix core (1 PFLOP/s with the shader clock these products run at).
-//   K splits: their fp32 planes and, where no consumer sums them, the reduce launch.
+//   K splits: their fp32 planes and, where no consumer sums them, the reduce launch; a consumer's block waits longer the more
+//   planes it asks for (0.15 us each; with 0 / 0.4 decode steps of 5 .. 16 rows are 1-4 % slower, 7.2B and 1.5B int8).
 static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred) {
   constexpr int kCus = 256;
   const int bm = c.rows();
@@ -561,7 +562,7 @@ static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, co
   } else {
     us = 6.0f + (full + (rest > 0 ? (full > 0 ? 0.75f + 0.25f * rest / kCus : 1.0f) : 0.0f)) * (11.0f + 58.0f * k_block / 4096.0f);
   }
-  if (c.splits > 1) us += (deferred ? 0.5f : 2.6f) + c.splits * M * n_total * (deferred ? 6.0f : 8.0f) / 5e6f;
+  if (c.splits > 1) us += (deferred ? 0.35f + 0.15f * c.splits : 2.6f) + c.splits * M * n_total * (deferred ? 6.0f : 8.0f) / 5e6f;
   return us;
 }
 

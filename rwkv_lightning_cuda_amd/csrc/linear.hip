@@ -1345,9 +1345,8 @@ __device__ __forceinline__ void rows_mfma_block(const LinearArgs& args, const Li
   const int steps = KP / (4 * KV);                    // vectors per lane: a step is 4 * KV values of a row
   const int n0 = (blk * G + g) * 16;
   const bool active = n0 < N;
-  const int64_t ldw = prob.ldw ? prob.ldw : K;
   const unsigned char* wrow = static_cast<const unsigned char*>(prob.w) +
-                              (static_cast<int64_t>(active ? n0 + r : r) * ldw + static_cast<int64_t>(kp) * KP + kq * KV) * EB;
+                              (static_cast<int64_t>(active ? n0 + r : r) * K + static_cast<int64_t>(kp) * KP + kq * KV) * EB;
   const half_t* xrow = xs + (r < M ? r : 0) * xstride + kp * KP + kq * KV;
   float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
   uint4_t w[NB];
@@ -1376,9 +1375,8 @@ __device__ __forceinline__ void rows_mfma_block(const LinearArgs& args, const Li
       }
     }
   };
-  // x of this problem: M rows of K / 8 vectors (the rows ldx values apart)
+  // x of this problem: M rows of K / 8 vectors
   const int kv = K >> 3;
-  const int64_t ldx = prob.ldx ? prob.ldx : K;
   constexpr int NTS = kRowsMfmaThreads / 2;  // staging threads: the first half of the wavefronts
   auto stage_x = [&]() {
     uint4_t xv[XV];
@@ -1388,7 +1386,7 @@ __device__ __forceinline__ void rows_mfma_block(const LinearArgs& args, const Li
       xv[j] = uint4_t{0u, 0u, 0u, 0u};
       if (i < M * kv) {
         const int m = i / kv, c = (i - m * kv) * 8;
-        xv[j] = *reinterpret_cast<const uint4_t*>(prob.x + m * ldx + c);
+        xv[j] = *reinterpret_cast<const uint4_t*>(prob.x + static_cast<int64_t>(m) * K + c);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1447,10 +1445,6 @@ __device__ __forceinline__ void rows_mfma_block(const LinearArgs& args, const Li
 #pragma unroll
       for (int q = 1; q < P; ++q) sum += ps[q * 256];
       const int64_t o = static_cast<int64_t>(m) * N + n;
-      if (prob.raw_f32) {  // (uniform per block)
-        static_cast<float*>(prob.y)[o] = sum;
-        return;
-      }
       if constexpr (FMT == RWKV_FMT_W8) sum *= h2f(prob.scale[n]);
       sum = round_h(sum);
       if (args.epilogue == RWKV_EPI_RELU_SQUARE) {
@@ -1585,37 +1579,6 @@ static int launch_rows_mfma_fmt(hipStream_t st, LinearArgs& args, int M) {
 static int launch_rows_mfma_any(hipStream_t st, LinearArgs& args, int M, int df) {
   if (df == RWKV_FMT_W8) return launch_rows_mfma_fmt<RWKV_FMT_W8>(st, args, M);
   return launch_rows_mfma_fmt<RWKV_FMT_F16>(st, args, M);
-}
-
-int linear_rows_mfma_sliced(hipStream_t st, int fmt, int M, int N, int K, int slice, const half_t* x, const void* w,
-                            float* partial, const RowCopy* copy) {
-  RWKV_REQUIRE(slice > 0 && K % slice == 0 && K / slice >= 1 && K / slice <= kMaxProblems,
-               "linear: %d columns in slices of %d", K, slice);
-  RWKV_REQUIRE(M >= 1 && M <= kRowsMfmaMax && linear_rows_mfma_supported(fmt, N, slice),
-               "linear: no few-row launch for %d rows of this format and shape (N = %d, K = %d)", M, N, slice);
-  RWKV_REQUIRE(x && w && partial, "linear: NULL tensor");
-  LinearArgs args = {};
-  args.n_problems = K / slice;
-  args.K = slice;
-  args.epilogue = RWKV_EPI_NONE;
-  args.out_f32 = 1;
-  const int eb = fmt == RWKV_FMT_F16 ? 2 : 1;
-  for (int i = 0; i < args.n_problems; ++i) {
-    LinearProblem& p = args.p[i];
-    p.w = static_cast<const unsigned char*>(w) + static_cast<int64_t>(i) * slice * eb;
-    p.x = x + static_cast<int64_t>(i) * slice;
-    p.y = partial + static_cast<int64_t>(i) * M * N;
-    p.N = N;
-    p.fmt = fmt;
-    p.ldw = K;
-    p.ldx = K;
-    p.raw_f32 = 1;
-  }
-  if (copy && copy->n > 0) {
-    RWKV_REQUIRE(copy->src && copy->dst && copy->n % 8 == 0, "linear: bad row copy");
-    args.copy = *copy;
-  }
-  return launch_rows_mfma_any(st, args, M, fmt);
 }
 
 int linear_ln_prologue_max_rows(int K) { return K <= 4096 && K % 8 == 0 ? kRow1MaxRowsLn : 0; }

@@ -88,30 +88,20 @@ struct GraphEntry {
 };
 
 constexpr size_t kMaxGraphs = 8;
-// Calls with at least this many rows stream the packed copy through MFMA.  Below: the weight-streaming GEMV that keeps
-// whole weight rows in flight for up to 4 rows of x (decode ms per step, GEMV / streaming GEMM: 7.2B shape, int8: 3 rows
-// 2.39 / 2.79, 4 rows 2.56 / 2.82; 1.5B shape: 3 rows 1.20 / 1.45, 4 rows 1.31 / 1.51, 5 rows 1.55 / 1.31; 0.1B shape,
-// fp16: 3 rows 0.51 / 0.63, 4 rows 0.57 / 0.67), and from 5 to 16 rows - for int8 and fp16 weights in rows of 1024,
-// 2048, 3072 or 4096 values - the same stream with the products on the matrix core (7.2B shape, int8, this / streaming
-// GEMM: 5 rows 2.84 / 3.01, 8 rows 2.69 / 2.87, 16 rows 2.99 / 3.06).  RWKV_PACKED_MIN_ROWS (tuning hook) overrides
-// the crossover.
+// Calls with at least packed_min_rows rows stream the packed copy through the matrix core; below, the weight-streaming GEMV
+// keeps whole weight rows in flight for up to 4 rows of x.  The GEMV pays a dot product per row and weight vector, the packed
+// product a K split's fp32 planes, so the line lies where the vectors are many: decode ms per step, GEMV / packed, 7.2B shape
+// int8 3 rows 2.42 / 2.37, 4 rows 2.65 / 2.51, int4 2.32 / 2.28 and 2.57 / 2.37, fp16 4 rows 3.33 / 3.44; 1.5B shape int8 4 rows
+// 1.35 / 1.36, fp16 1.28 / 1.41; 0.1B shape fp16 4 rows 0.51 / 0.54.  5 to 16 rows went through linear_rows_mfma before (weights
+// in plain order, a 16-byte load of a wavefront touching sixteen rows of the matrix; it stays for models without packed copies):
+// 7.2B int8 5 / 8 / 16 rows 2.65 / 2.57 / 2.95 -> 2.41 / 2.31 / 2.55, 1.5B int8 13 rows 1.24 -> 1.18.
+// RWKV_PACKED_MIN_ROWS (tuning hook) overrides the line.
 constexpr int kPackedMinRows = 3;  // what gets a packed copy at all: rows too long for the GEMV (ffn.value) use it from here
-constexpr int kFewRowsMax = 16;    // most rows of the few-row matrix-core launch
-inline bool few_rows_on_matrix_core(const rwkv_hip_model* m) {
-  if (m->layers.empty()) return false;
-  const Layer& l0 = m->layers[0];
-  const int mids[5] = {RWKV_M_ATT_R, RWKV_M_ATT_K, RWKV_M_ATT_V, RWKV_M_ATT_O, RWKV_M_FFN_KEY};
-  for (int id : mids)
-    if (!linear_rows_mfma_supported(l0.m[id].fmt, id == RWKV_M_FFN_KEY ? m->F : m->C, m->C)) return false;
-  const int ranks[4] = {m->Rw, m->Ra, m->Rg, m->Rv};
-  for (int r : ranks)
-    if (!linear_rows_mfma_supported(RWKV_FMT_F16, r, m->C)) return false;
-  return true;
-}
 inline int packed_min_rows(const rwkv_hip_model* m) {
   static const int forced = getenv("RWKV_PACKED_MIN_ROWS") ? atoi(getenv("RWKV_PACKED_MIN_ROWS")) : 0;
   if (forced >= kPackedMinRows) return forced;
-  return few_rows_on_matrix_core(m) ? kFewRowsMax + 1 : 5;
+  const bool long_quantised_rows = m->C >= 4096 && !m->layers.empty() && m->layers[0].m[RWKV_M_FFN_KEY].fmt != RWKV_FMT_F16;
+  return long_quantised_rows ? kPackedMinRows : 5;
 }
 // most blocks of a single-launch time-mix core beyond 8 rows (one round on the chip's compute units; us per layer at the 7.2B shape,
 // this launch / the row-tiled kernels: 16 rows 14 / 17, 32 rows 25 / 24)
@@ -280,8 +270,6 @@ int ensure_arena(rwkv_hip_session* s, int B, int T) {
     ws = std::max(ws, linear_packed_workspace_bytes(R, m->F, m->C));
     ws = std::max(ws, linear_packed_workspace_bytes(R, m->C, m->F));
     ws = std::max(ws, linear_packed_workspace_bytes(B, m->V, m->C));
-    // (the column slices of ffn.value on the few-row launch: F / C planes of fp32 partial sums)
-    if (R <= kFewRowsMax && m->F % m->C == 0) ws = std::max(ws, static_cast<size_t>(m->F / m->C) * R * m->C * sizeof(float));
     if (ws > s->gemm_ws_bytes) {
       for (auto& g : s->graphs) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
@@ -335,30 +323,6 @@ int apply_matrix(const rwkv_hip_session* s, const Matrix& mat, int M, int N, int
     RWKV_HIP_TRY(hipMemcpyAsync(copy->dst, copy->src, sizeof(half_t) * copy->n, hipMemcpyDeviceToDevice, s->stream));
   }
   return linear_any_m(s->stream, mat.fmt, M, N, K, x, mat.data, mat.scale, mat.zp, epilogue, out_f32, y);
-}
-
-// ffn.value of 5 to 16 rows on the few-row launch: F / C column slices of C values each, whose partial sums the
-// LayerNorm kernel that consumes the result adds up and scales (7.2B shape, 8 rows: 19.4 us for the packed product).
-bool sliced_value_ok(const rwkv_hip_session* s, const Matrix& mv, int rows) {
-  const rwkv_hip_model* m = s->model;
-  static const bool off = getenv("RWKV_SLICED_VALUE") && atoi(getenv("RWKV_SLICED_VALUE")) == 0;  // tuning hook
-  static const int min_rows = getenv("RWKV_ROWS_MFMA_MIN") ? atoi(getenv("RWKV_ROWS_MFMA_MIN")) : 5;  // tuning hook
-  return !off && rows >= min_rows && rows <= kFewRowsMax && m->F % m->C == 0 && m->F / m->C <= kMaxProblems &&
-         (mv.fmt == RWKV_FMT_W8 || mv.fmt == RWKV_FMT_F16) && linear_rows_mfma_supported(mv.fmt, m->C, m->C) &&
-         s->gemm_ws_bytes >= static_cast<size_t>(m->F / m->C) * rows * m->C * sizeof(float);
-}
-
-int sliced_value(const rwkv_hip_session* s, const Matrix& mv, int rows, const half_t* act, DeferredReduce* defer,
-                 const RowCopy* copy = nullptr) {
-  const rwkv_hip_model* m = s->model;
-  float* ws = static_cast<float*>(s->gemm_ws);
-  const int rc = linear_rows_mfma_sliced(s->stream, mv.fmt, rows, m->C, m->F, m->C, act, mv.data, ws, copy);
-  if (rc != RWKV_OK) return rc;
-  defer->partial = ws;
-  defer->scale = mv.fmt == RWKV_FMT_W8 ? mv.scale : nullptr;
-  defer->plane = static_cast<int64_t>(rows) * m->C;
-  defer->splits = m->F / m->C;
-  return RWKV_OK;
 }
 
 void take_deferred(LnArgs& a, const DeferredReduce& d) {
@@ -440,16 +404,16 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
   // channels.  The residual-stream tap needs the stand-alone kernels.
   const bool want_ln_in_linear = s->fused_ln > 0 || (s->fused_ln < 0 && rows <= linear_ln_prologue_max_rows(C));
   // (the shift row that the prologue leaves for later is stored by the single-launch time-mix core)
-  // (forced on, it also takes the rows that a launch with a prologue exists for: 5 to 8 on the few-row matrix-core
-  // launch, up to 8 through the tiled GEMV while the rows fit its LDS)
+  // (forced on, it also takes the rows below the packed product that a launch with a prologue exists for: 5 to 8 on the
+  // few-row matrix-core launch, up to 8 through the tiled GEMV while the rows fit its LDS)
   const bool ln_in_linear = want_ln_in_linear && step && small && !s->trace && fused_tmix &&
                             (rows <= linear_ln_prologue_max_rows(C) ||
                              (linear_ln_prologue_rows_ok(m->layers[0].m[RWKV_M_ATT_R].fmt, rows, C, C) &&
                               linear_ln_prologue_rows_ok(m->layers[0].m[RWKV_M_FFN_KEY].fmt, rows, F, C)) ||
                              (rows <= 8 && static_cast<size_t>(rows) * C * 2 + static_cast<size_t>(C) * 4 <= 49152));
-  // 5 to 8 rows on the few-row matrix-core launch: LN2 (+ its token shift) folds into the ffn.key launch.  LN1 stays a
-  // launch of its own there: it sums the split-K partials of the packed ffn.value product, which would otherwise
-  // cost the reduce launch that the folded LayerNorm saves.
+  // 5 to 8 rows on the few-row matrix-core launch (models without packed copies): LN2 (+ its token shift) folds into the
+  // ffn.key launch.  LN1 stays a launch of its own there: it sums the split-K partials of the packed ffn.value product, which
+  // would otherwise cost the reduce launch that the folded LayerNorm saves.
   const bool ln2_in_linear =
       ln_in_linear || (s->fused_ln != 0 && step && small && !s->trace && rows >= 5 &&
                        linear_ln_prologue_rows_ok(m->layers[0].m[RWKV_M_FFN_KEY].fmt, rows, F, C));
@@ -709,7 +673,8 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
       po.x_gate = b.g;
       TRY_PROF(linear_small_m(st, 1, C, 1, &po, RWKV_EPI_NONE, 0));
     } else {
-      TRY_PROF(apply_matrix(s, w.m[RWKV_M_ATT_O], rows, C, C, b.y2, RWKV_EPI_NONE, 0, b.att, defer_ok ? &att_partial : nullptr));
+      TRY_PROF(apply_matrix(s, w.m[RWKV_M_ATT_O], rows, C, C, b.y2, RWKV_EPI_NONE, 0, b.att,
+                            defer_ok && !ln2_in_linear ? &att_partial : nullptr));  // (the prologue reads b.att)
     }
 
     // residual add + LN2 + channel-mix token shift
@@ -757,8 +722,6 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
       if (sparse_value && mv.sparse_t) {
         TRY_AUX(ffn_sparse_launch(st, mv.fmt, rows, C, F, 1, b.act, mv.sparse_t, mv.scale, s->sparse_ws, s->sparse_ws_bytes, b.cm,
                                   &cp, true));
-      } else if (defer_ok && sliced_value_ok(s, mv, rows)) {
-        TRY_PROF(sliced_value(s, mv, rows, b.act, &cm_partial, &cp));
       } else if (rows > 8 || (mv.packed && rows >= kPackedMinRows)) {
         // (rows too long for the few-row launches: the packed product, whose first block moves the row too)
         TRY_PROF(apply_matrix(s, mv, rows, C, F, b.act, RWKV_EPI_NONE, 0, b.cm, defer_ok ? &cm_partial : nullptr, &cp));
@@ -774,8 +737,6 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
       if (sparse_value && mv.sparse_t) {
         TRY_AUX(ffn_sparse_launch(st, mv.fmt, rows, C, F, 1, b.act, mv.sparse_t, mv.scale, s->sparse_ws, s->sparse_ws_bytes, b.cm,
                                   nullptr, true));
-      } else if (defer_ok && step && sliced_value_ok(s, mv, rows)) {
-        TRY_PROF(sliced_value(s, mv, rows, b.act, &cm_partial));
       } else {
         TRY_PROF(apply_matrix(s, mv, rows, C, F, b.act, RWKV_EPI_NONE, 0, b.cm, defer_ok ? &cm_partial : nullptr));
       }

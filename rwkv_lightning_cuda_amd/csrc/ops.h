@@ -21,12 +21,6 @@ struct LinearProblem {
   // (the gate of the time-mix output, whose rank-out runs beside the heads' blocks instead of inside them).
   const float* x_f32 = nullptr;
   const half_t* x_gate = nullptr;
-  // The few-row matrix-core launch only: a problem may be a slice of K columns of longer rows - values between the
-  // starts of consecutive rows of W (ldw) and of x (ldx), 0 = K - and may leave its unscaled fp32 sums in y
-  // (raw_f32: one of several slices' partial products, for a consumer that adds them up and scales).
-  int ldw = 0;
-  int ldx = 0;
-  int raw_f32 = 0;
 };
 
 // LayerNorm + token-shift prologue of a small-M linear launch (decode steps): every block recomputes, for each
@@ -63,11 +57,6 @@ int linear_small_m(hipStream_t st, int M, int K, int n_problems, const LinearPro
                    int out_f32, const LnPrologue* ln = nullptr, const RowCopy* copy = nullptr);
 // Whether 5..16 rows of this format and shape run on the few-row matrix-core launch (weights in their plain order).
 bool linear_rows_mfma_supported(int fmt, int N, int K);
-// y = x W^T for rows of W longer than that launch takes (K a multiple of `slice`, a supported row length): one launch
-// over K / slice column slices, whose fp32 partial sums [K / slice][M][N] go to `partial` for the consumer to add
-// and scale (DeferredReduce).  M in 5..16.
-int linear_rows_mfma_sliced(hipStream_t st, int fmt, int M, int N, int K, int slice, const half_t* x, const void* w,
-                            float* partial, const RowCopy* copy = nullptr);
 // Rows of a decode step that linear_small_m takes with the LayerNorm prologue at this row length (0: none): through
 // the GEMV; and whether M rows of a format and shape go with it at all (the few-row matrix-core launch takes 5..8).
 int linear_ln_prologue_max_rows(int K);

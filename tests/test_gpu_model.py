@@ -862,6 +862,33 @@ def test_decode_step_of_five_to_eight_rows_folds_layernorm_into_the_few_row_laun
     sess.close()
 
 
+@pytest.mark.parametrize("B,C,ranks", [(3, 4096, 32), (4, 4096, 32), (5, 4096, 32), (16, 4096, 32), (13, 2048, 64), (5, 1024, 48),
+                                       (8, 2048, 48), (12, 1024, 48)])
+def test_decode_steps_of_three_to_sixteen_rows_match_the_rows_one_by_one(gpu, B, C, ranks):
+    """Decode steps on both sides of the line between the GEMV, the packed product (3 rows on at rows of 4096 int8 codes, 5 rows
+    at shorter ones) and the few-row launch in plain order (a rank of 48 has no packed copy): every row against the same row in
+    a batch of one, which only the GEMV takes.  The bar is the fp16 one of the batched decode tests: the routes differ in
+    summation order, which moves single activations by an fp16 step."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=2, C=C, H=C // 64, F=4 * C, V=512, Rw=ranks, Ra=ranks, Rg=64, Rv=32)
+    gmodel = HipModel.from_host_weights(dims, synth_weights(dims, 23), hip.FMT_W8)
+    tokens = np.random.default_rng(B).integers(0, dims.V, (B, 3))
+    sess = Session(gmodel)
+    st, lg = State(dims, B), hip.DeviceArray((B, dims.V), np.float32)
+    for t in range(3):
+        sess.forward(tokens[:, t:t + 1], st, lg)
+    logits, shift, wkv = lg.numpy(), st.shift.numpy().astype(np.float32), st.wkv.numpy()
+    for row in sorted({0, B // 2, B - 1}):
+        st1, lg1 = State(dims, 1), hip.DeviceArray((1, dims.V), np.float32)
+        for t in range(3):
+            sess.forward(tokens[row:row + 1, t:t + 1], st1, lg1)
+        assert rel_err(logits[row], lg1.numpy()[0]) <= 3e-3
+        assert rel_err(shift[:, :, row], st1.shift.numpy().astype(np.float32)[:, :, 0]) <= 3e-3
+        assert rel_err(wkv[:, row], st1.wkv.numpy()[:, 0]) <= 3e-3
+    sess.close()
+
+
 @pytest.mark.parametrize("B", [4, 8, 16, 12])
 def test_decode_time_mix_core_with_several_batch_rows_per_block(gpu, B):
     """The single-launch time-mix core of a decode step serves 1, 2 or 4 batch rows of a head per block (the head's
