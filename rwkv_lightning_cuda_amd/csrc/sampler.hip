@@ -6,7 +6,8 @@
 // {p >= t} still holds at least top_k entries or at least top_p mass; entries equal to t are scaled by
 // `comp` so the kept set has exactly top_k entries / top_p mass (:393-404).
 //
-// gfx950 re-design: one 1024-thread block (16 wavefronts) per row; each thread owns a fixed set of entries -
+// gfx950 re-design: rows with a small top_k take three launches (sample_stats_kernel and on, below).  Otherwise one 1024-thread
+// block (16 wavefronts) per row; each thread owns a fixed set of entries -
 // for rows of up to 65536 entries the float4 t, t + 1024, ..., loaded once (coalesced) and kept in registers
 // through the softmax, the bisection and the draw; for larger rows a contiguous slice that stays in `probs` -
 // so the draw is a single inverse-CDF walk with one uniform number over a fixed order of the row; block
@@ -111,6 +112,23 @@ struct SampleArgs {
   uint64_t seed, step;
 };
 
+__device__ __forceinline__ float penalised(float logit, float penalty, float log2_inv_temp) {
+  return sf((sf(logit) - penalty) * log2_inv_temp);
+}
+
+// how much of each of the n_eq entries at the threshold is kept, so that the kept set has top_k entries or top_p mass
+__device__ __forceinline__ float tie_share(const SampleArgs& a, float thr, unsigned n_eq, unsigned n_gt, float p_gt) {
+  float comp = fminf(sf((a.top_p - p_gt) / (thr * n_eq)), 1.0f);
+  comp = fminf(sf(static_cast<float>(a.top_k - static_cast<int>(n_gt)) / n_eq), comp);
+  return fmaxf(comp, 0.0f);
+}
+
+// uniform in (0,1]: never selects a zero-mass prefix
+__device__ __forceinline__ float uniform_of_row(const SampleArgs& a, int b) {
+  const Philox rnd = philox4x32_10(a.seed, static_cast<uint64_t>(b), a.step);
+  return (static_cast<float>(rnd.c[0] >> 8) + 1.0f) * (1.0f / 16777216.0f);
+}
+
 // count and mass of one bisection step through one LDS exchange (the same sums, in the same order, as
 // block_sum_u and block_reduce_f one after the other)
 __device__ __forceinline__ void block_count_mass(unsigned& c, float& m, BlockRed& red) {
@@ -138,14 +156,11 @@ constexpr int kSampleRegVecs = 16;  // float4 per thread held in registers: rows
 // the softmax, the ~30 bisection steps and the tie count touch no memory; `probs` is not written.  Larger
 // rows keep the slice in `probs` (L2) and re-read it in every pass.  Same arithmetic in the same order.
 template <bool REG>
-__global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
-  __shared__ BlockRed red;
-  __shared__ int s_pick;
-  const int b = blockIdx.x;
+__device__ __forceinline__ int sample_row(const SampleArgs& a, int b, BlockRed& red, int& s_pick) {
   const int t = threadIdx.x;
   const int V = a.V;
   const float* logits = a.logits + static_cast<int64_t>(b) * V;
-  float* pen = a.penalties ? a.penalties + static_cast<int64_t>(b) * V : nullptr;
+  const float* pen = a.penalties ? a.penalties + static_cast<int64_t>(b) * V : nullptr;
   float* probs = a.probs + static_cast<int64_t>(b) * V;
   // contiguous slice per thread, in units of 4 floats
   const int V4 = V / 4;
@@ -195,7 +210,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
     if (pen) p = reinterpret_cast<const float4_t*>(pen)[i];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      l[j] = sf((sf(l[j]) - p[j]) * a.log2_inv_temp);
+      l[j] = penalised(l[j], p[j], a.log2_inv_temp);
       if (l[j] > maxu) {
         maxu = l[j];
         maxi = i * 4 + j;
@@ -324,20 +339,13 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
     const unsigned n_gt = block_sum_u(gtk, red.u);
     const float p_gt = block_reduce_f(gtp, fadd_op, red.f);
     float comp = 1.0f;
-    if (n_eq > 0) {
-      comp = fminf(sf((a.top_p - p_gt) / (thr * n_eq)), comp);
-      comp = fminf(sf(static_cast<float>(a.top_k - static_cast<int>(n_gt)) / n_eq), comp);
-      comp = fmaxf(comp, 0.0f);
-    }
+    if (n_eq > 0) comp = tie_share(a, thr, n_eq, n_gt, p_gt);
 
     // 6. inverse-CDF draw over the kept set, thread by thread
     const float mine = gtp + (thr * eqk) * comp;
     float total;
     const float before = block_exclusive_scan(mine, red.f, &total);
-    const Philox rnd = philox4x32_10(a.seed, static_cast<uint64_t>(b), a.step);
-    // uniform in (0,1]: never selects a zero-mass prefix
-    const float u = (static_cast<float>(rnd.c[0] >> 8) + 1.0f) * (1.0f / 16777216.0f);
-    const float target = u * total;
+    const float target = uniform_of_row(a, b) * total;
     if (t == 0) s_pick = -1;
     __syncthreads();
     if (mine > 0.0f && target > before && target <= before + mine) {
@@ -375,18 +383,353 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
     pick = s_pick < 0 ? 0 : s_pick;
   }
 
-  if (t == 0) a.out[b] = pick;
-  // 7. penalty update (sampling.cu:461-470)
-  if (pen) {
-    for_each([&](int, int i) {
-      float4_t p = reinterpret_cast<float4_t*>(pen)[i];
+  return pick;
+}
+
+// 7. penalty update (sampling.cu:461-470) of one float4 of the row
+__device__ __forceinline__ float4_t decayed_penalty(float4_t p, int i, int pick, const SampleArgs& a) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float add = (pick != i * 4 + j) ? 0.0f : (p[j] == 0.0f ? a.presence : a.frequency);
-        p[j] = fmaf(p[j], a.decay, add);
+  for (int j = 0; j < 4; ++j) {
+    const float add = (pick != i * 4 + j) ? 0.0f : (p[j] == 0.0f ? a.presence : a.frequency);
+    p[j] = fmaf(p[j], a.decay, add);
+  }
+  return p;
+}
+
+template <bool REG>
+__global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
+  __shared__ BlockRed red;
+  __shared__ int s_pick;
+  const int b = blockIdx.x;
+  const int pick = sample_row<REG>(a, b, red, s_pick);
+  if (threadIdx.x == 0) a.out[b] = pick;
+  if (!a.penalties) return;
+  float4_t* pen = reinterpret_cast<float4_t*>(a.penalties + static_cast<int64_t>(b) * a.V);
+#pragma unroll 4
+  for (int i = threadIdx.x; i < a.V / 4; i += kSampleThreads) pen[i] = decayed_penalty(pen[i], i, pick, a);
+}
+
+// ---- top-k rows in three launches ------------------------------------------------------------------------------------
+// One block per row has one CU to move the row through and to do its arithmetic on (0.4 us per VALU operation and row of
+// 65536 entries), and at 64 rows three quarters of the chip idle.  With a top_k of at most kSplitMaxTopK the kept set is known to
+// lie among a few hundred entries before any probability is:
+//   sample_stats_kernel  the whole chip reads the rows: per 64 entries (a slot) the largest penalised logit, per 4096 entries
+//                        their maximum and the sum of their exponentials below it;
+//   sample_pick_kernel   one block per row: a value that at least top_k slot maxima reach bounds the top_k-th largest entry from
+//                        below, so only those slots (top_k and a few) are read again, and of them only the entries above it
+//                        compete: softmax, bisection, ties and draw of sample_row over these, in the order sample_row walks the
+//                        row in.  A row with more than kMaxCandidates of them (equal logits) goes through sample_row itself;
+//   sample_decay_kernel  the penalty rows, by the whole chip again.
+// Against the one-block kernel the sum of the exponentials and the masses are added in another order (fp32 both), no more.
+// Rows of 65536, penalties, top-k 50, top-p 0.6, one block per row / this: 1 row 53.4 / 19.8 us, 64 rows 66-70 / 27.7,
+// 128 rows 70.9 / 40.4; 8 rows, top-k 200, top-p 0.8: 64.5 / 27.7.
+// The slot maxima and the parts' sums lie in `probs`.
+constexpr int kSlot = 64;
+constexpr int kPartEntries = 4096;
+constexpr int kPartThreads = 256;
+constexpr int kSplitMaxTopK = 256;
+constexpr int kMaxCandidates = 1024;  // one per thread
+constexpr int kMaxSlots = kSampleRegVecs * kSampleThreads * 4 / kSlot;
+static_assert(kMaxSlots == kSampleThreads, "one slot per thread, sixteen per lane of a wavefront");
+
+// top_k slot maxima have to bound the kept set well (twice as many slots), one block has to hold a row's slots, and the greedy
+// pick of top_k == 1 compares logits, not probabilities.
+inline bool sample_split_ok(int V, int top_k) {
+  return top_k >= 2 && top_k <= kSplitMaxTopK && V <= kMaxSlots * kSlot && V / kSlot >= 2 * top_k;
+}
+
+__global__ __launch_bounds__(kPartThreads) void sample_stats_kernel(SampleArgs a) {
+  constexpr int kVecs = kPartEntries / 4 / kPartThreads;
+  __shared__ float red[kPartThreads / 64];
+  const int b = blockIdx.x;
+  const int part = blockIdx.y, parts = gridDim.y;
+  const int t = threadIdx.x;
+  const int V4 = a.V / 4;
+  const int n_slots = (a.V + kSlot - 1) / kSlot;
+  const float4_t* logits = reinterpret_cast<const float4_t*>(a.logits + static_cast<int64_t>(b) * a.V);
+  const float4_t* pen = a.penalties ? reinterpret_cast<const float4_t*>(a.penalties + static_cast<int64_t>(b) * a.V) : nullptr;
+  float* stats = a.probs + static_cast<int64_t>(b) * a.V;
+  float4_t l[kVecs], p[kVecs];
+#pragma unroll
+  for (int q = 0; q < kVecs; ++q) l[q] = logits[min(part * (kPartEntries / 4) + q * kPartThreads + t, V4 - 1)];
+#pragma unroll
+  for (int q = 0; q < kVecs; ++q) p[q] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  if (pen) {
+#pragma unroll
+    for (int q = 0; q < kVecs; ++q) p[q] = pen[min(part * (kPartEntries / 4) + q * kPartThreads + t, V4 - 1)];
+  }
+  auto fmax_op = [](float x, float y) { return fmaxf(x, y); };
+  float top = -INFINITY;
+#pragma unroll
+  for (int q = 0; q < kVecs; ++q) {
+    const bool live = part * (kPartEntries / 4) + q * kPartThreads + t < V4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) l[q][j] = live ? penalised(l[q][j], p[q][j], a.log2_inv_temp) : -INFINITY;
+    float m = fmaxf(fmaxf(l[q][0], l[q][1]), fmaxf(l[q][2], l[q][3]));
+    m = fmaxf(m, __builtin_bit_cast(float, lane_xor_dpp<8>(__builtin_bit_cast(int, m))));
+    m = fmaxf(m, __builtin_bit_cast(float, lane_xor_dpp<4>(__builtin_bit_cast(int, m))));
+    m = fmaxf(m, __builtin_bit_cast(float, lane_xor_dpp<2>(__builtin_bit_cast(int, m))));
+    m = fmaxf(m, __builtin_bit_cast(float, lane_xor_dpp<1>(__builtin_bit_cast(int, m))));
+    const int slot = part * (kPartEntries / kSlot) + (q * kPartThreads + t) / 16;
+    if ((t & 15) == 0 && slot < n_slots) stats[slot] = m;
+    top = fmaxf(top, m);
+  }
+  top = wave_reduce_dpp(top, fmax_op);
+  if ((t & 63) == 0) red[t >> 6] = top;
+  __syncthreads();
+  top = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  float sum = 0.0f;
+#pragma unroll
+  for (int q = 0; q < kVecs; ++q)
+    sum += (exp2f(l[q][0] - top) + exp2f(l[q][1] - top)) + (exp2f(l[q][2] - top) + exp2f(l[q][3] - top));
+  sum = wave_reduce_dpp(sum, [](float x, float y) { return x + y; });
+  __syncthreads();
+  if ((t & 63) == 0) red[t >> 6] = sum;
+  __syncthreads();
+  if (t == 0) {
+    stats[n_slots + part] = top;
+    stats[n_slots + parts + part] = (red[0] + red[1]) + (red[2] + red[3]);
+  }
+}
+static_assert(kPartThreads == 256, "sample_stats_kernel adds up four wavefronts");
+
+// order of finite floats as unsigned integers, and back
+__device__ __forceinline__ unsigned order_key(float x) {
+  const unsigned u = __float_as_uint(x);
+  return static_cast<int>(u) < 0 ? ~u : u | 0x80000000u;
+}
+__device__ __forceinline__ float from_order_key(unsigned k) {
+  return __uint_as_float(static_cast<int>(k) < 0 ? k & 0x7fffffffu : ~k);
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs a, int parts) {
+  __shared__ BlockRed red;
+  __shared__ int s_pick;
+  __shared__ unsigned counts[2][kSampleWaves];
+  __shared__ int slots[kMaxSlots];
+  __shared__ int n_cand;
+  __shared__ unsigned cand_at[kMaxCandidates], sorted_at[kMaxCandidates];
+  __shared__ float cand[kMaxCandidates], sorted[kMaxCandidates];
+  const int b = blockIdx.x;
+  const int t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int lane = t & 63;
+  const int V4 = a.V / 4;
+  const int n_slots = (a.V + kSlot - 1) / kSlot;
+  const unsigned top_k = static_cast<unsigned>(a.top_k);
+  const float* stats = a.probs + static_cast<int64_t>(b) * a.V;
+  auto fmax_op = [](float x, float y) { return fmaxf(x, y); };
+  auto fmin_op = [](float x, float y) { return fminf(x, y); };
+  auto fadd_op = [](float x, float y) { return x + y; };
+  auto umin_op = [](unsigned x, unsigned y) { return min(x, y); };
+
+  // every wavefront: the parts, and all slot maxima (sixteen per lane)
+  const int part = min(lane, parts - 1);
+  const float part_max = stats[n_slots + part];
+  const float part_sum = lane < parts ? stats[n_slots + parts + part] : 0.0f;
+  unsigned key[kMaxSlots / 64];
+#pragma unroll
+  for (int i = 0; i < kMaxSlots / 64; ++i) key[i] = order_key(stats[min(i * 64 + lane, n_slots - 1)]);
+  const float my_slot_max = stats[min(t, n_slots - 1)];
+  const float gmax = wave_reduce_dpp(part_max, fmax_op);
+  const float den = wave_reduce_dpp(part_sum * exp2f(part_max - gmax), fadd_op);
+
+  // a value that at least top_k slot maxima reach, and hardly more: sixteen thresholds at a time, one per wavefront
+  unsigned low_key = 0xffffffffu;
+#pragma unroll
+  for (int i = 0; i < kMaxSlots / 64; ++i) {
+    low_key = min(low_key, key[i]);
+    if (i * 64 + lane >= n_slots) key[i] = 0;  // (below every threshold; a lane past the end repeated the last slot)
+  }
+  unsigned lo = wave_reduce_dpp(low_key, umin_op);
+  unsigned hi = order_key(gmax) + 1u;
+  unsigned reach = static_cast<unsigned>(n_slots);  // maxima at or above lo
+  const unsigned enough = top_k + max(top_k / 4u, 16u);
+  for (int it = 0; reach > enough && hi - lo > 1u; it ^= 1) {
+    const unsigned span = hi - lo;
+    auto threshold = [&](int w) { return lo + max(static_cast<unsigned>(static_cast<uint64_t>(span) * (w + 1) / 17u), 1u); };
+    const unsigned mine = threshold(wave);
+    unsigned c = 0;
+#pragma unroll
+    for (int i = 0; i < kMaxSlots / 64; ++i) c += static_cast<unsigned>(__popcll(__ballot(key[i] >= mine)));
+    if (lane == 0) counts[it][wave] = c;
+    __syncthreads();
+    unsigned new_lo = lo, new_hi = hi;
+#pragma unroll
+    for (int w = 0; w < kSampleWaves; ++w) {
+      const unsigned cw = counts[it][w];
+      if (cw >= top_k) {
+        new_lo = threshold(w);
+        reach = cw;
+      } else {
+        new_hi = min(new_hi, threshold(w));
       }
-      reinterpret_cast<float4_t*>(pen)[i] = p;
-    });
+    }
+    lo = new_lo;
+    hi = new_hi;
+  }
+  // (two logits this close may round to the same probability, and entries of one probability share its fate)
+  const float floor_u = from_order_key(lo) - 4e-6f;
+
+  // the slots that reach it, then their entries that do
+  if (t == 0) n_cand = 0;
+  const bool chosen = t < n_slots && my_slot_max >= floor_u;
+  const uint64_t mask = __ballot(chosen);
+  __syncthreads();
+  if (lane == 0) red.u[wave] = static_cast<unsigned>(__popcll(mask));
+  __syncthreads();
+  int first = 0, n_chosen = 0;
+#pragma unroll
+  for (int w = 0; w < kSampleWaves; ++w) {
+    if (w < wave) first += static_cast<int>(red.u[w]);
+    n_chosen += static_cast<int>(red.u[w]);
+  }
+  if (chosen) slots[first + __popcll(mask & ((1ull << lane) - 1ull))] = t;
+  __syncthreads();
+  const float4_t* logits = reinterpret_cast<const float4_t*>(a.logits + static_cast<int64_t>(b) * a.V);
+  const float4_t* pen = a.penalties ? reinterpret_cast<const float4_t*>(a.penalties + static_cast<int64_t>(b) * a.V) : nullptr;
+  for (int s = t >> 4; s < n_chosen; s += kSampleThreads / 16) {
+    const int i = slots[s] * (kSlot / 4) + (t & 15);
+    if (i >= V4) continue;
+    const float4_t l = logits[i];
+    float4_t p = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (pen) p = pen[i];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float u = penalised(l[j], p[j], a.log2_inv_temp);
+      if (u >= floor_u) {
+        const int at = atomicAdd(&n_cand, 1);
+        if (at < kMaxCandidates) {
+          cand[at] = u;
+          // where sample_row's draw meets the entry: thread i % 1024, its slice's float4 i / 1024, element j
+          cand_at[at] = static_cast<unsigned>(((i % kSampleThreads) * kSampleRegVecs + i / kSampleThreads) * 4 + j);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const int n = n_cand;
+  int pick = 0;
+  if (n > kMaxCandidates) {
+    pick = sample_row<true>(a, b, red, s_pick);
+  } else {
+    if (t < n) {
+      const unsigned at = cand_at[t];
+      int rank = 0;
+      for (int i = 0; i < n; ++i) rank += cand_at[i] < at ? 1 : 0;
+      sorted_at[rank] = at;
+      sorted[rank] = exp2f(cand[t] - gmax) / den;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    // one wavefront, up to sixteen entries per lane: steps 4 to 6 of sample_row without a barrier
+    constexpr int kRounds = kMaxCandidates / 64;
+    const int rounds = (n + 63) / 64;
+    float p[kRounds];
+    float pmax = -INFINITY, pmin = INFINITY, mass = 0.0f;
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      p[r] = -1.0f;  // past the end: below every threshold
+      if (r < rounds && r * 64 + lane < n) {
+        p[r] = sorted[r * 64 + lane];
+        pmax = fmaxf(pmax, p[r]);
+        pmin = fminf(pmin, p[r]);
+        mass += p[r];
+      }
+    }
+    pmax = wave_reduce_dpp(pmax, fmax_op);
+    pmin = wave_reduce_dpp(pmin, fmin_op);
+    mass = wave_reduce_dpp(mass, fadd_op);
+    unsigned cnt = static_cast<unsigned>(n);
+    unsigned left = __float_as_uint(pmin), right = __float_as_uint(pmax) + 1u;
+    while ((cnt > top_k || mass > a.top_p) && left < right - 1u) {
+      const unsigned mid = left + (right - left) / 2u;
+      const float thr = __uint_as_float(mid);
+      unsigned c = 0;
+      float m = 0.0f;
+#pragma unroll
+      for (int r = 0; r < kRounds; ++r) {
+        if (r < rounds) {
+          c += static_cast<unsigned>(__popcll(__ballot(p[r] >= thr)));
+          m += p[r] >= thr ? p[r] : 0.0f;
+        }
+      }
+      m = wave_reduce_dpp(m, fadd_op);
+      if (c < top_k && m < a.top_p) {
+        right = mid;
+      } else {
+        left = mid;
+        cnt = c;
+        mass = m;
+      }
+    }
+    const float thr = __uint_as_float(left);
+    unsigned n_eq = 0, n_gt = 0;
+    float p_gt = 0.0f;
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      if (r < rounds) {
+        n_eq += static_cast<unsigned>(__popcll(__ballot(p[r] == thr)));
+        n_gt += static_cast<unsigned>(__popcll(__ballot(p[r] > thr)));
+        p_gt += p[r] > thr ? p[r] : 0.0f;
+      }
+    }
+    p_gt = wave_reduce_dpp(p_gt, fadd_op);
+    float comp = 1.0f;
+    if (n_eq > 0) comp = tie_share(a, thr, n_eq, n_gt, p_gt);
+    // running sums of the kept weights in the draw's order, then the first that reaches the target
+    float total = 0.0f;
+    float cum[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      cum[r] = 0.0f;
+      if (r < rounds) {
+        p[r] = p[r] < thr ? 0.0f : (p[r] == thr ? p[r] * comp : p[r]);
+        float inc = p[r];
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const float below = __shfl_up(inc, off, 64);
+          if (lane >= off) inc += below;
+        }
+        cum[r] = total + inc;
+        total = __shfl(cum[r], 63, 64);
+      }
+    }
+    const float target = uniform_of_row(a, b) * total;
+    int found = -1, last = -1;
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      if (r < rounds) {
+        const uint64_t kept = __ballot(p[r] > 0.0f);
+        const uint64_t hit = __ballot(p[r] > 0.0f && cum[r] >= target);
+        if (hit != 0 && found < 0) found = r * 64 + __ffsll(static_cast<unsigned long long>(hit)) - 1;
+        if (kept != 0) last = r * 64 + 63 - __clzll(static_cast<long long>(kept));
+      }
+    }
+    if (found < 0) found = last;  // rounding left the target past the last sum
+    if (found >= 0) {
+      const unsigned at = sorted_at[found];
+      const int i = static_cast<int>((at >> 2) % kSampleRegVecs) * kSampleThreads + static_cast<int>(at >> 2) / kSampleRegVecs;
+      pick = i * 4 + static_cast<int>(at & 3u);
+    }
+  }
+  if (t == 0) a.out[b] = pick;
+}
+
+__global__ __launch_bounds__(kPartThreads) void sample_decay_kernel(SampleArgs a) {
+  constexpr int kVecs = kPartEntries / 4 / kPartThreads;
+  const int b = blockIdx.x;
+  const int first = blockIdx.y * (kPartEntries / 4) + threadIdx.x;
+  const int V4 = a.V / 4;
+  float4_t* pen = reinterpret_cast<float4_t*>(a.penalties + static_cast<int64_t>(b) * a.V);
+  const int pick = a.out[b];
+  float4_t p[kVecs];
+#pragma unroll
+  for (int q = 0; q < kVecs; ++q) p[q] = pen[min(first + q * kPartThreads, V4 - 1)];
+#pragma unroll
+  for (int q = 0; q < kVecs; ++q) {
+    const int i = first + q * kPartThreads;
+    if (i < V4) pen[i] = decayed_penalty(p[q], i, pick, a);
   }
 }
 
@@ -500,7 +843,12 @@ int rwkv_hip_sample(rwkv_stream_t s, int B, int V, const void* logits, void* pen
   a.top_p = static_cast<float>(top_p);
   a.seed = seed;
   a.step = step;
-  if (V / 4 <= kSampleRegVecs * kSampleThreads) {
+  if (sample_split_ok(V, top_k)) {
+    const int parts = ceil_div(V, kPartEntries);
+    hipLaunchKernelGGL(sample_stats_kernel, dim3(B, parts), dim3(kPartThreads), 0, as_stream(s), a);
+    hipLaunchKernelGGL(sample_pick_kernel, dim3(B), dim3(kSampleThreads), 0, as_stream(s), a, parts);
+    if (penalties) hipLaunchKernelGGL(sample_decay_kernel, dim3(B, parts), dim3(kPartThreads), 0, as_stream(s), a);
+  } else if (V / 4 <= kSampleRegVecs * kSampleThreads) {
     hipLaunchKernelGGL(sample_kernel<true>, dim3(B), dim3(kSampleThreads), 0, as_stream(s), a);
   } else {
     hipLaunchKernelGGL(sample_kernel<false>, dim3(B), dim3(kSampleThreads), 0, as_stream(s), a);

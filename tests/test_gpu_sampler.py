@@ -75,6 +75,41 @@ def test_draws_stay_in_kept_set_and_follow_filtered_distribution(gpu, orc, top_k
     assert tv <= 0.5 * np.sqrt(max(kept, 1) / n) + 0.02
 
 
+@pytest.mark.parametrize("kind", ["normal", "ties", "equal"])
+@pytest.mark.parametrize("V,top_k,top_p", [(512, 4, 1.0), (516, 3, 0.7), (4100, 32, 0.9), (40004, 256, 0.99), (65536, 2, 0.6),
+                                          (65536, 256, 1.0)])
+def test_top_k_rows_in_three_launches(gpu, orc, V, top_k, top_p, kind):
+    """The three-launch route at its edges: as few slots as it takes (V = 128 top_k), a row that ends inside a slot and inside a
+    part, the smallest and the largest top_k, many entries at the threshold, and a row of equal logits, which has more candidates
+    than fit and goes through the whole-row selection.  Every pick has weight in the oracle's kept set and the penalty rows
+    follow the recurrence (two roundings of fp32)."""
+    hip = gpu
+    rng = np.random.default_rng(V + top_k)
+    logits = (rng.standard_normal(V) * 2.5).astype(np.float32)
+    if kind == "ties":
+        logits = np.round(logits * 2) / 2
+    if kind == "equal":
+        logits[:] = 1.25
+    B, steps = 5, 6
+    kept, probs = orc.sample_filter(logits, None, 0.8, top_k, top_p)
+    assert kept >= 1
+    draws = _draw(hip, logits, B, steps, seed=3, temperature=0.8, top_k=top_k, top_p=top_p)
+    weight = probs[draws.ravel()]
+    assert weight.min() > 0
+    again = _draw(hip, logits, B, steps, seed=3, temperature=0.8, top_k=top_k, top_p=top_p)
+    assert draws.tolist() == again.tolist()
+
+    start = np.where(rng.random((B, V)) < 0.1, rng.random((B, V)), 0.0).astype(np.float32)
+    d_pen = hip.DeviceArray.from_numpy(start)
+    picks = _draw(hip, logits, B, 1, seed=4, penalties=d_pen, presence=0.5, frequency=0.25, decay=0.9, top_k=top_k, top_p=top_p)[0]
+    want = start * np.float32(0.9)
+    for b in range(B):
+        assert orc.sample_filter(logits, start[b].copy(), 1.0, top_k, top_p)[1][picks[b]] > 0
+        want[b, picks[b]] += np.float32(0.5 if start[b, picks[b]] == 0 else 0.25)
+    err = float(np.max(np.abs(d_pen.numpy() - want)))
+    assert err <= 2.5e-7
+
+
 def test_rows_longer_than_the_register_path_follow_the_filtered_distribution(gpu, orc):
     """Rows of more than 65536 entries keep their slices in the probs scratch instead of registers: same kept set,
     same distribution; greedy picks the lowest index among tied maxima."""
