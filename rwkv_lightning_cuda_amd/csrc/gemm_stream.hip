@@ -572,6 +572,8 @@ static bool sums_at_consumer(int n_problems, int epilogue, int out_f32) {
   return n_problems == 1 && epilogue == RWKV_EPI_NONE && !out_f32;
 }
 
+// Blocks that occupy the 256 CUs well enough without a K split.
+constexpr int kFilledBlocks = 200;
 // Rows from which the wide tiles, whose wavefronts feed two MFMAs from every X fragment they read from LDS, are looked at.
 constexpr int kWideMinRows = 160;
 // Launches of int8 problems only have a wide tile of their own at these sizes (three blocks per CU).
@@ -603,7 +605,7 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
     c.ring = RingShape{0, 0, 0, 0};
     c.wide_mt = 4;
     // (from 1025 rows on, with most of the chip busy, the wide tile is the faster one whatever the estimates' last percent)
-    if (M > 1024 && ceil_div(M, 128) * count_col_blocks(c, n_problems, Ns, fmts) >= 200) best_us = 1e30f;
+    if (M > 1024 && ceil_div(M, 128) * count_col_blocks(c, n_problems, Ns, fmts) >= kFilledBlocks) best_us = 1e30f;
     consider(c);
     if (!any[RWKV_FMT_F16] && K <= 4096 && M <= 1024) {
       c.wide_mt = 2;
@@ -681,6 +683,10 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
   int64_t n_total = 0;
   for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
   const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
+  // A split is an offer, not a need, where blocks of 32 x 32 alone occupy the chip or K has no power of two of whole 512s
+  // (1024s up to 32 rows): such a call runs without a workspace too, with the split that fits.  Elsewhere a workspace too
+  // small for the split is an error.
+  fit_splits = fit_splits || K % (M <= 32 ? 1024 : 512) != 0 || static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
   const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace ? workspace_bytes / plane : 0)) : 32;
   const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, sums_at_consumer(n_problems, epilogue, out_f32), max_splits);
   int col_blocks = 0;

@@ -943,6 +943,28 @@ def test_linear_packed_tile_edges(gpu, orc, fmt_name, M, N, K):
     assert untouched
 
 
+@pytest.mark.parametrize("fmt_name", ["f16", "w8", "w4"])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 2560), (13, 96, 768), (32, 768, 1280), (33, 96, 1280), (100, 2560, 1024)])
+def test_linear_packed_without_a_workspace(gpu, orc, fmt_name, M, N, K):
+    """Where K has no power of two of whole 512s (1024s up to 32 rows), or blocks of 32 x 32 alone fill the chip, a K split is
+    taken only if its planes fit the workspace: no workspace, and one of a byte, give the product all the same."""
+    hip = gpu
+    rng = np.random.default_rng(M + N + K)
+    fmt = {"f16": hip.FMT_F16, "w8": hip.FMT_W8, "w4": hip.FMT_W4}[fmt_name]
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    parts = _quant_parts(orc, hip, fmt, (rng.standard_normal((N, K)) * 0.02).astype(np.float16))
+    dparts = [dev(hip, p) if p is not None else None for p in parts]
+    packed = hip.DeviceArray(parts[0].shape, parts[0].dtype)
+    hip.pack_weights(fmt, N, K, dparts[0], packed)
+    want = orc.gemv(fmt, x, parts[0], parts[1], parts[2]).astype(np.float32)
+    for ws in (None, hip.DeviceArray((1,), np.uint8)):
+        y = hip.DeviceArray((M, N), np.float16)
+        hip.linear_packed(fmt, M, N, K, dev(hip, x), packed, dparts[1], dparts[2], y, ws)
+        hip.device_sync()
+        err = rel_err(y.numpy().astype(np.float32), want)
+        assert err <= F16_TOL
+
+
 def test_pack_weights_is_the_documented_permutation(gpu):
     """Tile (band nt, k group kg) holds, for lane j + 32h, the KR consecutive k of row 32 nt + j starting at
     kg*G + h*KR, as 64 x 16-byte pieces (two pieces for fp16)."""
