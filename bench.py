@@ -192,8 +192,7 @@ def parity_legs(hip, fmt_name, with_others):
     if with_others:
         if fmt_name == "w8":
             others["w4_parity"] = leg(d8, w8, "w4", 8, 16, what)
-            # the few-row launches of 5 to 16 rows (products on the matrix core, LN2 folded into ffn.key, ffn.value in
-            # column slices) and of 2 to 4 rows (the GEMV with several rows of x, one walk of ffn.value)
+            # the packed GEMM of decode steps (8 rows, and 3 rows of long int8 rows with one walk of ffn.value)
             d2l = sliced("7.2B", 2)
             w2l = synth_weights(d2l, 90)
             two = "7.2B shape, 2 of 32 layers (C 4096, full 65536-row head)"
