@@ -110,6 +110,29 @@ def test_top_k_rows_in_three_launches(gpu, orc, V, top_k, top_p, kind):
     assert err <= 2.5e-7
 
 
+@pytest.mark.parametrize("kind", ["normal", "ties", "equal"])
+@pytest.mark.parametrize("V,top_k,top_p", [(4, 0, 0.5), (256, 0, 0.5), (260, 0, 0.9), (1028, 700, 0.8), (40004, 0, 0.3),
+                                          (65536, 0, 0.9), (65536, 500, 1.0), (65536, 65535, 1.0)])
+def test_threshold_of_rows_in_registers(gpu, orc, V, top_k, top_p, kind):
+    """The threshold search hands its last 256 candidates to single wavefronts: a row that is no longer than that, one entry
+    group more, more equal entries at the threshold than fit (the whole-row search then runs to its end), and the whole
+    range.  Every draw has weight in the oracle's kept set, and draws repeat."""
+    hip = gpu
+    rng = np.random.default_rng(V + top_k)
+    logits = (rng.standard_normal(V) * 2.5).astype(np.float32)
+    if kind == "ties":
+        logits = np.round(logits * 2) / 2
+    if kind == "equal":
+        logits[:] = 1.25
+    kept, probs = orc.sample_filter(logits, None, 0.8, top_k, top_p)
+    assert kept >= 1
+    draws = _draw(hip, logits, 7, 6, seed=3, temperature=0.8, top_k=top_k, top_p=top_p)
+    weight = probs[draws.ravel()]
+    assert weight.min() > 0
+    again = _draw(hip, logits, 7, 6, seed=3, temperature=0.8, top_k=top_k, top_p=top_p)
+    assert draws.tolist() == again.tolist()
+
+
 def test_rows_longer_than_the_register_path_follow_the_filtered_distribution(gpu, orc):
     """Rows of more than 65536 entries keep their slices in the probs scratch instead of registers: same kept set,
     same distribution; greedy picks the lowest index among tied maxima."""
