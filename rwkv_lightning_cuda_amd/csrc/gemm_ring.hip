@@ -338,7 +338,7 @@ __device__ __forceinline__ void ring_block(const StreamArgs& g, const StreamProb
 
   if (wave >= kRingWorkers) {
     ring_feed<MT, NB, WP, KC>(g, pr, m0, kbeg, nstages, lds, wave - kRingWorkers, lane);
-    ride_along_copy(g.copy, 64 * kRingFeeders);
+    ride_along_copy(g.copy, g.col_blocks * g.splits, 64 * kRingFeeders);  // (a block past the last pair has left)
   } else {
     ring_work<FMT, MT, NB, WP, KC>(g, pr, col_block, kbeg, nstages, lds, wave, lane);
   }

@@ -34,12 +34,12 @@ struct StreamArgs {
   RowCopy copy;  // rides on the launch: its first blocks move these rows (they are no operand of the product)
 };
 
-// shared out between the first blocks of the launch (those with y == z == 0), so that no single block carries it on its
-// critical path; in a launch whose other wavefronts are busy, called by the last `threads` of the block
-__device__ __forceinline__ void ride_along_copy(const RowCopy& cp, unsigned threads = 0) {
+// shared out between the first blocks of the launch (those with y == z == 0 among the first `blocks` of x, every one of which
+// has to come here: a share nobody takes is never copied), so that no single block carries it on its critical path; called by
+// the last `threads` of the block
+__device__ __forceinline__ void ride_along_copy(const RowCopy& cp, unsigned blocks, unsigned threads) {
   constexpr unsigned kCopyBlocks = 8;
-  const unsigned nb = gridDim.x < kCopyBlocks ? gridDim.x : kCopyBlocks;
-  if (threads == 0) threads = blockDim.x;
+  const unsigned nb = blocks < kCopyBlocks ? blocks : kCopyBlocks;
   if (blockIdx.x < nb && blockIdx.y == 0 && blockIdx.z == 0 && cp.n > 0) {
     const unsigned t = threadIdx.x - (blockDim.x - threads);
     for (int i = (blockIdx.x * threads + t) * 8; i < cp.n; i += nb * threads * 8)

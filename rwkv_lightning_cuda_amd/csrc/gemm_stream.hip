@@ -400,7 +400,7 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
 template <bool MIXED, int MT>
 __global__ __launch_bounds__(256, MIXED ? 1 : 2) void gemm_stream_wide_kernel(StreamArgs g) {
   __shared__ __align__(16) half_t xs[2 * 32 * MT * (128 + 8)];
-  ride_along_copy(g.copy);
+  ride_along_copy(g.copy, gridDim.x, blockDim.x);
   const int id = blockIdx.x;
   const int row_tile = (id >> 3) % g.row_tiles;
   const int pair = (id / (8 * g.row_tiles)) * 8 + (id & 7);

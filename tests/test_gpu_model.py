@@ -162,6 +162,41 @@ def test_matrices_of_different_formats_side_by_side(gpu):
     assert cos >= 0.9995
 
 
+@pytest.mark.parametrize("F,projections", [(256, ("w8", "w8", "w8")), (1024, ("w8", "w4", "w4")), (448, ("w4", "w4", "w4"))])
+def test_shift_rows_that_ride_on_a_launch_of_few_blocks(gpu, F, projections):
+    """The new shift rows of a short chunk move into the state with the next packed launch.  40 sequences of 256 channels are
+    five blocks' shares of that copy; ffn.key of 256 or 448 columns, or the one int8 projection beside two int4 ones, is a
+    launch of four blocks (seven at 64 columns each).  Every row of the state against the same tokens one by one, whose
+    LayerNorm kernels write the rows themselves (the bar is the fp16 one of the decode tests: sums in another order)."""
+    from rwkv_lightning_cuda_amd.model import DeviceMatrix, HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=3, C=256, H=4, F=F, V=512, Rw=32, Ra=32, Rg=32, Rv=32)
+    weights = synth_weights(dims, 41)
+    fmts = {"w8": hip.FMT_W8, "w4": hip.FMT_W4}
+    model = HipModel.from_host_weights(dims, weights, hip.FMT_W8)
+    for layer in range(dims.L):
+        for (name, mid), fmt in zip((("att_r", hip.M_ATT_R), ("att_k", hip.M_ATT_K), ("att_v", hip.M_ATT_V)), projections):
+            N, K = dims.mat_shape(name)
+            w = hip.DeviceArray.from_numpy(weights["layers"][layer][name])
+            model.set_matrix(layer, mid, DeviceMatrix.from_f16_device(fmts[fmt], N, K, w))
+    B, T = 40, 2
+    tokens = np.random.default_rng(F).integers(0, dims.V, (B, T))
+    states, logits = [], []
+    for step in (T, 1):
+        sess = Session(model)
+        st = State(dims, B)
+        lg = hip.DeviceArray((B, dims.V), np.float32)
+        for t in range(0, T, step):
+            sess.forward(tokens[:, t:t + step], st, lg)
+        states.append(st.shift.numpy().astype(np.float32))
+        logits.append(lg.numpy())
+        sess.close()
+    for row in range(B):
+        err = rel_err(states[0][:, :, row], states[1][:, :, row])
+        assert err <= 3e-3, "shift rows of sequence %d" % row
+    assert rel_err(logits[0], logits[1]) <= 3e-3
+
+
 @pytest.mark.parametrize("H", [3, 5])
 def test_odd_head_count_on_the_row_tiled_rank_out(gpu, orc, H):
     """C = 64 H with H odd leaves the last 128-channel block of the LoRA rank-out half empty: the packed copy of the
