@@ -684,9 +684,9 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
   for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
   const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
   // A split is an offer, not a need, where blocks of 32 x 32 alone occupy the chip or K has no power of two of whole 512s
-  // (1024s up to 32 rows): such a call runs without a workspace too, with the split that fits.  Elsewhere a workspace too
-  // small for the split is an error.
-  fit_splits = fit_splits || K % (M <= 32 ? 1024 : 512) != 0 || static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
+  // (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a workspace too, with the split that
+  // fits.  Elsewhere a workspace too small for the split is an error.
+  fit_splits = fit_splits || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 || static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
   const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace ? workspace_bytes / plane : 0)) : 32;
   const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, sums_at_consumer(n_problems, epilogue, out_f32), max_splits);
   int col_blocks = 0;

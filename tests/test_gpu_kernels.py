@@ -965,6 +965,26 @@ def test_linear_packed_without_a_workspace(gpu, orc, fmt_name, M, N, K):
         assert err <= F16_TOL
 
 
+@pytest.mark.parametrize("fmt_name", ["f16", "w8", "w4"])
+@pytest.mark.parametrize("M,N,K", [(33, 96, 1536), (48, 64, 512), (64, 3168, 1536)])
+def test_linear_packed_of_33_to_64_rows_without_a_workspace(gpu, orc, fmt_name, M, N, K):
+    """33 to 64 rows of K up to 2048 need a split only where K is a multiple of 1024: 512 and 1536 run without a workspace, up
+    to the last width whose blocks of 32 x 32 do not fill the chip."""
+    hip = gpu
+    rng = np.random.default_rng(M + N + K)
+    fmt = {"f16": hip.FMT_F16, "w8": hip.FMT_W8, "w4": hip.FMT_W4}[fmt_name]
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    parts = _quant_parts(orc, hip, fmt, (rng.standard_normal((N, K)) * 0.02).astype(np.float16))
+    dparts = [dev(hip, p) if p is not None else None for p in parts]
+    packed = hip.DeviceArray(parts[0].shape, parts[0].dtype)
+    hip.pack_weights(fmt, N, K, dparts[0], packed)
+    y = hip.DeviceArray((M, N), np.float16)
+    hip.linear_packed(fmt, M, N, K, dev(hip, x), packed, dparts[1], dparts[2], y, None)
+    hip.device_sync()
+    err = rel_err(y.numpy().astype(np.float32), orc.gemv(fmt, x, parts[0], parts[1], parts[2]).astype(np.float32))
+    assert err <= F16_TOL
+
+
 def test_pack_weights_is_the_documented_permutation(gpu):
     """Tile (band nt, k group kg) holds, for lane j + 32h, the KR consecutive k of row 32 nt + j starting at
     kg*G + h*KR, as 64 x 16-byte pieces (two pieces for fp16)."""
