@@ -110,6 +110,31 @@ def test_top_k_rows_in_three_launches(gpu, orc, V, top_k, top_p, kind):
     assert err <= 2.5e-7
 
 
+@pytest.mark.parametrize("shared", ["logits", "penalties", "second row"])
+def test_top_k_rows_whose_scratch_is_an_input(gpu, orc, shared):
+    """Rows of up to 65536 entries leave the scratch alone when it is the logits or the penalty rows (or reaches into them):
+    every draw has weight in the oracle's kept set, the logits stay as they are and the penalties follow the recurrence."""
+    hip = gpu
+    V, B, top_k, top_p = 8192, 6, 40, 0.8
+    rng = np.random.default_rng(11)
+    logits = (rng.standard_normal((B, V)) * 2.5).astype(np.float32)
+    start = np.where(rng.random((B, V)) < 0.1, rng.random((B, V)), 0.0).astype(np.float32)
+    room = hip.DeviceArray((B + 1, V), np.float32)
+    d_logits, d_pen = room.view(0, (B, V)), hip.DeviceArray.from_numpy(start)
+    d_logits.upload(logits)
+    probs = {"logits": d_logits, "penalties": d_pen, "second row": room.view(V, (B, V))}[shared]
+    picked = hip.DeviceArray((B,), np.int32)
+    hip.sample(B, V, d_logits, d_pen, probs, picked, presence=0.5, frequency=0.25, decay=0.9, top_k=top_k, top_p=top_p, seed=7)
+    hip.device_sync()
+    picks = picked.numpy()
+    assert np.array_equal(d_logits.numpy(), logits)
+    want = start * np.float32(0.9)
+    for b in range(B):
+        assert orc.sample_filter(logits[b], start[b].copy(), 1.0, top_k, top_p)[1][picks[b]] > 0
+        want[b, picks[b]] += np.float32(0.5 if start[b, picks[b]] == 0 else 0.25)
+    assert float(np.max(np.abs(d_pen.numpy() - want))) <= 2.5e-7
+
+
 @pytest.mark.parametrize("kind", ["normal", "ties", "equal"])
 @pytest.mark.parametrize("V,top_k,top_p", [(4, 0, 0.5), (256, 0, 0.5), (260, 0, 0.9), (1028, 700, 0.8), (40004, 0, 0.3),
                                           (65536, 0, 0.9), (65536, 500, 1.0), (65536, 65535, 1.0)])
