@@ -485,7 +485,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
 //   sample_decay_kernel  the penalty rows, by the whole chip again.
 // Against the one-block kernel the sum of the exponentials and the masses are added in another order (fp32 both), no more.
 // Rows of 65536, penalties, top-k 50, top-p 0.6, one block per row / this: 1 row 53.4 / 19.8 us, 64 rows 66-70 / 27.7,
-// 128 rows 70.9 / 40.4; 8 rows, top-k 200, top-p 0.8: 64.5 / 27.7.
+// 128 rows 70.9 / 40.4; 8 rows, top-k 200, top-p 0.8: 64.5 / 27.7.  The same rows masked down to 20 entries: 64 rows 75.1 /
+// 28.8.  Rows of equal logits, which pay for the launches on top of sample_row, lose: 1 row 87 / 95, 256 rows 112 / 144.
 // The slot maxima and the parts' sums lie in `probs`.
 constexpr int kSlot = 64;
 constexpr int kPartEntries = 4096;
@@ -608,6 +609,18 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
   unsigned hi = order_key(gmax) + 1u;
   unsigned reach = static_cast<unsigned>(n_slots);  // maxima at or above lo
   const unsigned enough = top_k + max(top_k / 4u, 16u);
+  // Entries 150 octaves below the maximum have probability zero: they never carry weight.  Where fewer than top_k slots reach
+  // higher than that - a row masked down to a few entries - there is nothing to search for, and the zeros need not compete one
+  // by one; that they are there the threshold search below has to know: it then starts at zero with a count above any top_k.
+  const float zero_u = gmax - 150.0f;
+  const unsigned zero_key = order_key(zero_u);
+  if (lo < zero_key) {
+    unsigned c = 0;
+#pragma unroll
+    for (int i = 0; i < kMaxSlots / 64; ++i) c += static_cast<unsigned>(__popcll(__ballot(key[i] >= zero_key)));
+    reach = c;
+    if (c >= top_k) lo = zero_key;
+  }
   for (int it = 0; reach > enough && hi - lo > 1u; it ^= 1) {
     const unsigned span = hi - lo;
     auto threshold = [&](int w) { return lo + max(static_cast<unsigned>(static_cast<uint64_t>(span) * (w + 1) / 17u), 1u); };
@@ -632,7 +645,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
     hi = new_hi;
   }
   // (two logits this close may round to the same probability, and entries of one probability share its fate)
-  const float floor_u = from_order_key(lo) - 4e-6f;
+  const float bound_u = from_order_key(lo) - 4e-6f;
+  const bool zeros_below = bound_u < zero_u;
+  const float floor_u = fmaxf(bound_u, zero_u);
 
   // the slots that reach it, then their entries that do
   if (t == 0) n_cand = 0;
@@ -652,6 +667,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
   const float4_t* logits = reinterpret_cast<const float4_t*>(a.logits + static_cast<int64_t>(b) * a.V);
   const float4_t* pen = a.penalties ? reinterpret_cast<const float4_t*>(a.penalties + static_cast<int64_t>(b) * a.V) : nullptr;
   for (int s = t >> 4; s < n_chosen; s += kSampleThreads / 16) {
+    // (more candidates than fit: the row goes another way, whatever the rest of them is)
+    if (s >= kSampleThreads / 16 && *static_cast<volatile int*>(&n_cand) > kMaxCandidates) break;
     const int i = slots[s] * (kSlot / 4) + (t & 15);
     if (i >= V4) continue;
     const float4_t l = logits[i];
@@ -703,8 +720,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
     pmax = wave_reduce_dpp(pmax, fmax_op);
     pmin = wave_reduce_dpp(pmin, fmin_op);
     mass = wave_reduce_dpp(mass, fadd_op);
-    unsigned cnt = static_cast<unsigned>(n);
-    unsigned left = __float_as_uint(pmin), right = __float_as_uint(pmax) + 1u;
+    unsigned cnt = zeros_below ? static_cast<unsigned>(V4) * 4u : static_cast<unsigned>(n);
+    unsigned left = zeros_below ? 0u : __float_as_uint(pmin), right = __float_as_uint(pmax) + 1u;
     while ((cnt > top_k || mass > a.top_p) && left < right - 1u) {
       const unsigned mid = left + (right - left) / 2u;
       const float thr = __uint_as_float(mid);

@@ -135,6 +135,51 @@ def test_top_k_rows_whose_scratch_is_an_input(gpu, orc, shared):
     assert float(np.max(np.abs(d_pen.numpy() - want))) <= 2.5e-7
 
 
+@pytest.mark.parametrize("low", [-np.inf, -3.0e38, -200.0])
+@pytest.mark.parametrize("live", [1, 3, 39, 40, 41, 900, 1500])
+def test_top_k_rows_masked_to_a_few_entries(gpu, orc, live, low):
+    """A row masked down to fewer entries than top_k, to as many, to more, and to more than one block holds as candidates; the
+    rest at minus infinity, near the type's lowest value, or just low enough for a probability of zero.  Every draw has weight
+    in the oracle's kept set, and draws repeat."""
+    hip = gpu
+    V, top_k = 8192, 40
+    rng = np.random.default_rng(live)
+    logits = np.full(V, low, np.float32)
+    logits[100:100 + live] = (rng.standard_normal(live) * 2.5).astype(np.float32)
+    for top_p in (1.0, 0.6):
+        kept, probs = orc.sample_filter(logits, None, 1.0, top_k, top_p)
+        draws = _draw(hip, logits, 5, 12, seed=3, temperature=1.0, top_k=top_k, top_p=top_p)
+        assert probs[draws.ravel()].min() > 0
+        assert draws.tolist() == _draw(hip, logits, 5, 12, seed=3, temperature=1.0, top_k=top_k, top_p=top_p).tolist()
+
+
+def test_masked_rows_take_no_longer_than_others(gpu):
+    """Rows that leave 20 of 65536 entries and a top_k of 50 (constrained decoding) against unmasked ones: the few entries that
+    are left compete, not the masked ones (90 against 28 us with the masked entries competing)."""
+    hip = gpu
+    B, V = 64, 65536
+    rng = np.random.default_rng(5)
+    logits = (rng.standard_normal((B, V)) * 3).astype(np.float32)
+    masked = np.full((B, V), -np.inf, np.float32)
+    masked[:, :20] = logits[:, :20]
+    pen, probs, picked = (hip.DeviceArray.zeros(s, d) for s, d in (((B, V), np.float32), ((B, V), np.float32), ((B,), np.int32)))
+    best = []
+    for rows in (logits, masked):
+        d = hip.DeviceArray.from_numpy(rows)
+        start, stop = hip.Event(), hip.Event()
+        us = []
+        for _ in range(8):
+            start.record()
+            for step in range(20):
+                hip.sample(B, V, d, pen, probs, picked, presence=0.5, frequency=0.1, decay=0.99, top_k=50, top_p=0.6, step=step)
+            stop.record()
+            hip.device_sync()
+            us.append(start.elapsed_ms(stop) * 50)
+        best.append(min(us))
+    print("unmasked %.1f us, masked %.1f us" % tuple(best))
+    assert best[1] <= 1.5 * best[0]
+
+
 @pytest.mark.parametrize("kind", ["normal", "ties", "equal"])
 @pytest.mark.parametrize("V,top_k,top_p", [(4, 0, 0.5), (256, 0, 0.5), (260, 0, 0.9), (1028, 700, 0.8), (40004, 0, 0.3),
                                           (65536, 0, 0.9), (65536, 500, 1.0), (65536, 65535, 1.0)])
