@@ -615,22 +615,46 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
   return best;
 }
 
-// The formats are not known here, nor whether a consumer sums the planes: the largest that any of the choices would need.
-size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const int* Ns) {
-  int64_t n_total = 0;
-  for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
-  int fmts[kMaxProblems];
+// Neither the format is known here nor the epilogue: the largest that any of the choices would need.
+size_t linear_packed_workspace_bytes(int M, int N, int K) {
   int splits = 1;
-  for (int mix = 0; mix < 5; ++mix) {  // one format, or int8 / int4 problems with fp16 ones behind them
-    const int first = mix == 0 || mix == 3 ? RWKV_FMT_W8 : (mix == 1 || mix == 4 ? RWKV_FMT_W4 : RWKV_FMT_F16);
-    for (int i = 0; i < n_problems && i < kMaxProblems; ++i) fmts[i] = mix >= 3 && i >= std::min(3, n_problems - 1) ? RWKV_FMT_F16 : first;
-    for (const bool deferred : {false, true})
-      splits = std::max(splits, choose_config(M, K, n_problems, Ns, fmts, deferred, 32).splits);
-  }
-  return splits > 1 ? static_cast<size_t>(splits) * M * n_total * sizeof(float) : 0;
+  for (const int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16})
+    for (const bool deferred : {false, true}) splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, deferred, 32).splits);
+  return splits > 1 ? static_cast<size_t>(splits) * M * N * sizeof(float) : 0;
 }
 
-size_t linear_packed_workspace_bytes(int M, int N, int K) { return linear_packed_multi_workspace_bytes(M, K, 1, &N); }
+// int8 and int4 matrices side by side have no launch in common: f is called with the problems of each format.
+template <typename F>
+static int for_each_launch(int n_problems, const PackedProblem* problems, F&& f) {
+  bool any[3] = {false, false, false};
+  for (int i = 0; i < n_problems; ++i) any[problems[i].fmt] = true;
+  if (!(any[RWKV_FMT_W8] && any[RWKV_FMT_W4])) return f(n_problems, problems);
+  for (const int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16}) {
+    PackedProblem part[kMaxProblems];
+    int n = 0;
+    for (int i = 0; i < n_problems; ++i)
+      if (problems[i].fmt == fmt) part[n++] = problems[i];
+    const int rc = n > 0 ? f(n, part) : RWKV_OK;
+    if (rc != RWKV_OK) return rc;
+  }
+  return RWKV_OK;
+}
+
+size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32) {
+  size_t bytes = 0;
+  for_each_launch(n_problems, problems, [&](int n, const PackedProblem* part) -> int {
+    int Ns[kMaxProblems], fmts[kMaxProblems];
+    int64_t n_total = 0;
+    for (int i = 0; i < n; ++i) {
+      n_total += Ns[i] = part[i].N;
+      fmts[i] = part[i].fmt;
+    }
+    const int splits = choose_config(M, K, n, Ns, fmts, sums_at_consumer(n, epilogue, out_f32), 32).splits;
+    if (splits > 1) bytes = std::max(bytes, static_cast<size_t>(splits) * M * n_total * sizeof(float));
+    return RWKV_OK;
+  });
+  return bytes;
+}
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
                          void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy, bool fit_splits);
@@ -639,27 +663,16 @@ int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const Pack
                         int out_f32, void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy) {
   RWKV_REQUIRE(n_problems >= 1 && n_problems <= kMaxProblems, "linear_packed: %d problems (1..%d allowed)", n_problems,
                kMaxProblems);
-  bool any[3] = {false, false, false};
-  for (int i = 0; i < n_problems; ++i) {
+  for (int i = 0; i < n_problems; ++i)
     RWKV_REQUIRE(linear_packed_supported(problems[i].fmt, M, problems[i].N, K), "linear_packed: unsupported shape M=%d N=%d K=%d fmt=%d",
                  M, problems[i].N, K, problems[i].fmt);
-    any[problems[i].fmt] = true;
-  }
-  if (!(any[RWKV_FMT_W8] && any[RWKV_FMT_W4]))
-    return packed_launch(st, M, K, n_problems, problems, epilogue, out_f32, workspace, workspace_bytes, defer, copy, n_problems > 1);
-  // int8 and int4 matrices side by side have no launch in common: one per format.  (fit_splits: formats may come in any mix, the
-  // workspace was sized without knowing it: no more K splits than fit)
-  for (const int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16}) {
-    PackedProblem part[kMaxProblems];
-    int n = 0;
-    for (int i = 0; i < n_problems; ++i)
-      if (problems[i].fmt == fmt) part[n++] = problems[i];
-    if (n == 0) continue;
-    const int rc = packed_launch(st, M, K, n, part, epilogue, out_f32, workspace, workspace_bytes, nullptr, copy, true);
-    if (rc != RWKV_OK) return rc;
-    copy = nullptr;
-  }
-  return RWKV_OK;
+  return for_each_launch(n_problems, problems, [&](int n, const PackedProblem* part) {
+    // (several problems take no more K splits than fit the workspace)
+    const int rc = packed_launch(st, M, K, n, part, epilogue, out_f32, workspace, workspace_bytes, n == n_problems ? defer : nullptr,
+                                 copy, n_problems > 1);
+    copy = nullptr;  // the rows ride on the first launch
+    return rc;
+  });
 }
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,

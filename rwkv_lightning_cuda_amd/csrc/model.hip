@@ -196,6 +196,77 @@ int model_ready(const rwkv_hip_model* m) {
   return RWKV_OK;
 }
 
+// The launch of the three projections and the rank-ins of a layer (ranks: w, a, g and, past layer 0, v) in its packed form: how
+// many problems, 0 if a matrix has no packed copy; x and y stay NULL.
+int packed_projections(const rwkv_hip_model* m, int layer, PackedProblem* p) {
+  const Layer& w = m->layers[layer];
+  const int mids[3] = {RWKV_M_ATT_R, RWKV_M_ATT_K, RWKV_M_ATT_V};
+  const int ranks[4] = {m->Rw, m->Ra, m->Rg, m->Rv};
+  const int n_lora = layer == 0 ? 3 : 4;
+  bool all = true;
+  for (int i = 0; i < 3; ++i) {
+    p[i] = w.m[mids[i]].packed_problem(m->C, nullptr, nullptr);
+    all = all && p[i].packed != nullptr;
+  }
+  for (int i = 0; i < n_lora; ++i) {
+    p[3 + i] = PackedProblem{w.lora_in_packed[i], nullptr, nullptr, nullptr, nullptr, ranks[i], RWKV_FMT_F16};
+    all = all && p[3 + i].packed != nullptr;
+  }
+  return all ? 3 + n_lora : 0;
+}
+
+// Where a launch of int8 problems only has a tile of its own (several wavefronts per SIMD), three int8 projections go without
+// the fp16 rank-ins, which follow in a launch of their own.
+bool projections_apart(const PackedProblem* p, int rows, int C) {
+  bool apart = linear_packed_int8_tile(rows, C);
+  for (int i = 0; i < 3; ++i) apart = apart && p[i].fmt == RWKV_FMT_W8;
+  return apart;
+}
+
+// What the packed launches of a forward call of `rows` rows (B sequences) keep their K splits in: exactly what they ask for, from
+// the formats the layers have - a workspace that only bounds it would let a launch of several problems take the split that fits
+// what an earlier, larger call of the session has left, and its sums depend on that call.
+size_t packed_workspace_bytes(const rwkv_hip_model* m, int B, int rows) {
+  const int C = m->C, F = m->F;
+  size_t ws = 0;
+  auto ask = [&](int M, int K, int n, const PackedProblem* p, int epilogue, int out_f32) {
+    ws = std::max(ws, linear_packed_multi_workspace_bytes(M, K, n, p, epilogue, out_f32));
+  };
+  auto ask_matrix = [&](const Matrix& mat, int M, int N, int K, int epilogue, int out_f32) {
+    if (!mat.packed) return;
+    const PackedProblem p = mat.packed_problem(N, nullptr, nullptr);
+    ask(M, K, 1, &p, epilogue, out_f32);
+  };
+  auto formats = [&](int l) {  // of the launches of a layer
+    unsigned f = l == 0 ? 1u : 2u;
+    for (const Matrix& mat : m->layers[l].m) f = f * 4 + (mat.packed ? static_cast<unsigned>(mat.fmt) : 3u);
+    for (const void* rank_in : m->layers[l].lora_in_packed) f = f * 2 + (rank_in ? 1u : 0u);
+    return f;
+  };
+  unsigned done = ~0u;
+  for (int l = 0; l < m->L; ++l) {
+    const unsigned f = formats(l);
+    if (f == done) continue;
+    done = f;
+    const Layer& w = m->layers[l];
+    PackedProblem p[7];
+    const int n = packed_projections(m, l, p);
+    if (n == 0) {
+      for (const int id : {RWKV_M_ATT_R, RWKV_M_ATT_K, RWKV_M_ATT_V}) ask_matrix(w.m[id], rows, C, C, RWKV_EPI_NONE, 0);
+    } else if (projections_apart(p, rows, C)) {
+      ask(rows, C, 3, p, RWKV_EPI_NONE, 0);
+      ask(rows, C, n - 3, p + 3, RWKV_EPI_NONE, 0);
+    } else {
+      ask(rows, C, n, p, RWKV_EPI_NONE, 0);
+    }
+    ask_matrix(w.m[RWKV_M_ATT_O], rows, C, C, RWKV_EPI_NONE, 0);
+    ask_matrix(w.m[RWKV_M_FFN_KEY], rows, F, C, RWKV_EPI_RELU_SQUARE, 0);
+    ask_matrix(w.m[RWKV_M_FFN_VALUE], rows, C, F, RWKV_EPI_NONE, 0);
+  }
+  ask_matrix(m->head, B, m->V, C, RWKV_EPI_NONE, 1);
+  return ws;
+}
+
 int ensure_arena(rwkv_hip_session* s, int B, int T) {
   const rwkv_hip_model* m = s->model;
   const size_t rows = static_cast<size_t>(B) * T;
@@ -258,18 +329,7 @@ int ensure_arena(rwkv_hip_session* s, int B, int T) {
   // (from the smallest row count that any matrix takes through its packed copy: ffn.value's rows are too long for
   // the few-row launches)
   if (rows >= static_cast<size_t>(kPackedMinRows)) {
-    const int R = static_cast<int>(rows);
-    const int qkv_ns[7] = {m->C, m->C, m->C, m->Rw, m->Ra, m->Rg, m->Rv};
-    size_t ws = std::max(linear_packed_multi_workspace_bytes(R, m->C, 7, qkv_ns),
-                         linear_packed_multi_workspace_bytes(R, m->C, 6, qkv_ns));  // layer 0 has no v rank-in
-    // (the same launch in two parts: the projections, then the rank-ins)
-    ws = std::max(ws, linear_packed_multi_workspace_bytes(R, m->C, 3, qkv_ns));
-    ws = std::max(ws, linear_packed_multi_workspace_bytes(R, m->C, 4, qkv_ns + 3));
-    ws = std::max(ws, linear_packed_multi_workspace_bytes(R, m->C, 3, qkv_ns + 3));
-    ws = std::max(ws, linear_packed_workspace_bytes(R, m->C, m->C));
-    ws = std::max(ws, linear_packed_workspace_bytes(R, m->F, m->C));
-    ws = std::max(ws, linear_packed_workspace_bytes(R, m->C, m->F));
-    ws = std::max(ws, linear_packed_workspace_bytes(B, m->V, m->C));
+    const size_t ws = packed_workspace_bytes(m, B, static_cast<int>(rows));
     if (ws > s->gemm_ws_bytes) {
       for (auto& g : s->graphs) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
@@ -535,23 +595,20 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
           TRY_PROF(linear_small_m(st, rows, C, 3 + n_lora, p, RWKV_EPI_NONE, 0));
         }
       } else {
-        bool all_packed = rows >= packed_min_rows(m);
-        for (int i = 0; i < 3; ++i) all_packed = all_packed && w.m[mids[i]].packed != nullptr;
-        for (int i = 0; i < n_lora; ++i) all_packed = all_packed && w.lora_in_packed[i] != nullptr;
-        if (all_packed) {
+        PackedProblem p[7];
+        if (rows >= packed_min_rows(m) && packed_projections(m, l, p) > 0) {
           // one streaming-GEMM launch (+ one split-K reduce) for the three projections and the rank-ins
-          PackedProblem p[7];
-          for (int i = 0; i < 3; ++i)
-            p[i] = w.m[mids[i]].packed_problem(C, xs[i], ys[i]);
-          for (int i = 0; i < n_lora; ++i)
-            p[3 + i] = PackedProblem{w.lora_in_packed[i], nullptr, nullptr, lx[i], lh[i], ranks[i], RWKV_FMT_F16};
-          // Where a launch of int8 problems only has a tile of its own (several wavefronts per SIMD), three int8
-          // projections go without the fp16 rank-ins, which follow in a launch of their own.
-          bool w8_only = linear_packed_int8_tile(rows, C);
-          for (int i = 0; i < 3; ++i) w8_only = w8_only && p[i].fmt == RWKV_FMT_W8;
+          for (int i = 0; i < 3; ++i) {
+            p[i].x = xs[i];
+            p[i].y = ys[i];
+          }
+          for (int i = 0; i < n_lora; ++i) {
+            p[3 + i].x = lx[i];
+            p[3 + i].y = lh[i];
+          }
           const RowCopy moved = pending;
           pending = RowCopy{};
-          if (w8_only) {
+          if (projections_apart(p, rows, C)) {
             TRY_PROF(linear_packed_multi(st, rows, C, 3, p, RWKV_EPI_NONE, 0, s->gemm_ws, s->gemm_ws_bytes, nullptr, &moved));
             TRY_PROF(linear_packed_multi(st, rows, C, n_lora, p + 3, RWKV_EPI_NONE, 0, s->gemm_ws, s->gemm_ws_bytes));
           } else {

@@ -101,7 +101,8 @@ struct PackedProblem {
 // Row counts and K at which a launch of int8 problems only gets a tile of its own (several wavefronts per SIMD):
 // callers with int8 and fp16 problems for one launch do better with two launches there.
 bool linear_packed_int8_tile(int M, int K);
-size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const int* Ns);
+// Exactly what linear_packed_multi takes for these problems (their N, format and layout; the pointers are not looked at).
+size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32);
 int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue,
                         int out_f32, void* workspace, size_t workspace_bytes, DeferredReduce* defer = nullptr,
                         const RowCopy* copy = nullptr);  // copy: rows moved by the launch's first block (n % 8 == 0)

@@ -162,6 +162,37 @@ def test_matrices_of_different_formats_side_by_side(gpu):
     assert cos >= 0.9995
 
 
+@pytest.mark.parametrize("C,F,projections,rows,before", [(2048, 8192, ("w8", "f16", "f16"), 327, 513),
+                                                         (4096, 4096, ("w4", "w8", "f16"), 18, 19)])
+def test_a_call_does_not_depend_on_what_the_session_ran_before(gpu, C, F, projections, rows, before):
+    """Projections of different formats: their launches of several products take a K split where the workspace has room for its
+    planes.  The same call in a fresh session and behind a longer one, which leaves a larger workspace, bit by bit."""
+    from rwkv_lightning_cuda_amd.model import DeviceMatrix, HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    ranks = dict(Rw=96, Ra=96, Rg=256, Rv=64) if C == 2048 else dict(Rw=32, Ra=32, Rg=64, Rv=32)
+    dims = ModelDims(L=1, C=C, H=C // 64, F=F, V=512, **ranks)
+    weights = synth_weights(dims, 3)
+    model = HipModel.from_host_weights(dims, weights, hip.FMT_F16)
+    fmts = {"f16": hip.FMT_F16, "w8": hip.FMT_W8, "w4": hip.FMT_W4}
+    for (name, mid), fmt in zip((("att_r", hip.M_ATT_R), ("att_k", hip.M_ATT_K), ("att_v", hip.M_ATT_V)), projections):
+        w = hip.DeviceArray.from_numpy(weights["layers"][0][name])
+        model.set_matrix(0, mid, DeviceMatrix.from_f16_device(fmts[fmt], C, C, w))
+    rng = np.random.default_rng(2)
+    tokens, longer = rng.integers(0, dims.V, (1, rows)), rng.integers(0, dims.V, (1, before))
+    out = []
+    for first in (None, longer):
+        sess = Session(model)
+        lg = hip.DeviceArray((1, dims.V), np.float32)
+        if first is not None:
+            sess.forward(first, State(dims, 1), lg)
+        st = State(dims, 1)
+        sess.forward(tokens, st, lg)
+        out.append((lg.numpy().view(np.uint32), st.wkv.numpy().view(np.uint32), st.shift.numpy().view(np.uint16)))
+        sess.close()
+    for name, a, b in zip(("logits", "wkv", "shift"), *out):
+        assert np.array_equal(a, b), name
+
+
 @pytest.mark.parametrize("F,projections", [(256, ("w8", "w8", "w8")), (1024, ("w8", "w4", "w4")), (448, ("w4", "w4", "w4"))])
 def test_shift_rows_that_ride_on_a_launch_of_few_blocks(gpu, F, projections):
     """The new shift rows of a short chunk move into the state with the next packed launch.  40 sequences of 256 channels are
