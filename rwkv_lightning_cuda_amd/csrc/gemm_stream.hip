@@ -567,8 +567,9 @@ static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, co
   return us;
 }
 
-// Whether the planes of a K split may be left to the launch's consumer.  The choice of tile and split goes by this alone and
-// not by whether this call leaves them: a product has the same sums either way.
+// Whether the planes of a K split may be left to the launch's consumer.  Inside a model the choice of tile and split goes by this
+// alone and not by whether this call leaves them: a product has the same sums either way.  (linear_packed has no consumer and
+// goes by the reduce launch it pays for.)
 static bool sums_at_consumer(int n_problems, int epilogue, int out_f32) {
   return n_problems == 1 && epilogue == RWKV_EPI_NONE && !out_f32;
 }
@@ -646,11 +647,11 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
   return e.config;
 }
 
-// Neither the format is known here nor the epilogue: the largest that any of the choices would need.
+// The format is not known here: the largest that any of the choices would need.
 size_t linear_packed_workspace_bytes(int M, int N, int K) {
   int splits = 1;
   for (const int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16})
-    for (const bool deferred : {false, true}) splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, deferred, 32).splits);
+    splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, false, 32).splits);
   return splits > 1 ? static_cast<size_t>(splits) * M * N * sizeof(float) : 0;
 }
 
@@ -688,26 +689,33 @@ size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const P
 }
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
-                         void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy, bool fit_splits);
+                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer,
+                         DeferredReduce* defer, const RowCopy* copy);
 
-int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue,
-                        int out_f32, void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy) {
+static int require_supported(int M, int K, int n_problems, const PackedProblem* problems) {
   RWKV_REQUIRE(n_problems >= 1 && n_problems <= kMaxProblems, "linear_packed: %d problems (1..%d allowed)", n_problems,
                kMaxProblems);
   for (int i = 0; i < n_problems; ++i)
     RWKV_REQUIRE(linear_packed_supported(problems[i].fmt, M, problems[i].N, K), "linear_packed: unsupported shape M=%d N=%d K=%d fmt=%d",
                  M, problems[i].N, K, problems[i].fmt);
+  return RWKV_OK;
+}
+
+int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue,
+                        int out_f32, void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy) {
+  if (const int rc = require_supported(M, K, n_problems, problems)) return rc;
   return for_each_launch(n_problems, problems, [&](int n, const PackedProblem* part) {
     // (several problems take no more K splits than fit the workspace)
-    const int rc = packed_launch(st, M, K, n, part, epilogue, out_f32, workspace, workspace_bytes, n == n_problems ? defer : nullptr,
-                                 copy, n_problems > 1);
+    const int rc = packed_launch(st, M, K, n, part, epilogue, out_f32, workspace, workspace_bytes, n_problems > 1,
+                                 sums_at_consumer(n, epilogue, out_f32), n == n_problems ? defer : nullptr, copy);
     copy = nullptr;  // the rows ride on the first launch
     return rc;
   });
 }
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
-                         void* workspace, size_t workspace_bytes, DeferredReduce* defer, const RowCopy* copy, bool fit_splits) {
+                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, DeferredReduce* defer,
+                         const RowCopy* copy) {
   StreamArgs g;
   ReduceArgs r;
   if (copy) {
@@ -732,7 +740,7 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
   // fits.  Elsewhere a workspace too small for the split is an error.
   fit_splits = fit_splits || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 || static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
   const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace ? workspace_bytes / plane : 0)) : 32;
-  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, sums_at_consumer(n_problems, epilogue, out_f32), max_splits);
+  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, at_consumer, max_splits);
   int col_blocks = 0;
   for (int i = 0; i < n_problems; ++i) {
     const PackedProblem& q = problems[i];
@@ -795,10 +803,10 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
 }
 
 int linear_packed(hipStream_t st, int fmt, int M, int N, int K, const half_t* x, const void* packed, const half_t* scale,
-                  const uint8_t* zp, int epilogue, int out_f32, void* y, void* workspace, size_t workspace_bytes,
-                  DeferredReduce* defer, const RowCopy* copy) {
+                  const uint8_t* zp, int epilogue, int out_f32, void* y, void* workspace, size_t workspace_bytes) {
   const PackedProblem q = {packed, scale, zp, x, y, N, fmt};
-  return linear_packed_multi(st, M, K, 1, &q, epilogue, out_f32, workspace, workspace_bytes, defer, copy);
+  if (const int rc = require_supported(M, K, 1, &q)) return rc;
+  return packed_launch(st, M, K, 1, &q, epilogue, out_f32, workspace, workspace_bytes, false, false, nullptr, nullptr);
 }
 
 }  // namespace rwkv

@@ -81,12 +81,10 @@ struct DeferredReduce {
 int pack_weights_launch(hipStream_t st, int fmt, int N, int K, const void* w, void* packed);
 // int4 scales and zero points [N][groups] -> [groups][N]
 int transpose_groups_launch(hipStream_t st, int N, int groups, const half_t* scale, const uint8_t* zp, half_t* scale_t, uint8_t* zp_t);
-// Workspace for one call: fp32 split-K partials (0 when the shape needs no split).
+// Workspace for one call of linear_packed: fp32 split-K partials (0 when the shape needs no split).
 size_t linear_packed_workspace_bytes(int M, int N, int K);
-// defer (single problem, fp16 output, no epilogue): the consumer sums the partials instead of a reduce launch.
 int linear_packed(hipStream_t st, int fmt, int M, int N, int K, const half_t* x, const void* packed, const half_t* scale,
-                  const uint8_t* zp, int epilogue, int out_f32, void* y, void* workspace, size_t workspace_bytes,
-                  DeferredReduce* defer = nullptr, const RowCopy* copy = nullptr);
+                  const uint8_t* zp, int epilogue, int out_f32, void* y, void* workspace, size_t workspace_bytes);
 // Up to kMaxProblems products sharing M and K (own weights, format, x, y each) in one launch (+ one reduce launch).
 struct PackedProblem {
   const void* packed;
@@ -103,6 +101,7 @@ struct PackedProblem {
 bool linear_packed_int8_tile(int M, int K);
 // Exactly what linear_packed_multi takes for these problems (their N, format and layout; the pointers are not looked at).
 size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32);
+// defer (single problem, fp16 output, no epilogue): the consumer sums the partials instead of a reduce launch.
 int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue,
                         int out_f32, void* workspace, size_t workspace_bytes, DeferredReduce* defer = nullptr,
                         const RowCopy* copy = nullptr);  // copy: rows moved by the launch's first block (n % 8 == 0)

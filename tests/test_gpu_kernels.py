@@ -985,6 +985,27 @@ def test_linear_packed_of_33_to_64_rows_without_a_workspace(gpu, orc, fmt_name, 
     assert err <= F16_TOL
 
 
+@pytest.mark.parametrize("fmt_name", ["f16", "w8", "w4"])
+@pytest.mark.parametrize("M,N,K", [(8, 2048, 2048), (13, 4096, 4096), (33, 768, 3072), (129, 4096, 4096)])
+def test_linear_packed_gives_one_product_for_both_output_types(gpu, orc, fmt_name, M, N, K):
+    """The operator pays for the reduce launch of a K split whatever the type of its output: both types take the same split, so
+    the same sums (to fp16 outputs it once took the splits that pay only where a LayerNorm kernel adds the planes up)."""
+    hip = gpu
+    rng = np.random.default_rng(M + N + K)
+    fmt = {"f16": hip.FMT_F16, "w8": hip.FMT_W8, "w4": hip.FMT_W4}[fmt_name]
+    x = dev(hip, rng.standard_normal((M, K)).astype(np.float16))
+    parts = _quant_parts(orc, hip, fmt, (rng.standard_normal((N, K)) * 0.02).astype(np.float16))
+    dparts = [dev(hip, p) if p is not None else None for p in parts]
+    packed = hip.DeviceArray(parts[0].shape, parts[0].dtype)
+    hip.pack_weights(fmt, N, K, dparts[0], packed)
+    ws = hip.DeviceArray((max(hip.linear_packed_workspace(M, N, K), 16),), np.uint8)
+    y16, y32 = hip.DeviceArray((M, N), np.float16), hip.DeviceArray((M, N), np.float32)
+    hip.linear_packed(fmt, M, N, K, x, packed, dparts[1], dparts[2], y16, ws)
+    hip.linear_packed(fmt, M, N, K, x, packed, dparts[1], dparts[2], y32, ws, out_f32=1)
+    hip.device_sync()
+    assert np.array_equal(y16.numpy(), y32.numpy().astype(np.float16))
+
+
 def test_pack_weights_is_the_documented_permutation(gpu):
     """Tile (band nt, k group kg) holds, for lane j + 32h, the KR consecutive k of row 32 nt + j starting at
     kg*G + h*KR, as 64 x 16-byte pieces (two pieces for fp16)."""
