@@ -543,7 +543,11 @@ static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, co
     n_total += Ns[i];
   }
   const float k_block = static_cast<float>(K) / c.splits;
-  blocks *= ceil_div(M, bm) * c.splits;
+  blocks *= c.splits;
+  // (each eighth pair of column block and split goes to the same XCD, whose 32 CUs run all its row tiles: twelve pairs of 18
+  // row tiles leave four XCDs with 36 blocks.  Launches of several problems have too many pairs for it to matter.)
+  if (n_problems == 1) blocks = ceil_div(blocks, 8) * 8;
+  blocks *= ceil_div(M, bm);
   block_bytes *= k_block;
   w_bytes *= static_cast<float>(K);
   const int full = blocks / kCus, rest = blocks % kCus;
@@ -556,7 +560,7 @@ static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, co
     const float gflop = 2e-9f * bm * bn_max * k_block * kCus;
     const bool two_per_cu = c.ring.mt == 1 && c.ring.kc == 128;
     const bool wide_ring = c.ring.mt == 4 || c.ring.wp == 4;
-    us += rounds * gflop * (c.fmt == RWKV_FMT_W4 ? (wide_ring ? 0.73f : 0.57f) : (c.ring.mt == 4 && c.fmt == RWKV_FMT_W8 ? 0.55f : (c.ring.nb == 2 ? 0.38f : 0.28f)));
+    us += rounds * gflop * (c.fmt == RWKV_FMT_W4 ? (wide_ring ? 0.73f : 0.57f) : (c.ring.mt == 4 && c.fmt == RWKV_FMT_W8 ? 0.55f : (c.ring.nb == 2 ? 0.37f : (c.ring.mt == 1 && c.ring.wp == 4 ? 0.30f : 0.28f))));
     us += (two_per_cu ? 1.5f : 4.5f) * (rounds - 1);
   } else if (c.wide_mt == 2) {
     us = 7.0f + 34.0f * std::max(1.0f, blocks * 1.05f / kCus) * k_block / 4096.0f;
@@ -735,10 +739,10 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
   int64_t n_total = 0;
   for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
   const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
-  // A split is an offer, not a need, where blocks of 32 x 32 alone occupy the chip or K has no power of two of whole 512s
-  // (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a workspace too, with the split that
-  // fits.  Elsewhere a workspace too small for the split is an error.
-  fit_splits = fit_splits || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 || static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
+  // A split is an offer, not a need, from 513 rows on, where blocks of 32 x 32 alone occupy the chip and where K has no power of
+  // two of whole 512s (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a workspace too, with
+  // the split that fits.  Elsewhere a workspace too small for the split is an error.
+  fit_splits = fit_splits || M > 512 || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 || static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
   const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace ? workspace_bytes / plane : 0)) : 32;
   const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, at_consumer, max_splits);
   int col_blocks = 0;
