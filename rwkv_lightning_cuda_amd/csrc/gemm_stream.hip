@@ -528,7 +528,10 @@ static int count_col_blocks(const StreamConfig& c, int n_problems, const int* Ns
 //   wide: bound by the matrix core (1 PFLOP/s with the shader clock these products run at).
 //   K splits: their fp32 planes and, where no consumer sums them, the reduce launch; a consumer's block waits longer the more
 //   planes it asks for (0.15 us each; with 0 / 0.4 decode steps of 5 .. 16 rows are 1-4 % slower, 7.2B and 1.5B int8).
-static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred) {
+//   int4 scales and zero points as [N][K/128] (group_rows): a cache line each per column and stage, of which the stage uses a few
+//   bytes.  Two bytes per code of what a CU takes in, 1.5 with stages of 256 k; up to 2048 k a column's lie in 48 bytes.
+static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred,
+                         bool group_rows) {
   constexpr int kCus = 256;
   const int bm = c.rows();
   int blocks = 0, bn_max = 0;
@@ -537,7 +540,8 @@ static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, co
     const int bn = c.cols(fmts[i]);
     const float per = fmts[i] == RWKV_FMT_F16 ? 2.0f : (fmts[i] == RWKV_FMT_W8 ? 1.0f : 0.55f);
     blocks += ceil_div(Ns[i], bn);
-    block_bytes = std::max(block_bytes, bn * per + bm * 2.0f);
+    const float lines = group_rows && K > 2048 && fmts[i] == RWKV_FMT_W4 ? (c.k_step() == 128 ? 2.0f : 1.5f) : 0.0f;
+    block_bytes = std::max(block_bytes, bn * (per + lines) + bm * 2.0f);
     bn_max = std::max(bn_max, bn);
     w_bytes += per * Ns[i];
     n_total += Ns[i];
@@ -585,14 +589,15 @@ constexpr int kWideMinRows = 160;
 // Launches of int8 problems only have a wide tile of their own at these sizes (three blocks per CU).
 bool linear_packed_int8_tile(int M, int K) { return M > 512 && M <= 1024 && K <= 4096 && K > 2048; }
 
-static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, int max_splits) {
+static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, bool group_rows,
+                                  int max_splits) {
   bool any[3] = {false, false, false};
   for (int i = 0; i < n_problems; ++i) any[fmts[i]] = true;
   StreamConfig best;
   float best_us = 1e30f;
   auto consider = [&](StreamConfig c) {
     for (c.splits = 1; c.splits == 1 || (c.splits <= max_splits && K % (c.splits * c.k_step()) == 0); c.splits *= 2) {
-      const float us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred);
+      const float us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred, group_rows);
       if (us < best_us) {
         best_us = us;
         best = c;
@@ -624,7 +629,8 @@ static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, c
 // The search over tiles and splits takes 1 to 6 us of host time, and a decode step asks for about ten choices before its first
 // launch: each thread keeps the latest by all that they depend on (us per step, searching / kept: 1.5B shape fp16 4 rows
 // 1270 / 1236, int8 13 rows 1189 / 1158; 7.2B shape int8 8 rows 2239 / 2198; 0.1B shape fp16 8 rows 460 / 447).
-static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, int max_splits) {
+static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, bool group_rows,
+                                  int max_splits) {
   struct Entry {
     int key[5 + 2 * kMaxProblems];
     bool used;
@@ -633,7 +639,7 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
   constexpr unsigned kSets = 32, kWays = 4;
   static thread_local Entry table[kSets][kWays];
   static thread_local unsigned oldest[kSets];
-  int key[5 + 2 * kMaxProblems] = {M, K, n_problems, deferred ? 1 : 0, max_splits};
+  int key[5 + 2 * kMaxProblems] = {M, K, n_problems, (deferred ? 1 : 0) + (group_rows ? 2 : 0), max_splits};
   for (int i = 0; i < n_problems; ++i) {
     key[5 + 2 * i] = Ns[i];
     key[6 + 2 * i] = fmts[i];
@@ -645,7 +651,7 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
     if (e.used && memcmp(e.key, key, sizeof key) == 0) return e.config;
   Entry& e = table[set][oldest[set]];
   oldest[set] = (oldest[set] + 1) % kWays;
-  e.config = search_config(M, K, n_problems, Ns, fmts, deferred, max_splits);
+  e.config = search_config(M, K, n_problems, Ns, fmts, deferred, group_rows, max_splits);
   memcpy(e.key, key, sizeof key);
   e.used = true;
   return e.config;
@@ -655,7 +661,7 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
 size_t linear_packed_workspace_bytes(int M, int N, int K) {
   int splits = 1;
   for (const int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16})
-    splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, false, 32).splits);
+    splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, false, fmt == RWKV_FMT_W4, 32).splits);
   return splits > 1 ? static_cast<size_t>(splits) * M * N * sizeof(float) : 0;
 }
 
@@ -681,11 +687,13 @@ size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const P
   for_each_launch(n_problems, problems, [&](int n, const PackedProblem* part) -> int {
     int Ns[kMaxProblems], fmts[kMaxProblems];
     int64_t n_total = 0;
+    bool group_rows = false;
     for (int i = 0; i < n; ++i) {
       n_total += Ns[i] = part[i].N;
       fmts[i] = part[i].fmt;
+      group_rows = group_rows || (fmts[i] == RWKV_FMT_W4 && !part[i].groups_first);
     }
-    const int splits = choose_config(M, K, n, Ns, fmts, sums_at_consumer(n, epilogue, out_f32), 32).splits;
+    const int splits = choose_config(M, K, n, Ns, fmts, sums_at_consumer(n, epilogue, out_f32), group_rows, 32).splits;
     if (splits > 1) bytes = std::max(bytes, static_cast<size_t>(splits) * M * n_total * sizeof(float));
     return RWKV_OK;
   });
@@ -732,19 +740,21 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
   g.epilogue = r.epilogue = epilogue;
   g.out_f32 = r.out_f32 = out_f32;
   int Ns[kMaxProblems], fmts[kMaxProblems];
-  for (int i = 0; i < n_problems; ++i) {
-    Ns[i] = problems[i].N;
-    fmts[i] = problems[i].fmt;
-  }
   int64_t n_total = 0;
-  for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
+  bool group_rows = false;
+  for (int i = 0; i < n_problems; ++i) {
+    n_total += Ns[i] = problems[i].N;
+    fmts[i] = problems[i].fmt;
+    group_rows = group_rows || (fmts[i] == RWKV_FMT_W4 && !problems[i].groups_first);
+  }
   const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
-  // A split is an offer, not a need, from 513 rows on, where blocks of 32 x 32 alone occupy the chip and where K has no power of
-  // two of whole 512s (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a workspace too, with
-  // the split that fits.  Elsewhere a workspace too small for the split is an error.
-  fit_splits = fit_splits || M > 512 || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 || static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
+  // A split is an offer, not a need, for int4 codes, from 513 rows on, where blocks of 32 x 32 alone occupy the chip and where K
+  // has no power of two of whole 512s (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a
+  // workspace too, with the split that fits.  Elsewhere a workspace too small for the split is an error.
+  fit_splits = fit_splits || fmts[0] == RWKV_FMT_W4 || M > 512 || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 ||
+               static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
   const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace ? workspace_bytes / plane : 0)) : 32;
-  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, at_consumer, max_splits);
+  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, max_splits);
   int col_blocks = 0;
   for (int i = 0; i < n_problems; ++i) {
     const PackedProblem& q = problems[i];

@@ -1006,10 +1006,13 @@ def test_linear_packed_gives_one_product_for_both_output_types(gpu, orc, fmt_nam
     assert np.array_equal(y16.numpy(), y32.numpy().astype(np.float16))
 
 
-@pytest.mark.parametrize("fmt_name,N,K,fewer,more", [("f16", 768, 3072, 1152, 1536), ("w8", 768, 3072, 1152, 1536)])
+@pytest.mark.parametrize("fmt_name,N,K,fewer,more", [("f16", 768, 3072, 1152, 1536), ("w8", 768, 3072, 1152, 1536),
+                                                     ("w4", 4096, 16384, 96, 128), ("w4", 4096, 16384, 352, 448),
+                                                     ("w4", 4096, 16384, 640, 1024)])
 def test_linear_packed_of_fewer_rows_takes_no_longer(gpu, fmt_name, N, K, fewer, more):
-    """The tile and split of a call are chosen by estimate.  Where the estimate missed the XCDs' uneven share of the blocks,
-    1152 rows took 1.2 times as long as 1536.  (A bar of 1.15: neighbouring tiles' own steps.)"""
+    """The tile and split of a call are chosen by estimate.  Where the estimate missed the XCDs' uneven share of the blocks or the
+    cache lines of int4 scales in rows, 1152 rows took 1.2 times as long as 1536, 640 rows 1.6 times as long as 1024.  (A bar of
+    1.15: neighbouring tiles' own steps.)"""
     hip = gpu
     rng = np.random.default_rng(N + K)
     fmt, per = {"f16": (hip.FMT_F16, 2), "w8": (hip.FMT_W8, 1), "w4": (hip.FMT_W4, 0.5)}[fmt_name]
