@@ -892,17 +892,18 @@ def test_decode_step_with_layernorm_folded_into_linear_matches_the_unfused_step(
 
 @pytest.mark.parametrize("B,C", [(5, 1024), (8, 1024), (7, 2048), (8, 4096), (12, 1024)])
 def test_decode_step_of_five_to_eight_rows_folds_layernorm_into_the_few_row_launch(gpu, B, C):
-    """Decode steps of 5 to 8 rows run their int8 and fp16 products with rows of 1024 .. 4096 values on the few-row
-    matrix-core launch, and by default fold LN2 + its token shift into the ffn.key launch: a staging wavefront per row
-    computes LayerNorm with the stand-alone kernel's formulas and rounding points (sums associated differently), so
-    the step agrees with the one through the stand-alone kernels to fp16 rounding (logits and shift rows within 2e-3
-    of their scale, WKV state within 1e-3).  The same bars with LN1 folded as well (forced: the r/k/v launch, with
-    layer 0 gathering its embedding rows itself; the ffn.value product is then reduced by a launch of its own
-    instead of by the LayerNorm kernel).  Twelve rows have no launch with a prologue: asked to fold, the session
-    runs the stand-alone kernels."""
+    """Models whose rank-ins have no packed copy (a rank that is no multiple of 32) run the int8 and fp16 products of decode
+    steps of 5 to 8 rows, in rows of 1024 .. 4096 values, on the few-row matrix-core launch, and by default fold LN2 + its
+    token shift into the ffn.key launch: a staging wavefront per row computes LayerNorm with the stand-alone kernel's
+    formulas and rounding points (sums associated differently), so the step agrees with the one through the stand-alone
+    kernels to fp16 rounding (logits and shift rows within 2e-3 of their scale, WKV state within 1e-3).  The same bars with
+    LN1 folded as well (forced: the r/k/v launch, with layer 0 gathering its embedding rows itself; the ffn.value product is
+    then reduced by a launch of its own instead of by the LayerNorm kernel).  That the three modes are three routes shows in
+    their last bits.  Twelve rows have no launch with a prologue: asked to fold, the session runs the stand-alone kernels,
+    bit by bit."""
     from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
     hip = gpu
-    dims = ModelDims(L=2, C=C, H=C // 64, F=4 * C, V=512, Rw=32, Ra=32, Rg=64, Rv=32)
+    dims = ModelDims(L=2, C=C, H=C // 64, F=4 * C, V=512, Rw=48, Ra=48, Rg=64, Rv=32)
     gmodel = HipModel.from_host_weights(dims, synth_weights(dims, 19), hip.FMT_W8)
     rng = np.random.default_rng(B)
     prompt = rng.integers(0, dims.V, (B, 3))
@@ -925,6 +926,8 @@ def test_decode_step_of_five_to_eight_rows_folds_layernorm_into_the_few_row_laun
             err = rel_err(states[i].wkv.numpy(), states[1].wkv.numpy())
             assert err <= 1e-3, "%s: wkv state at step %d" % (name, step)
     assert states[0].elapsed.numpy().tolist() == [6] * B
+    bits = [st.wkv.numpy().view(np.uint32) for st in states]
+    assert len({b.tobytes() for b in bits}) == (3 if B <= 8 else 1)
     sess.close()
 
 
