@@ -871,10 +871,9 @@ def _quant_parts(orc, hip, fmt, w):
                                    (20, 96, 1024), (32, 4160, 512), (5, 64, 2048),
                                    (1030, 3872, 512), (3000, 2336, 256)])
 def test_linear_packed_matches_oracle(gpu, orc, fmt_name, M, N, K):
-    """Every tile variant (32-, 64- and 128-row tiles; one, two and four wavefront groups; 64-, 128- and 256-column
-    blocks - the last two shapes take the 128 x 256 tile for int8 and fp16 weights, once split and once not;
-    several row tiles), with and without K splits, chunk counts that are not a power of two, ragged M and column
-    counts that are not a multiple of the column block."""
+    """Tiles of 32, 64 and 128 rows and of 64, 128 and 256 columns (the last shape: the 128 x 256 tile of int8 and fp16 weights),
+    with and without K splits, stage counts that are not a power of two, ragged M and column counts that are not a multiple of
+    the column block."""
     hip = gpu
     if fmt_name == "w4" and K % 128:
         pytest.skip("W4 groups are 128 wide")
@@ -917,7 +916,8 @@ def test_linear_packed_matches_oracle(gpu, orc, fmt_name, M, N, K):
 
 @pytest.mark.parametrize("fmt_name", ["f16", "w8", "w4"])
 @pytest.mark.parametrize("M,N,K", [(1, 32, 256), (31, 64, 256), (32, 96, 768), (33, 4128, 512), (63, 2080, 1280), (65, 8256, 256),
-                                   (97, 16416, 256), (128, 64, 3840), (129, 8224, 768), (255, 16416, 256), (257, 352, 1792)])
+                                   (97, 16416, 256), (128, 64, 3840), (129, 8224, 768), (255, 16416, 256), (257, 352, 1792),
+                                   (1030, 544, 256), (1030, 1184, 256), (260, 224, 8192)])
 def test_linear_packed_tile_edges(gpu, orc, fmt_name, M, N, K):
     """The LDS-ring tiles where they can go wrong: one row, rows on both sides of a tile's edge, one band of columns and a
     block that is cut, as few stages as there are (K = 256) and stage counts that are no multiple of the rings."""
@@ -982,6 +982,28 @@ def test_linear_packed_of_33_to_64_rows_without_a_workspace(gpu, orc, fmt_name, 
     hip.linear_packed(fmt, M, N, K, dev(hip, x), packed, dparts[1], dparts[2], y, None)
     hip.device_sync()
     err = rel_err(y.numpy().astype(np.float32), orc.gemv(fmt, x, parts[0], parts[1], parts[2]).astype(np.float32))
+    assert err <= F16_TOL
+
+
+@pytest.mark.parametrize("fmt_name,M,N,K", [("w8", 330, 5184, 3072), ("w8", 1300, 4704, 2560), ("f16", 1300, 4704, 2560)])
+def test_linear_packed_wide_tiles_with_a_k_split(gpu, orc, fmt_name, M, N, K):
+    """The tiles of 64 x 256 and 128 x 256 where they split K (no other shape here makes them), rows on both sides of the tiles'
+    edges against the oracle."""
+    hip = gpu
+    rng = np.random.default_rng(M + N)
+    fmt = {"f16": hip.FMT_F16, "w8": hip.FMT_W8}[fmt_name]
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    parts = _quant_parts(orc, hip, fmt, (rng.standard_normal((N, K)) * 0.02).astype(np.float16))
+    dparts = [dev(hip, p) if p is not None else None for p in parts]
+    packed = hip.DeviceArray(parts[0].shape, parts[0].dtype)
+    hip.pack_weights(fmt, N, K, dparts[0], packed)
+    assert hip.linear_packed_workspace(M, N, K) > 0
+    ws = hip.DeviceArray((hip.linear_packed_workspace(M, N, K),), np.uint8)
+    y = hip.DeviceArray((M, N), np.float16)
+    hip.linear_packed(fmt, M, N, K, dev(hip, x), packed, dparts[1], dparts[2], y, ws)
+    hip.device_sync()
+    rows = [0, 1, 63, 64, 127, 128, 255, M - 2, M - 1]
+    err = rel_err(y.numpy()[rows].astype(np.float32), orc.gemv(fmt, x[rows], parts[0], parts[1], parts[2]).astype(np.float32))
     assert err <= F16_TOL
 
 
