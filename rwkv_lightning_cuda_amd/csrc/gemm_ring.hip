@@ -82,13 +82,8 @@ struct RingWeights {
 #pragma unroll
       for (int i = 0; i < 2 * GPW; ++i) put(i * 4, __builtin_nontemporal_load(wband + (static_cast<int64_t>(k32) * 2 + i) * 64));
     } else {
-      const uint4_t* piece = wband + static_cast<int64_t>(k32 >> 1) * 64;
-      if constexpr (GPW == 1) {
-        const uint2_t v = __builtin_nontemporal_load(reinterpret_cast<const uint2_t*>(piece) + (k32 & 1));
-        d[0] = v[0]; d[1] = v[1];
-      } else {
-        put(0, __builtin_nontemporal_load(piece));
-      }
+      static_assert(KW == 64, "a worker of int4 codes takes whole pieces");
+      put(0, __builtin_nontemporal_load(wband + static_cast<int64_t>(k32 >> 1) * 64));
       const int q = n * pr.group_n + (k32 >> 2) * pr.group_k;
       sc = pr.scale[q];
       zb = pr.zp[q];
@@ -110,8 +105,7 @@ struct RingWeights {
 template <int FMT, int KW>
 __device__ __forceinline__ int ring_x_piece(int st, int kg, int h) {
   if constexpr (FMT == RWKV_FMT_W4) {
-    if constexpr (KW == 32) return (kg >> 1) * 8 + h * 4 + (kg & 1) * 2 + st;
-    else return kg * 8 + h * 4 + st;
+    return kg * 8 + h * 4 + st;
   } else {
     return kg * (KW / 8) + (st >> 1) * 4 + h * 2 + (st & 1);
   }
