@@ -504,6 +504,7 @@ struct StreamConfig {
   int fmt = RWKV_FMT_F16;         // ring: the launch's format
   bool mixed = false;             // ring: fp16 problems beside it
   int splits = 1;
+  float us = 1e30f;               // estimate
   bool is_ring() const { return ring.mt > 0; }
   int rows() const { return 32 * (is_ring() ? ring.mt : wide_mt); }
   int cols(int problem_fmt) const {
@@ -586,22 +587,16 @@ static bool sums_at_consumer(int n_problems, int epilogue, int out_f32) {
 constexpr int kFilledBlocks = 200;
 // Rows from which the wide tiles, whose wavefronts feed two MFMAs from every X fragment they read from LDS, are looked at.
 constexpr int kWideMinRows = 160;
-// Launches of int8 problems only have a wide tile of their own at these sizes (three blocks per CU).
-bool linear_packed_int8_tile(int M, int K) { return M > 512 && M <= 1024 && K <= 4096 && K > 2048; }
 
 static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, bool group_rows,
                                   int max_splits) {
   bool any[3] = {false, false, false};
   for (int i = 0; i < n_problems; ++i) any[fmts[i]] = true;
   StreamConfig best;
-  float best_us = 1e30f;
   auto consider = [&](StreamConfig c) {
     for (c.splits = 1; c.splits == 1 || (c.splits <= max_splits && K % (c.splits * c.k_step()) == 0); c.splits *= 2) {
-      const float us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred, group_rows);
-      if (us < best_us) {
-        best_us = us;
-        best = c;
-      }
+      c.us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred, group_rows);
+      if (c.us < best.us) best = c;
     }
   };
   StreamConfig c;
@@ -616,7 +611,7 @@ static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, c
     c.ring = RingShape{0, 0, 0, 0};
     c.wide_mt = 4;
     // (from 1025 rows on, with most of the chip busy, the wide tile is the faster one whatever the estimates' last percent)
-    if (M > 1024 && ceil_div(M, 128) * count_col_blocks(c, n_problems, Ns, fmts) >= kFilledBlocks) best_us = 1e30f;
+    if (M > 1024 && ceil_div(M, 128) * count_col_blocks(c, n_problems, Ns, fmts) >= kFilledBlocks) best.us = 1e30f;
     consider(c);
     if (!any[RWKV_FMT_F16] && K <= 4096 && M <= 1024) {
       c.wide_mt = 2;
@@ -698,6 +693,21 @@ size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const P
     return RWKV_OK;
   });
   return bytes;
+}
+
+// (0.9: a second launch's start and end are a guess.  7.2B shape int8, ms per chunk, together / apart: 260 rows 9.76 / 9.28, 340
+// rows 10.53 / 10.30, 384 rows 10.42 / 10.56; 1.5B shape: 516 rows 4.79 / 4.86, 640 rows 5.23 / 5.18, 1200 rows 8.73 / 8.53)
+bool linear_packed_apart(int M, int K, int n_first, int n_problems, const PackedProblem* problems) {
+  int Ns[kMaxProblems], fmts[kMaxProblems];
+  for (int i = 0; i < n_problems; ++i) {
+    Ns[i] = problems[i].N;
+    fmts[i] = problems[i].fmt;
+    if (i < n_first && fmts[i] != RWKV_FMT_W8) return false;
+  }
+  const float together = choose_config(M, K, n_problems, Ns, fmts, false, false, 32).us;
+  const float apart = choose_config(M, K, n_first, Ns, fmts, false, false, 32).us +
+                      choose_config(M, K, n_problems - n_first, Ns + n_first, fmts + n_first, false, false, 32).us;
+  return apart < 0.9f * together;
 }
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,

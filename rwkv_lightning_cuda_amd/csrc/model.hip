@@ -215,14 +215,6 @@ int packed_projections(const rwkv_hip_model* m, int layer, PackedProblem* p) {
   return all ? 3 + n_lora : 0;
 }
 
-// Where a launch of int8 problems only has a tile of its own (several wavefronts per SIMD), three int8 projections go without
-// the fp16 rank-ins, which follow in a launch of their own.
-bool projections_apart(const PackedProblem* p, int rows, int C) {
-  bool apart = linear_packed_int8_tile(rows, C);
-  for (int i = 0; i < 3; ++i) apart = apart && p[i].fmt == RWKV_FMT_W8;
-  return apart;
-}
-
 // What the packed launches of a forward call of `rows` rows (B sequences) keep their K splits in: exactly what they ask for, from
 // the formats the layers have - a workspace that only bounds it would let a launch of several problems take the split that fits
 // what an earlier, larger call of the session has left, and its sums depend on that call.
@@ -253,7 +245,7 @@ size_t packed_workspace_bytes(const rwkv_hip_model* m, int B, int rows) {
     const int n = packed_projections(m, l, p);
     if (n == 0) {
       for (const int id : {RWKV_M_ATT_R, RWKV_M_ATT_K, RWKV_M_ATT_V}) ask_matrix(w.m[id], rows, C, C, RWKV_EPI_NONE, 0);
-    } else if (projections_apart(p, rows, C)) {
+    } else if (linear_packed_apart(rows, C, 3, n, p)) {
       ask(rows, C, 3, p, RWKV_EPI_NONE, 0);
       ask(rows, C, n - 3, p + 3, RWKV_EPI_NONE, 0);
     } else {
@@ -608,7 +600,7 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
           }
           const RowCopy moved = pending;
           pending = RowCopy{};
-          if (projections_apart(p, rows, C)) {
+          if (linear_packed_apart(rows, C, 3, 3 + n_lora, p)) {
             TRY_PROF(linear_packed_multi(st, rows, C, 3, p, RWKV_EPI_NONE, 0, s->gemm_ws, s->gemm_ws_bytes, nullptr, &moved));
             TRY_PROF(linear_packed_multi(st, rows, C, n_lora, p + 3, RWKV_EPI_NONE, 0, s->gemm_ws, s->gemm_ws_bytes));
           } else {

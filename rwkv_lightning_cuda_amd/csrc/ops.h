@@ -96,9 +96,9 @@ struct PackedProblem {
   int fmt;
   bool groups_first = false;  // int4: scale and zp are [K/128][N] (one 64-byte piece per 32 columns) instead of [N][K/128]
 };
-// Row counts and K at which a launch of int8 problems only gets a tile of its own (several wavefronts per SIMD):
-// callers with int8 and fp16 problems for one launch do better with two launches there.
-bool linear_packed_int8_tile(int M, int K);
+// Whether the first n_first problems, all int8, and the fp16 ones behind them do better in a launch each: a launch of int8
+// problems only has a tile of its own from a few hundred rows on (the pointers are not looked at).
+bool linear_packed_apart(int M, int K, int n_first, int n_problems, const PackedProblem* problems);
 // Exactly what linear_packed_multi takes for these problems (their N, format and layout; the pointers are not looked at).
 size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32);
 // defer (single problem, fp16 output, no epilogue): the consumer sums the partials instead of a reduce launch.

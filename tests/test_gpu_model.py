@@ -162,6 +162,27 @@ def test_matrices_of_different_formats_side_by_side(gpu):
     assert cos >= 0.9995
 
 
+def test_projections_and_rank_ins_in_launches_of_their_own(gpu):
+    """1200 rows of 1024 channels, int8: the projections go without the rank-ins.  The same tokens in chunks of 400 rows, which go
+    together (the bar is the fp16 one of the decode tests: sums in another order)."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=2, C=1024, H=16, F=2048, V=512, Rw=32, Ra=32, Rg=64, Rv=32)
+    model = HipModel.from_host_weights(dims, synth_weights(dims, 7), hip.FMT_W8)
+    B, T = 40, 30
+    tokens = np.random.default_rng(4).integers(0, dims.V, (B, T))
+    out = []
+    for chunk in (T, T // 3):
+        sess, st = Session(model), State(dims, B)
+        lg = hip.DeviceArray((B, dims.V), np.float32)
+        for t in range(0, T, chunk):
+            sess.forward(tokens[:, t:t + chunk], st, lg)
+        out.append((lg.numpy(), st.shift.numpy().astype(np.float32), st.wkv.numpy()))
+        sess.close()
+    for name, a, b in zip(("logits", "shift", "wkv"), *out):
+        assert rel_err(a, b) <= 3e-3, name
+
+
 @pytest.mark.parametrize("C,F,projections,rows,before", [(2048, 8192, ("w8", "f16", "f16"), 327, 513),
                                                          (4096, 4096, ("w4", "w8", "f16"), 18, 19)])
 def test_a_call_does_not_depend_on_what_the_session_ran_before(gpu, C, F, projections, rows, before):
