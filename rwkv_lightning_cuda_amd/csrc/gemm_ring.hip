@@ -1,4 +1,4 @@
-// Packed-weight MFMA GEMM for batched decode and prefill chunks (17 .. some hundred rows; any number of rows of int4 codes):
+// Packed-weight MFMA GEMM for batched decode and prefill chunks (up to some hundred rows; any number of rows of int4 codes):
 // X through a ring of LDS stages that feeder wavefronts fill with direct-to-LDS loads, weights through registers.
 //
 // Reference: as gemm_stream.hip (cuda/rwkv7_v3a_ops.cu:2235-2368).
@@ -6,12 +6,12 @@
 // What bounds it.  256 CUs that stream the weights once take 12.8 us for 67 MB (6.5 TB/s and 2 us of launch); every block also
 // needs its rows of X, out of L2, and the two add up: 15.4 us with 64 rows of X per CU (512 KB), 19.3 with 128, whatever
 // the number of loads in flight.  So a block (a) reads every weight byte once - up to 64 rows no two blocks share weights -
-// and (b) has no other traffic: one block per CU, 12 wavefronts.
-//   * Four feeders only move X: 16-byte direct-to-LDS loads (no registers, no ds_write), up to seven stages ahead, waits by
-//     count.  A separate wavefront counts X alone: in the wavefronts that also load weights, loads return in order and every
+// and (b) has no other traffic: 12 wavefronts, one block per CU (two of the tiles of 32 rows and 128 k, 64 KB of LDS each).
+//   * Four feeders only move X: 16-byte direct-to-LDS loads (no registers, no ds_write), seven stages ahead - three where a
+//     stage is 32 KB - waits by count.  A separate wavefront counts X alone: in the wavefronts that also load weights, loads return in order and every
 //     wait for X (L2) would be one for older weights (HBM).
 //   * Eight workers multiply.  A worker owns NB bands of 32 columns and 1 / KG of each stage's k; its weights come as whole
-//     1 KiB pieces, non-temporally, three stages ahead.  KG groups of workers share the k of a stage, so that 64 columns still
+//     1 KiB pieces, non-temporally, one to three stages ahead (what the registers hold).  KG groups of workers share the k of a stage, so that 64 columns still
 //     occupy eight wavefronts; their sums meet in LDS once, at the end, in group order.
 //   * One barrier per stage for all twelve, placed before the last MFMA step, whose fragments are in registers by then: the
 //     first fragments of the next stage are read under that step's products.

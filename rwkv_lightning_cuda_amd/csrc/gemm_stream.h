@@ -1,6 +1,5 @@
 // What the two files of the packed-weight GEMM share: the launch arguments and the exact expansion of int8 / int4 codes
-// to fp16 (gemm_stream.hip: packing, dispatch, split-K reduce and the register-staged tiles; gemm_ring.hip: the
-// LDS-ring tiles).
+// to fp16 (gemm_stream.hip: packing, dispatch, split-K reduce and the wide tiles; gemm_ring.hip: the LDS-ring tiles).
 #pragma once
 
 #include "ops.h"
@@ -22,7 +21,7 @@ struct StreamProblem {
 };
 
 // Up to kMaxProblems products that share M, K and the split (each with its own weights, format, x and y) in one
-// launch: grid.y runs over the column blocks of all problems, block_end[] are the prefix sums.
+// launch: its column blocks run over all problems, block_end[] are the prefix sums.
 struct StreamArgs {
   StreamProblem p[kMaxProblems];
   int block_end[kMaxProblems];

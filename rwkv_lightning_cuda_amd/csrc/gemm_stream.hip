@@ -1,5 +1,5 @@
 // Weight-streaming MFMA GEMM Y[M,N] = X[M,K] . W[N,K]^T over weights stored in an MFMA-native packed order.
-// This is the M >= 16 path of the model: batched decode (M = batch) and prefill chunks (M = batch * 128).
+// This is the path of prefill chunks and of batched decode, from 5 rows on (from 3 for int8 / int4 rows of 4096 and more).
 //
 // Reference: the cuBLAS / cuBLASLt calls behind rwkv7_v3a_linear_f16_orig_launch and
 // rwkv7_v3a_linear_f16_orig_lt_cfg_launch (cuda/rwkv7_v3a_ops.cu:2235-2368): fp16 in, fp32 accumulate, fp16
@@ -15,7 +15,7 @@
 // traffic for the weights; every weight byte leaves HBM once per 32*MT rows of X.
 //
 // Two kernels stream that order.  gemm_ring.hip: up to a few hundred rows (all rows for int4 codes), where the product is
-// bound by the weights' and X's way into the CUs.  Here: the wide tiles for more rows, bound by the matrix core.  With more
+// bound by the weights' and X's way into the CUs.  Here: the wide tiles for more rows, bound by LDS and issue.  With more
 // than one K split each block writes an fp32 partial tile and a second small kernel sums the partials in split order (a
 // fixed order: results do not depend on scheduling) and applies scale and epilogue - or the LayerNorm kernel that consumes
 // the result does (DeferredReduce).
@@ -192,7 +192,7 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
     n[nb] = band * 32 + j;
     wband[nb] = pr.wp + (static_cast<int64_t>(band) * (g.K / T::G)) * (P::PIECES * 64) + lane;
   }
-  half_t scale_h[NB];  // the columns' int8 scales, requested before the main loop (see stream_block)
+  half_t scale_h[NB];  // the columns' int8 scales, requested before the main loop (in the epilogue: 1.2 us per launch)
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
     scale_h[nb] = static_cast<half_t>(1.0f);
@@ -334,7 +334,8 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
   };
 
   constexpr int U = (D % 2 == 0) ? D : 2 * D;
-  // whole rounds of U chunks as one basic block, the chunks left over with exits between them (see stream_block)
+  // whole rounds of U chunks as one basic block (with exits between them the compiler waits for every load in flight at the
+  // head of each round), the chunks left over with exits
   const int whole = nchunks - nchunks % U;
   int c0 = 0;
   for (; c0 < whole; c0 += U) {
@@ -520,9 +521,10 @@ static int count_col_blocks(const StreamConfig& c, int n_problems, const int* Ns
   return col_blocks;
 }
 
-// Estimated microseconds of a launch: what the choice between tiles and K splits goes by.  Fitted to sweeps of every tile over
-// 17 .. 2048 rows x the matrices of the presets (2048 .. 65536 columns, 768 .. 16384 k, three formats); the tile it picks is
-// within a few percent of the best one of the sweep.
+// Estimated microseconds of a launch: what the choice between tiles and K splits goes by.  Fitted to sweeps of every tile and
+// split over 5 .. 3000 rows x the matrices of the presets (768 .. 65536 columns, 768 .. 16384 k, three formats: 969 launches).
+// Its pick takes the best one's time in half of them; in geometric mean 1.04 (int8), 1.02 (fp16), 1.01 (int4 scales by row)
+// and 1.03 (by group) times, in one of ten more than 1.16 / 1.09 / 1.02 / 1.13 times.
 //   ring: a fixed part (launch, first stage, epilogue); the bytes of the busiest CU at what a CU takes in while all of them
 //   stream (94 GB/s; 130 while half of the chip idles); what of the HBM stream of the weights does not hide behind that; the
 //   products; per further round of blocks its start and end, which a second block hides where two fit a CU.

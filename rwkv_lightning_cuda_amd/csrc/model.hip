@@ -25,7 +25,7 @@ struct Matrix {
   const void* data = nullptr;
   const half_t* scale = nullptr;
   const uint8_t* zp = nullptr;
-  void* packed = nullptr;  // owned: the same codes in the MFMA-native order, for calls with >= 16 rows
+  void* packed = nullptr;  // owned: the same codes in the MFMA-native order, for calls of packed_min_rows rows and more
   half_t* scale_by_group = nullptr;  // int4, in the same block behind the codes: scale and zero point as [K/128][N]
   uint8_t* zp_by_group = nullptr;
   void free_copies() {
@@ -711,7 +711,7 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
                        w.t[RWKV_T_LNX_B], b.g, b.y2));
       }
     }
-    // From 16 rows on (the streaming GEMM) the LayerNorm kernels that consume the output projection and
+    // On the packed path the LayerNorm kernels that consume the output projection and
     // ffn.value sum the split-K partials themselves instead of a reduce launch; att / cm then stay unwritten.
     const bool defer_ok = !s->trace && !ln_in_linear;
     DeferredReduce att_partial;
