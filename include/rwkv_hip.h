@@ -267,7 +267,7 @@ int rwkv_hip_advance_i32(rwkv_stream_t s, int n, int amount, void* x);
 /* ---- sampler.  Replaces rwkv_sampling::setup_rand_raw / batch_sampling_repetition_temperature_topk_topp_raw
  * / batch_sampling_temperature_topk_topp_raw (src/utils/sampling.h:14-46).
  * logits f32 [B,V]; penalties f32 [B,V] in/out (NULL = no penalty, as the no-penalty reference entry);
- * probs f32 [B,V] scratch; out i32 [B].  The random stream is a counter-based Philox4x32-10 keyed by
+ * probs f32 [B,V] scratch (calls that share it must not overlap); out i32 [B].  The random stream is a counter-based Philox4x32-10 keyed by
  * (seed, row, step): same arguments give the same tokens.  V % 4 == 0, V <= 1048576,
  * temperature in [0.001, 1000], as the reference checks (src/utils/sampling.cu:492-512). */
 int rwkv_hip_sample(rwkv_stream_t s, int B, int V, const void* logits, void* penalties, void* probs, void* out,

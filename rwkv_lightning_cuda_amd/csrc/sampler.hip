@@ -925,15 +925,16 @@ int rwkv_hip_sample(rwkv_stream_t s, int B, int V, const void* logits, void* pen
   a.top_p = static_cast<float>(top_p);
   a.seed = seed;
   a.step = step;
-  // The three launches keep their sums in `probs` while the logits and penalties are still being read.  The one-block kernel
-  // does not touch the scratch of a row it holds in registers: a caller whose scratch is one of the inputs stays there.
-  const auto apart = [&](const void* input) {
+  // The three launches keep their sums in `probs` while the logits and penalties are still being read and other rows' picks are
+  // written.  The one-block kernel does not touch the scratch of a row it holds in registers: a caller whose scratch reaches
+  // into one of these stays there.
+  const int64_t row_bytes = static_cast<int64_t>(B) * V * 4;
+  const auto apart = [&](const void* other, int64_t bytes) {
     const char* p = static_cast<const char*>(probs);
-    const char* q = static_cast<const char*>(input);
-    const int64_t bytes = static_cast<int64_t>(B) * V * 4;
-    return !input || p + bytes <= q || q + bytes <= p;
+    const char* q = static_cast<const char*>(other);
+    return !other || p + row_bytes <= q || q + bytes <= p;
   };
-  if (sample_split_ok(V, top_k) && apart(logits) && apart(penalties)) {
+  if (sample_split_ok(V, top_k) && apart(logits, row_bytes) && apart(penalties, row_bytes) && apart(out, static_cast<int64_t>(B) * 4)) {
     const int parts = ceil_div(V, kPartEntries);
     hipLaunchKernelGGL(sample_stats_kernel, dim3(B, parts), dim3(kPartThreads), 0, as_stream(s), a);
     hipLaunchKernelGGL(sample_pick_kernel, dim3(B), dim3(kSampleThreads), 0, as_stream(s), a, parts);

@@ -135,6 +135,22 @@ def test_top_k_rows_whose_scratch_is_an_input(gpu, orc, shared):
     assert float(np.max(np.abs(d_pen.numpy() - want))) <= 2.5e-7
 
 
+def test_top_k_rows_whose_picks_lie_in_the_scratch(gpu, orc):
+    """The picks of 3000 rows over the scratch of the last rows, whose blocks start when most picks are written: the last rows'
+    draws have weight in the oracle's kept set all the same."""
+    hip = gpu
+    V, B, top_k, top_p = 512, 3000, 4, 0.8
+    logits = (np.random.default_rng(2).standard_normal((B, V)) * 2.5).astype(np.float32)
+    room = hip.DeviceArray((B + 4, V), np.float32)
+    picked = room.view((B - 2) * V, (B,), np.int32)
+    hip.sample(B, V, hip.DeviceArray.from_numpy(logits), None, room.view(0, (B, V)), picked, top_k=top_k, top_p=top_p, seed=7)
+    hip.device_sync()
+    picks = picked.numpy()
+    assert picks.min() >= 0 and picks.max() < V
+    for b in range(B - 8, B):
+        assert orc.sample_filter(logits[b], None, 1.0, top_k, top_p)[1][picks[b]] > 0
+
+
 @pytest.mark.parametrize("low", [-np.inf, -3.0e38, -200.0])
 @pytest.mark.parametrize("live", [1, 3, 39, 40, 41, 900, 1500])
 def test_top_k_rows_masked_to_a_few_entries(gpu, orc, live, low):
