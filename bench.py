@@ -540,7 +540,7 @@ def main():
             also["prefill_gemm"] = {"bound": "mfma", "achieved": flops / (total_ms * 1e-3) / 1e12,
                                     "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
                                     "frac": flops / (total_ms * 1e-3) / 1e12 / MFMA_F16_PEAK_TFLOPS,
-                                    "kernel": "gemm_stream_kernel (+ split-K reduce), M = %d rows" % rows,
+                                    "kernel": "gemm_ring_kernel (+ split-K reduce), M = %d rows" % rows,
                                     "launches": launches, "sum_launch_ms": total_ms,
                                     # at M = 128 the launches are weight-streaming bound: the same time against HBM
                                     "weights_gb_s": model.weight_bytes() / (total_ms * 1e-3) / 1e9,

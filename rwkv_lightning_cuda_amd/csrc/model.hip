@@ -159,7 +159,7 @@ struct rwkv_hip_session {
   bool wkv_fp16 = false;      // the WKV state tensor is fp16 [L,B,H,64,64] (the reference's use_wkv32 == false)
   int tmix_rows = -1;         // decode steps' single-launch time-mix core: rows per block 1/2/4, 0 never, < 0 by batch
   int fused_ln = -1;          // decode steps fold LayerNorm + token shift into the linear launches: 1 always, 0 never,
-                              // -1 for one row of at most 4096 channels (the row-resident GEMV hides the prologue
+                              // -1 for one or two rows of at most 4096 channels (the row-resident GEMV hides the prologue
                               // behind its weight requests: 7.2B shape 2.04 -> 1.92 ms per step, 0.1B 0.413 -> 0.373)
 };
 
@@ -452,7 +452,7 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
   }
   const bool fused_tmix = tmix_rows > 0;
   // Decode steps on the GEMV path can fold both LayerNorm + token-shift kernels of a layer into the prologue of the
-  // linear launch that consumes them (r/k/v + LoRA rank-ins; ffn.key): by default for one row of up to 4096
+  // linear launch that consumes them (r/k/v + LoRA rank-ins; ffn.key): by default for one or two rows of up to 4096
   // channels.  The residual-stream tap needs the stand-alone kernels.
   const bool want_ln_in_linear = s->fused_ln > 0 || (s->fused_ln < 0 && rows <= linear_ln_prologue_max_rows(C));
   // (the shift row that the prologue leaves for later is stored by the single-launch time-mix core)
