@@ -439,13 +439,9 @@ __global__ __launch_bounds__(256) void kk_a_gate_kernel(KkArgs p) {
   if (p.new_k) p.new_k[idx] = nk;
   if (p.neg_kk) p.neg_kk[idx] = nkk;
   if (p.kka) p.kka[idx] = kka;
-  if (p.k32) {
-    p.k32[idx] = h2f(nk);
-    p.a32[idx] = h2f(nkk);
-    p.b32[idx] = h2f(kka);
+  if (p.d32) {
     const float wraw = round_h(h2f(p.w12[idx]) + h2f(p.w0[c]));  // rwkv7_add_vec_launch rounding point
     p.d32[idx] = exp2f(-0.8750387749145276f / (1.0f + exp2f(-1.4426950408889634f * wraw)));
-    p.r32[idx] = h2f(p.r[idx]);
   }
   if (p.w_sum16) p.w_sum16[idx] = f2h(h2f(p.w12[idx]) + h2f(p.w0[c]));
 }

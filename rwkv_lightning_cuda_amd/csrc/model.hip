@@ -700,13 +700,11 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
         // bitwise the same)
         KkArgs p = {};
         p.k = b.k; p.k_k = w.t[RWKV_T_K_K]; p.a0 = w.t[RWKV_T_A0]; p.a12 = b.a12; p.k_a = w.t[RWKV_T_K_A];
-        p.new_k = b.k2; p.neg_kk = nullptr; p.kka = nullptr;
-        p.w12 = b.w12; p.w0 = w.t[RWKV_T_W0]; p.r = b.r;
-        p.k32 = b.k32; p.a32 = b.a32; p.b32 = b.b32; p.d32 = b.d32; p.r32 = b.r32;
+        p.new_k = b.k2; p.neg_kk = b.nkk; p.kka = b.kka;
+        p.w12 = b.w12; p.w0 = w.t[RWKV_T_W0]; p.d32 = b.d32;
         p.rows_heads = static_cast<int64_t>(rows) * H; p.H = H;
         TRY_AUX(kk_a_gate_launch(st, p));
-        TRY_AUX(wkv7_seq_f16_launch(st, B, T, C, H, S, b.r32, b.d32, b.k32, b.a32, b.b32, static_cast<int64_t>(T) * C, v_cur,
-                                b.y, static_cast<int64_t>(T) * C));
+        TRY_AUX(wkv7_seq_f16_launch(st, B, T, C, H, S, b.r, b.d32, b.k2, b.nkk, b.kka, v_cur, b.y));
         TRY_AUX(lnx_launch(st, static_cast<int64_t>(rows) * H, H, b.y, b.r, b.k2, v_cur, w.t[RWKV_T_R_K], w.t[RWKV_T_LNX_W],
                        w.t[RWKV_T_LNX_B], b.g, b.y2));
       }

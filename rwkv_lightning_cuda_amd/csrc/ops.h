@@ -163,15 +163,10 @@ struct KkArgs {
   half_t* new_k;
   half_t* neg_kk;
   half_t* kka;
-  // optional extras (all may be NULL): decay logits w12 (+ w0) and r, widened for the WKV kernel
+  // optional extras (all may be NULL): the decay of w12 + w0 for the WKV kernel
   const half_t* w12;
   const half_t* w0;
-  const half_t* r;
-  float* k32;
-  float* a32;
-  float* b32;
   float* d32;
-  float* r32;
   // optional (needs w12 and w0): f16(w12 + w0), the decay logit as the fp16-state recurrence takes it for calls of
   // more than 16 tokens (src/rwkv7_fast_v4.cu:1266-1271) - what add_vec_launch would write in a launch of its own
   half_t* w_sum16;
@@ -231,8 +226,7 @@ int ffn_sparse_launch(hipStream_t st, int fmt, int rows, int C, int F, int activ
 int argmax_launch(hipStream_t st, int B, int V, const float* logits, int* out, int64_t* next = nullptr, int* history = nullptr);
 
 // ---- wkv7.hip -----------------------------------------------------------------------------------
-// T tokens of the recurrence from fp32 operands (decay applied); v, y fp16.  op_bs / io_bs: elements
-// between batch rows of the operand / io tensors.
+// T tokens of the recurrence, all tensors [B,T,C]; d is the decay itself in fp32.
 // The model's row-tiled time-mix pass in one launch: kk normalise / a-gate / decay while staging, the WKV recurrence,
 // then per-head GroupNorm + (r.k.r_k) v bonus + gate on the way out.  All fp16 tensors [B,T,C] contiguous.
 struct TmixSeqArgs {
@@ -244,9 +238,8 @@ int tmix_seq_launch(hipStream_t st, int B, int T, int C, int H, float* state, co
 // false: few heads in flight and more than one token - the stand-alone kernels are faster there (the recurrence
 // then runs a head's row ranges on separate CUs, which the fused pass cannot: its GroupNorm needs whole heads)
 bool tmix_seq_whole_heads(int B, int T, int H);
-int wkv7_seq_f16_launch(hipStream_t st, int B, int T, int C, int H, float* state, const float* r, const float* d,
-                        const float* k, const float* a, const float* b, int64_t op_bs, const half_t* v, half_t* y,
-                        int64_t io_bs);
+int wkv7_seq_f16_launch(hipStream_t st, int B, int T, int C, int H, float* state, const half_t* r, const float* d,
+                        const half_t* k, const half_t* a, const half_t* b, const half_t* v, half_t* y);
 
 // ---- wkv7_f16state.hip: the recurrence with an fp16 state (w raw decay logits, w0 [C] or NULL added unrounded) ----
 int wkv7_f16state_launch(hipStream_t st, int B, int T, int C, int H, half_t* state, const half_t* r, const half_t* w,

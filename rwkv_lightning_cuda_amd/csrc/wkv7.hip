@@ -4,11 +4,11 @@
 //   sa = sum_j S[i][j]*a[j];  S[i][j] = S[i][j]*d[j] + sa*b[j] + k[j]*v[i];  y[i] = sum_j S[i][j]*r[j]
 // with the decay map d = exp(-e^-1/2 * sigmoid(w)) of :13-14,26-28.
 //
-// Sequence kernel (any T): four to sixteen wavefronts per (batch, head), each lane keeps a few rows x 4 columns of
-// the 64 x 64 state in registers for the whole call.  The per-column operands r,d,k,a,b of a token are staged in
-// LDS as fp32 and each lane reads only the four columns it owns; the two row sums of a step (sa and y) are
-// reduced over the 16 lanes that share a row with DPP adds.  The staging converts what the caller has (fp16 or
-// fp32 tensors, raw decay logits or decays, or the model's own fp16 rows) on the way into LDS.
+// Lanes keep a few rows x 4 or 8 columns of the 64 x 64 state in registers for the whole call.  The per-column operands of a
+// token are staged in LDS and each lane reads only the columns it owns; the two row sums of a step (sa and y) are reduced over
+// the lanes that share a row with DPP adds.  The staging converts what the caller has (raw decay logits or decays, or the
+// model's own fp16 rows) on the way into LDS.  Calls of several tokens: wkv7_feed_kernel; single tokens and the model's fused
+// pass: wkv7_seq_kernel.  Every variant and every split of T over several calls gives bitwise the same result.
 #include <type_traits>
 #include "ops.h"
 
@@ -21,34 +21,21 @@ __device__ __forceinline__ float decay_from_logit(float w) {
   return exp2f(kWScaleLog2e / (1.0f + exp2f(kNLog2e * w)));
 }
 
-// ---- sequence kernel -------------------------------------------------------------------------
-// grid = B*H, block = 1024/RPL threads: 16/RPL wavefronts per head, RPL = 4, 2 or 1 state rows per lane.  Lane
-// (g, c) = (lane / 16, lane % 16) of wavefront q owns rows 4*RPL*q + RPL*g .. +RPL-1 and columns 4c .. 4c+3, so
-// the 16 lanes of one DPP row hold complete state rows and the wavefronts never exchange data.  r,d,k,a,b are
-// fp32 with `op_bs` elements between batch rows; v,y are IO with `io_bs` elements between batch rows.  The
-// block stages the operands kSeqChunk tokens at a time with coalesced 16-byte loads, double-buffered (the
-// loads of chunk c+1 are in flight while chunk c computes); a step costs each lane six LDS reads (its four
-// columns of the five operands and its v values) against 28*RPL VALU operations.  y goes back through LDS so
-// that the global stores are coalesced.  The arithmetic of a state element does not depend on RPL or on the
-// chunking: every variant and every split of T over several calls gives bitwise the same result.  Smaller RPL
-// means less serial work per token and wavefront and is used while the grid is small enough to leave SIMDs
-// idle (RPL = 1 up to 64 heads, 2 up to 128); RPL = 4 reads each operand least often.
-constexpr int kSeqChunk = 8;
-
-// Where the five operand vectors of a token come from (SRC):
-//   kSrcFp32  - fp32 tensors r, d, k, a, b (decay applied), `op_bs` elements between batch rows, staged with 16-byte
-//               loads: what kk_a_gate_kernel writes for the model's stand-alone path;
-//   kSrcRaw   - the caller's r, w, k, a, b in the io type, converted (and the decay derived from w, by w_mode)
-//               while staging, one wavefront per token, lane = channel: the C-ABI operator, which so reads every
-//               operand once instead of through an fp32 copy (14 instead of 56 bytes per token and channel);
-//   kSrcFused - the model's fused pass, below.
-constexpr int kSrcFp32 = 0;
-constexpr int kSrcFused = 1;
-constexpr int kSrcRaw = 2;
-struct RawOperands {
-  const void *r, *w, *k, *a, *b;
+// Operands of the stand-alone recurrence, all [B,T,C]: w as raw decay logits or decays (w_mode).
+template <typename IO, typename WT>
+struct SeqOperands {
+  const IO *r, *k, *v, *a, *b;
+  const WT* w;
   int w_mode;
 };
+
+// ---- sequence kernel -------------------------------------------------------------------------
+// grid = B*H, block = 1024/RPL threads: 16/RPL wavefronts per head, RPL state rows per lane.  Lane (g, c) = (lane / 16,
+// lane % 16) of wavefront q owns rows 4*RPL*q + RPL*g .. +RPL-1 and columns 4c .. 4c+3, so the 16 lanes of one DPP row hold
+// complete state rows and the wavefronts never exchange data.  v,y have `io_bs` elements between batch rows.  The block stages
+// the operands kSeqChunk tokens at a time, double-buffered; a step costs each lane six LDS reads (its four columns of the five
+// operands and its v values) against 28*RPL VALU operations.  y goes back through LDS so that the global stores are coalesced.
+constexpr int kSeqChunk = 8;
 
 // FUSED (the model's row-tiled time-mix path, fp16 io): the operands are not read as fp32 tensors but derived
 // while staging from the fp16 rows r, k, a12, w12 - the arithmetic of kk_a_gate_kernel, one wavefront per token,
@@ -56,26 +43,14 @@ struct RawOperands {
 // gate - the arithmetic of lnx_rkvres_xg_kernel on the fp16-rounded y - so that three launches and the fp32
 // operand tensors between them become one launch.  Bitwise the same results as the three kernels.
 //
-// PARTS > 1: the rows of a head's state are independent of each other (row i needs only its own sum over the
-// columns, v_i and the per-column operands), so a head is cut into PARTS row ranges that run as separate blocks on
-// separate CUs - with few heads in flight the step is bound by one CU's VALU rate, not by memory.  Not with FUSED
-// (the GroupNorm needs the whole head's y).  Same lanes, same rows, same arithmetic: bitwise the same results.
-//
 // STRAIGHT = false leaves out the unrolled eight-step body: single-token calls move a head's state once and are
 // bound by that traffic, so they want the registers for more blocks per CU instead (148 -> under 100 VGPRs).
-template <typename IO, int RPL, int PARTS, int SRC, bool STRAIGHT = true>
-__global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int C, int H, float* __restrict__ state,
-                                                              const float* __restrict__ r, const float* __restrict__ d,
-                                                              const float* __restrict__ k, const float* __restrict__ a,
-                                                              const float* __restrict__ b, int64_t op_bs,
+template <typename IO, typename WT, int RPL, bool FUSED, bool STRAIGHT = true>
+__global__ __launch_bounds__(1024 / RPL) void wkv7_seq_kernel(int T, int C, int H, float* __restrict__ state,
                                                               const IO* __restrict__ v, IO* __restrict__ y,
-                                                              int64_t io_bs, TmixSeqArgs fa, RawOperands ro) {
-  constexpr bool FUSED = SRC == kSrcFused;
-  constexpr bool RAW = SRC == kSrcRaw;
-  static_assert(PARTS == 1 || !FUSED, "the fused pass needs whole heads");
-  constexpr int NT = 1024 / RPL / PARTS;
-  constexpr int kOpVecs = 5 * kSeqChunk * (kHead / 4);         // float4 of operands per chunk
-  constexpr int kOpSlots = (kOpVecs + NT - 1) / NT;
+                                                              int64_t io_bs, TmixSeqArgs fa, SeqOperands<IO, WT> ro) {
+  constexpr bool RAW = !FUSED;
+  constexpr int NT = 1024 / RPL;
   constexpr int kVSlots = (kSeqChunk * kHead + NT - 1) / NT;
   typedef float rows_t __attribute__((ext_vector_type(RPL)));
   __shared__ __align__(16) float ops[2][kSeqChunk][5][kHead];  // [buffer][token][a,b,d,k,r][column]
@@ -87,14 +62,12 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
   __shared__ __align__(16) float spare[kSpare ? NT * RPL : 4];
   __shared__ __align__(16) float gs[FUSED ? 2 : 1][FUSED ? kSeqChunk : 1][kHead];  // FUSED: the gate rows
 
-  const int bh = blockIdx.x / PARTS;
-  const int part = blockIdx.x % PARTS;
+  const int bh = blockIdx.x;
   const int bi = bh / H;
   const int h = bh - bi * H;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int row_lo = part * (kHead / PARTS);                         // this block's rows
-  const int i0 = row_lo + 4 * RPL * (tid >> 6) + RPL * (lane >> 4);  // first of this lane's rows
+  const int i0 = 4 * RPL * (tid >> 6) + RPL * (lane >> 4);  // first of this lane's rows
   const int j0 = 4 * (lane & 15);                           // first of its 4 columns
   float* sblk = state + (static_cast<int64_t>(bh) * kHead + i0) * kHead + j0;
 
@@ -102,37 +75,15 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
 #pragma unroll
   for (int i = 0; i < RPL; ++i) S[i] = __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(sblk + i * kHead));
 
-  const int64_t base = static_cast<int64_t>(bi) * op_bs + h * kHead;
   const int64_t iob = static_cast<int64_t>(bi) * io_bs + h * kHead;
-  // staging slot i of thread t: float4 number t + i*NT of the chunk = (operand, token, 4 columns)
-  const float* st_src[kOpSlots];
-  int st_tok[kOpSlots];
-  int st_dst[kOpSlots];  // offset inside ops[buf], -1: slot unused
-#pragma unroll
-  for (int i = 0; i < kOpSlots; ++i) {
-    const int idx = tid + i * NT;
-    const int o = idx / (kSeqChunk * 16);
-    const int tok = (idx >> 4) % kSeqChunk;
-    const int col = (idx & 15) * 4;
-    const float* src = o == 0 ? a : (o == 1 ? b : (o == 2 ? d : (o == 3 ? k : r)));
-    st_src[i] = src + base + col;
-    st_tok[i] = tok;
-    st_dst[i] = idx < kOpVecs ? (tok * 5 + o) * kHead + col : -1;
-  }
-
   // Two sets of staging registers: a chunk is requested two chunks before it is needed - eight steps are shorter
   // than a trip to memory.
-  float4_t stage[2][kOpSlots];
   float v_stage[2][kVSlots];
   // FUSED: raw fp16 values of this thread's (token, channel) slots: r, k, a12, w12, g; and its channel's constants
   half_t raw[2][kVSlots][5];
   // RAW: the caller's r, w, k, a, b values of the slots, still in the io type
-  IO rio[2][RAW ? kVSlots : 1][5];
-  const IO* ro_r = static_cast<const IO*>(ro.r);
-  const IO* ro_w = static_cast<const IO*>(ro.w);
-  const IO* ro_k = static_cast<const IO*>(ro.k);
-  const IO* ro_a = static_cast<const IO*>(ro.a);
-  const IO* ro_b = static_cast<const IO*>(ro.b);
+  IO rio[2][RAW ? kVSlots : 1][4];
+  WT wio[2][RAW ? kVSlots : 1];
   float c_kk = 0.0f, c_a0 = 0.0f, c_ka = 0.0f, c_w0 = 0.0f, c_rk = 0.0f, c_lnw = 0.0f, c_lnb = 0.0f;
   if constexpr (FUSED) {
     const int c = h * kHead + lane;
@@ -144,12 +95,6 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
   // under a branch makes the compiler's s_waitcnt accounting wait for everything in flight, the younger set too.
   auto request = [&](int t0, auto set_c) {
     constexpr int set = decltype(set_c)::value;
-    if constexpr (SRC == kSrcFp32) {
-#pragma unroll
-      for (int i = 0; i < kOpSlots; ++i) {
-        stage[set][i] = *reinterpret_cast<const float4_t*>(st_src[i] + static_cast<int64_t>(min(t0 + st_tok[i], T - 1)) * C);
-      }
-    }
 #pragma unroll
     for (int i = 0; i < kVSlots; ++i) {
       const int tok = min((tid + i * NT) >> 6, kSeqChunk - 1);
@@ -160,18 +105,13 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
         raw[set][i][4] = fa.g[at];
       }
       if constexpr (RAW) {
-        rio[set][i][0] = ro_a[at]; rio[set][i][1] = ro_b[at]; rio[set][i][2] = ro_w[at]; rio[set][i][3] = ro_k[at];
-        rio[set][i][4] = ro_r[at];
+        rio[set][i][0] = ro.a[at]; rio[set][i][1] = ro.b[at]; rio[set][i][2] = ro.k[at]; rio[set][i][3] = ro.r[at];
+        wio[set][i] = ro.w[at];
       }
     }
   };
   auto commit = [&](int buf, auto set_c) {
     constexpr int set = decltype(set_c)::value;
-    if constexpr (SRC == kSrcFp32) {
-#pragma unroll
-      for (int i = 0; i < kOpSlots; ++i)
-        if (st_dst[i] >= 0) *reinterpret_cast<float4_t*>(&ops[buf][0][0][0] + st_dst[i]) = stage[set][i];
-    }
 #pragma unroll
     for (int i = 0; i < kVSlots; ++i) {
       const int tok = (tid + i * NT) >> 6;  // wave-uniform: one wavefront per token, lane = channel
@@ -197,12 +137,12 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
           gs[buf][tok][lane] = h2f(raw[set][i][4]);
         }
         if constexpr (RAW) {
-          const float wv = static_cast<float>(rio[set][i][2]);
+          const float wv = static_cast<float>(wio[set][i]);
           ops[buf][tok][0][lane] = static_cast<float>(rio[set][i][0]);
           ops[buf][tok][1][lane] = static_cast<float>(rio[set][i][1]);
           ops[buf][tok][2][lane] = (ro.w_mode == RWKV_W_RAW_LOGIT) ? decay_from_logit(wv) : wv;
-          ops[buf][tok][3][lane] = static_cast<float>(rio[set][i][3]);
-          ops[buf][tok][4][lane] = static_cast<float>(rio[set][i][4]);
+          ops[buf][tok][3][lane] = static_cast<float>(rio[set][i][2]);
+          ops[buf][tok][4][lane] = static_cast<float>(rio[set][i][3]);
         }
       }
     }
@@ -234,7 +174,7 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
           const float rkv = wave_sum(ops[buf][tt][4][lane] * ops[buf][tt][3][lane] * c_rk);
           const float o = (dd * rstd * c_lnw + c_lnb + rkv * vs[buf][tt][lane]) * gs[buf][tt][lane];
           y[iob + static_cast<int64_t>(t0 + tt) * C + lane] = static_cast<IO>(o);
-        } else if (PARTS == 1 || (lane >= row_lo && lane < row_lo + kHead / PARTS)) {
+        } else {
           y[iob + static_cast<int64_t>(t0 + tt) * C + lane] = static_cast<IO>(ys[buf][tt][lane]);
         }
       }
@@ -348,65 +288,489 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
   for (int i = 0; i < RPL; ++i) __builtin_nontemporal_store(S[i], reinterpret_cast<float4_t*>(sblk + i * kHead));
 }
 
-// Heads in flight up to which a head is cut into four (two) row ranges of four wavefronts each, one block per
-// range; above, one block of four wavefronts per head fills the chip.  Single-token calls move a head's state once
-// and are bound by that traffic: whole heads.
-constexpr int kSeqSmallGrid = 128;
-constexpr int kSeqTinyGrid = 64;
 
-bool tmix_seq_whole_heads(int B, int T, int H) { return !(B * H <= kSeqSmallGrid && T > 1); }
+// ---- sequence kernel with feeders (T > 1) ---------------------------------------------------------------------------
+// NC wavefronts own the state and do nothing but steps; NF feeders bring the operands of the next chunk of kSeqChunk tokens
+// into LDS (requested SETS chunks ahead, the decay derived where the caller has logits) and take the finished y rows out.  All
+// meet once per chunk, ahead of the chunk's last step, whose operands are in registers by then.  A block owns 1 / PARTS of a
+// head's rows - they are independent of each other: row i needs its own sum over the columns, v_i and the per-column operands -
+// a lane RPL rows x G groups of four columns.
+//
+// What bounds it.  Few heads (a wavefront per SIMD): a wavefront issues an instruction every 5 to 6 clocks at best and every 8.5
+// where it needs the one before (16 through DPP), so the step is its instruction count, 36, times six: 0.11 us measured.  The
+// staging used to stand in the same instruction stream, and five fp32 vectors per token and wavefront took the CU's LDS 170 of
+// a step's 350 clocks; fp16 operands now stay fp16 in LDS (the mixed-precision multiply-add takes them as they are): 104.  Many
+// heads: VALU issue, four clocks per instruction and SIMD; eight columns per lane put one of a row's four adds over lanes into the
+// lane (24 instead of 28 operations per four elements).  us per call, before / now:
+//   1 x 64 tokens x 12 heads, fp32 tensors 13.4 / 10.6   1 x 512 x 64, fp16 84.8 / 57   3 x 333 x 32 72 / 56
+//   4 x 256 x 64 83.7 / 70   8 x 256 x 64 125 / 113   16 x 256 x 64 223 / 213
+template <typename E, int N>
+struct Loose {  // N elements that are aligned like one
+  typedef E type __attribute__((ext_vector_type(N), aligned(sizeof(E))));
+};
 
-template <typename IO, int SRC>
-static void launch_seq(hipStream_t st, int B, int T, int C, int H, float* state, const float* r, const float* d,
-                       const float* k, const float* a, const float* b, int64_t op_bs, const IO* v, IO* y, int64_t io_bs,
-                       const TmixSeqArgs& fa, const RawOperands& ro) {
-  if constexpr (SRC != kSrcFused) {
-    if (B * H <= kSeqTinyGrid && T > 1) {
-      hipLaunchKernelGGL((wkv7_seq_kernel<IO, 1, 4, SRC>), dim3(B * H * 4), dim3(256), 0, st, T, C, H, state, r, d, k, a, b,
-                         op_bs, v, y, io_bs, fa, ro);
-      return;
+// A chunk's operands in LDS.  The 16 groups of four columns of a token lie in the order in which the lanes of a row read
+// them: lane e takes groups G e .. G e + G - 1, its m-th at place m * 16 / G + e, so that the lanes' pieces are neighbours.
+template <typename OT>
+struct SeqStage;
+template <>
+struct SeqStage<half_t> {  // a and b (k and r) of a group share a 16-byte piece
+  half_t ab[kSeqChunk][16][8];
+  half_t kr[kSeqChunk][16][8];
+  float d[kSeqChunk][16][4];
+  half_t v[kSeqChunk][kHead];
+  __device__ __forceinline__ half_t* a_at(int t, int p) { return &ab[t][p][0]; }
+  __device__ __forceinline__ half_t* b_at(int t, int p) { return &ab[t][p][4]; }
+  __device__ __forceinline__ half_t* k_at(int t, int p) { return &kr[t][p][0]; }
+  __device__ __forceinline__ half_t* r_at(int t, int p) { return &kr[t][p][4]; }
+};
+template <>
+struct SeqStage<float> {
+  float a[kSeqChunk][16][4], b[kSeqChunk][16][4], k[kSeqChunk][16][4], r[kSeqChunk][16][4];
+  float d[kSeqChunk][16][4];
+  float v[kSeqChunk][kHead];
+  __device__ __forceinline__ float* a_at(int t, int p) { return &a[t][p][0]; }
+  __device__ __forceinline__ float* b_at(int t, int p) { return &b[t][p][0]; }
+  __device__ __forceinline__ float* k_at(int t, int p) { return &k[t][p][0]; }
+  __device__ __forceinline__ float* r_at(int t, int p) { return &r[t][p][0]; }
+};
+
+// The operands of one step in a lane's registers.
+template <typename OT, int G, int RPL>
+struct SeqStep {
+  typedef OT vec4 __attribute__((ext_vector_type(4)));
+  typedef OT vec8 __attribute__((ext_vector_type(8)));
+  typedef OT rows_t __attribute__((ext_vector_type(RPL)));
+  vec4 a[G], b[G], k[G], r[G];
+  float4_t d[G];
+  rows_t v;
+  __device__ __forceinline__ void load(SeqStage<OT>& st, int t, int e, int row) {
+#pragma unroll
+    for (int m = 0; m < G; ++m) {
+      const int p = m * (16 / G) + e;
+      if constexpr (sizeof(OT) == 2) {
+        const vec8 ab = *reinterpret_cast<const vec8*>(st.a_at(t, p));
+        const vec8 kr = *reinterpret_cast<const vec8*>(st.k_at(t, p));
+        a[m] = __builtin_shufflevector(ab, ab, 0, 1, 2, 3);
+        b[m] = __builtin_shufflevector(ab, ab, 4, 5, 6, 7);
+        k[m] = __builtin_shufflevector(kr, kr, 0, 1, 2, 3);
+        r[m] = __builtin_shufflevector(kr, kr, 4, 5, 6, 7);
+      } else {
+        a[m] = *reinterpret_cast<const vec4*>(st.a_at(t, p));
+        b[m] = *reinterpret_cast<const vec4*>(st.b_at(t, p));
+        k[m] = *reinterpret_cast<const vec4*>(st.k_at(t, p));
+        r[m] = *reinterpret_cast<const vec4*>(st.r_at(t, p));
+      }
+      d[m] = *reinterpret_cast<const float4_t*>(&st.d[t][p][0]);
     }
-    if (B * H <= kSeqSmallGrid && T > 1) {
-      hipLaunchKernelGGL((wkv7_seq_kernel<IO, 2, 2, SRC>), dim3(B * H * 2), dim3(256), 0, st, T, C, H, state, r, d, k, a, b,
-                         op_bs, v, y, io_bs, fa, ro);
-      return;
-    }
+    v = *reinterpret_cast<const rows_t*>(&st.v[t][row]);
   }
-  if (T == 1) {
-    hipLaunchKernelGGL((wkv7_seq_kernel<IO, 4, 1, SRC, false>), dim3(B * H), dim3(256), 0, st, T, C, H, state, r, d, k, a, b,
-                       op_bs, v, y, io_bs, fa, ro);
+};
+
+__device__ __forceinline__ void seq_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// x * y where either may be fp16.  minus_zero holds -0.0 in a register the compiler cannot see through: the mixed-precision
+// multiply-add then takes fp16 operands as they are (x * y + -0.0 is x * y to the bit), where a product would convert first.
+template <typename X, typename Y>
+__device__ __forceinline__ float seq_product(X x, Y y, float minus_zero) {
+  if constexpr (sizeof(X) == 2 || sizeof(Y) == 2) return fmaf(static_cast<float>(x), static_cast<float>(y), minus_zero);
+  else return x * y;
+}
+
+template <typename IO, typename WT, int G, int RPL, int NC, int PARTS, int NF, int SETS, int WAVES, bool AHEAD>
+__global__ __launch_bounds__(64 * (NC + NF), WAVES) void wkv7_feed_kernel(int T, int C, int H, float* __restrict__ state, SeqOperands<IO, WT> op,
+                                                                         IO* __restrict__ y) {
+  constexpr int kRows = kHead / PARTS;        // rows of the state per block
+  constexpr int LPR = 16 / G;                 // lanes per row
+  static_assert(NC * RPL * (64 / LPR) == kRows, "the compute wavefronts own the block's rows");
+  __shared__ __align__(16) SeqStage<IO> stage[2];
+  // y of a chunk: one buffer written, one read by the feeders, and the one between, whose last token is still being written
+  __shared__ __align__(16) float ys[3][kSeqChunk][kRows];
+  __shared__ __align__(16) float spare[kSeqChunk * kRows + 64 * RPL];  // where the idle lanes of a row store
+  const int bh = blockIdx.x / PARTS;
+  const int row_lo = (blockIdx.x % PARTS) * kRows;
+  const int bi = bh / H;
+  const int h = bh - bi * H;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int64_t base = static_cast<int64_t>(bi) * T * C + h * kHead;
+  const int chunks = (T + kSeqChunk - 1) / kSeqChunk;
+
+  if (wave >= NC) {
+    // feeder f: tokens f * TPF .. of a chunk, CPF columns of one of them per lane
+    constexpr int TPF = kSeqChunk / NF, LPT = 64 / TPF, CPF = kHead / LPT;
+    using vec = typename Loose<IO, CPF>::type;
+    using wvec = typename Loose<WT, CPF>::type;
+    struct Set {
+      vec a, b, k, r, v;
+      wvec w;
+    };
+    Set set[SETS];
+    const int f = wave - NC;
+    const int tok = f * TPF + lane / LPT;
+    const int col = (lane % LPT) * CPF;
+    // (every load unconditional: tokens past the end repeat the last one, their steps never run)
+    auto request = [&](Set& s, int c) {
+      const int64_t at = base + static_cast<int64_t>(min(c * kSeqChunk + tok, T - 1)) * C + col;
+      s.a = *reinterpret_cast<const vec*>(op.a + at);
+      s.b = *reinterpret_cast<const vec*>(op.b + at);
+      s.w = *reinterpret_cast<const wvec*>(op.w + at);
+      s.k = *reinterpret_cast<const vec*>(op.k + at);
+      s.r = *reinterpret_cast<const vec*>(op.r + at);
+      s.v = *reinterpret_cast<const vec*>(op.v + at);
+    };
+    auto commit = [&](const Set& s, SeqStage<IO>& st) {
+      constexpr int PW = CPF < 4 ? CPF : 4;  // columns of a piece
+      typedef IO piece __attribute__((ext_vector_type(PW)));
+      typedef float fpiece __attribute__((ext_vector_type(PW)));
+#pragma unroll
+      for (int g = 0; g < CPF / PW; ++g) {
+        const int c = (col + g * PW) >> 2;
+        const int p = (c % G) * LPR + c / G;
+        const int in = (col + g * PW) & 3;
+        piece a, b, k, r;
+        fpiece d;
+#pragma unroll
+        for (int i = 0; i < PW; ++i) {
+          a[i] = s.a[g * PW + i];
+          b[i] = s.b[g * PW + i];
+          k[i] = s.k[g * PW + i];
+          r[i] = s.r[g * PW + i];
+          d[i] = static_cast<float>(s.w[g * PW + i]);
+        }
+        if (op.w_mode == RWKV_W_RAW_LOGIT) {
+#pragma unroll
+          for (int i = 0; i < PW; ++i) d[i] = decay_from_logit(d[i]);
+        }
+        *reinterpret_cast<piece*>(st.a_at(tok, p) + in) = a;
+        *reinterpret_cast<piece*>(st.b_at(tok, p) + in) = b;
+        *reinterpret_cast<piece*>(st.k_at(tok, p) + in) = k;
+        *reinterpret_cast<piece*>(st.r_at(tok, p) + in) = r;
+        *reinterpret_cast<fpiece*>(&st.d[tok][p][in]) = d;
+      }
+      typedef IO store_v __attribute__((ext_vector_type(CPF)));
+      *reinterpret_cast<store_v*>(&st.v[tok][col]) = s.v;
+    };
+    // the finished y rows of a chunk: EW neighbouring rows per lane
+    auto write_out = [&](int c, int slot) {
+      constexpr int EW = PARTS == 1 ? CPF : 2;
+      constexpr int kPieces = kSeqChunk * kRows / EW;
+      typedef float fvec __attribute__((ext_vector_type(EW)));
+      using ovec = typename Loose<IO, EW>::type;
+      const int n = min(kSeqChunk, T - c * kSeqChunk);
+#pragma unroll
+      for (int i = 0; i < (kPieces + 64 * NF - 1) / (64 * NF); ++i) {
+        const int idx = f * 64 + lane + i * 64 * NF;
+        const int t = idx / (kRows / EW);
+        const int r = idx % (kRows / EW) * EW;
+        if (t < n) {
+          const fvec yv = *reinterpret_cast<const fvec*>(&ys[slot][t][r]);
+          ovec o;
+#pragma unroll
+          for (int e = 0; e < EW; ++e) o[e] = static_cast<IO>(yv[e]);
+          *reinterpret_cast<ovec*>(y + base + static_cast<int64_t>(c * kSeqChunk + t) * C + row_lo + r) = o;
+        }
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < SETS; ++i) request(set[i], i);
+    commit(set[0], stage[0]);
+    request(set[0], SETS);
+    commit(set[1 % SETS], stage[1]);
+    request(set[1 % SETS], SETS + 1);
+    seq_barrier();  // chunks 0 and 1 are staged
+    int slot = 2;   // of chunk c - 1
+    // chunk c has been read (its last step runs from registers): chunk c + 2 takes its place
+    auto turn = [&](int u, int c) {
+      seq_barrier();
+      commit(set[(u + 2) % SETS], stage[u & 1]);
+      request(set[(u + 2) % SETS], c + 2 + SETS);
+      if (c > 0) write_out(c - 1, slot);
+      slot = slot == 2 ? 0 : slot + 1;
+    };
+    const int whole = chunks - chunks % SETS;
+    int c0 = 0;
+    for (; c0 < whole; c0 += SETS) {
+#pragma unroll
+      for (int u = 0; u < SETS; ++u) turn(u, c0 + u);
+    }
+#pragma unroll
+    for (int u = 0; u < SETS - 1; ++u) {
+      if (c0 + u >= chunks) break;
+      turn(u, c0 + u);
+    }
+    seq_barrier();  // all steps are done
+    write_out(chunks - 1, slot);
+    return;
+  }
+
+  const int e = lane % LPR;
+  const int row = RPL * ((64 / LPR) * wave + lane / LPR);  // first of this lane's rows in the block
+  float* sblk = state + (static_cast<int64_t>(bh) * kHead + row_lo + row) * kHead + 4 * G * e;
+  float4_t S[RPL][G];
+#pragma unroll
+  for (int i = 0; i < RPL; ++i)
+#pragma unroll
+    for (int m = 0; m < G; ++m) S[i][m] = __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(sblk + i * kHead + 4 * m));
+
+  float minus_zero = -0.0f;
+  asm volatile("" : "+s"(minus_zero));
+  using Step = SeqStep<IO, G, RPL>;
+  typedef typename Step::vec4 vec4;
+  typedef float frows __attribute__((ext_vector_type(RPL)));
+  // One step of the recurrence together with the output sums of the step before it, which read the same state:
+  //   y' = S r' of the step before, sa = S a, S = S d + sa b + k v
+  // The sum over a row's 64 columns: four columns in a chain, then groups 2n and 2n + 1, and so on up - in the lane as far as
+  // it holds them, over the lanes of the row from there - the same tree whatever G.
+  // A wavefront that is alone on its SIMD waits 8 clocks for the result of the instruction before (12 where a DPP move reads
+  // it), so the order is laid down here: the two chains of products alternate, the products k v stand between the DPP adds,
+  // and no instruction needs one of the two before it.
+  auto step = [&](const Step& q, const vec4 (&r_before)[G], float* dst) {
+    float sa[RPL], out[RPL], p[RPL][G], o[RPL][G], kv[RPL][G][4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+#pragma unroll
+      for (int i = 0; i < RPL; ++i)
+#pragma unroll
+        for (int m = 0; m < G; ++m) {
+          p[i][m] = x == 0 ? seq_product(S[i][m][0], q.a[m][0], minus_zero) : fmaf(S[i][m][x], static_cast<float>(q.a[m][x]), p[i][m]);
+          o[i][m] = x == 0 ? seq_product(S[i][m][0], r_before[m][0], minus_zero)
+                           : fmaf(S[i][m][x], static_cast<float>(r_before[m][x]), o[i][m]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    auto in_lane = [](const float (&t)[G]) {
+      if constexpr (G == 1) return t[0];
+      else if constexpr (G == 2) return t[0] + t[1];
+      else return (t[0] + t[1]) + (t[2] + t[3]);
+    };
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+      sa[i] = in_lane(p[i]);
+      out[i] = in_lane(o[i]);
+    }
+    constexpr int kLevels = G == 1 ? 4 : (G == 2 ? 3 : 2);
+    constexpr int kProducts = RPL * G * 4;
+    auto products = [&](int from, int to) {
+#pragma unroll
+      for (int j = from; j < to; ++j) {
+        const int x = j % 4, m = j / 4 % G, i = j / (4 * G);
+        kv[i][m][x] = seq_product(q.k[m][x], q.v[i], minus_zero);
+        asm volatile("" : "+v"(kv[i][m][x]));  // here, not at its use
+      }
+    };
+#pragma unroll
+    for (int l = 0; l < kLevels; ++l) {
+      products(l * kProducts / kLevels, (l + 1) * kProducts / kLevels);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < RPL; ++i) {
+        auto add = [&](float v) {
+          if (l == 0) return dpp_add<0xB1>(v);   // quad_perm [1,0,3,2]
+          if (l == 1) return dpp_add<0x4E>(v);   // quad_perm [2,3,0,1]
+          if (l == 2) return dpp_add<0x141>(v);  // row_half_mirror
+          return dpp_add<0x140>(v);              // row_mirror
+        };
+        sa[i] = add(sa[i]);
+        out[i] = add(out[i]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < RPL; ++i)
+#pragma unroll
+      for (int m = 0; m < G; ++m)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) kv[i][m][x] = fmaf(sa[i], static_cast<float>(q.b[m][x]), kv[i][m][x]);
+    frows yy;
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) yy[i] = out[i];
+    *reinterpret_cast<frows*>(dst) = yy;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < RPL; ++i)
+#pragma unroll
+      for (int m = 0; m < G; ++m)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) S[i][m][x] = fmaf(S[i][m][x], q.d[m][x], kv[i][m][x]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto row_sums = [&](const vec4 (&x)[G], float (&sum)[RPL]) {
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+      float p[G];
+#pragma unroll
+      for (int m = 0; m < G; ++m) {
+        p[m] = seq_product(S[i][m].x, x[m][0], minus_zero);
+        p[m] = fmaf(S[i][m].y, static_cast<float>(x[m][1]), p[m]);
+        p[m] = fmaf(S[i][m].z, static_cast<float>(x[m][2]), p[m]);
+        p[m] = fmaf(S[i][m].w, static_cast<float>(x[m][3]), p[m]);
+      }
+      if constexpr (G == 1) sum[i] = p[0];
+      else if constexpr (G == 2) sum[i] = p[0] + p[1];
+      else sum[i] = (p[0] + p[1]) + (p[2] + p[3]);
+    }
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+      sum[i] = dpp_add<0xB1>(sum[i]);
+      sum[i] = dpp_add<0x4E>(sum[i]);
+      if constexpr (LPR >= 8) sum[i] = dpp_add<0x141>(sum[i]);
+      if constexpr (LPR >= 16) sum[i] = dpp_add<0x140>(sum[i]);
+    }
+  };
+  // All lanes of a row hold its sums: the first stores them, the others store to a spare area (a store under a branch would
+  // end the scheduling region).
+  float* idle = &spare[lane * RPL];
+  int slot = 0;
+  seq_barrier();  // chunks 0 and 1 are staged
+  if constexpr (AHEAD) {
+    float* y_before = idle;  // where the sums of the step before go
+    vec4 r_before[G];
+#pragma unroll
+    for (int m = 0; m < G; ++m) r_before[m] = vec4{};
+    Step cur;
+    cur.load(stage[0], 0, e, row_lo + row);
+    for (int c = 0; c < chunks; ++c) {
+      SeqStage<IO>& st = stage[c & 1];
+      SeqStage<IO>& after = stage[(c & 1) ^ 1];
+      float* dst = e == 0 ? &ys[slot][0][row] : idle;
+      slot = slot == 2 ? 0 : slot + 1;
+      const int n = T - c * kSeqChunk;
+      if (n >= kSeqChunk) {
+        // the operands of step t + 1 are read from LDS while step t computes
+#pragma unroll
+        for (int t = 0; t < kSeqChunk; ++t) {
+          Step next;
+          if (t + 1 < kSeqChunk) {
+            next.load(st, t + 1, e, row_lo + row);
+          } else {
+            seq_barrier();
+            next.load(after, 0, e, row_lo + row);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          step(cur, r_before, t == 0 ? y_before : dst + (t - 1) * kRows);
+#pragma unroll
+          for (int m = 0; m < G; ++m) r_before[m] = cur.r[m];
+          cur = next;
+        }
+        y_before = dst + (kSeqChunk - 1) * kRows;
+      } else {  // the last, partial chunk
+#pragma unroll 1
+        for (int t = 0; t < n; ++t) {
+          cur.load(st, t, e, row_lo + row);
+          step(cur, r_before, y_before);
+#pragma unroll
+          for (int m = 0; m < G; ++m) r_before[m] = cur.r[m];
+          y_before = dst + t * kRows;
+        }
+        seq_barrier();
+      }
+    }
+    float out[RPL];  // the output sums of the last step
+    row_sums(r_before, out);
+    frows yy;
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) yy[i] = out[i];
+    *reinterpret_cast<frows*>(y_before) = yy;
   } else {
-    hipLaunchKernelGGL((wkv7_seq_kernel<IO, 4, 1, SRC>), dim3(B * H), dim3(256), 0, st, T, C, H, state, r, d, k, a, b, op_bs,
-                       v, y, io_bs, fa, ro);
+    // many wavefronts per SIMD: they hide each other's latencies, and registers are what limits their number
+    for (int c = 0; c < chunks; ++c) {
+      SeqStage<IO>& st = stage[c & 1];
+      float* dst = e == 0 ? &ys[slot][0][row] : idle;
+      slot = slot == 2 ? 0 : slot + 1;
+      auto token = [&](int t) {
+        Step q;
+        q.load(st, t, e, row_lo + row);
+        float sa[RPL], out[RPL];
+        row_sums(q.a, sa);
+#pragma unroll
+        for (int i = 0; i < RPL; ++i)
+#pragma unroll
+          for (int m = 0; m < G; ++m)
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              S[i][m][x] = fmaf(S[i][m][x], q.d[m][x], fmaf(sa[i], static_cast<float>(q.b[m][x]), seq_product(q.k[m][x], q.v[i], minus_zero)));
+        row_sums(q.r, out);
+        frows yy;
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) yy[i] = out[i];
+        *reinterpret_cast<frows*>(dst + t * kRows) = yy;
+      };
+      const int n = T - c * kSeqChunk;
+      if (n >= kSeqChunk) {
+#pragma unroll
+        for (int t = 0; t < kSeqChunk; ++t) token(t);
+      } else {
+#pragma unroll 1
+        for (int t = 0; t < n; ++t) token(t);
+      }
+      seq_barrier();
+    }
+  }
+  seq_barrier();  // all steps are done
+#pragma unroll
+  for (int i = 0; i < RPL; ++i)
+#pragma unroll
+    for (int m = 0; m < G; ++m) __builtin_nontemporal_store(S[i][m], reinterpret_cast<float4_t*>(sblk + i * kHead + 4 * m));
+}
+
+template <typename IO, typename WT, bool FUSED>
+static void launch_seq(hipStream_t st, int B, int T, int C, int H, float* state, const IO* v, IO* y, const TmixSeqArgs& fa,
+                       const SeqOperands<IO, WT>& ro) {
+  const int64_t io_bs = static_cast<int64_t>(T) * C;
+  if (T == 1) {
+    hipLaunchKernelGGL((wkv7_seq_kernel<IO, WT, 4, FUSED, false>), dim3(B * H), dim3(256), 0, st, T, C, H, state, v, y, io_bs, fa, ro);
+  } else if constexpr (FUSED) {
+    hipLaunchKernelGGL((wkv7_seq_kernel<IO, WT, 4, FUSED>), dim3(B * H), dim3(256), 0, st, T, C, H, state, v, y, io_bs, fa, ro);
   }
 }
 
-// The C-ABI operator: operands in the io type, read once by the sequence kernel itself.
-template <typename IO>
-static int launch_wkv7(hipStream_t st, int B, int T, int C, int H, int w_mode, float* state, const IO* r,
-                       const IO* w, const IO* k, const IO* v, const IO* a, const IO* b, IO* y) {
-  const int64_t row = static_cast<int64_t>(T) * C;
-  const RawOperands ro = {r, w, k, a, b, w_mode};
-  launch_seq<IO, kSrcRaw>(st, B, T, C, H, state, nullptr, nullptr, nullptr, nullptr, nullptr, 0, v, y, row, TmixSeqArgs{}, ro);
+template <typename IO, typename WT, int G, int RPL, int NC, int PARTS, int NF, int SETS, int WAVES, bool AHEAD>
+static void launch_feed(hipStream_t st, int B, int T, int C, int H, float* state, const SeqOperands<IO, WT>& op, IO* y) {
+  hipLaunchKernelGGL((wkv7_feed_kernel<IO, WT, G, RPL, NC, PARTS, NF, SETS, WAVES, AHEAD>), dim3(B * H * PARTS), dim3(64 * (NC + NF)), 0, st, T, C, H,
+                     state, op, y);
+}
+
+// Which tile a call of more than one token takes.  Up to 128 heads the chip has CUs to spare: a head is cut into row ranges of
+// four wavefronts each, one state row per lane, and every wavefront is alone on its SIMD.  Up to 512 heads (two per CU) whole
+// heads, 2 x 8 elements per lane, the next step's operands read ahead; with more heads, or fp32 operands (twice the
+// registers), wavefronts are worth more than reading ahead (us per token of 16 x 64 heads, 6 per SIMD / 3 reading ahead: 0.83 /
+// 1.05; of 4 x 64 heads 0.29 / 0.27, of 8 x 64 0.46 / 0.44).
+constexpr int kSeqQuarterHeads = 64;
+constexpr int kSeqHalfHeads = 128;
+constexpr int kSeqAheadHeads = 512;
+
+// false: few heads in flight and more than one token, so that the recurrence runs a head's row ranges on separate CUs, which
+// the fused pass cannot: its GroupNorm needs whole heads
+bool tmix_seq_whole_heads(int B, int T, int H) { return !(B * H <= kSeqHalfHeads && T > 1); }
+
+template <typename IO, typename WT>
+static int launch_recurrence(hipStream_t st, int B, int T, int C, int H, float* state, const SeqOperands<IO, WT>& op, IO* y) {
+  if (T == 1) {
+    launch_seq<IO, WT, false>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
+  } else if (B * H <= kSeqQuarterHeads) {
+    launch_feed<IO, WT, 1, 1, 4, 4, 2, 2, 1, true>(st, B, T, C, H, state, op, y);
+  } else if (B * H <= kSeqHalfHeads) {
+    launch_feed<IO, WT, 2, 1, 4, 2, 2, 4, 1, true>(st, B, T, C, H, state, op, y);
+  } else {
+    constexpr bool kHalf = sizeof(IO) == 2;
+    if (kHalf && B * H <= kSeqAheadHeads) launch_feed<IO, WT, 2, 2, 4, 1, 2, 2, kHalf ? 4 : 6, kHalf>(st, B, T, C, H, state, op, y);
+    else launch_feed<IO, WT, 2, 2, 4, 1, 2, 2, 6, false>(st, B, T, C, H, state, op, y);
+  }
   RWKV_LAUNCH_CHECK();
   return RWKV_OK;
 }
 
-int wkv7_seq_f16_launch(hipStream_t st, int B, int T, int C, int H, float* state, const float* r, const float* d,
-                        const float* k, const float* a, const float* b, int64_t op_bs, const half_t* v, half_t* y,
-                        int64_t io_bs) {
-  launch_seq<half_t, kSrcFp32>(st, B, T, C, H, state, r, d, k, a, b, op_bs, v, y, io_bs, TmixSeqArgs{}, RawOperands{});
-  RWKV_LAUNCH_CHECK();
-  return RWKV_OK;
+int wkv7_seq_f16_launch(hipStream_t st, int B, int T, int C, int H, float* state, const half_t* r, const float* d,
+                        const half_t* k, const half_t* a, const half_t* b, const half_t* v, half_t* y) {
+  return launch_recurrence<half_t, float>(st, B, T, C, H, state, SeqOperands<half_t, float>{r, k, v, a, b, d, RWKV_W_DECAY}, y);
 }
 
 int tmix_seq_launch(hipStream_t st, int B, int T, int C, int H, float* state, const TmixSeqArgs& fa, const half_t* v,
                     half_t* y2) {
   RWKV_REQUIRE(fa.r && fa.k && fa.a12 && fa.w12 && fa.g && fa.k_k && fa.a0 && fa.k_a && fa.w0 && fa.r_k && fa.lnx_w && fa.lnx_b,
                "tmix_seq: NULL tensor");
-  const int64_t row = static_cast<int64_t>(T) * C;
-  launch_seq<half_t, kSrcFused>(st, B, T, C, H, state, nullptr, nullptr, nullptr, nullptr, nullptr, 0, v, y2, row, fa,
-                                RawOperands{});
+  launch_seq<half_t, half_t, true>(st, B, T, C, H, state, v, y2, fa, SeqOperands<half_t, half_t>{});
   RWKV_LAUNCH_CHECK();
   return RWKV_OK;
 }
@@ -422,16 +786,13 @@ extern "C" int rwkv_hip_wkv7(rwkv_stream_t s, int B, int T, int C, int H, int w_
   RWKV_REQUIRE(C == H * kHead, "wkv7: C (%d) must equal H*64 (%d)", C, H * kHead);
   RWKV_REQUIRE(w_mode == RWKV_W_RAW_LOGIT || w_mode == RWKV_W_DECAY, "wkv7: bad w_mode %d", w_mode);
   RWKV_REQUIRE(state && r && w && k && v && a && b && y, "wkv7: NULL tensor");
-  if (io == RWKV_IO_F16) {
-    return launch_wkv7<half_t>(as_stream(s), B, T, C, H, w_mode, static_cast<float*>(state),
-                               static_cast<const half_t*>(r), static_cast<const half_t*>(w),
-                               static_cast<const half_t*>(k), static_cast<const half_t*>(v),
-                               static_cast<const half_t*>(a), static_cast<const half_t*>(b),
-                               static_cast<half_t*>(y));
-  }
+  auto run = [&](auto type) {
+    using IO = decltype(type);
+    const SeqOperands<IO, IO> op = {static_cast<const IO*>(r), static_cast<const IO*>(k), static_cast<const IO*>(v),
+                                    static_cast<const IO*>(a), static_cast<const IO*>(b), static_cast<const IO*>(w), w_mode};
+    return launch_recurrence<IO, IO>(as_stream(s), B, T, C, H, static_cast<float*>(state), op, static_cast<IO*>(y));
+  };
+  if (io == RWKV_IO_F16) return run(half_t{});
   RWKV_REQUIRE(io == RWKV_IO_F32, "wkv7: bad io %d", io);
-  return launch_wkv7<float>(as_stream(s), B, T, C, H, w_mode, static_cast<float*>(state),
-                            static_cast<const float*>(r), static_cast<const float*>(w),
-                            static_cast<const float*>(k), static_cast<const float*>(v),
-                            static_cast<const float*>(a), static_cast<const float*>(b), static_cast<float*>(y));
+  return run(float{});
 }

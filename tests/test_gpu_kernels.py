@@ -231,6 +231,43 @@ def test_wkv7_small_and_large_grids_agree_bitwise(gpu):
         assert same
 
 
+@pytest.mark.parametrize("B,H", [(1, 3), (2, 32), (5, 13), (4, 32), (3, 43), (8, 64), (9, 57)])
+@pytest.mark.parametrize("io", ["f16", "f32"])
+def test_wkv7_call_of_several_tokens_is_bitwise_its_single_tokens(gpu, B, H, io):
+    """At the heads on either side of every change of tile (64, 128, 512), at lengths around its chunks of eight tokens: a call
+    of T tokens against T calls of one token, which take another kernel.  The operands start one element behind a 16-byte
+    boundary."""
+    hip = gpu
+    T, C = 35, H * 64
+    dt = np.float16 if io == "f16" else np.float32
+    inp = wkv_inputs(B, T, H, seed=B + H, dtype=dt)
+    names = ["r", "w_raw", "k", "v", "a", "b"]
+    mode = hip.IO_F16 if io == "f16" else hip.IO_F32
+    item = np.dtype(dt).itemsize
+    state1 = hip.DeviceArray.zeros((B, H, 64, 64), np.float32)
+    rows = []
+    for t in range(T):
+        d = [dev(hip, np.ascontiguousarray(inp[n][:, t])) for n in names]
+        y = hip.DeviceArray((B, 1, C), dt)
+        hip.wkv7(B, 1, C, H, hip.W_RAW_LOGIT, mode, state1, *d, y)
+        rows.append(y.numpy())
+    want = np.concatenate(rows, axis=1)
+    want_state = state1.numpy()
+    state = hip.DeviceArray.zeros((B, H, 64, 64), np.float32)
+    t0 = 0
+    for n_tok in (2, 7, 8, 9, 1, 8):          # 35 tokens
+        shifted = [dev(hip, np.concatenate([np.zeros(1, dt), np.ascontiguousarray(inp[n][:, t0:t0 + n_tok]).reshape(-1)])) for n in names]
+        y = hip.DeviceArray.zeros((1 + B * n_tok * C,), dt)
+        hip.wkv7(B, n_tok, C, H, hip.W_RAW_LOGIT, mode, state, *[s.ptr + item for s in shifted], y.ptr + item)
+        got = y.numpy()
+        assert got[0] == 0
+        same = np.array_equal(got[1:].reshape(B, n_tok, C), want[:, t0:t0 + n_tok])
+        assert same, (n_tok, t0)
+        t0 += n_tok
+    same = np.array_equal(state.numpy(), want_state)
+    assert t0 == T and same
+
+
 # ------------------------------------------------------------------------------- checkpoint tensors
 def test_bf16_to_f16_every_pattern_and_transposes_bit_exact(gpu, orc):
     hip = gpu
