@@ -12,9 +12,9 @@
 // two fp16 terms, hi = f16(a) and lo = f16(a - hi): hi + lo carries 22 bits of a, both products with the fp16
 // weight are exact in fp32, and the result differs from an fp32 dot only by summation order.  Without an
 // activation the hidden is fp16 already and the lo term is skipped.  One launch takes up to four problems
-// (w, a, g, v of a layer): grid = (C/128, row blocks, problems), block = 2 groups of 4 wavefronts x 32 output
+// (w, a, g, v of a layer): grid = (C/128, row tiles, problems), block = 2 groups of 4 wavefronts x 32 output
 // channels (the groups take alternate 16-wide steps of the rank and add up through LDS), the 32 x R slice of
-// act(h) of a row tile staged in LDS.
+// act(h) of a row tile staged in LDS; many rows take wider blocks (lora_out_wide_kernel).
 #include <algorithm>
 #include <cstdint>
 
@@ -31,9 +31,8 @@ constexpr int kLoraKG = 2;       // wavefront groups that split the rank between
 constexpr int kLoraThreads = 2 * kLoraCols * kLoraKG;
 constexpr int kLoraStage = (kLoraRows * (kLoraMaxR / 8 + 1) + kLoraThreads - 1) / kLoraThreads;  // pieces per thread
 
-// Per row tile: every lane requests its whole weight row (up to 16 pieces of 8; once per block - a block keeps
-// its weights over all its row tiles), its pieces of the 32 x R hidden slice and its piece of the epilogue
-// operands (v, v_first) in one go; the block turns the hidden slice into hi / lo fp16 in LDS (one barrier), each
+// Every lane requests its whole weight row (up to 16 pieces of 8), its pieces of the 32 x R hidden slice and its
+// piece of the epilogue operands (v, v_first) in one go; the block turns the hidden slice into hi / lo fp16 in LDS (one barrier), each
 // wavefront runs its MFMA steps, both groups lay their 32 x 128 sums out in LDS (over the hi / lo tiles, free by
 // then) and all threads add the two in group order, apply the epilogue and write 16 bytes of a row each.
 //
@@ -89,113 +88,241 @@ __global__ __launch_bounds__(kLoraThreads) void lora_out_kernel(LoraOutMultiArgs
   uint4_t bias_raw = *reinterpret_cast<const uint4_t*>((p.bias ? p.bias : p.w2) + (ocol_ok ? ocol : 0));
 
   const int pieces = (R >> 3) + 1;  // R/8 pieces of 8 per row + the zeroed pad
-  const int row_tiles = (a.M + kLoraRows - 1) / kLoraRows;
-  auto row_tile = [&](int rt, bool more) {
-    const int m0 = rt * kLoraRows;
-    const int mn = min(kLoraRows, a.M - m0);
-    uint4_t hv[kLoraStage];  // all of them loaded, whatever the rank: a value left undefined costs more than the load
+  const int m0 = blockIdx.y * kLoraRows;
+  const int mn = min(kLoraRows, a.M - m0);
+  uint4_t hv[kLoraStage];  // all of them loaded, whatever the rank: a value left undefined costs more than the load
 #pragma unroll
-    for (int i = 0; i < kLoraStage; ++i) {
+  for (int i = 0; i < kLoraStage; ++i) {
+    const int idx = threadIdx.x + i * kLoraThreads;
+    const int m = idx / pieces;
+    const int ks = (idx - m * pieces) * 8;
+    hv[i] = *reinterpret_cast<const uint4_t*>(p.h + static_cast<int64_t>(m0 + (m < mn ? m : mn - 1)) * R +
+                                              (ks < R ? ks : R - 8));
+  }
+  const int64_t o = static_cast<int64_t>(m0 + (orow < mn ? orow : mn - 1)) * a.C + (ocol_ok ? ocol : 0);
+  // without the v-residual gate: the output row itself, readable and unused
+  half8_t v8 = *reinterpret_cast<const half8_t*>((p.vres ? p.v : p.out) + o);
+  half8_t vf8 = *reinterpret_cast<const half8_t*>((p.vres ? p.v_first : p.out) + o);
+  __builtin_amdgcn_sched_barrier(0);
+  // keeps the conversion of the bias below the loads above: moved up beside its own load, it would wait for the
+  // weights before the hidden slice is even requested
+  asm volatile("" : "+v"(bias_raw));
+  const half8_t bias8 = __builtin_bit_cast(half8_t, bias_raw);
+
+#pragma unroll
+  for (int i = 0; i < kLoraStage; ++i) {
+    if (i * kLoraThreads < kLoraRows * pieces) {
       const int idx = threadIdx.x + i * kLoraThreads;
       const int m = idx / pieces;
       const int ks = (idx - m * pieces) * 8;
-      hv[i] = *reinterpret_cast<const uint4_t*>(p.h + static_cast<int64_t>(m0 + (m < mn ? m : mn - 1)) * R +
-                                                (ks < R ? ks : R - 8));
+      if (m < kLoraRows) {
+        const bool live = m < mn && ks < R;  // rows past M and the pad hold exact zeros
+        const half8_t raw = __builtin_bit_cast(half8_t, hv[i]);
+        half8_t hi, lo;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          float f = h2f(raw[e]);
+          if (p.act == RWKV_ACT_TANH) f = tanh_f(f);
+          if (p.act == RWKV_ACT_SIGMOID) f = sigmoid_f(f);
+          if (!live) f = 0.0f;
+          hi[e] = f2h(f);
+          lo[e] = f2h(f - h2f(hi[e]));
+        }
+        *reinterpret_cast<half8_t*>(&hi_s[m * ld + ks]) = hi;
+        if (split) *reinterpret_cast<half8_t*>(&lo_s[m * ld + ks]) = lo;
+      }
     }
-    const int64_t o = static_cast<int64_t>(m0 + (orow < mn ? orow : mn - 1)) * a.C + (ocol_ok ? ocol : 0);
-    // without the v-residual gate: the output row itself, readable and unused
-    half8_t v8 = *reinterpret_cast<const half8_t*>((p.vres ? p.v : p.out) + o);
-    half8_t vf8 = *reinterpret_cast<const half8_t*>((p.vres ? p.v_first : p.out) + o);
-    __builtin_amdgcn_sched_barrier(0);
-    // keeps the conversion of the bias below the loads above: moved up beside its own load, it would wait for the
-    // weights before the hidden slice is even requested
-    asm volatile("" : "+v"(bias_raw));
-    const half8_t bias8 = __builtin_bit_cast(half8_t, bias_raw);
+  }
+  __syncthreads();
 
+  float16_t acc;
 #pragma unroll
-    for (int i = 0; i < kLoraStage; ++i) {
-      if (i * kLoraThreads < kLoraRows * pieces) {
-        const int idx = threadIdx.x + i * kLoraThreads;
-        const int m = idx / pieces;
-        const int ks = (idx - m * pieces) * 8;
-        if (m < kLoraRows) {
-          const bool live = m < mn && ks < R;  // rows past M and the pad hold exact zeros
-          const half8_t raw = __builtin_bit_cast(half8_t, hv[i]);
-          half8_t hi, lo;
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            float f = h2f(raw[e]);
-            if (p.act == RWKV_ACT_TANH) f = tanh_f(f);
-            if (p.act == RWKV_ACT_SIGMOID) f = sigmoid_f(f);
-            if (!live) f = 0.0f;
-            hi[e] = f2h(f);
-            lo[e] = f2h(f - h2f(hi[e]));
-          }
-          *reinterpret_cast<half8_t*>(&hi_s[m * ld + ks]) = hi;
-          if (split) *reinterpret_cast<half8_t*>(&lo_s[m * ld + ks]) = lo;
+  for (int i = 0; i < kSteps; ++i) {
+    const int k = (i * kLoraKG + kg) * 16;
+    if (k < R) {
+      const half8_t ah = *reinterpret_cast<const half8_t*>(&hi_s[j * ld + k + h * 8]);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, w[i], acc, 0, 0, 0);
+      if (split) {
+        const half8_t al = *reinterpret_cast<const half8_t*>(&lo_s[j * ld + k + h * 8]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, w[i], acc, 0, 0, 0);
+      }
+    }
+  }
+  __syncthreads();  // the hidden tiles are free: group 0 lays its sums over hi_s, group 1 over lo_s
+  // accumulator v of lane (j, h): row 8*(v/4) + 4h + v%4, column wave*32 + j
+  float* tile = reinterpret_cast<float*>(kg == 0 ? hi_s : lo_s);
+#pragma unroll
+  for (int v = 0; v < 16; ++v) tile[(8 * (v / 4) + 4 * h + (v % 4)) * kLoraOutLd + wave * 32 + j] = acc[v];
+  __syncthreads();
+
+  const float* t0 = reinterpret_cast<const float*>(hi_s) + orow * kLoraOutLd + (threadIdx.x & 15) * 8;
+  const float* t1 = reinterpret_cast<const float*>(lo_s) + orow * kLoraOutLd + (threadIdx.x & 15) * 8;
+  float sum[8];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const float4_t s0 = *reinterpret_cast<const float4_t*>(t0 + 4 * q);
+    const float4_t s1 = *reinterpret_cast<const float4_t*>(t1 + 4 * q);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum[4 * q + e] = s0[e] + s1[e];
+  }
+  half8_t res;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float b = p.bias ? h2f(bias8[e]) : 0.0f;
+    if (p.vres) {
+      const float vv = h2f(v8[e]);
+      const float gate = sigmoid_f(b + sum[e]);
+      res[e] = f2h(vv + (h2f(vf8[e]) - vv) * gate);
+    } else {
+      res[e] = f2h(sum[e] + b);
+    }
+  }
+  if (orow < mn && ocol_ok) *reinterpret_cast<half8_t*>(p.out + o) = res;
+}
+
+// The same products for many rows.  The kernel above evaluates the activation of a hidden value once per 128 output channels
+// and takes the sums through LDS and two barriers; this one takes 32 rows x 32*NW channels per block.  The weights are the
+// A operand: accumulator v of lane (j, h) is row j of the tile, and the channels are dealt to A's rows so that a lane's 16
+// values are 16 consecutive channels (16*h + v of the wavefront's 32) and leave in 16-byte stores straight from the registers.
+// A wavefront walks the whole rank with the weights of four steps in flight; its sums are built as above (even and odd
+// steps apart, hi before lo, then added), so the bits are the same.
+// Per rank step a CU's wavefronts ask as many cycles of LDS (the hidden) and of the vector memory path (the weights) as of
+// the matrix core.  Tiles of 64 rows or 64 channels per wavefront ask for half of one of them and lose as much to occupancy
+// (2048 rows x 4096 channels, ranks 128 / 128 / 480 / 96: 66-92 us against 57).
+template <int NW>
+__global__ __launch_bounds__(NW * 64) void lora_out_wide_kernel(LoraOutMultiArgs a) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  constexpr int kTpr = NW * 64 / kLoraRows;                      // threads that stage one row
+  constexpr int kStage = (kLoraMaxR / 8 + 1 + kTpr - 1) / kTpr;  // pieces of 8 per thread, the zeroed pad among them
+  constexpr int kDepth = 4;                                      // rank steps whose weights are in flight
+  const LoraOutProblem& p = a.p[blockIdx.z];
+  const int R = p.R;
+  const int ld = R + 8;
+  const int steps = (R + 15) >> 4;
+  const bool split = p.act != RWKV_ACT_NONE;
+  half_t* hi_s = reinterpret_cast<half_t*>(lds_raw);
+  half_t* lo_s = hi_s + kLoraRows * ld;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int j = lane & 31;
+  const int h = lane >> 5;
+  const int m0 = blockIdx.y * kLoraRows;
+  const int mn = min(kLoraRows, a.M - m0);
+  const int c0 = (blockIdx.x * NW + wave) * 32;  // the wavefront's channels
+  const bool busy = c0 < a.C;                    // C % 32 == 0: all of them exist, or none
+
+  // this lane's row of A
+  const int cl = 16 * ((j >> 2) & 1) + 4 * (j >> 3) + (j & 3);
+  const half_t* wp = p.w2p ? p.w2p + (static_cast<int64_t>(busy ? c0 >> 5 : 0) * steps * 64 + cl + 32 * h) * 8
+                           : p.w2 + static_cast<int64_t>(busy ? c0 + cl : cl) * R + 8 * h;
+  const int stride = p.w2p ? 512 : 16;
+  // the half step past a rank of 8 mod 16 meets zeros of the hidden: any finite weights do (the packed ones exist and are zero)
+  const int tail = !p.w2p && h && (R & 15) ? 8 : 0;
+  half8_t w[kDepth];
+  auto request = [&](int s) { return *reinterpret_cast<const half8_t*>(wp + s * stride - (s == steps - 1 ? tail : 0)); };
+
+  // the hidden slice is requested first, then the weights of the first steps, all without a branch per lane (see above)
+  {
+    const int row = threadIdx.x / kTpr;
+    const int ks0 = (threadIdx.x % kTpr) * 8;
+    const half_t* src = p.h + static_cast<int64_t>(m0 + (row < mn ? row : mn - 1)) * R;
+    uint4_t hv[kStage];
+#pragma unroll
+    for (int i = 0; i < kStage; ++i) {
+      const int ks = ks0 + i * kTpr * 8;
+      if (i * kTpr * 8 <= R) hv[i] = *reinterpret_cast<const uint4_t*>(src + (ks < R ? ks : R - 8));
+    }
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) w[u] = request(min(u, steps - 1));
+#pragma unroll
+    for (int i = 0; i < kStage; ++i) {
+      if (i * kTpr * 8 <= R) {
+        const int ks = ks0 + i * kTpr * 8;
+        const bool live = row < mn && ks < R;  // rows past M and the pad hold exact zeros
+        const half8_t raw = __builtin_bit_cast(half8_t, hv[i]);
+        half8_t hi, lo;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          float f = h2f(raw[e]);
+          if (p.act == RWKV_ACT_TANH) f = tanh_f(f);
+          if (p.act == RWKV_ACT_SIGMOID) f = sigmoid_f(f);
+          if (!live) f = 0.0f;
+          hi[e] = f2h(f);
+          lo[e] = f2h(f - h2f(hi[e]));
+        }
+        if (ks <= R) {
+          *reinterpret_cast<half8_t*>(&hi_s[row * ld + ks]) = hi;
+          if (split) *reinterpret_cast<half8_t*>(&lo_s[row * ld + ks]) = lo;
         }
       }
     }
-    __syncthreads();
+  }
+  __syncthreads();
+  if (!busy) return;
 
-    float16_t acc;
+  float16_t acc[2];  // even and odd rank steps
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+  for (int v = 0; v < 16; ++v) acc[0][v] = acc[1][v] = 0.0f;
+  const half_t* hp = hi_s + j * ld + 8 * h;
+  const half_t* lp = lo_s + j * ld + 8 * h;
+  for (int s0 = 0; s0 < steps; s0 += kDepth) {
 #pragma unroll
-    for (int i = 0; i < kSteps; ++i) {
-      const int k = (i * kLoraKG + kg) * 16;
-      if (k < R) {
-        const half8_t ah = *reinterpret_cast<const half8_t*>(&hi_s[j * ld + k + h * 8]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, w[i], acc, 0, 0, 0);
-        if (split) {
-          const half8_t al = *reinterpret_cast<const half8_t*>(&lo_s[j * ld + k + h * 8]);
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, w[i], acc, 0, 0, 0);
-        }
+    for (int u = 0; u < kDepth; ++u) {
+      const int s = s0 + u;
+      if (s < steps) {  // the same for the whole block
+        acc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[u], *reinterpret_cast<const half8_t*>(hp + 16 * s), acc[u & 1], 0, 0, 0);
+        if (split)
+          acc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[u], *reinterpret_cast<const half8_t*>(lp + 16 * s), acc[u & 1], 0, 0, 0);
+        w[u] = request(min(s + kDepth, steps - 1));
       }
     }
-    __syncthreads();  // the hidden tiles are free: group 0 lays its sums over hi_s, group 1 over lo_s
-    // accumulator v of lane (j, h): row 8*(v/4) + 4h + v%4, column wave*32 + j
-    float* tile = reinterpret_cast<float*>(kg == 0 ? hi_s : lo_s);
-#pragma unroll
-    for (int v = 0; v < 16; ++v) tile[(8 * (v / 4) + 4 * h + (v % 4)) * kLoraOutLd + wave * 32 + j] = acc[v];
-    __syncthreads();
+  }
 
-    const float* t0 = reinterpret_cast<const float*>(hi_s) + orow * kLoraOutLd + (threadIdx.x & 15) * 8;
-    const float* t1 = reinterpret_cast<const float*>(lo_s) + orow * kLoraOutLd + (threadIdx.x & 15) * 8;
-    float sum[8];
+  if (j >= mn) return;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const float4_t s0 = *reinterpret_cast<const float4_t*>(t0 + 4 * q);
-      const float4_t s1 = *reinterpret_cast<const float4_t*>(t1 + 4 * q);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum[4 * q + e] = s0[e] + s1[e];
+  for (int q = 0; q < 2; ++q) {
+    const int c = c0 + 16 * h + 8 * q;
+    const int64_t o = static_cast<int64_t>(m0 + j) * a.C + c;
+    half8_t bias8 = {}, v8 = {}, vf8 = {}, res;
+    if (p.bias) bias8 = *reinterpret_cast<const half8_t*>(p.bias + c);
+    if (p.vres) {
+      v8 = *reinterpret_cast<const half8_t*>(p.v + o);
+      vf8 = *reinterpret_cast<const half8_t*>(p.v_first + o);
     }
-    half8_t res;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
+      const float sum = acc[0][8 * q + e] + acc[1][8 * q + e];
       const float b = p.bias ? h2f(bias8[e]) : 0.0f;
       if (p.vres) {
         const float vv = h2f(v8[e]);
-        const float gate = sigmoid_f(b + sum[e]);
-        res[e] = f2h(vv + (h2f(vf8[e]) - vv) * gate);
+        res[e] = f2h(vv + (h2f(vf8[e]) - vv) * sigmoid_f(b + sum));
       } else {
-        res[e] = f2h(sum[e] + b);
+        res[e] = f2h(sum + b);
       }
     }
-    if (orow < mn && ocol_ok) *reinterpret_cast<half8_t*>(p.out + o) = res;
-    if (more) __syncthreads();  // the tiles are rewritten by the next row tile
-  };
-  // One tile per block (up to 256 rows) as straight-line code: inside a loop the compiler makes the requests of a
-  // tile wait for the weights, for the sake of registers that the previous trip round the loop has long released.
-  if (static_cast<int>(gridDim.y) >= row_tiles) {
-    row_tile(blockIdx.y, false);
-  } else {
-    for (int rt = blockIdx.y; rt < row_tiles; rt += gridDim.y) row_tile(rt, true);
+    *reinterpret_cast<half8_t*>(p.out + o) = res;
   }
 }
 
-// Row tiles per block: one up to 256 rows; beyond that the blocks of a problem walk the row tiles with a stride, so
-// that the weights of a block are requested once for several tiles and the grid stays at a few blocks per CU.
+template <int NW>
+int lora_out_wide_launch(hipStream_t st, const LoraOutMultiArgs& a) {
+  // the longest problem first: its blocks would be the launch's tail otherwise
+  LoraOutMultiArgs o = a;
+  const auto cost = [](const LoraOutProblem& p) { return p.R * (p.act != RWKV_ACT_NONE ? 2 : 1); };
+  std::stable_sort(o.p, o.p + o.n, [&](const LoraOutProblem& x, const LoraOutProblem& y) { return cost(x) > cost(y); });
+  size_t lds = 0;
+  for (int i = 0; i < o.n; ++i)
+    lds = std::max(lds, static_cast<size_t>(kLoraRows) * (o.p[i].R + 8) * (o.p[i].act != RWKV_ACT_NONE ? 4 : 2));
+  if (lds > 65536)
+    RWKV_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&lora_out_wide_kernel<NW>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+  hipLaunchKernelGGL((lora_out_wide_kernel<NW>), dim3(ceil_div(o.C, 32 * NW), ceil_div(o.M, kLoraRows), o.n), dim3(NW * 64), lds, st, o);
+  RWKV_LAUNCH_CHECK();
+  return RWKV_OK;
+}
+
 __global__ __launch_bounds__(256) void lora_pack_w2_kernel(int C, int R, const half_t* __restrict__ w2, half_t* __restrict__ packed,
                                                            int64_t n_pieces) {
   const int64_t piece = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;  // (band, step, lane)
@@ -242,9 +369,39 @@ int lora_out_multi(hipStream_t st, const LoraOutMultiArgs& a) {
                   reinterpret_cast<uintptr_t>(p.v_first) | reinterpret_cast<uintptr_t>(p.w2p)) % 16 == 0,
                  "lora_out: tensors must be 16-byte aligned");
   }
+  // the grid's second dimension ends at 65535
+  constexpr int kMostRows = 65535 * kLoraRows;
+  if (a.M > kMostRows) {
+    LoraOutMultiArgs part = a;
+    for (int m0 = 0; m0 < a.M; m0 += part.M) {
+      part.M = std::min(kMostRows, a.M - m0);
+      for (int i = 0; i < a.n; ++i) {
+        part.p[i].h = a.p[i].h + static_cast<int64_t>(m0) * a.p[i].R;
+        part.p[i].out = a.p[i].out + static_cast<int64_t>(m0) * a.C;
+        if (a.p[i].vres) {
+          part.p[i].v = a.p[i].v + static_cast<int64_t>(m0) * a.C;
+          part.p[i].v_first = a.p[i].v_first + static_cast<int64_t>(m0) * a.C;
+        }
+      }
+      const int rc = lora_out_multi(st, part);
+      if (rc != RWKV_OK) return rc;
+    }
+    return RWKV_OK;
+  }
+  // Up to one and a half blocks per CU the small tile is the faster one (its rank is walked by two groups of wavefronts); past
+  // that, what the blocks repeat counts.  us of the four problems of a layer, small tile / 32 x 256: 4096 channels, 64 rows
+  // (256 blocks) 8.3 / 11.1, 128 (512) 12.0 / 11.5, 144 (640) 14.9 / 11.7, 256 20.1 / 14.8; 2048 channels, 128 rows (256) 6.9 / 7.2,
+  // 192 (384) 9.1 / 8.0, 256 (512) 9.7 / 8.3; 768 channels, 256 rows (192) 4.6 / 6.3.
   const int row_tiles = ceil_div(a.M, kLoraRows);
-  const int row_blocks = row_tiles <= 8 ? row_tiles : std::max(8, ceil_div(row_tiles, 8));
-  hipLaunchKernelGGL(lora_out_kernel, dim3(ceil_div(a.C, kLoraCols), row_blocks, a.n), dim3(kLoraThreads), 0, st, a);
+  const int64_t cus = device_cu_count();
+  if (static_cast<int64_t>(ceil_div(a.C, kLoraCols)) * row_tiles * a.n * 2 > 3 * cus) {
+    // twice as many channels per block where that still leaves two blocks per CU and no channel of a block unused: 32 x 256 / 32 x
+    // 512 at 4096 channels and 256 rows 14.6 / 15.8, 500 22.5 / 19.0, 2048 68.8 / 56.7; 2048 channels and 999 rows 14.4 / 14.0
+    // (before, with the small tile's blocks walking several row tiles: 20.6, 34.5, 108.5; 27.3)
+    const bool wide = a.C % 512 == 0 && static_cast<int64_t>(a.C / 512) * row_tiles * a.n >= 2 * cus;
+    return wide ? lora_out_wide_launch<16>(st, a) : lora_out_wide_launch<8>(st, a);
+  }
+  hipLaunchKernelGGL(lora_out_kernel, dim3(ceil_div(a.C, kLoraCols), row_tiles, a.n), dim3(kLoraThreads), 0, st, a);
   RWKV_LAUNCH_CHECK();
   return RWKV_OK;
 }

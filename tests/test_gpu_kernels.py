@@ -616,8 +616,7 @@ def test_kk_gate_groupnorm_lora(gpu, orc):
 
 
 def test_lora_out_blocks_walk_several_row_tiles(gpu, orc):
-    """Beyond 256 rows a block keeps its weights and walks several 32-row tiles; the last tile here is partial.  The
-    v-residual epilogue is checked on the same rows."""
+    """Ten row tiles, the last one partial; the v-residual epilogue is checked on the same rows."""
     hip = gpu
     rng = np.random.default_rng(77)
     rows, C, R = 300 + 13, 256, 40
@@ -635,6 +634,46 @@ def test_lora_out_blocks_walk_several_row_tiles(gpu, orc):
     assert rel_err(o.numpy().astype(np.float32), o32) <= F16_TOL
     ref = orc.vres_gate(v, v_first, v0, o32)
     assert rel_err(og.numpy().astype(np.float32), ref.astype(np.float32)) <= F16_TOL
+
+
+@pytest.mark.parametrize("C,R,rows", [(4064, 24, 417), (4096, 480, 1025), (4096, 40, 2050), (96, 8, 12321), (2048, 512, 4097),
+                                      (352, 136, 4100)])
+def test_lora_out_blocks_of_many_channels(gpu, C, R, rows):
+    """Both widths of the many-row rank-out: channels that leave wavefronts of the last block idle, a last row tile of one, two
+    or four rows, ranks that end in a half step, and the v-residual epilogue.  The result is within half an fp16 ulp (plus the
+    fp32 sums' own error) of the float64 one, and bitwise what the few-row kernel gives for the same rows."""
+    hip = gpu
+    rng = np.random.default_rng(rows + C)
+    h = rng.standard_normal((rows, R)).astype(np.float16)
+    w2 = (rng.standard_normal((C, R)) * 0.1).astype(np.float16)
+    v, v_first = (rng.standard_normal((rows, C)).astype(np.float16) for _ in range(2))
+    v0 = (rng.standard_normal(C) * 0.3).astype(np.float16)
+    dh, dw, dv, df, d0 = (dev(hip, x) for x in (h, w2, v, v_first, v0))
+    few = 32 if C > 512 else 64  # rows of one launch that keeps the few-row kernel
+    first = (rows - 1) // 32 * 32 - (few - 32)  # the last tiles, the partial one among them
+    n = rows - first
+    for act, vres in ((hip.ACT_SIGMOID, 0), (hip.ACT_NONE, 1), (hip.ACT_TANH, 0)):
+        more = dict(bias=d0, vres=1) if vres else {}
+        o = hip.DeviceArray((rows, C), np.float16)
+        hip.lora_out(rows, C, R, act, dh, dw, o, **more, **(dict(v=dv, v_first=df) if vres else {}))
+        part = hip.DeviceArray((n, C), np.float16)
+        hip.lora_out(n, C, R, act, dev(hip, h[first:]), dw, part, **more,
+                     **(dict(v=dev(hip, v[first:]), v_first=dev(hip, v_first[first:])) if vres else {}))
+        hip.device_sync()
+        got = o.numpy()
+        assert np.array_equal(got[first:].view(np.uint16), part.numpy().view(np.uint16))
+        hf = h.astype(np.float32)
+        if act == hip.ACT_TANH:
+            hf = np.tanh(hf)
+        elif act == hip.ACT_SIGMOID:
+            hf = (1.0 / (1.0 + np.exp(-hf))).astype(np.float32)
+        exact = hf.astype(np.float64) @ w2.astype(np.float64).T
+        if vres:
+            gate = 1.0 / (1.0 + np.exp(-(exact + v0.astype(np.float64))))
+            exact = v + (v_first.astype(np.float64) - v) * gate
+        mags = np.abs(hf).astype(np.float64) @ np.abs(w2).astype(np.float64).T + (2.0 if vres else 0.0)
+        bound = 0.5 * np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64) + 1e-6 * mags
+        assert np.all(np.abs(got.astype(np.float64) - exact) <= bound)
 
 
 @pytest.mark.parametrize("rows,C,R", [(1, 96, 8), (33, 256, 136), (70, 768, 480), (128, 4096, 512), (64, 4096, 96),
