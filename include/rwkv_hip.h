@@ -343,11 +343,12 @@ int rwkv_hip_graph_capture_count(int64_t* count);
 int rwkv_hip_session_set_profile(rwkv_hip_session* s, int mode);
 int rwkv_hip_session_read_profile(rwkv_hip_session* s, int64_t* launches, double* total_ms);
 /* Decode steps of up to max_rows rows (0..12) use the row-skipping ffn.value product (CmixMode::NoFcOne / NoFcRows2
- * of the reference, include/rwkv7_fast_v4_common.hpp:198-211, whose default is 12 rows at C = 4096).  Default 4: two
- * to four rows share one walk that reads every row that is non-zero for any of them once (with a fraction z of zero
- * activations per row that is 1 - z^rows of the matrix: at the z = 0.5 of random-init weights about what the dense
- * product reads, far less with trained weights; 7.2B shape, 2 / 3 / 4 rows: 2.19 / 2.39 / 2.56 ms per step against
- * 2.61 / 2.79 / 2.82 before).  From five rows on every row walks its own rows, which pays only while rows x (1 - z)
+ * of the reference, include/rwkv7_fast_v4_common.hpp:198-211, whose default is 12 rows at C = 4096).  Two to four rows
+ * share one walk that reads every row that is non-zero for any of them once (with a fraction z of zero activations per row
+ * that is 1 - z^rows of the matrix: at the z = 0.5 of random-init weights about what the dense product reads at three and four
+ * rows, far less with trained weights).  Without a call steps of up to four rows use it where the matrix is large enough for
+ * its second launch: from 8 MB on for one and two rows, above 32 MB for three and four (0.1B fp16, one row: 22.0 us per layer
+ * dense, 24.3 with the walk).  From five rows on every row walks its own rows, which pays only while rows x (1 - z)
  * stays below 1.  0 selects the dense product. */
 int rwkv_hip_session_set_sparse_ffn(rwkv_hip_session* s, int max_rows);
 /* on != 0: the `wkv` tensor of rwkv_hip_forward / rwkv_hip_decode_greedy is the fp16 state, f16 [L,B,H,64,64], and

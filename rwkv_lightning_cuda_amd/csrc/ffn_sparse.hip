@@ -11,13 +11,18 @@
 // Weights: the [C,F] matrix transposed to [F,C]: fp16 values as they are, or int8 codes stored offset by 128
 // (u = q + 128, one byte each) with the same per-output-channel fp16 scale.
 //
-// Kernel 1: grid = (F/256, column chunks, tokens), block = 8 wavefronts.  A wavefront owns 32 consecutive f and one 16-byte
-// piece of the row per lane (1024 int8 or 512 fp16 columns per chunk): it ballots the non-zero activations, walks
-// the set bits eight rows at a time (missing rows of the last batch repeat a row already read, with coefficient
-// zero, so no load sits under a branch), and accumulates two rows per v_dot2_f32_f16: v_perm_b32 pairs the
-// values of the two rows (int8: bytes under exponent 0x64, then one packed subtract gives the exact codes).  The eight wavefronts' sums meet in LDS in wavefront
-// order and the block writes one fp32 partial row.  Kernel 2 sums the F/256 partial rows in a fixed order,
-// applies the scale and rounds to fp16.
+// Kernel 1: grid = (row blocks, column chunks, tokens), block = 8 wavefronts.  A wavefront owns 32 .. 128 consecutive f and a
+// chunk of 256 columns (fp16: 128), one row's piece of it per lane group of 16 lanes: it lists the rows with a non-zero
+// activation in LDS, its four lane groups walk the list two rows each at a time (v_dot2_f32_f16: v_perm_b32 pairs the values of
+// the two rows; int8: bytes under exponent 0x64, then one packed subtract gives the exact codes), the groups' sums meet by
+// lane swaps, the wavefronts' in LDS in wavefront order, and the block writes one fp32 partial row.  Kernel 2 sums the
+// partial rows in a fixed order, applies the scale and rounds to fp16.
+//
+// Narrow chunks make few partial rows: 7.2B int8 has 16 of them (256 blocks; a chunk of a whole wavefront's 1024 columns had
+// 64) and 1.5B int8 still a block per CU.  us per layer, one / two tokens, in the decode step: 7.2B int8 54.1 / 62.6 ->
+// 52.9 / 60.5, int4 44.9 / 56.7 -> 42.0 / 52.6, fp16 79.1 / 89.8 -> 76.8 / 85.6; 1.5B int8 35.0 / 43.0 -> 32.1 / 37.8, int4 36.2 /
+// 45.8 -> 32.6 / 39.4.  Measured and left: the block that draws a chunk's last ticket sums the partial rows instead of the
+// second launch (3.4 us of tail against the launch's 4.4 in a trace, but 0.9 us per layer slower in the replayed step).
 #include <mutex>
 
 #include "ops.h"
@@ -30,10 +35,8 @@ namespace rwkv {
 constexpr size_t kStaticScratchBytes = static_cast<size_t>(16) << 20;
 static __device__ __align__(256) float scratch[kStaticScratchBytes / sizeof(float)];
 
-constexpr int kSparseRowsPerWave = 32;
 constexpr int kSparseWaves = 8;
-constexpr int kSparseRowsPerBlock = kSparseRowsPerWave * kSparseWaves;  // 256
-constexpr int kSparseBatch = 8;
+constexpr int kSparseRowsPerBlock = 32 * kSparseWaves;  // 256: the fewest rows of a block that the entry points' workspace is sized for
 
 // columns per lane = values in a 16-byte piece
 constexpr int sparse_lane_cols(int fmt) { return fmt == RWKV_FMT_F16 ? 8 : 16; }
@@ -150,382 +153,172 @@ int ffn_sparse_pack_w4_launch(hipStream_t st, int C, int F, const void* q, const
 }
 
 // ---- kernel 1 ------------------------------------------------------------------------------------------------------------
-// `activated` != 0: `in` already holds f16(relu(preact)^2) (the model's ffn.key launch applies it).
+constexpr int kSparseSteps = 2;  // steps of a batch (4: the same within 1 %; 8, or loads under branches: 2-6 % of the step slower)
+constexpr int kSparseGroups = 4;  // lane groups of a wavefront, each with a row's piece of the chunk
+constexpr int kSparseListed = 128 + 8;  // entries of a wavefront's list, the pad of the last step among them
+
 template <int FMT>
-__global__ __launch_bounds__(64 * kSparseWaves) void ffn_sparse_kernel(int C, int F, int activated,
-                                                                       const half_t* __restrict__ in,
-                                                                       const uint4_t* __restrict__ wt,
-                                                                       float* __restrict__ partial) {
-  constexpr int LC = sparse_lane_cols(FMT);  // columns per lane
-  constexpr int kCols = 64 * LC;             // columns per block
-  __shared__ __align__(16) float red[kSparseWaves][kCols];
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int f0 = blockIdx.x * kSparseRowsPerBlock + wave * kSparseRowsPerWave;
-  const int c0 = blockIdx.y * kCols;
-  const bool col_ok = c0 + LC * lane < C;
-  // 16-byte pieces: row f has C/LC of them, this lane's piece of the row is (c0/LC + lane)
-  const int row_pieces = C / LC;
-  const uint4_t* wlane = wt + c0 / LC + (col_ok ? lane : 0);
-  in += static_cast<int64_t>(blockIdx.z) * F;                       // this token's activations ...
-  partial += static_cast<int64_t>(blockIdx.z) * gridDim.x * C;      // ... and partial rows
+struct SparsePiece {
+  typedef uint4_t type;
+};
+template <>
+struct SparsePiece<RWKV_FMT_W4> {
+  typedef uint2_t type;
+};
 
-  float a = 0.0f;
-  if (lane < kSparseRowsPerWave) {
-    a = h2f(in[f0 + lane]);
-    if (!activated) {
-      a = fmaxf(round_h(a), 0.0f);
-      a = round_h(a * a);
-    }
-  }
-  const half_t ah = f2h(a);
-  const uint32_t abits = __builtin_bit_cast(uint16_t, ah);
-  uint64_t mask = __ballot((abits << 17) != 0u);  // +0 and -0 both count as zero
-
-  float acc[LC];
-#pragma unroll
-  for (int i = 0; i < LC; ++i) acc[i] = 0.0f;
-  const half2_t bias = {static_cast<half_t>(1152.0f), static_cast<half_t>(1152.0f)};
-
-  while (mask != 0) {
-    int row[kSparseBatch];
-    uint32_t coef[kSparseBatch];
-    const int first = __builtin_ctzll(mask);
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; ++p) {
-      if (mask != 0) {
-        row[p] = __builtin_ctzll(mask);
-        mask &= mask - 1;
-        coef[p] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(abits), row[p]));
-      } else {
-        row[p] = first;
-        coef[p] = 0u;
-      }
-    }
-    uint4_t q[kSparseBatch];
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; ++p) q[p] = __builtin_nontemporal_load(&wlane[static_cast<int64_t>(f0 + row[p]) * row_pieces]);
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; p += 2) {
-      const half2_t ap = as_half2(coef[p] | (coef[p + 1] << 16));
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const uint32_t lo = q[p][d];
-        const uint32_t hi = q[p + 1][d];
-        if constexpr (FMT == RWKV_FMT_W8) {
-          const half2_t w0 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c040c00u) | 0x64006400u) - bias;
-          const half2_t w1 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c050c01u) | 0x64006400u) - bias;
-          const half2_t w2 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c060c02u) | 0x64006400u) - bias;
-          const half2_t w3 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c070c03u) | 0x64006400u) - bias;
-          acc[4 * d + 0] = __builtin_amdgcn_fdot2(ap, w0, acc[4 * d + 0], false);
-          acc[4 * d + 1] = __builtin_amdgcn_fdot2(ap, w1, acc[4 * d + 1], false);
-          acc[4 * d + 2] = __builtin_amdgcn_fdot2(ap, w2, acc[4 * d + 2], false);
-          acc[4 * d + 3] = __builtin_amdgcn_fdot2(ap, w3, acc[4 * d + 3], false);
-        } else {
-          // a dword holds two fp16 columns of a row: pair the low halves and the high halves of the two rows
-          const half2_t w0 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x05040100u));
-          const half2_t w1 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x07060302u));
-          acc[2 * d + 0] = __builtin_amdgcn_fdot2(ap, w0, acc[2 * d + 0], false);
-          acc[2 * d + 1] = __builtin_amdgcn_fdot2(ap, w1, acc[2 * d + 1], false);
-        }
-      }
-    }
-  }
-
-#pragma unroll
-  for (int i = 0; i < LC / 4; ++i)
-    *reinterpret_cast<float4_t*>(&red[wave][LC * lane + 4 * i]) =
-        float4_t{acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]};
-  __syncthreads();
-  if (threadIdx.x < kCols / 4) {
-    const int c = 4 * threadIdx.x;
-    float4_t sum = *reinterpret_cast<const float4_t*>(&red[0][c]);
-#pragma unroll
-    for (int w = 1; w < kSparseWaves; ++w) sum = sum + *reinterpret_cast<const float4_t*>(&red[w][c]);
-    if (c0 + c < C) *reinterpret_cast<float4_t*>(partial + static_cast<int64_t>(blockIdx.x) * C + c0 + c) = sum;
-  }
-}
-
-// int4 codes: the same walk with 8-byte pieces (16 columns per lane, 1024 per block).  The two rows of a
-// v_dot2_f32_f16 are paired nibble by nibble: even and odd nibbles of each dword are masked into bytes, v_perm_b32
-// puts row A's byte under exponent 0x64 in the low half and row B's in the high half, one packed subtract of
-// 1024 gives the exact codes.  sum_f a_f (q_fc - zp_c) = sum_f a_f q_fc - zp_c sum_f a_f: the zero point and the
-// scale of the wavefront's 128-group are applied once, after the walk.
-__global__ __launch_bounds__(64 * kSparseWaves) void ffn_sparse_w4_kernel(int C, int F, int activated,
-                                                                          const half_t* __restrict__ in,
-                                                                          const uint8_t* __restrict__ blob,
-                                                                          float* __restrict__ partial) {
-  constexpr int LC = 16;
-  constexpr int kCols = 64 * LC;
-  __shared__ __align__(16) float red[kSparseWaves][kCols];
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int f0 = blockIdx.x * kSparseRowsPerBlock + wave * kSparseRowsPerWave;
-  const int c0 = blockIdx.y * kCols;
-  const bool col_ok = c0 + LC * lane < C;
-  const int cl = c0 + (col_ok ? LC * lane : 0);  // this lane's first column
-  const int row_pieces = C / LC;                 // 8-byte pieces per row
-  const uint2_t* wlane = reinterpret_cast<const uint2_t*>(blob) + cl / LC;
-  const int G = F / 128;
-  const half_t* scale_t = reinterpret_cast<const half_t*>(blob + static_cast<size_t>(C) * F / 2);
-  const uint8_t* zp_t = reinterpret_cast<const uint8_t*>(scale_t + static_cast<size_t>(G) * C);
-  const int64_t gat = static_cast<int64_t>(f0 / 128) * C + cl;
-  const half8_t sc0 = *reinterpret_cast<const half8_t*>(scale_t + gat);
-  const half8_t sc1 = *reinterpret_cast<const half8_t*>(scale_t + gat + 8);
-  const uint4_t zq = *reinterpret_cast<const uint4_t*>(zp_t + gat);
-  in += static_cast<int64_t>(blockIdx.z) * F;
-  partial += static_cast<int64_t>(blockIdx.z) * gridDim.x * C;
-
-  float a = 0.0f;
-  if (lane < kSparseRowsPerWave) {
-    a = h2f(in[f0 + lane]);
-    if (!activated) {
-      a = fmaxf(round_h(a), 0.0f);
-      a = round_h(a * a);
-    }
-  }
-  const half_t ah = f2h(a);
-  const uint32_t abits = __builtin_bit_cast(uint16_t, ah);
-  uint64_t mask = __ballot((abits << 17) != 0u);
-
-  float acc[LC];
-#pragma unroll
-  for (int i = 0; i < LC; ++i) acc[i] = 0.0f;
-  float asum = 0.0f;
-  const half2_t bias = {static_cast<half_t>(1024.0f), static_cast<half_t>(1024.0f)};
-
-  while (mask != 0) {
-    int row[kSparseBatch];
-    uint32_t coef[kSparseBatch];
-    const int first = __builtin_ctzll(mask);
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; ++p) {
-      if (mask != 0) {
-        row[p] = __builtin_ctzll(mask);
-        mask &= mask - 1;
-        coef[p] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(abits), row[p]));
-      } else {
-        row[p] = first;
-        coef[p] = 0u;
-      }
-    }
-    uint2_t q[kSparseBatch];
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; ++p)
-      q[p] = __builtin_nontemporal_load(&wlane[static_cast<int64_t>(f0 + row[p]) * row_pieces]);
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; p += 2) {
-      const half2_t ap = as_half2(coef[p] | (coef[p + 1] << 16));
-      asum += h2f(ap[0]) + h2f(ap[1]);
-#pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        const uint32_t lo = q[p][d];
-        const uint32_t hi = q[p + 1][d];
-        const uint32_t ea = lo & 0x0f0f0f0fu, oa = (lo >> 4) & 0x0f0f0f0fu;
-        const uint32_t eb = hi & 0x0f0f0f0fu, ob = (hi >> 4) & 0x0f0f0f0fu;
-        // nibble n of the dword is column 8 d + n: byte n / 2 of the even (n even) or odd word
-        const half2_t w0 = as_half2(__builtin_amdgcn_perm(eb, ea, 0x0c040c00u) | 0x64006400u) - bias;
-        const half2_t w1 = as_half2(__builtin_amdgcn_perm(ob, oa, 0x0c040c00u) | 0x64006400u) - bias;
-        const half2_t w2 = as_half2(__builtin_amdgcn_perm(eb, ea, 0x0c050c01u) | 0x64006400u) - bias;
-        const half2_t w3 = as_half2(__builtin_amdgcn_perm(ob, oa, 0x0c050c01u) | 0x64006400u) - bias;
-        const half2_t w4 = as_half2(__builtin_amdgcn_perm(eb, ea, 0x0c060c02u) | 0x64006400u) - bias;
-        const half2_t w5 = as_half2(__builtin_amdgcn_perm(ob, oa, 0x0c060c02u) | 0x64006400u) - bias;
-        const half2_t w6 = as_half2(__builtin_amdgcn_perm(eb, ea, 0x0c070c03u) | 0x64006400u) - bias;
-        const half2_t w7 = as_half2(__builtin_amdgcn_perm(ob, oa, 0x0c070c03u) | 0x64006400u) - bias;
-        acc[8 * d + 0] = __builtin_amdgcn_fdot2(ap, w0, acc[8 * d + 0], false);
-        acc[8 * d + 1] = __builtin_amdgcn_fdot2(ap, w1, acc[8 * d + 1], false);
-        acc[8 * d + 2] = __builtin_amdgcn_fdot2(ap, w2, acc[8 * d + 2], false);
-        acc[8 * d + 3] = __builtin_amdgcn_fdot2(ap, w3, acc[8 * d + 3], false);
-        acc[8 * d + 4] = __builtin_amdgcn_fdot2(ap, w4, acc[8 * d + 4], false);
-        acc[8 * d + 5] = __builtin_amdgcn_fdot2(ap, w5, acc[8 * d + 5], false);
-        acc[8 * d + 6] = __builtin_amdgcn_fdot2(ap, w6, acc[8 * d + 6], false);
-        acc[8 * d + 7] = __builtin_amdgcn_fdot2(ap, w7, acc[8 * d + 7], false);
-      }
-    }
-  }
-
-#pragma unroll
-  for (int i = 0; i < LC; ++i) {
-    const float zpf = static_cast<float>((zq[i >> 2] >> (8 * (i & 3))) & 0xffu);
-    const float scf = h2f(i < 8 ? sc0[i] : sc1[i - 8]);
-    acc[i] = (acc[i] - zpf * asum) * scf;
-  }
-#pragma unroll
-  for (int i = 0; i < LC / 4; ++i)
-    *reinterpret_cast<float4_t*>(&red[wave][LC * lane + 4 * i]) =
-        float4_t{acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]};
-  __syncthreads();
-  if (threadIdx.x < kCols / 4) {
-    const int c = 4 * threadIdx.x;
-    float4_t sum = *reinterpret_cast<const float4_t*>(&red[0][c]);
-#pragma unroll
-    for (int w = 1; w < kSparseWaves; ++w) sum = sum + *reinterpret_cast<const float4_t*>(&red[w][c]);
-    if (c0 + c < C) *reinterpret_cast<float4_t*>(partial + static_cast<int64_t>(blockIdx.x) * C + c0 + c) = sum;
-  }
-}
-
-// ---- kernel 1 for several tokens at once ------------------------------------------------------------------------------
-// TOK tokens share one walk: a wavefront ballots the rows that are non-zero for ANY of its tokens and reads each of
-// them once; a token for which a row is zero takes it with coefficient zero (an exact zero product).  With a
-// fraction z of zero activations per token the walk reads 1 - z^TOK of the matrix once, where one walk per token
-// reads TOK * (1 - z) of it.  Per token the rows still add up in increasing order, but a token's rows pair up
-// differently than in its own walk (a pair is one v_dot2), so the last bits of the fp32 sums can differ from the
-// one-token kernel's; the result repeats bitwise from call to call.
-template <int TOK>
-__device__ __forceinline__ void sparse_union_heads(const half_t* __restrict__ in, int F, int f0, int lane, int activated,
-                                                  uint32_t (&abits)[TOK], uint64_t& mask) {
-  mask = 0;
-#pragma unroll
-  for (int t = 0; t < TOK; ++t) {
-    float a = 0.0f;
-    if (lane < kSparseRowsPerWave) {
-      a = h2f(in[static_cast<int64_t>(t) * F + f0 + lane]);
-      if (!activated) {
-        a = fmaxf(round_h(a), 0.0f);
-        a = round_h(a * a);
-      }
-    }
-    const half_t ah = f2h(a);
-    abits[t] = __builtin_bit_cast(uint16_t, ah);
-    mask |= __ballot((abits[t] << 17) != 0u);  // +0 and -0 both count as zero
-  }
-}
-
-// the wavefronts' sums of one token meet in LDS in wavefront order; the block writes the token's partial row
-template <int LC>
-__device__ __forceinline__ void sparse_block_row(const float (&acc)[LC], float (*red)[64 * LC], int wave, int lane, int C, int c0,
-                                                 float* __restrict__ partial_row) {
-  constexpr int kCols = 64 * LC;
-#pragma unroll
-  for (int i = 0; i < LC / 4; ++i)
-    *reinterpret_cast<float4_t*>(&red[wave][LC * lane + 4 * i]) =
-        float4_t{acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]};
-  __syncthreads();
-  if (threadIdx.x < kCols / 4) {
-    const int c = 4 * threadIdx.x;
-    float4_t sum = *reinterpret_cast<const float4_t*>(&red[0][c]);
-#pragma unroll
-    for (int w = 1; w < kSparseWaves; ++w) sum = sum + *reinterpret_cast<const float4_t*>(&red[w][c]);
-    if (c0 + c < C) *reinterpret_cast<float4_t*>(partial_row + c0 + c) = sum;
-  }
-  __syncthreads();  // red is written again for the next token
-}
-
+// acc += a_lo * (the piece's columns of row lo) + a_hi * (those of row hi), for every token's pair ap = (a_lo, a_hi)
 template <int FMT, int TOK>
-__global__ __launch_bounds__(64 * kSparseWaves) void ffn_sparse_union_kernel(int C, int F, int activated,
-                                                                             const half_t* __restrict__ in,
-                                                                             const uint4_t* __restrict__ wt,
-                                                                             float* __restrict__ partial) {
-  constexpr int LC = sparse_lane_cols(FMT);
-  constexpr int kCols = 64 * LC;
-  __shared__ __align__(16) float red[kSparseWaves][kCols];
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int f0 = blockIdx.x * kSparseRowsPerBlock + wave * kSparseRowsPerWave;
-  const int c0 = blockIdx.y * kCols;
-  const bool col_ok = c0 + LC * lane < C;
-  const int row_pieces = C / LC;
-  const uint4_t* wlane = wt + c0 / LC + (col_ok ? lane : 0);
-
-  uint32_t abits[TOK];
-  uint64_t mask;
-  sparse_union_heads<TOK>(in, F, f0, lane, activated, abits, mask);
-
-  float acc[TOK][LC];
+__device__ __forceinline__ void sparse_pair(const typename SparsePiece<FMT>::type& qlo, const typename SparsePiece<FMT>::type& qhi,
+                                            const half2_t (&ap)[TOK], float (&acc)[TOK][sparse_lane_cols(FMT)]) {
+  constexpr int kDwords = sizeof(qlo) / 4;
 #pragma unroll
-  for (int t = 0; t < TOK; ++t)
-#pragma unroll
-    for (int i = 0; i < LC; ++i) acc[t][i] = 0.0f;
-  const half2_t bias = {static_cast<half_t>(1152.0f), static_cast<half_t>(1152.0f)};
-
-  while (mask != 0) {
-    int row[kSparseBatch];
-    bool live[kSparseBatch];
-    const int first = __builtin_ctzll(mask);
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; ++p) {
-      live[p] = mask != 0;
-      if (live[p]) {
-        row[p] = __builtin_ctzll(mask);
-        mask &= mask - 1;
-      } else {
-        row[p] = first;  // a row already read, taken with coefficient zero: no load sits under a branch
-      }
-    }
-    uint4_t q[kSparseBatch];
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; ++p) q[p] = __builtin_nontemporal_load(&wlane[static_cast<int64_t>(f0 + row[p]) * row_pieces]);
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; p += 2) {
-      half2_t ap[TOK];
+  for (int d = 0; d < kDwords; ++d) {
+    const uint32_t lo = qlo[d];
+    const uint32_t hi = qhi[d];
+    if constexpr (FMT == RWKV_FMT_F16) {
+      // a dword holds two columns of a row: pair the low halves and the high halves of the two rows
+      const half2_t w0 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x05040100u));
+      const half2_t w1 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x07060302u));
 #pragma unroll
       for (int t = 0; t < TOK; ++t) {
-        const uint32_t c0b = live[p] ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(abits[t]), row[p])) : 0u;
-        const uint32_t c1b = live[p + 1] ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(abits[t]), row[p + 1])) : 0u;
-        ap[t] = as_half2(c0b | (c1b << 16));
+        acc[t][2 * d + 0] = __builtin_amdgcn_fdot2(ap[t], w0, acc[t][2 * d + 0], false);
+        acc[t][2 * d + 1] = __builtin_amdgcn_fdot2(ap[t], w1, acc[t][2 * d + 1], false);
+      }
+    } else if constexpr (FMT == RWKV_FMT_W8) {
+      const half2_t bias = {static_cast<half_t>(1152.0f), static_cast<half_t>(1152.0f)};
+      half2_t w[4];
+      w[0] = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c040c00u) | 0x64006400u) - bias;
+      w[1] = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c050c01u) | 0x64006400u) - bias;
+      w[2] = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c060c02u) | 0x64006400u) - bias;
+      w[3] = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c070c03u) | 0x64006400u) - bias;
+#pragma unroll
+      for (int t = 0; t < TOK; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[t][4 * d + i] = __builtin_amdgcn_fdot2(ap[t], w[i], acc[t][4 * d + i], false);
+    } else {
+      // nibble n of the dword is column 8 d + n.  The bytes of the two rows are paired once for both of their nibbles; under exponent
+      // 0x64 the low one is 1024 + q, the high one in place 1024 + 16 q, exact after the subtract (the 16 comes off after the walk).
+      // (Codes as fp16 denormals would save the subtract, but v_dot2_f32_f16 keeps fewer bits of such products: 2.26e-4
+      // instead of 2.09e-4 from the 64-bit result at 4096 x 16384.)
+      const half2_t bias = {static_cast<half_t>(1024.0f), static_cast<half_t>(1024.0f)};
+      half2_t w[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t both = __builtin_amdgcn_perm(hi, lo, 0x0c040c00u + 0x00010001u * i);
+        w[2 * i] = as_half2((both & 0x000f000fu) | 0x64006400u) - bias;
+        w[2 * i + 1] = as_half2((both & 0x00f000f0u) | 0x64006400u) - bias;
       }
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const uint32_t lo = q[p][d];
-        const uint32_t hi = q[p + 1][d];
-        if constexpr (FMT == RWKV_FMT_W8) {
-          const half2_t w0 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c040c00u) | 0x64006400u) - bias;
-          const half2_t w1 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c050c01u) | 0x64006400u) - bias;
-          const half2_t w2 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c060c02u) | 0x64006400u) - bias;
-          const half2_t w3 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x0c070c03u) | 0x64006400u) - bias;
+      for (int t = 0; t < TOK; ++t)
 #pragma unroll
-          for (int t = 0; t < TOK; ++t) {
-            acc[t][4 * d + 0] = __builtin_amdgcn_fdot2(ap[t], w0, acc[t][4 * d + 0], false);
-            acc[t][4 * d + 1] = __builtin_amdgcn_fdot2(ap[t], w1, acc[t][4 * d + 1], false);
-            acc[t][4 * d + 2] = __builtin_amdgcn_fdot2(ap[t], w2, acc[t][4 * d + 2], false);
-            acc[t][4 * d + 3] = __builtin_amdgcn_fdot2(ap[t], w3, acc[t][4 * d + 3], false);
-          }
-        } else {
-          const half2_t w0 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x05040100u));
-          const half2_t w1 = as_half2(__builtin_amdgcn_perm(hi, lo, 0x07060302u));
-#pragma unroll
-          for (int t = 0; t < TOK; ++t) {
-            acc[t][2 * d + 0] = __builtin_amdgcn_fdot2(ap[t], w0, acc[t][2 * d + 0], false);
-            acc[t][2 * d + 1] = __builtin_amdgcn_fdot2(ap[t], w1, acc[t][2 * d + 1], false);
-          }
-        }
-      }
+        for (int i = 0; i < 8; ++i) acc[t][8 * d + i] = __builtin_amdgcn_fdot2(ap[t], w[i], acc[t][8 * d + i], false);
     }
   }
-#pragma unroll
-  for (int t = 0; t < TOK; ++t)
-    sparse_block_row<LC>(acc[t], red, wave, lane, C, c0,
-                         partial + (static_cast<int64_t>(t) * gridDim.x + blockIdx.x) * C);
 }
 
-// int4 codes, several tokens at once: the walk of ffn_sparse_w4_kernel over the union of the tokens' rows
-template <int TOK>
-__global__ __launch_bounds__(64 * kSparseWaves) void ffn_sparse_w4_union_kernel(int C, int F, int activated,
-                                                                                const half_t* __restrict__ in,
-                                                                                const uint8_t* __restrict__ blob,
-                                                                                float* __restrict__ partial) {
-  constexpr int LC = 16;
-  constexpr int kCols = 64 * LC;
-  __shared__ __align__(16) float red[kSparseWaves][kCols];
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int f0 = blockIdx.x * kSparseRowsPerBlock + wave * kSparseRowsPerWave;
-  const int c0 = blockIdx.y * kCols;
-  const bool col_ok = c0 + LC * lane < C;
-  const int cl = c0 + (col_ok ? LC * lane : 0);
-  const int row_pieces = C / LC;
-  const uint2_t* wlane = reinterpret_cast<const uint2_t*>(blob) + cl / LC;
-  const int G = F / 128;
-  const half_t* scale_t = reinterpret_cast<const half_t*>(blob + static_cast<size_t>(C) * F / 2);
-  const uint8_t* zp_t = reinterpret_cast<const uint8_t*>(scale_t + static_cast<size_t>(G) * C);
-  const int64_t gat = static_cast<int64_t>(f0 / 128) * C + cl;
-  const half8_t sc0 = *reinterpret_cast<const half8_t*>(scale_t + gat);
-  const half8_t sc1 = *reinterpret_cast<const half8_t*>(scale_t + gat + 8);
-  const uint4_t zq = *reinterpret_cast<const uint4_t*>(zp_t + gat);
+// Sums over the four lane groups of a wavefront, each group keeping a quarter of the columns (v[0 .. N/4) afterwards): after the
+// swap of v[i] and v[i + N/2] the lower half of the wavefront holds both halves' v[i], the upper half both halves' v[i + N/2];
+// then the same between neighbouring rows of 16 lanes.  (Two idle slots between a register's write and the swap that reads it.)
+template <int N>
+__device__ __forceinline__ void sum_scatter_groups(float (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(v[i]), "+v"(v[i + N / 2]));
+    v[i] += v[i + N / 2];
+  }
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) {
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(v[i]), "+v"(v[i + N / 4]));
+    v[i] += v[i + N / 4];
+  }
+}
 
-  uint32_t abits[TOK];
-  uint64_t mask;
-  sparse_union_heads<TOK>(in, F, f0, lane, activated, abits, mask);
+struct SparseArgs {
+  int C, F;
+  int rpw;        // rows of ffn.value per wavefront: 32, 64 or 128 (int4: within one 128-group)
+  int activated;  // `in` already holds f16(relu(preact)^2) (the model's ffn.key launch applies it)
+  const half_t* in;
+  const uint8_t* wt;
+  float* partial;
+};
+
+template <int FMT, int TOK>
+__global__ __launch_bounds__(64 * kSparseWaves) void ffn_sparse_kernel(SparseArgs a) {
+  typedef typename SparsePiece<FMT>::type piece_t;
+  constexpr int LC = sparse_lane_cols(FMT);  // columns per lane
+  constexpr int G = kSparseGroups;
+  constexpr int kLanes = 64 / G;             // lanes of a group: one row's piece of the column chunk
+  constexpr int kCols = kLanes * LC;         // columns per block
+  constexpr int kKept = LC / G;              // columns a lane keeps (sum_scatter_groups)
+  constexpr int kThreads = 64 * kSparseWaves;
+  __shared__ __align__(16) float red[kSparseWaves][kCols];
+  __shared__ __align__(8) uint16_t row_s[kSparseWaves][kSparseListed];
+  __shared__ __align__(8) uint16_t coef_s[TOK][kSparseWaves][kSparseListed];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int group = lane / kLanes;
+  const int C = a.C;
+  const int f0 = (blockIdx.x * kSparseWaves + wave) * a.rpw;
+  const int c0 = blockIdx.y * kCols;
+  const int cl = c0 + LC * (lane % kLanes);  // this lane's first column
+  const half_t* in = a.in + static_cast<int64_t>(blockIdx.z) * a.F;                   // this token's activations ...
+  float* partial = a.partial + static_cast<int64_t>(blockIdx.z) * gridDim.x * C;      // ... and partial rows
+  const uint32_t row_bytes = static_cast<uint32_t>(C / LC) * sizeof(piece_t);
+  const uint8_t* wlane = a.wt + static_cast<int64_t>(f0) * row_bytes + (cl < C ? cl / LC : 0) * sizeof(piece_t);
+
+  // the columns this lane ends with
+  const int cq = LC * (lane % kLanes) + (LC / 2) * (lane >> 5) + (LC / 4) * ((lane >> 4) & 1);
+  half4_t w4_scale[kKept / 4 + 1];
+  uint32_t w4_zp[kKept / 4 + 1];
+  if constexpr (FMT == RWKV_FMT_W4) {
+    const int n_groups = a.F / 128;
+    const half_t* scale_t = reinterpret_cast<const half_t*>(a.wt + static_cast<size_t>(C) * a.F / 2);
+    const uint8_t* zp_t = reinterpret_cast<const uint8_t*>(scale_t + static_cast<size_t>(n_groups) * C);
+    const int64_t gat = static_cast<int64_t>(f0 / 128) * C + (c0 + cq < C ? c0 + cq : 0);
+#pragma unroll
+    for (int i = 0; i < kKept / 4; ++i) {
+      w4_scale[i] = *reinterpret_cast<const half4_t*>(scale_t + gat + 4 * i);
+      w4_zp[i] = *reinterpret_cast<const uint32_t*>(zp_t + gat + 4 * i);
+    }
+  }
+
+  // the wavefront's list: rows that are non-zero for any of its tokens, in increasing order, with every token's coefficient
+  int n = 0;
+  for (int r0 = 0; r0 < a.rpw; r0 += 64) {
+    const int r = r0 + lane;
+    uint16_t bits[TOK];
+    bool any = false;
+#pragma unroll
+    for (int t = 0; t < TOK; ++t) {
+      float x = h2f(in[static_cast<int64_t>(t) * a.F + f0 + (r < a.rpw ? r : 0)]);
+      if (!a.activated) {
+        x = fmaxf(round_h(x), 0.0f);
+        x = round_h(x * x);
+      }
+      bits[t] = __builtin_bit_cast(uint16_t, f2h(x));
+      any |= (bits[t] & 0x7fffu) != 0u;  // +0 and -0 both count as zero
+    }
+    any &= r < a.rpw;
+    const uint64_t mask = __ballot(any);
+    if (any) {
+      const int at = n + __builtin_popcountll(mask & ((1ull << lane) - 1));
+      row_s[wave][at] = static_cast<uint16_t>(r);
+#pragma unroll
+      for (int t = 0; t < TOK; ++t) coef_s[t][wave][at] = bits[t];
+    }
+    n += __builtin_popcountll(mask);
+  }
+  // a step takes two rows per lane group; the last one is filled up with a row that is read anyway, at coefficient zero
+  const int steps = (n + 2 * G - 1) / (2 * G);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (n > 0 && n + lane < 2 * G * steps) {
+    row_s[wave][n + lane] = row_s[wave][0];
+#pragma unroll
+    for (int t = 0; t < TOK; ++t) coef_s[t][wave][n + lane] = 0;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 
   float acc[TOK][LC];
   float asum[TOK];
@@ -535,81 +328,82 @@ __global__ __launch_bounds__(64 * kSparseWaves) void ffn_sparse_w4_union_kernel(
 #pragma unroll
     for (int i = 0; i < LC; ++i) acc[t][i] = 0.0f;
   }
-  const half2_t bias = {static_cast<half_t>(1024.0f), static_cast<half_t>(1024.0f)};
-
-  while (mask != 0) {
-    int row[kSparseBatch];
-    bool live[kSparseBatch];
-    const int first = __builtin_ctzll(mask);
+  // Batches of kSparseSteps steps, the next one in flight under the products of this one.  No load sits under a branch (the compiler
+  // would wait for all of them at the first use): steps past the last repeat it.
+  auto request = [&](int s0, piece_t (&q)[kSparseSteps][2]) {
 #pragma unroll
-    for (int p = 0; p < kSparseBatch; ++p) {
-      live[p] = mask != 0;
-      if (live[p]) {
-        row[p] = __builtin_ctzll(mask);
-        mask &= mask - 1;
-      } else {
-        row[p] = first;
-      }
+    for (int u = 0; u < kSparseSteps; ++u) {
+      const uint32_t rows = *reinterpret_cast<const uint32_t*>(&row_s[wave][2 * (G * min(s0 + u, steps - 1) + group)]);
+      q[u][0] = __builtin_nontemporal_load(reinterpret_cast<const piece_t*>(wlane + static_cast<uint64_t>(rows & 0xffffu) * row_bytes));
+      q[u][1] = __builtin_nontemporal_load(reinterpret_cast<const piece_t*>(wlane + static_cast<uint64_t>(rows >> 16) * row_bytes));
     }
-    uint2_t q[kSparseBatch];
+  };
+  auto take = [&](int s, const piece_t (&q)[2]) {
+    half2_t ap[TOK];
 #pragma unroll
-    for (int p = 0; p < kSparseBatch; ++p)
-      q[p] = __builtin_nontemporal_load(&wlane[static_cast<int64_t>(f0 + row[p]) * row_pieces]);
-#pragma unroll
-    for (int p = 0; p < kSparseBatch; p += 2) {
-      half2_t ap[TOK];
-#pragma unroll
-      for (int t = 0; t < TOK; ++t) {
-        const uint32_t c0b = live[p] ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(abits[t]), row[p])) : 0u;
-        const uint32_t c1b = live[p + 1] ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(abits[t]), row[p + 1])) : 0u;
-        ap[t] = as_half2(c0b | (c1b << 16));
-        asum[t] += h2f(ap[t][0]) + h2f(ap[t][1]);
-      }
-#pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        const uint32_t lo = q[p][d];
-        const uint32_t hi = q[p + 1][d];
-        const uint32_t ea = lo & 0x0f0f0f0fu, oa = (lo >> 4) & 0x0f0f0f0fu;
-        const uint32_t eb = hi & 0x0f0f0f0fu, ob = (hi >> 4) & 0x0f0f0f0fu;
-        half2_t w[8];
-        w[0] = as_half2(__builtin_amdgcn_perm(eb, ea, 0x0c040c00u) | 0x64006400u) - bias;
-        w[1] = as_half2(__builtin_amdgcn_perm(ob, oa, 0x0c040c00u) | 0x64006400u) - bias;
-        w[2] = as_half2(__builtin_amdgcn_perm(eb, ea, 0x0c050c01u) | 0x64006400u) - bias;
-        w[3] = as_half2(__builtin_amdgcn_perm(ob, oa, 0x0c050c01u) | 0x64006400u) - bias;
-        w[4] = as_half2(__builtin_amdgcn_perm(eb, ea, 0x0c060c02u) | 0x64006400u) - bias;
-        w[5] = as_half2(__builtin_amdgcn_perm(ob, oa, 0x0c060c02u) | 0x64006400u) - bias;
-        w[6] = as_half2(__builtin_amdgcn_perm(eb, ea, 0x0c070c03u) | 0x64006400u) - bias;
-        w[7] = as_half2(__builtin_amdgcn_perm(ob, oa, 0x0c070c03u) | 0x64006400u) - bias;
-#pragma unroll
-        for (int t = 0; t < TOK; ++t)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc[t][8 * d + i] = __builtin_amdgcn_fdot2(ap[t], w[i], acc[t][8 * d + i], false);
-      }
+    for (int t = 0; t < TOK; ++t) {
+      ap[t] = as_half2(*reinterpret_cast<const uint32_t*>(&coef_s[t][wave][2 * (G * s + group)]));
+      if constexpr (FMT == RWKV_FMT_W4) asum[t] += h2f(ap[t][0]) + h2f(ap[t][1]);
     }
+    sparse_pair<FMT, TOK>(q[0], q[1], ap, acc);
+  };
+  if (steps > 0) {
+    piece_t q[kSparseSteps][2];
+    request(0, q);
+    int s0 = 0;
+    for (; s0 + kSparseSteps < steps; s0 += kSparseSteps) {
+      piece_t next[kSparseSteps][2];
+      request(s0 + kSparseSteps, next);
+#pragma unroll
+      for (int u = 0; u < kSparseSteps; ++u) take(s0 + u, q[u]);
+#pragma unroll
+      for (int u = 0; u < kSparseSteps; ++u)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) q[u][i] = next[u][i];
+    }
+#pragma unroll
+    for (int u = 0; u < kSparseSteps; ++u)
+      if (s0 + u < steps) take(s0 + u, q[u]);
   }
+
 #pragma unroll
   for (int t = 0; t < TOK; ++t) {
+    sum_scatter_groups(acc[t]);
+    if constexpr (FMT == RWKV_FMT_W4) {
+      // sum_f a_f (q_fc - zp_c) = sum_f a_f q_fc - zp_c sum_f a_f, and the scale of the wavefront's 128-group
+      asum[t] = add_swapped_rows<false>(add_swapped_rows<true>(asum[t]));
 #pragma unroll
-    for (int i = 0; i < LC; ++i) {
-      const float zpf = static_cast<float>((zq[i >> 2] >> (8 * (i & 3))) & 0xffu);
-      const float scf = h2f(i < 8 ? sc0[i] : sc1[i - 8]);
-      acc[t][i] = (acc[t][i] - zpf * asum[t]) * scf;
+      for (int i = 0; i < kKept; ++i) {
+        const float zp = static_cast<float>((w4_zp[i >> 2] >> (8 * (i & 3))) & 0xffu);
+        acc[t][i] = (acc[t][i] * (i & 1 ? 0.0625f : 1.0f) - zp * asum[t]) * h2f(w4_scale[i >> 2][i & 3]);
+      }
     }
-    sparse_block_row<LC>(acc[t], red, wave, lane, C, c0,
-                         partial + (static_cast<int64_t>(t) * gridDim.x + blockIdx.x) * C);
+    if (t > 0) __syncthreads();  // the sums of the token before have been read
+#pragma unroll
+    for (int i = 0; i < kKept; ++i) red[wave][cq + i] = acc[t][i];
+    __syncthreads();
+    // the wavefronts' sums meet in wavefront order
+    for (int c = threadIdx.x; c < kCols && c0 + c < C; c += kThreads) {
+      float sum = red[0][c];
+#pragma unroll
+      for (int w = 1; w < kSparseWaves; ++w) sum += red[w][c];
+      partial[(static_cast<int64_t>(t) * gridDim.x + blockIdx.x) * C + c0 + c] = sum;
+    }
   }
 }
 
-// ---- kernel 2: out[c] = f16(scale[c] * sum of the partial rows); block 0 also does the optional row copy --------
-// grid = (ceil(C/64), tokens), block = 256 = 16 groups of partial rows x 16 column quads.  Group g sums rows g, g+16, ... (its
+// ---- kernel 2: out[c] = f16(scale[c] * sum of the partial rows) -----------------------------------
+// grid = (ceil(C/64) and one for the optional row copy, tokens), block = 256 = 16 groups of partial rows x 16 column quads.  Group g sums rows g, g+16, ... (its
 // loads are independent, so they are all in flight together), the 16 group sums meet in LDS in group order.
 __global__ __launch_bounds__(256) void ffn_sparse_finish_kernel(int C, int n_partial, const float* __restrict__ partial,
                                                                 const half_t* __restrict__ scale,
                                                                 half_t* __restrict__ out, RowCopy copy) {
   __shared__ __align__(16) float red[16][64];
-  if (blockIdx.x == 0 && blockIdx.y == 0 && copy.n > 0) {
-    for (int i = threadIdx.x * 8; i < copy.n; i += 256 * 8)
-      *reinterpret_cast<uint4_t*>(copy.dst + i) = *reinterpret_cast<const uint4_t*>(copy.src + i);
+  if (static_cast<int>(blockIdx.x) * 64 >= C) {  // the block past the columns
+    if (blockIdx.y == 0)
+      for (int i = threadIdx.x * 8; i < copy.n; i += 256 * 8)
+        *reinterpret_cast<uint4_t*>(copy.dst + i) = *reinterpret_cast<const uint4_t*>(copy.src + i);
+    return;
   }
   const int g = threadIdx.x >> 4;
   const int cq = (threadIdx.x & 15) * 4;
@@ -635,19 +429,23 @@ __global__ __launch_bounds__(256) void ffn_sparse_finish_kernel(int C, int n_par
   *reinterpret_cast<half4_t*>(out + c) = o;
 }
 
-template <int TOK>
-static void launch_union(hipStream_t st, int fmt, dim3 grid, int C, int F, int activated, const half_t* in, const void* wt,
-                         float* ws) {
+template <int FMT>
+static void launch_walk(hipStream_t st, dim3 grid, int tokens, const SparseArgs& a) {
   const dim3 block(64 * kSparseWaves);
-  if (fmt == RWKV_FMT_W4) {
-    hipLaunchKernelGGL((ffn_sparse_w4_union_kernel<TOK>), grid, block, 0, st, C, F, activated, in, static_cast<const uint8_t*>(wt), ws);
-  } else if (fmt == RWKV_FMT_W8) {
-    hipLaunchKernelGGL((ffn_sparse_union_kernel<RWKV_FMT_W8, TOK>), grid, block, 0, st, C, F, activated, in,
-                       static_cast<const uint4_t*>(wt), ws);
-  } else {
-    hipLaunchKernelGGL((ffn_sparse_union_kernel<RWKV_FMT_F16, TOK>), grid, block, 0, st, C, F, activated, in,
-                       static_cast<const uint4_t*>(wt), ws);
-  }
+  if (tokens == 1) hipLaunchKernelGGL((ffn_sparse_kernel<FMT, 1>), grid, block, 0, st, a);
+  else if (tokens == 2) hipLaunchKernelGGL((ffn_sparse_kernel<FMT, 2>), grid, block, 0, st, a);
+  else if (tokens == 3) hipLaunchKernelGGL((ffn_sparse_kernel<FMT, 3>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((ffn_sparse_kernel<FMT, 4>), grid, block, 0, st, a);
+}
+
+// Bytes of ffn.value from which the walk beats the dense product at the half zeros of random-init weights (walk / dense, us per
+// layer): one and two tokens 1.5B int4 (9 MB) 32.6 / 33.0 and 39.4 / 41.1, int8 32.1 / 34.6, but 0.1B fp16 (5 MB) 24.3 / 22.0 and
+// 27.8 / 25.2 - the second launch costs more than half of the matrix.  Three and four tokens, whose walk reads most of the rows:
+// 1.5B int8 43.4 / 40.8 and 45.2 / 42.6, fp16 (34 MB) 46.9 / 45.2 and 49.2 / 46.6; 7.2B int8 (67 MB) 68.0 / 66.9 and 69.3 / 67.2, int4
+// (35 MB) 62.8 / 61.8 and 65.2 / 61.7: the fewer rows of trained weights decide there.
+bool ffn_sparse_pays(int fmt, int rows, int C, int F) {
+  const size_t bytes = ffn_sparse_packed_bytes(fmt, C, F);
+  return rows <= 2 ? bytes >= (8u << 20) : rows <= kSparseUnionMaxRows && bytes > (32u << 20);
 }
 
 int ffn_sparse_launch(hipStream_t st, int fmt, int rows, int C, int F, int activated, const half_t* in, const void* wt,
@@ -663,27 +461,20 @@ int ffn_sparse_launch(hipStream_t st, int fmt, int rows, int C, int F, int activ
     RWKV_REQUIRE(copy->n % 8 == 0, "ffn_sparse: row copy length %d must be a multiple of 8", copy->n);
     cp = *copy;
   }
-  const int n_partial = F / kSparseRowsPerBlock;
-  const dim3 grid(n_partial, ceil_div(C, 64 * sparse_lane_cols(fmt)), rows);
-  if (one_walk && rows >= 2 && rows <= kSparseUnionMaxRows) {
-    // the tokens share one walk over the rows that are non-zero for any of them
-    const dim3 g2(grid.x, grid.y, 1);
-    float* ws = static_cast<float*>(workspace);
-    if (rows == 2) launch_union<2>(st, fmt, g2, C, F, activated, in, wt, ws);
-    else if (rows == 3) launch_union<3>(st, fmt, g2, C, F, activated, in, wt, ws);
-    else launch_union<4>(st, fmt, g2, C, F, activated, in, wt, ws);
-  } else if (fmt == RWKV_FMT_W4) {
-    hipLaunchKernelGGL(ffn_sparse_w4_kernel, grid, dim3(64 * kSparseWaves), 0, st, C, F, activated, in,
-                       static_cast<const uint8_t*>(wt), static_cast<float*>(workspace));
-  } else if (fmt == RWKV_FMT_W8) {
-    hipLaunchKernelGGL(ffn_sparse_kernel<RWKV_FMT_W8>, grid, dim3(64 * kSparseWaves), 0, st, C, F, activated, in,
-                       static_cast<const uint4_t*>(wt), static_cast<float*>(workspace));
-  } else {
-    hipLaunchKernelGGL(ffn_sparse_kernel<RWKV_FMT_F16>, grid, dim3(64 * kSparseWaves), 0, st, C, F, activated, in,
-                       static_cast<const uint4_t*>(wt), static_cast<float*>(workspace));
-  }
+  // 2 .. 4 tokens share one walk over the rows that are non-zero for any of them; otherwise a walk per token
+  const int tokens = one_walk && rows >= 2 && rows <= kSparseUnionMaxRows ? rows : 1;
+  // rows per wavefront: as many as leave a block per CU (fewer partial rows; twice the blocks 1-3 % of the step slower)
+  const int chunks = ceil_div(C, 64 / kSparseGroups * sparse_lane_cols(fmt));
+  int rpw = 128;
+  while (rpw > 32 && (F % (kSparseWaves * rpw) != 0 || static_cast<int64_t>(chunks) * (F / (kSparseWaves * rpw)) < device_cu_count())) rpw /= 2;
+  const SparseArgs a = {C, F, rpw, activated, in, static_cast<const uint8_t*>(wt), static_cast<float*>(workspace)};
+  const int n_partial = F / (kSparseWaves * rpw);
+  const dim3 grid(n_partial, chunks, rows / tokens);
+  if (fmt == RWKV_FMT_W4) launch_walk<RWKV_FMT_W4>(st, grid, tokens, a);
+  else if (fmt == RWKV_FMT_W8) launch_walk<RWKV_FMT_W8>(st, grid, tokens, a);
+  else launch_walk<RWKV_FMT_F16>(st, grid, tokens, a);
   RWKV_LAUNCH_CHECK();
-  hipLaunchKernelGGL(ffn_sparse_finish_kernel, dim3(ceil_div(C, 64), rows), dim3(256), 0, st, C, n_partial,
+  hipLaunchKernelGGL(ffn_sparse_finish_kernel, dim3(ceil_div(C, 64) + (cp.n > 0 ? 1 : 0), rows), dim3(256), 0, st, C, n_partial,
                      static_cast<const float*>(workspace), fmt == RWKV_FMT_W8 ? scale : nullptr, out, cp);
   RWKV_LAUNCH_CHECK();
   return RWKV_OK;

@@ -154,7 +154,7 @@ struct rwkv_hip_session {
   size_t gemm_ws_bytes = 0;
   void* sparse_ws = nullptr;  // partial rows of the row-skipping ffn.value product
   size_t sparse_ws_bytes = 0;
-  int sparse_ffn_rows = 4;    // decode steps of up to this many rows read only the ffn.value rows with a non-zero activation
+  int sparse_ffn_rows = -1;   // decode steps of up to this many rows read only the ffn.value rows with a non-zero activation; -1: where it pays
                               // (2..4 rows share one walk over the rows that are non-zero for any of them)
   bool wkv_fp16 = false;      // the WKV state tensor is fp16 [L,B,H,64,64] (the reference's use_wkv32 == false)
   int tmix_rows = -1;         // decode steps' single-launch time-mix core: rows per block 1/2/4, 0 never, < 0 by batch
@@ -473,9 +473,12 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
   // output projection's launch applies the gate while it stages x.
   const bool gate_split = fused_tmix && rows == 1 && C <= 4096 && !s->trace;
 
-  // Decode steps of a few rows (one by default) read, per row, only the ffn.value rows whose relu^2 activation is
-  // non-zero (int8 or fp16 weights).
-  const bool sparse_value = step && rows <= s->sparse_ffn_rows && s->sparse_ws != nullptr;
+  // Decode steps of a few rows read only the ffn.value rows whose relu^2 activation is non-zero.
+  const bool sparse_step = step && s->sparse_ws != nullptr;
+  const auto sparse_value = [&](const Matrix& mv) {
+    if (!sparse_step || !mv.sparse_t) return false;
+    return s->sparse_ffn_rows >= 0 ? rows <= s->sparse_ffn_rows : rows <= kSparseUnionMaxRows && ffn_sparse_pays(mv.fmt, rows, C, F);
+  };
 
   // Prefill chunks of up to 256 rows: residual add + LayerNorm + token shift as one launch per LayerNorm (the block
   // of a row also normalises the previous row).  The new shift rows come out in a buffer of their own - the blocks
@@ -766,7 +769,7 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
       const Matrix& mv = w.m[RWKV_M_FFN_VALUE];
       RowCopy cp;
       cp.src = b.ln2; cp.dst = shift1; cp.n = rows * C;
-      if (sparse_value && mv.sparse_t) {
+      if (sparse_value(mv)) {
         TRY_AUX(ffn_sparse_launch(st, mv.fmt, rows, C, F, 1, b.act, mv.sparse_t, mv.scale, s->sparse_ws, s->sparse_ws_bytes, b.cm,
                                   &cp, true));
       } else if (rows > 8 || (mv.packed && rows >= kPackedMinRows)) {
@@ -781,7 +784,7 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
       pending = RowCopy{};
       TRY_PROF(apply_matrix(s, w.m[RWKV_M_FFN_KEY], rows, F, C, b.mixed, RWKV_EPI_RELU_SQUARE, 0, b.act, nullptr, &moved));
       const Matrix& mv = w.m[RWKV_M_FFN_VALUE];
-      if (sparse_value && mv.sparse_t) {
+      if (sparse_value(mv)) {
         TRY_AUX(ffn_sparse_launch(st, mv.fmt, rows, C, F, 1, b.act, mv.sparse_t, mv.scale, s->sparse_ws, s->sparse_ws_bytes, b.cm,
                                   nullptr, true));
       } else {

@@ -217,6 +217,8 @@ int ffn_sparse_pack_launch(hipStream_t st, int fmt, int C, int F, const void* w,
 // one_walk: 2 .. kSparseUnionMaxRows tokens share one walk over the rows that are non-zero for any of them (each such
 // row is read once); otherwise every token walks its own rows.
 constexpr int kSparseUnionMaxRows = 4;
+// whether the walk is the faster product (one_walk, 1 .. kSparseUnionMaxRows tokens)
+bool ffn_sparse_pays(int fmt, int rows, int C, int F);
 int ffn_sparse_launch(hipStream_t st, int fmt, int rows, int C, int F, int activated, const half_t* in, const void* wt,
                       const half_t* scale, void* workspace, size_t workspace_bytes, half_t* out, const RowCopy* copy,
                       bool one_walk);

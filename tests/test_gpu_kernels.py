@@ -895,6 +895,16 @@ def test_cmix_sparse_down_shared_walk_matches_oracle_and_per_token_walks(gpu, or
         hip.cmix_sparse_down_relu_rows_shared(fmt, 5, C, F, dev(hip, pre), wt, sd, ws, out)   # more tokens than one walk takes
 
 
+@pytest.mark.parametrize("fmt_name", ["w8", "f16", "w4"])
+@pytest.mark.parametrize("C,F", [(16, 256), (272, 768), (400, 5120), (4112, 8192)])
+def test_cmix_sparse_down_at_the_edges_of_chunks_and_lists(gpu, orc, C, F, fmt_name):
+    """A last column chunk of 16 columns, wavefronts of 32, 64 and 128 rows, lists from empty to full: one token, and walks of two
+    and four that share it."""
+    test_cmix_sparse_down_matches_dense_product_and_oracle(gpu, orc, C, F, fmt_name)
+    for rows in (2, 4):
+        test_cmix_sparse_down_shared_walk_matches_oracle_and_per_token_walks(gpu, orc, fmt_name, C, F, rows)
+
+
 def test_cmix_sparse_rejects_bad_arguments(gpu):
     hip = gpu
     with pytest.raises(hip.RwkvHipError):

@@ -355,6 +355,29 @@ def test_fused_launches_match_the_standalone_kernels_bitwise(gpu, fmt, B, T):
     sess.close()
 
 
+def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
+    """Without set_sparse_ffn a decode step walks the non-zero rows only where the matrix pays for the second launch: a
+    small model gives the bits of the dense product, and those of the walk once it is asked for."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=2, C=512, H=8, F=2048, V=512, Rw=32, Ra=32, Rg=64, Rv=32)
+    model = HipModel.from_host_weights(dims, synth_weights(dims, 11), hip.FMT_W8)
+    for rows in (1, 2, 4):
+        tokens = np.arange(rows).reshape(rows, 1)
+        out = []
+        for most in (None, 0, 4):
+            sess = Session(model)
+            if most is not None:
+                sess.set_sparse_ffn(most)
+            st, lg = State(dims, rows), hip.DeviceArray((rows, dims.V), np.float32)
+            for _ in range(3):
+                sess.forward(tokens, st, lg)
+            out.append(lg.numpy().copy())
+            sess.close()
+        assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+        assert rel_err(out[2], out[1]) <= 2.0 ** -8  # the same products, fp32 sums in another order, rounded to fp16 per layer
+
+
 def test_chunked_prefill_resume_bitwise_and_chunk_size_invariance(gpu, orc):
     """State carried in HBM across chunks.  (a) Saving the state to the host between chunks and resuming from
     the restored copy is bitwise identical to the uninterrupted run (same chunking).  (b) A different chunking
