@@ -186,7 +186,8 @@ __global__ __launch_bounds__(kLoraThreads) void lora_out_kernel(LoraOutMultiArgs
 // and takes the sums through LDS and two barriers; this one takes 32 rows x 32*NW channels per block.  The weights are the
 // A operand: accumulator v of lane (j, h) is row j of the tile, and the channels are dealt to A's rows so that a lane's 16
 // values are 16 consecutive channels (16*h + v of the wavefront's 32) and leave in 16-byte stores straight from the registers.
-// A wavefront walks the whole rank with the weights of four steps in flight; its sums are built as above (even and odd
+// A wavefront walks the whole rank with the weights of eight steps in flight (16 wavefronts: four, which their registers allow; with
+// four the 8-wavefront block takes 14.2 us instead of 12.1 for 125 rows in a 7.2B prefill, whose weights come out of HBM); its sums are built as above (even and odd
 // steps apart, hi before lo, then added), so the bits are the same.
 // Per rank step a CU's wavefronts ask as many cycles of LDS (the hidden) and of the vector memory path (the weights) as of
 // the matrix core.  Tiles of 64 rows or 64 channels per wavefront ask for half of one of them and lose as much to occupancy
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(NW * 64) void lora_out_wide_kernel(LoraOutMultiArgs
   extern __shared__ __align__(16) unsigned char lds_raw[];
   constexpr int kTpr = NW * 64 / kLoraRows;                      // threads that stage one row
   constexpr int kStage = (kLoraMaxR / 8 + 1 + kTpr - 1) / kTpr;  // pieces of 8 per thread, the zeroed pad among them
-  constexpr int kDepth = 4;                                      // rank steps whose weights are in flight
+  constexpr int kDepth = NW == 8 ? 8 : 4;                        // rank steps whose weights are in flight
   const LoraOutProblem& p = a.p[blockIdx.z];
   const int R = p.R;
   const int ld = R + 8;
@@ -390,14 +391,14 @@ int lora_out_multi(hipStream_t st, const LoraOutMultiArgs& a) {
   }
   // Up to one and a half blocks per CU the small tile is the faster one (its rank is walked by two groups of wavefronts); past
   // that, what the blocks repeat counts.  us of the four problems of a layer, small tile / 32 x 256: 4096 channels, 64 rows
-  // (256 blocks) 8.3 / 11.1, 128 (512) 12.0 / 11.5, 144 (640) 14.9 / 11.7, 256 20.1 / 14.8; 2048 channels, 128 rows (256) 6.9 / 7.2,
-  // 192 (384) 9.1 / 8.0, 256 (512) 9.7 / 8.3; 768 channels, 256 rows (192) 4.6 / 6.3.
+  // (256 blocks) 8.3 / 11.1, 128 (512) 12.0 / 10.7, 160 15.0 / 12.3, 256 20.0 / 13.2; 2048 channels, 128 rows (256) 6.9 / 7.2,
+  // 192 (384) 9.4 / 7.3, 256 (512) 9.8 / 8.2; 768 channels, 256 rows (192) 4.6 / 6.3.
   const int row_tiles = ceil_div(a.M, kLoraRows);
   const int64_t cus = device_cu_count();
   if (static_cast<int64_t>(ceil_div(a.C, kLoraCols)) * row_tiles * a.n * 2 > 3 * cus) {
     // twice as many channels per block where that still leaves two blocks per CU and no channel of a block unused: 32 x 256 / 32 x
-    // 512 at 4096 channels and 256 rows 14.6 / 15.8, 500 22.5 / 19.0, 2048 68.8 / 56.7; 2048 channels and 999 rows 14.4 / 14.0
-    // (before, with the small tile's blocks walking several row tiles: 20.6, 34.5, 108.5; 27.3)
+    // 512 at 4096 channels and 500 rows 21.4 / 19.2, 1000 39.0 / 37.4, 2048 68.4 / 57.9; 2048 channels and 999 rows 17.9 / 13.1, 2048
+    // 29.2 / 28.7 (before, with the small tile's blocks walking several row tiles: 33.7, 60.5, 107.6; 26.5, 50.1)
     const bool wide = a.C % 512 == 0 && static_cast<int64_t>(a.C / 512) * row_tiles * a.n >= 2 * cus;
     return wide ? lora_out_wide_launch<16>(st, a) : lora_out_wide_launch<8>(st, a);
   }
