@@ -416,64 +416,169 @@ int token_shift_mix_launch(hipStream_t st, const MixArgs& a) {
   return RWKV_OK;
 }
 
-// ---- kk normalise + a-gate: one wave per (row, head), lane = channel --------------------------------
-// Optional fp32 outputs feed the WKV sequence kernel directly (values are the fp16-rounded ones).
-
-__global__ __launch_bounds__(256) void kk_a_gate_kernel(KkArgs p) {
-  const int64_t rh = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (rh >= p.rows_heads) return;
-  const int lane = threadIdx.x & 63;
-  const int h = static_cast<int>(rh % p.H);
-  const int64_t idx = rh * kHead + lane;
-  const int c = h * kHead + lane;
-  const float kv = h2f(p.k[idx]);
-  const float u = kv * h2f(p.k_k[c]);
-  const float total = wave_sum(u * u);
-  const float inv = 1.0f / fmaxf(sqrtf(total), kKkEps);
-  const float kk = u * inv;
-  const float av = sigmoid_f(h2f(p.a0[c]) + h2f(p.a12[idx]));
-  const float ka = h2f(p.k_a[c]);
-  const half_t nk = f2h(kv * fmaf(av, ka, 1.0f - ka));
-  const half_t nkk = f2h(-kk);
-  const half_t kka = f2h(kk * av);
-  if (p.new_k) p.new_k[idx] = nk;
-  if (p.neg_kk) p.neg_kk[idx] = nkk;
-  if (p.kka) p.kka[idx] = kka;
-  if (p.d32) {
-    const float wraw = round_h(h2f(p.w12[idx]) + h2f(p.w0[c]));  // rwkv7_add_vec_launch rounding point
-    p.d32[idx] = exp2f(-0.8750387749145276f / (1.0f + exp2f(-1.4426950408889634f * wraw)));
+// ---- kk normalise + a-gate, GroupNorm + rkv residual + gate: 16 lanes per (row, head), four channels per lane ------------
+// Both read and write a few fp16 rows once: with one channel per lane their requests were 128 bytes per wavefront and the
+// sums six trips through LDS each.  Four channels per lane make requests of 512 bytes and keep the sums in the registers of a DPP row;
+// eight would halve the blocks of a 128-row chunk, which are two per CU.  us, before -> now: 999 rows x 32 heads 12.5 and 9.7
+// -> 9.4 and 5.8; 128 rows x 64 heads 5.2 and 4.6 -> 5.3 and 4.7 (launch and latency).
+//
+// The sums are those of a wavefront with one channel per lane (wave_sum: channel i adds what i ^ 32, 16, 8, 4, 2, 1 holds), so
+// that the kernels that do this inside a larger one agree bitwise: the first four levels are lane exchanges, the last two lie
+// within a lane.
+__device__ __forceinline__ float head_sum_tail(float (&t)[4]) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    t[e] += __builtin_bit_cast(float, lane_xor_dpp<4>(__builtin_bit_cast(int, t[e])));
+    t[e] = dpp_add<0x4E>(t[e]);  // lane ^ 2
+    t[e] = dpp_add<0xB1>(t[e]);  // lane ^ 1
   }
-  if (p.w_sum16) p.w_sum16[idx] = f2h(h2f(p.w12[idx]) + h2f(p.w0[c]));
+  return (t[0] + t[2]) + (t[1] + t[3]);
+}
+__device__ __forceinline__ float head_sum(const float (&v)[4]) {
+  float t[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) t[e] = dpp_add<0x128>(v[e]);  // lane ^ 8
+  return head_sum_tail(t);
+}
+// sum of a * b with a fused first level (wave_sum_dpp_of_product)
+__device__ __forceinline__ float head_sum_of_product(const float (&a)[4], const float (&b)[4]) {
+  float t[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float p;
+    {
+#pragma clang fp contract(off)
+      p = a[e] * b[e];
+    }
+    t[e] = fmaf(a[e], b[e], __builtin_bit_cast(float, lane_xor_dpp<8>(__builtin_bit_cast(int, p))));
+  }
+  return head_sum_tail(t);
+}
+// f16(a * b) of four values with one rounding each, what the compiler makes of a product that is only converted
+// (v_fma_mixlo_f16) where a lane has one channel; with four it would convert pairs, which rounds twice.
+__device__ __forceinline__ half4_t mul_f16(const float (&a)[4], const float (&b)[4]) {
+  uint2_t r;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    uint32_t d;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\tv_fma_mixhi_f16 %0, %3, %4, 0"
+        : "=&v"(d)
+        : "v"(a[2 * i]), "v"(b[2 * i]), "v"(a[2 * i + 1]), "v"(b[2 * i + 1]));
+    r[i] = d;
+  }
+  return __builtin_bit_cast(half4_t, r);
+}
+// four values at p; VEC: p is aligned to them
+template <bool VEC>
+__device__ __forceinline__ half4_t load4(const half_t* p) {
+  if constexpr (VEC) return *reinterpret_cast<const half4_t*>(p);
+  return half4_t{p[0], p[1], p[2], p[3]};
+}
+template <bool VEC>
+__device__ __forceinline__ void store4(half_t* p, half4_t v) {
+  if constexpr (VEC) {
+    *reinterpret_cast<half4_t*>(p) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = v[e];
+  }
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void kk_a_gate_kernel(KkArgs p) {
+  const int64_t rh = static_cast<int64_t>(blockIdx.x) * 16 + (threadIdx.x >> 4);
+  if (rh >= p.rows_heads) return;  // whole groups of 16 lanes
+  const int h = static_cast<int>(rh % p.H);
+  const int64_t idx = rh * kHead + 4 * (threadIdx.x & 15);
+  const int c = h * kHead + 4 * (threadIdx.x & 15);
+  const half4_t k4 = load4<VEC>(p.k + idx), a4 = load4<VEC>(p.a12 + idx);
+  const half4_t kk4 = load4<VEC>(p.k_k + c), a04 = load4<VEC>(p.a0 + c), ka4 = load4<VEC>(p.k_a + c);
+  half4_t w4 = {}, w04 = {};
+  if (p.d32 || p.w_sum16) {
+    w4 = load4<VEC>(p.w12 + idx);
+    w04 = load4<VEC>(p.w0 + c);
+  }
+  float u[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) u[e] = h2f(k4[e]) * h2f(kk4[e]);
+  const float total = head_sum_of_product(u, u);
+  const float inv = 1.0f / fmaxf(sqrtf(total), kKkEps);
+  half4_t pkk, ws;
+  float4_t d;
+  float kv[4], kf[4], kk[4], av[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    kk[e] = u[e] * inv;
+    av[e] = sigmoid_f(h2f(a04[e]) + h2f(a4[e]));
+    const float ka = h2f(ka4[e]);
+    kv[e] = h2f(k4[e]);
+    kf[e] = fmaf(av[e], ka, 1.0f - ka);
+    pkk[e] = f2h(kk[e]);
+    ws[e] = f2h(h2f(w4[e]) + h2f(w04[e]));  // rwkv7_add_vec_launch rounding point
+  }
+  if (p.new_k) store4<VEC>(p.new_k + idx, mul_f16(kv, kf));
+  // (negated as halves: the compiler does not get a vector of negated floats through without packed fp32)
+  const uint2_t flipped = __builtin_bit_cast(uint2_t, pkk) ^ uint2_t{0x80008000u, 0x80008000u};
+  if (p.neg_kk) store4<VEC>(p.neg_kk + idx, __builtin_bit_cast(half4_t, flipped));
+  if (p.kka) store4<VEC>(p.kka + idx, mul_f16(kk, av));
+  if (p.d32) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d[e] = exp2f(-0.8750387749145276f / (1.0f + exp2f(-1.4426950408889634f * h2f(ws[e]))));
+    *reinterpret_cast<float4_t*>(p.d32 + idx) = d;
+  }
+  if (p.w_sum16) store4<VEC>(p.w_sum16 + idx, ws);
 }
 
 int kk_a_gate_launch(hipStream_t st, const KkArgs& p) {
   RWKV_REQUIRE(p.rows_heads > 0 && p.H > 0, "kk_a_gate: bad shape");
   RWKV_REQUIRE(p.w_sum16 == nullptr || (p.w12 && p.w0), "kk_a_gate: the rounded decay logit needs w12 and w0");
-  hipLaunchKernelGGL(kk_a_gate_kernel, dim3(ceil_div(p.rows_heads, 4)), dim3(256), 0, st, p);
+  RWKV_REQUIRE(reinterpret_cast<uintptr_t>(p.d32) % 16 == 0, "kk_a_gate: the decay must be 16-byte aligned");
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(p.k) | reinterpret_cast<uintptr_t>(p.a12) | reinterpret_cast<uintptr_t>(p.k_k) |
+                         reinterpret_cast<uintptr_t>(p.a0) | reinterpret_cast<uintptr_t>(p.k_a) | reinterpret_cast<uintptr_t>(p.w12) |
+                         reinterpret_cast<uintptr_t>(p.w0) | reinterpret_cast<uintptr_t>(p.new_k) |
+                         reinterpret_cast<uintptr_t>(p.neg_kk) | reinterpret_cast<uintptr_t>(p.kka) |
+                         reinterpret_cast<uintptr_t>(p.w_sum16);
+  const dim3 grid(ceil_div(p.rows_heads, 16));
+  if (bits % 8 == 0) hipLaunchKernelGGL(kk_a_gate_kernel<true>, grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(kk_a_gate_kernel<false>, grid, dim3(256), 0, st, p);
   RWKV_LAUNCH_CHECK();
   return RWKV_OK;
 }
 
-// ---- per-head GroupNorm + rkv residual + gate: one wave per (row, head) --------------------------------
+template <bool VEC>
 __global__ __launch_bounds__(256) void lnx_rkvres_xg_kernel(int64_t rows_heads, int H, const half_t* __restrict__ y,
                                                             const half_t* __restrict__ r, const half_t* __restrict__ k,
                                                             const half_t* __restrict__ v, const half_t* __restrict__ r_k,
                                                             const half_t* __restrict__ lnw, const half_t* __restrict__ lnb,
-                                                            const half_t* __restrict__ g, half_t* __restrict__ out) {
-  const int64_t rh = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (rh >= rows_heads) return;
-  const int lane = threadIdx.x & 63;
+                                                            const half_t* __restrict__ g, half_t* out) {
+  const int64_t rh = static_cast<int64_t>(blockIdx.x) * 16 + (threadIdx.x >> 4);
+  if (rh >= rows_heads) return;  // whole groups of 16 lanes
   const int h = static_cast<int>(rh % H);
-  const int64_t idx = rh * kHead + lane;
-  const int c = h * kHead + lane;
-  const float yv = h2f(y[idx]);
-  const float mean = wave_sum(yv) * (1.0f / 64.0f);
-  const float d = yv - mean;
-  const float var = wave_sum(d * d) * (1.0f / 64.0f);
+  const int64_t idx = rh * kHead + 4 * (threadIdx.x & 15);
+  const int c = h * kHead + 4 * (threadIdx.x & 15);
+  const half4_t y4 = load4<VEC>(y + idx), r4 = load4<VEC>(r + idx), k4 = load4<VEC>(k + idx), v4 = load4<VEC>(v + idx),
+                g4 = load4<VEC>(g + idx);
+  const half4_t rk4 = load4<VEC>(r_k + c), lw4 = load4<VEC>(lnw + c), lb4 = load4<VEC>(lnb + c);
+  float yv[4], d[4], rk[4], w[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) yv[e] = h2f(y4[e]);
+  const float mean = head_sum(yv) * (1.0f / 64.0f);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    d[e] = yv[e] - mean;
+    rk[e] = mul_f32(h2f(r4[e]), h2f(k4[e]));
+    w[e] = h2f(rk4[e]);
+  }
+  const float var = head_sum_of_product(d, d) * (1.0f / 64.0f);
   const float rstd = rsqrtf(var + kLnxEps);
-  const float rkv = wave_sum(h2f(r[idx]) * h2f(k[idx]) * h2f(r_k[c]));
-  const float o = (d * rstd * h2f(lnw[c]) + h2f(lnb[c]) + rkv * h2f(v[idx])) * h2f(g[idx]);
-  out[idx] = f2h(o);
+  const float rkv = head_sum_of_product(rk, w);
+  float o[4], gate[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    o[e] = d[e] * rstd * h2f(lw4[e]) + h2f(lb4[e]) + rkv * h2f(v4[e]);
+    gate[e] = h2f(g4[e]);
+  }
+  store4<VEC>(out + idx, mul_f16(o, gate));
 }
 
 // ---- small element-wise kernels ---------------------------------------------------------------------
@@ -519,8 +624,14 @@ int embed_gather_launch(hipStream_t st, int rows, int C, const int64_t* tokens, 
 
 int lnx_launch(hipStream_t st, int64_t rows_heads, int H, const half_t* y, const half_t* r, const half_t* k,
                const half_t* v, const half_t* r_k, const half_t* lnw, const half_t* lnb, const half_t* g, half_t* out) {
-  hipLaunchKernelGGL(lnx_rkvres_xg_kernel, dim3(ceil_div(rows_heads, 4)), dim3(256), 0, st, rows_heads, H, y, r, k, v,
-                     r_k, lnw, lnb, g, out);
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(r) | reinterpret_cast<uintptr_t>(k) |
+                         reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(r_k) | reinterpret_cast<uintptr_t>(lnw) |
+                         reinterpret_cast<uintptr_t>(lnb) | reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(out);
+  const dim3 grid(ceil_div(rows_heads, 16));
+  if (bits % 8 == 0)
+    hipLaunchKernelGGL(lnx_rkvres_xg_kernel<true>, grid, dim3(256), 0, st, rows_heads, H, y, r, k, v, r_k, lnw, lnb, g, out);
+  else
+    hipLaunchKernelGGL(lnx_rkvres_xg_kernel<false>, grid, dim3(256), 0, st, rows_heads, H, y, r, k, v, r_k, lnw, lnb, g, out);
   RWKV_LAUNCH_CHECK();
   return RWKV_OK;
 }

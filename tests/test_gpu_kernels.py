@@ -615,6 +615,34 @@ def test_kk_gate_groupnorm_lora(gpu, orc):
             assert err <= F16_TOL
 
 
+@pytest.mark.parametrize("rows,H", [(1, 1), (3, 5), (129, 64)])
+def test_kk_gate_groupnorm_of_tensors_that_are_not_aligned(gpu, rows, H):
+    """16 lanes per head with a last block that is partial; every tensor one half behind a 16-byte boundary gives the bits
+    of aligned ones."""
+    hip = gpu
+    rng = np.random.default_rng(rows + H)
+    C = H * 64
+    n = rows * C
+
+    def pair(size):
+        x = rng.standard_normal(size).astype(np.float16)
+        shifted = dev(hip, np.concatenate([np.zeros(1, np.float16), x]))
+        return dev(hip, x), shifted, shifted.ptr + 2
+
+    k, a12, y, r, v, g = (pair(n) for _ in range(6))
+    k_k, a0, k_a, r_k, lnw, lnb = (pair(C) for _ in range(6))
+    outs = []
+    for i in (0, 2):
+        o = [hip.DeviceArray((n + 1,), np.float16) for _ in range(4)]
+        to = [x.ptr + i for x in o]
+        hip.kk_a_gate(rows, C, H, k[i], k_k[i], a0[i], a12[i], k_a[i], *to[:3])
+        hip.lnx_rkvres_xg(rows, C, H, y[i], r[i], k[i], v[i], r_k[i], lnw[i], lnb[i], g[i], to[3])
+        hip.device_sync()
+        outs.append([x.numpy()[i // 2:][:n].view(np.uint16) for x in o])
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+
+
 def test_lora_out_blocks_walk_several_row_tiles(gpu, orc):
     """Ten row tiles, the last one partial; the v-residual epilogue is checked on the same rows."""
     hip = gpu
