@@ -12,12 +12,15 @@
 // 1024 threads by row length - decode steps have few rows, so the wavefronts of a row are the only parallelism the
 // launch has: 512 threads instead of 256 with two slices each make a 4096-wide row 15-25 % faster), so a row is
 // read from HBM once for the two-pass mean/variance and the normalise+lerp epilogue.
+#include <algorithm>
 #include <type_traits>
 
 #include "ops.h"
 
 namespace rwkv {
 
+constexpr int kMixSeqRows = 256;  // rows of the launch with a block per row; more: blocks of several rows
+constexpr int kMixRows = 4;       // rows of a block at most
 constexpr int kLnMaxThreads = 1024;  // one 8-element vector per thread -> C <= 8192
 
 
@@ -332,6 +335,152 @@ __global__ __launch_bounds__(NT) void ln_mix_seq_kernel(LnArgs a) {
   if (t == a.T - 1) *reinterpret_cast<half8_t*>(a.shift_next + static_cast<int64_t>(bi) * C + c) = yv;
 }
 
+// The same for many rows: a block walks several consecutive rows, so that only the row before its first one is normalised a
+// second time, and keeps the LayerNorm output of the row before in registers.  Bound by memory: against a LayerNorm and a
+// token-shift launch the LN rows are neither written nor read again.  The loads of the next row are in flight during the
+// reductions of this one.  Statements and order of ln_mix_seq_kernel: the same bits.  Two rows per block, four from 2048 rows on,
+// us of LN1 + LN2 with 1 / 2 / 4 / 8 rows per block: 2048 rows x 4096 63.9 / 50.4 / 46.8 / 47.8 (two launches each 66.3), 999 x 2048 21.5 /
+// 18.1 / 19.1 / 26.7 (25.4).
+// PLANES: split-K planes of the residual requested ahead (0: a plain fp16 residual); further ones are read in line.
+template <int NT, int PLANES>
+__global__ __launch_bounds__(NT) void ln_mix_rows_kernel(LnArgs a, int rows, int rows_per_block) {
+  constexpr int NW = NT / 64;
+  __shared__ float red[2][2][NW];  // by row parity: a buffer is written again two barriers after it was read
+  const int C = a.C;
+  const int first = blockIdx.x * rows_per_block;
+  const int n = min(rows_per_block, rows - first);
+  int bi = first / a.T;
+  int t = first - bi * a.T;
+  const bool live = static_cast<int>(threadIdx.x) * 8 < C;
+  const int c = live ? threadIdx.x * 8 : 0;  // idle threads repeat slice 0 and store nothing
+  const int wave = threadIdx.x >> 6;
+
+  struct Raw {
+    half8_t x, r;
+    float4_t q[PLANES > 0 ? 2 * PLANES : 1];
+  };
+  auto request = [&](int row, Raw& o) {
+    const int64_t at = static_cast<int64_t>(row) * C + c;
+    o.x = *reinterpret_cast<const half8_t*>(a.x + at);
+    if constexpr (PLANES == 0) {
+      o.r = *reinterpret_cast<const half8_t*>(a.res + at);
+    } else {
+#pragma unroll
+      for (int u = 0; u < PLANES; ++u) {
+        const float* p = a.res_partial + at + (u < a.res_splits ? u : a.res_splits - 1) * a.res_plane;
+        o.q[2 * u] = *reinterpret_cast<const float4_t*>(p);
+        o.q[2 * u + 1] = *reinterpret_cast<const float4_t*>(p + 4);
+      }
+    }
+  };
+  const half8_t wv = *reinterpret_cast<const half8_t*>(a.w + c);
+  const half8_t bv = *reinterpret_cast<const half8_t*>(a.b + c);
+  half8_t mv[6];
+#pragma unroll
+  for (int s = 0; s < 6; ++s) mv[s] = *reinterpret_cast<const half8_t*>(a.mu[s < a.n_mix ? s : a.n_mix - 1] + c);
+  half8_t sv8 = wv;
+  if constexpr (PLANES > 0) {
+    if (a.res_scale) sv8 = *reinterpret_cast<const half8_t*>(a.res_scale + c);
+  }
+  half8_t prev = *reinterpret_cast<const half8_t*>(a.shift + static_cast<int64_t>(bi) * C + c);
+  Raw cur, next;
+  int i = t > 0 ? -1 : 0;  // -1: the row before, for its output alone
+  request(first + i, cur);
+  for (; i < n; ++i) {
+    request(first + min(i + 1, n - 1), next);
+    half8_t rv = cur.r;
+    if constexpr (PLANES > 0) {
+      float4_t s0 = cur.q[0], s1 = cur.q[1];
+#pragma unroll
+      for (int u = 1; u < PLANES; ++u) {
+        if (u < a.res_splits) {
+          s0 = s0 + cur.q[2 * u];
+          s1 = s1 + cur.q[2 * u + 1];
+        }
+      }
+      for (int u = PLANES; u < a.res_splits; ++u) {
+        const float* p = a.res_partial + static_cast<int64_t>(first + i) * C + c + u * a.res_plane;
+        s0 = s0 + *reinterpret_cast<const float4_t*>(p);
+        s1 = s1 + *reinterpret_cast<const float4_t*>(p + 4);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        rv[e] = f2h(mul_f32(s0[e], a.res_scale ? h2f(sv8[e]) : 1.0f));
+        rv[4 + e] = f2h(mul_f32(s1[e], a.res_scale ? h2f(sv8[4 + e]) : 1.0f));
+      }
+    }
+    float v[8];
+    float sum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = live ? h2f(cur.x[e]) + h2f(rv[e]) : 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum += v[e];
+    auto block_total = [&](float x, float* scratch) {  // block_sum's order
+      x = wave_sum_dpp(x);
+      if ((threadIdx.x & 63) == 0) scratch[wave] = x;
+      __syncthreads();
+      float total = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) total += scratch[w];
+      return total;
+    };
+    const float mean = block_total(sum, red[i & 1][0]) / static_cast<float>(C);
+    float sq = 0.0f;
+    if (live) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float d = v[e] - mean;
+        sq = fmaf(d, d, sq);
+      }
+    }
+    const float rstd = rsqrtf(block_total(sq, red[i & 1][1]) / static_cast<float>(C) + a.eps);
+    half8_t yv;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) yv[e] = f2h_apart(fmaf((v[e] - mean) * rstd, h2f(wv[e]), h2f(bv[e])));
+    cur = next;
+    if (i < 0) {
+      prev = yv;
+      continue;
+    }
+    if (live) {
+      const int64_t o = static_cast<int64_t>(first + i) * C + c;
+      half8_t xo;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xo[e] = f2h(v[e]);
+      *reinterpret_cast<half8_t*>(a.x_out + o) = xo;
+      // lerps read the fp16-rounded LN output (rwkv7_v3a_ops.cu:1978-1983)
+#pragma unroll
+      for (int s = 0; s < 6; ++s) {
+        if (s < a.n_mix) {
+          half8_t ov;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float yf = h2f(yv[e]);
+            ov[e] = f2h_apart(fmaf(h2f(prev[e]) - yf, h2f(mv[s][e]), yf));
+          }
+          *reinterpret_cast<half8_t*>(a.out[s] + o) = ov;
+        }
+      }
+      if (t == a.T - 1) *reinterpret_cast<half8_t*>(a.shift_next + static_cast<int64_t>(bi) * C + c) = yv;
+    }
+    prev = yv;
+    if (++t == a.T) {
+      t = 0;
+      ++bi;
+      if (i + 1 < n) prev = *reinterpret_cast<const half8_t*>(a.shift + static_cast<int64_t>(bi) * C + c);
+    }
+  }
+}
+
+template <int NT>
+static void ln_mix_rows_launch(hipStream_t st, int rows, const LnArgs& a) {
+  const int per = std::max(2, std::min(kMixRows, rows / (2 * device_cu_count())));
+  const dim3 grid(ceil_div(rows, per));
+  if (!a.res_partial) hipLaunchKernelGGL((ln_mix_rows_kernel<NT, 0>), grid, dim3(NT), 0, st, a, rows, per);
+  else if (a.res_splits <= 2) hipLaunchKernelGGL((ln_mix_rows_kernel<NT, 2>), grid, dim3(NT), 0, st, a, rows, per);
+  else hipLaunchKernelGGL((ln_mix_rows_kernel<NT, 4>), grid, dim3(NT), 0, st, a, rows, per);
+}
+
 static int check_ln_shape(int rows, int C) {
   RWKV_REQUIRE(rows > 0, "layer norm: rows must be positive");
   RWKV_REQUIRE(C > 0 && C % 8 == 0 && C <= kLnMaxThreads * 8,
@@ -364,7 +513,10 @@ int ln_launch(hipStream_t st, int mode, int rows, const LnArgs& a) {
     // no output may share memory with an input
     RWKV_REQUIRE(a.x_out != a.x && a.y != a.x && (a.res == nullptr || (a.x_out != a.res && a.y != a.res)),
                  "layer norm + token shift over a sequence: outputs must not alias x or the residual");
-    if (a.C <= 256 * 8) hipLaunchKernelGGL(ln_mix_seq_kernel<256>, dim3(rows), dim3(256), 0, st, a);
+    if (rows > kMixSeqRows) {
+      if (a.C <= 256 * 8) ln_mix_rows_launch<256>(st, rows, a);
+      else ln_mix_rows_launch<512>(st, rows, a);
+    } else if (a.C <= 256 * 8) hipLaunchKernelGGL(ln_mix_seq_kernel<256>, dim3(rows), dim3(256), 0, st, a);
     else hipLaunchKernelGGL(ln_mix_seq_kernel<512>, dim3(rows), dim3(512), 0, st, a);
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;

@@ -480,14 +480,13 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
     return s->sparse_ffn_rows >= 0 ? rows <= s->sparse_ffn_rows : rows <= kSparseUnionMaxRows && ffn_sparse_pays(mv.fmt, rows, C, F);
   };
 
-  // Prefill chunks of up to 256 rows: residual add + LayerNorm + token shift as one launch per LayerNorm (the block
-  // of a row also normalises the previous row).  The new shift rows come out in a buffer of their own - the blocks
-  // of the first tokens still read the old ones - and the next packed launch moves them into the state.  The block
-  // reads the residual and the split-K partials of two rows, which from a few hundred rows on costs more than the
-  // launch it saves (prefill of a 4096-token prompt in chunks of 128: 22.6 -> 23.2 k tok/s at batch 1, 54.2 ->
-  // 53.4 k at batch 16).  RWKV_SEQ_LN=0 (tuning hook) switches it off.
+  // Prefill calls: residual add + LayerNorm + token shift as one launch per LayerNorm (a block also normalises the row
+  // before its first; up to 256 rows a block per row, more in blocks of several rows).  The new shift rows come out in a
+  // buffer of their own - the blocks of the first tokens still read the old ones - and the next packed launch moves them into
+  // the state (prefill of a 4096-token prompt in chunks of 128: 22.6 -> 23.2 k tok/s at batch 1; of 16 x 128 tokens 0.6 of 37 ms).
+  // RWKV_SEQ_LN=0 (tuning hook) switches it off.
   static const bool seq_ln_on = !(getenv("RWKV_SEQ_LN") && atoi(getenv("RWKV_SEQ_LN")) == 0);
-  const bool seq_fused = seq_ln_on && !step && !s->trace && C <= 4096 && rows >= packed_min_rows(m) && rows <= 256;
+  const bool seq_fused = seq_ln_on && !step && !s->trace && C <= 4096 && rows >= packed_min_rows(m);
   RowCopy pending;  // shift rows waiting to be moved
   auto flush_pending = [&]() -> int {
     if (pending.n > 0) {

@@ -355,6 +355,13 @@ def test_fused_launches_match_the_standalone_kernels_bitwise(gpu, fmt, B, T):
     sess.close()
 
 
+@pytest.mark.parametrize("B,T", [(1, 300), (600, 2), (40, 31), (5, 411), (16, 130)])
+def test_layer_norm_blocks_of_several_rows_match_the_standalone_kernels_bitwise(gpu, B, T):
+    """More than 256 rows: a LayerNorm block walks 1, 2 or 4 rows, with the first row of a sequence at its start, inside it or
+    nowhere, and a last block that is partial."""
+    test_fused_launches_match_the_standalone_kernels_bitwise(gpu, 1, B, T)
+
+
 def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
     """Without set_sparse_ffn a decode step walks the non-zero rows only where the matrix pays for the second launch: a
     small model gives the bits of the dense product, and those of the walk once it is asked for."""
