@@ -482,8 +482,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
 //                        their maximum and the sum of their exponentials below it;
 //   sample_pick_kernel   one block per row: a value that at least top_k slot maxima reach bounds the top_k-th largest entry from
 //                        below, so only those slots (top_k and a few) are read again, and of them only the entries above it
-//                        compete: softmax, bisection, ties and draw of sample_row over these, in the order sample_row walks the
-//                        row in.  A row with more than kMaxCandidates of them (equal logits) goes through sample_row itself;
+//                        compete: softmax, threshold, ties and draw of sample_row over these, in the order sample_row walks the
+//                        row in (14.8 of the 27 us of 64 rows of 65536, top-k 50, top-p 0.6; 20.8 with sample_row's bisection).  A row with more than kMaxCandidates of them (equal logits) goes through sample_row itself;
 //   sample_decay_kernel  the penalty rows, by the whole chip again.
 // Against the one-block kernel the sum of the exponentials and the masses are added in another order (fp32 both), no more.
 // Rows of 65536, penalties, top-k 50, top-p 0.6, one block per row / this: 1 row 53.4 / 19.8 us, 64 rows 66-70 / 27.7,
@@ -571,11 +571,11 @@ __device__ __forceinline__ float from_order_key(unsigned k) {
 __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs a, int parts) {
   __shared__ BlockRed red;
   __shared__ int s_pick;
-  __shared__ unsigned counts[2][kSampleWaves];
+  __shared__ __align__(16) unsigned counts[2][kSampleWaves];
   __shared__ int slots[kMaxSlots];
   __shared__ int n_cand;
   __shared__ unsigned cand_at[kMaxCandidates], sorted_at[kMaxCandidates];
-  __shared__ float cand[kMaxCandidates], sorted[kMaxCandidates];
+  __shared__ float cand[kMaxCandidates], sorted[kMaxCandidates], by_value[kMaxCandidates];
   const int b = blockIdx.x;
   const int t = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -624,8 +624,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
     if (c >= top_k) lo = zero_key;
   }
   for (int it = 0; reach > enough && hi - lo > 1u; it ^= 1) {
-    const unsigned span = hi - lo;
-    auto threshold = [&](int w) { return lo + max(static_cast<unsigned>(static_cast<uint64_t>(span) * (w + 1) / 17u), 1u); };
+    const unsigned apart = max((hi - lo) / 17u, 1u);
+    auto threshold = [&](int w) { return lo + apart * (w + 1); };
     const unsigned mine = threshold(wave);
     unsigned c = 0;
 #pragma unroll
@@ -655,7 +655,6 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
   if (t == 0) n_cand = 0;
   const bool chosen = t < n_slots && my_slot_max >= floor_u;
   const uint64_t mask = __ballot(chosen);
-  __syncthreads();
   if (lane == 0) red.u[wave] = static_cast<unsigned>(__popcll(mask));
   __syncthreads();
   int first = 0, n_chosen = 0;
@@ -697,10 +696,16 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
   } else {
     if (t < n) {
       const unsigned at = cand_at[t];
-      int rank = 0;
-      for (int i = 0; i < n; ++i) rank += cand_at[i] < at ? 1 : 0;
+      const float u = cand[t];
+      int rank = 0, larger = 0;
+      for (int i = 0; i < n; ++i) {
+        rank += cand_at[i] < at ? 1 : 0;
+        larger += cand[i] > u || (cand[i] == u && i < t) ? 1 : 0;
+      }
+      const float prob = exp2f(u - gmax) / den;
       sorted_at[rank] = at;
-      sorted[rank] = exp2f(cand[t] - gmax) / den;
+      sorted[rank] = prob;
+      by_value[larger] = prob;  // (not increasing: the exponential is monotone)
     }
     __syncthreads();
     if (wave != 0) return;
@@ -708,44 +713,50 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
     constexpr int kRounds = kMaxCandidates / 64;
     const int rounds = (n + 63) / 64;
     float p[kRounds];
-    float pmax = -INFINITY, pmin = INFINITY, mass = 0.0f;
+    float pmin = INFINITY, mass = 0.0f;
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
       p[r] = -1.0f;  // past the end: below every threshold
       if (r < rounds && r * 64 + lane < n) {
         p[r] = sorted[r * 64 + lane];
-        pmax = fmaxf(pmax, p[r]);
         pmin = fminf(pmin, p[r]);
         mass += p[r];
       }
     }
-    pmax = wave_reduce_dpp(pmax, fmax_op);
     pmin = wave_reduce_dpp(pmin, fmin_op);
     mass = wave_reduce_dpp(mass, fadd_op);
     unsigned cnt = zeros_below ? static_cast<unsigned>(V4) * 4u : static_cast<unsigned>(n);
-    unsigned left = zeros_below ? 0u : __float_as_uint(pmin), right = __float_as_uint(pmax) + 1u;
-    while ((cnt > top_k || mass > a.top_p) && left < right - 1u) {
-      const unsigned mid = left + (right - left) / 2u;
-      const float thr = __uint_as_float(mid);
-      unsigned c = 0;
-      float m = 0.0f;
+    // The threshold of sample_row's bisection is the largest value that still leaves top_k entries or top_p mass at or above it,
+    // and that changes only at an entry: instead of some 25 halvings of the bit pattern (0.3 us each; a row that needs them all
+    // held up the launch) the entries in order of value are halved, 6 or 7 times for 50 to 100 of them, with the same sums at each.
+    float thr = zeros_below ? 0.0f : pmin;
+    bool fits = false;  // the kept set has top_k entries or top_p mass as it is
+    if (cnt > top_k || mass > a.top_p) {
+      int low = 0, high = n;  // entries from `high` on leave enough, those before `low` do not
+      while (low < high) {
+        const int mid = (low + high) / 2;
+        const float v = by_value[mid];
+        unsigned c = 0;
+        float m = 0.0f;
 #pragma unroll
-      for (int r = 0; r < kRounds; ++r) {
-        if (r < rounds) {
-          c += static_cast<unsigned>(__popcll(__ballot(p[r] >= thr)));
-          m += p[r] >= thr ? p[r] : 0.0f;
+        for (int r = 0; r < kRounds; ++r) {
+          if (r < rounds) {
+            c += static_cast<unsigned>(__popcll(__ballot(p[r] >= v)));
+            m += p[r] >= v ? p[r] : 0.0f;
+          }
+        }
+        m = wave_reduce_dpp(m, fadd_op);
+        if (c < top_k && m < a.top_p) {
+          low = mid + 1;
+        } else {
+          high = mid;
+          cnt = c;
+          mass = m;
         }
       }
-      m = wave_reduce_dpp(m, fadd_op);
-      if (c < top_k && m < a.top_p) {
-        right = mid;
-      } else {
-        left = mid;
-        cnt = c;
-        mass = m;
-      }
+      if (high < n) thr = by_value[high];
+      fits = cnt <= top_k && mass <= a.top_p;
     }
-    const float thr = __uint_as_float(left);
     unsigned n_eq = 0, n_gt = 0;
     float p_gt = 0.0f;
 #pragma unroll
@@ -758,7 +769,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
     }
     p_gt = wave_reduce_dpp(p_gt, fadd_op);
     float comp = 1.0f;
-    if (n_eq > 0) comp = tie_share(a, thr, n_eq, n_gt, p_gt);
+    if (n_eq > 0 && !fits) comp = tie_share(a, thr, n_eq, n_gt, p_gt);
     // running sums of the kept weights in the draw's order, then the first that reaches the target
     float total = 0.0f;
     float cum[kRounds];
