@@ -16,6 +16,7 @@
 // bisection.  Randomness is counter-based Philox4x32-10 keyed by (seed; row, step) instead of a
 // per-row cuRAND state seeded from the wall clock (src/rwkv_sampler.cpp:14-19), so a run is reproducible.
 #include <cfloat>
+#include <type_traits>
 
 #include "ops.h"
 
@@ -483,7 +484,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
 //   sample_pick_kernel   one block per row: a value that at least top_k slot maxima reach bounds the top_k-th largest entry from
 //                        below, so only those slots (top_k and a few) are read again, and of them only the entries above it
 //                        compete: softmax, threshold, ties and draw of sample_row over these, in the order sample_row walks the
-//                        row in (14.8 of the 27 us of 64 rows of 65536, top-k 50, top-p 0.6; 20.8 with sample_row's bisection).  A row with more than kMaxCandidates of them (equal logits) goes through sample_row itself;
+//                        row in (13.3 of the 26 us of 64 rows of 65536, top-k 50, top-p 0.6; 20.8 with sample_row's bisection).  A row with more than kMaxCandidates of them (equal logits) goes through sample_row itself;
 //   sample_decay_kernel  the penalty rows, by the whole chip again.
 // Against the one-block kernel the sum of the exponentials and the masses are added in another order (fp32 both), no more.
 // Rows of 65536, penalties, top-k 50, top-p 0.6, one block per row / this: 1 row 53.4 / 19.8 us, 64 rows 66-70 / 27.7,
@@ -574,8 +575,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
   __shared__ __align__(16) unsigned counts[2][kSampleWaves];
   __shared__ int slots[kMaxSlots];
   __shared__ int n_cand;
-  __shared__ unsigned cand_at[kMaxCandidates], sorted_at[kMaxCandidates];
-  __shared__ float cand[kMaxCandidates], sorted[kMaxCandidates], by_value[kMaxCandidates];
+  __shared__ __align__(16) unsigned cand_at[kMaxCandidates];
+  __shared__ __align__(16) float cand[kMaxCandidates];
+  __shared__ unsigned sorted_at[kMaxCandidates];
+  __shared__ float sorted[kMaxCandidates], by_value[kMaxCandidates];
   const int b = blockIdx.x;
   const int t = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -632,19 +635,15 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
     for (int i = 0; i < kMaxSlots / 64; ++i) c += static_cast<unsigned>(__popcll(__ballot(key[i] >= mine)));
     if (lane == 0) counts[it][wave] = c;
     __syncthreads();
-    unsigned new_lo = lo, new_hi = hi;
-#pragma unroll
-    for (int w = 0; w < kSampleWaves; ++w) {
-      const unsigned cw = counts[it][w];
-      if (cw >= top_k) {
-        new_lo = threshold(w);
-        reach = cw;
-      } else {
-        new_hi = min(new_hi, threshold(w));
-      }
+    // (counts fall from one threshold to the next: the first `held` of them are held by top_k maxima)
+    const unsigned cw = counts[it][lane & (kSampleWaves - 1)];
+    const int held = __popcll(__ballot(lane < kSampleWaves && cw >= top_k));
+    const unsigned below = lo;
+    if (held > 0) {
+      lo = threshold(held - 1);
+      reach = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(cw), held - 1));
     }
-    lo = new_lo;
-    hi = new_hi;
+    if (held < kSampleWaves) hi = min(hi, below + apart * (held + 1));
   }
   // (two logits this close may round to the same probability, and entries of one probability share its fate)
   const float bound_u = from_order_key(lo) - 4e-6f;
@@ -653,6 +652,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
 
   // the slots that reach it, then their entries that do
   if (t == 0) n_cand = 0;
+  cand_at[t] = 0xffffffffu;  // past the last candidate: behind every position, below every value
+  cand[t] = -INFINITY;
   const bool chosen = t < n_slots && my_slot_max >= floor_u;
   const uint64_t mask = __ballot(chosen);
   if (lane == 0) red.u[wave] = static_cast<unsigned>(__popcll(mask));
@@ -698,9 +699,21 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
       const unsigned at = cand_at[t];
       const float u = cand[t];
       int rank = 0, larger = 0;
-      for (int i = 0; i < n; ++i) {
-        rank += cand_at[i] < at ? 1 : 0;
-        larger += cand[i] > u || (cand[i] == u && i < t) ? 1 : 0;
+      // sixteen at a time: the reads of a trip are in flight together (one by one they took 2.1 us for 55 candidates)
+      for (int i0 = 0; i0 < n; i0 += 16) {
+        uint4_t where[4];
+        float4_t value[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          where[q] = *reinterpret_cast<const uint4_t*>(&cand_at[i0 + 4 * q]);
+          value[q] = *reinterpret_cast<const float4_t*>(&cand[i0 + 4 * q]);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float x = value[i / 4][i % 4];
+          rank += where[i / 4][i % 4] < at ? 1 : 0;
+          larger += x > u || (x == u && i0 + i < t) ? 1 : 0;
+        }
       }
       const float prob = exp2f(u - gmax) / den;
       sorted_at[rank] = at;
@@ -709,102 +722,106 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
     }
     __syncthreads();
     if (wave != 0) return;
-    // one wavefront, up to sixteen entries per lane: steps 4 to 6 of sample_row without a barrier
-    constexpr int kRounds = kMaxCandidates / 64;
-    const int rounds = (n + 63) / 64;
-    float p[kRounds];
-    float pmin = INFINITY, mass = 0.0f;
+    // one wavefront, up to two or up to sixteen entries per lane: steps 4 to 6 of sample_row without a barrier
+    auto draw = [&](auto rounds_c) {
+      constexpr int kRounds = decltype(rounds_c)::value;
+      const int rounds = (n + 63) / 64;
+      float p[kRounds];
+      float pmin = INFINITY, mass = 0.0f;
 #pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      p[r] = -1.0f;  // past the end: below every threshold
-      if (r < rounds && r * 64 + lane < n) {
-        p[r] = sorted[r * 64 + lane];
-        pmin = fminf(pmin, p[r]);
-        mass += p[r];
+      for (int r = 0; r < kRounds; ++r) {
+        p[r] = -1.0f;  // past the end: below every threshold
+        if (r < rounds && r * 64 + lane < n) {
+          p[r] = sorted[r * 64 + lane];
+          pmin = fminf(pmin, p[r]);
+          mass += p[r];
+        }
       }
-    }
-    pmin = wave_reduce_dpp(pmin, fmin_op);
-    mass = wave_reduce_dpp(mass, fadd_op);
-    unsigned cnt = zeros_below ? static_cast<unsigned>(V4) * 4u : static_cast<unsigned>(n);
-    // The threshold of sample_row's bisection is the largest value that still leaves top_k entries or top_p mass at or above it,
-    // and that changes only at an entry: instead of some 25 halvings of the bit pattern (0.3 us each; a row that needs them all
-    // held up the launch) the entries in order of value are halved, 6 or 7 times for 50 to 100 of them, with the same sums at each.
-    float thr = zeros_below ? 0.0f : pmin;
-    bool fits = false;  // the kept set has top_k entries or top_p mass as it is
-    if (cnt > top_k || mass > a.top_p) {
-      int low = 0, high = n;  // entries from `high` on leave enough, those before `low` do not
-      while (low < high) {
-        const int mid = (low + high) / 2;
-        const float v = by_value[mid];
-        unsigned c = 0;
-        float m = 0.0f;
+      pmin = wave_reduce_dpp(pmin, fmin_op);
+      mass = wave_reduce_dpp(mass, fadd_op);
+      unsigned cnt = zeros_below ? static_cast<unsigned>(V4) * 4u : static_cast<unsigned>(n);
+      // The threshold of sample_row's bisection is the largest value that still leaves top_k entries or top_p mass at or above it,
+      // and that changes only at an entry: instead of some 25 halvings of the bit pattern (0.3 us each; a row that needs them all
+      // held up the launch) the entries in order of value are halved, 6 or 7 times for 50 to 100 of them, with the same sums at each.
+      float thr = zeros_below ? 0.0f : pmin;
+      bool fits = false;  // the kept set has top_k entries or top_p mass as it is
+      if (cnt > top_k || mass > a.top_p) {
+        int low = 0, high = n;  // entries from `high` on leave enough, those before `low` do not
+        while (low < high) {
+          const int mid = (low + high) / 2;
+          const float v = by_value[mid];
+          unsigned c = 0;
+          float m = 0.0f;
 #pragma unroll
-        for (int r = 0; r < kRounds; ++r) {
-          if (r < rounds) {
-            c += static_cast<unsigned>(__popcll(__ballot(p[r] >= v)));
-            m += p[r] >= v ? p[r] : 0.0f;
+          for (int r = 0; r < kRounds; ++r) {
+            if (r < rounds) {
+              c += static_cast<unsigned>(__popcll(__ballot(p[r] >= v)));
+              m += p[r] >= v ? p[r] : 0.0f;
+            }
+          }
+          m = wave_reduce_dpp(m, fadd_op);
+          if (c < top_k && m < a.top_p) {
+            low = mid + 1;
+          } else {
+            high = mid;
+            cnt = c;
+            mass = m;
           }
         }
-        m = wave_reduce_dpp(m, fadd_op);
-        if (c < top_k && m < a.top_p) {
-          low = mid + 1;
-        } else {
-          high = mid;
-          cnt = c;
-          mass = m;
+        if (high < n) thr = by_value[high];
+        fits = cnt <= top_k && mass <= a.top_p;
+      }
+      unsigned n_eq = 0, n_gt = 0;
+      float p_gt = 0.0f;
+#pragma unroll
+      for (int r = 0; r < kRounds; ++r) {
+        if (r < rounds) {
+          n_eq += static_cast<unsigned>(__popcll(__ballot(p[r] == thr)));
+          n_gt += static_cast<unsigned>(__popcll(__ballot(p[r] > thr)));
+          p_gt += p[r] > thr ? p[r] : 0.0f;
         }
       }
-      if (high < n) thr = by_value[high];
-      fits = cnt <= top_k && mass <= a.top_p;
-    }
-    unsigned n_eq = 0, n_gt = 0;
-    float p_gt = 0.0f;
+      p_gt = wave_reduce_dpp(p_gt, fadd_op);
+      float comp = 1.0f;
+      if (n_eq > 0 && !fits) comp = tie_share(a, thr, n_eq, n_gt, p_gt);
+      // running sums of the kept weights in the draw's order, then the first that reaches the target
+      float total = 0.0f;
+      float cum[kRounds];
 #pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      if (r < rounds) {
-        n_eq += static_cast<unsigned>(__popcll(__ballot(p[r] == thr)));
-        n_gt += static_cast<unsigned>(__popcll(__ballot(p[r] > thr)));
-        p_gt += p[r] > thr ? p[r] : 0.0f;
-      }
-    }
-    p_gt = wave_reduce_dpp(p_gt, fadd_op);
-    float comp = 1.0f;
-    if (n_eq > 0 && !fits) comp = tie_share(a, thr, n_eq, n_gt, p_gt);
-    // running sums of the kept weights in the draw's order, then the first that reaches the target
-    float total = 0.0f;
-    float cum[kRounds];
+      for (int r = 0; r < kRounds; ++r) {
+        cum[r] = 0.0f;
+        if (r < rounds) {
+          p[r] = p[r] < thr ? 0.0f : (p[r] == thr ? p[r] * comp : p[r]);
+          float inc = p[r];
 #pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      cum[r] = 0.0f;
-      if (r < rounds) {
-        p[r] = p[r] < thr ? 0.0f : (p[r] == thr ? p[r] * comp : p[r]);
-        float inc = p[r];
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const float below = __shfl_up(inc, off, 64);
-          if (lane >= off) inc += below;
+          for (int off = 1; off < 64; off <<= 1) {
+            const float below = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += below;
+          }
+          cum[r] = total + inc;
+          total = __shfl(cum[r], 63, 64);
         }
-        cum[r] = total + inc;
-        total = __shfl(cum[r], 63, 64);
       }
-    }
-    const float target = uniform_of_row(a, b) * total;
-    int found = -1, last = -1;
+      const float target = uniform_of_row(a, b) * total;
+      int found = -1, last = -1;
 #pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      if (r < rounds) {
-        const uint64_t kept = __ballot(p[r] > 0.0f);
-        const uint64_t hit = __ballot(p[r] > 0.0f && cum[r] >= target);
-        if (hit != 0 && found < 0) found = r * 64 + __ffsll(static_cast<unsigned long long>(hit)) - 1;
-        if (kept != 0) last = r * 64 + 63 - __clzll(static_cast<long long>(kept));
+      for (int r = 0; r < kRounds; ++r) {
+        if (r < rounds) {
+          const uint64_t kept = __ballot(p[r] > 0.0f);
+          const uint64_t hit = __ballot(p[r] > 0.0f && cum[r] >= target);
+          if (hit != 0 && found < 0) found = r * 64 + __ffsll(static_cast<unsigned long long>(hit)) - 1;
+          if (kept != 0) last = r * 64 + 63 - __clzll(static_cast<long long>(kept));
+        }
       }
-    }
-    if (found < 0) found = last;  // rounding left the target past the last sum
-    if (found >= 0) {
-      const unsigned at = sorted_at[found];
-      const int i = static_cast<int>((at >> 2) % kSampleRegVecs) * kSampleThreads + static_cast<int>(at >> 2) / kSampleRegVecs;
-      pick = i * 4 + static_cast<int>(at & 3u);
-    }
+      if (found < 0) found = last;  // rounding left the target past the last sum
+      if (found >= 0) {
+        const unsigned at = sorted_at[found];
+        const int i = static_cast<int>((at >> 2) % kSampleRegVecs) * kSampleThreads + static_cast<int>(at >> 2) / kSampleRegVecs;
+        pick = i * 4 + static_cast<int>(at & 3u);
+      }
+    };
+    if (n <= 128) draw(std::integral_constant<int, 2>{});
+    else draw(std::integral_constant<int, kMaxCandidates / 64>{});
   }
   if (t == 0) a.out[b] = pick;
 }
