@@ -7,8 +7,8 @@
 // Lanes keep a few rows x 4 or 8 columns of the 64 x 64 state in registers for the whole call.  The per-column operands of a
 // token are staged in LDS and each lane reads only the columns it owns; the two row sums of a step (sa and y) are reduced over
 // the lanes that share a row with DPP adds.  The staging converts what the caller has (raw decay logits or decays, or the
-// model's own fp16 rows) on the way into LDS.  Calls of several tokens: wkv7_feed_kernel; single tokens and the model's fused
-// pass: wkv7_seq_kernel.  Every variant and every split of T over several calls gives bitwise the same result.
+// model's own fp16 rows) on the way into LDS.  Long calls: wkv7_feed_kernel; single tokens, short calls, very many heads and the
+// model's fused pass: wkv7_seq_kernel.  Every variant and every split of T over several calls gives bitwise the same result.
 #include <type_traits>
 #include "ops.h"
 
@@ -30,7 +30,7 @@ struct SeqOperands {
 };
 
 // ---- sequence kernel -------------------------------------------------------------------------
-// grid = B*H, block = 1024/RPL threads: 16/RPL wavefronts per head, RPL state rows per lane.  Lane (g, c) = (lane / 16,
+// grid = B*H*PARTS, block = 1024/RPL/PARTS threads: 16/RPL wavefronts per head, RPL state rows per lane.  Lane (g, c) = (lane / 16,
 // lane % 16) of wavefront q owns rows 4*RPL*q + RPL*g .. +RPL-1 and columns 4c .. 4c+3, so the 16 lanes of one DPP row hold
 // complete state rows and the wavefronts never exchange data.  v,y have `io_bs` elements between batch rows.  The block stages
 // the operands kSeqChunk tokens at a time, double-buffered; a step costs each lane six LDS reads (its four columns of the five
@@ -43,14 +43,19 @@ constexpr int kSeqChunk = 8;
 // gate - the arithmetic of lnx_rkvres_xg_kernel on the fp16-rounded y - so that three launches and the fp32
 // operand tensors between them become one launch.  Bitwise the same results as the three kernels.
 //
+// PARTS > 1: the rows of a head's state are independent of each other (row i needs only its own sum over the columns, v_i and
+// the per-column operands), so with few heads a head is cut into PARTS row ranges that run on separate CUs.  Not with FUSED: the
+// GroupNorm needs whole heads.
+//
 // STRAIGHT = false leaves out the unrolled eight-step body: single-token calls move a head's state once and are
 // bound by that traffic, so they want the registers for more blocks per CU instead (148 -> under 100 VGPRs).
-template <typename IO, typename WT, int RPL, bool FUSED, bool STRAIGHT = true>
-__global__ __launch_bounds__(1024 / RPL) void wkv7_seq_kernel(int T, int C, int H, float* __restrict__ state,
+template <typename IO, typename WT, int RPL, int PARTS, bool FUSED, bool STRAIGHT = true>
+__global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int C, int H, float* __restrict__ state,
                                                               const IO* __restrict__ v, IO* __restrict__ y,
                                                               int64_t io_bs, TmixSeqArgs fa, SeqOperands<IO, WT> ro) {
   constexpr bool RAW = !FUSED;
-  constexpr int NT = 1024 / RPL;
+  static_assert(PARTS == 1 || !FUSED, "the fused pass needs whole heads");
+  constexpr int NT = 1024 / RPL / PARTS;
   constexpr int kVSlots = (kSeqChunk * kHead + NT - 1) / NT;
   typedef float rows_t __attribute__((ext_vector_type(RPL)));
   __shared__ __align__(16) float ops[2][kSeqChunk][5][kHead];  // [buffer][token][a,b,d,k,r][column]
@@ -62,13 +67,14 @@ __global__ __launch_bounds__(1024 / RPL) void wkv7_seq_kernel(int T, int C, int 
   __shared__ __align__(16) float spare[kSpare ? NT * RPL : 4];
   __shared__ __align__(16) float gs[FUSED ? 2 : 1][FUSED ? kSeqChunk : 1][kHead];  // FUSED: the gate rows
 
-  const int bh = blockIdx.x;
+  const int bh = blockIdx.x / PARTS;
   const int bi = bh / H;
   const int h = bh - bi * H;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int i0 = 4 * RPL * (tid >> 6) + RPL * (lane >> 4);  // first of this lane's rows
-  const int j0 = 4 * (lane & 15);                           // first of its 4 columns
+  const int row_lo = (blockIdx.x % PARTS) * (kHead / PARTS);         // this block's rows
+  const int i0 = row_lo + 4 * RPL * (tid >> 6) + RPL * (lane >> 4);  // first of this lane's rows
+  const int j0 = 4 * (lane & 15);                                    // first of its 4 columns
   float* sblk = state + (static_cast<int64_t>(bh) * kHead + i0) * kHead + j0;
 
   float4_t S[RPL];
@@ -174,7 +180,7 @@ __global__ __launch_bounds__(1024 / RPL) void wkv7_seq_kernel(int T, int C, int 
           const float rkv = wave_sum(ops[buf][tt][4][lane] * ops[buf][tt][3][lane] * c_rk);
           const float o = (dd * rstd * c_lnw + c_lnb + rkv * vs[buf][tt][lane]) * gs[buf][tt][lane];
           y[iob + static_cast<int64_t>(t0 + tt) * C + lane] = static_cast<IO>(o);
-        } else {
+        } else if (PARTS == 1 || (lane >= row_lo && lane < row_lo + kHead / PARTS)) {
           y[iob + static_cast<int64_t>(t0 + tt) * C + lane] = static_cast<IO>(ys[buf][tt][lane]);
         }
       }
@@ -289,7 +295,7 @@ __global__ __launch_bounds__(1024 / RPL) void wkv7_seq_kernel(int T, int C, int 
 }
 
 
-// ---- sequence kernel with feeders (T > 1) ---------------------------------------------------------------------------
+// ---- sequence kernel with feeders ---------------------------------------------------------------------------
 // NC wavefronts own the state and do nothing but steps; NF feeders bring the operands of the next chunk of kSeqChunk tokens
 // into LDS (requested SETS chunks ahead, the decay derived where the caller has logits) and take the finished y rows out.  All
 // meet once per chunk, ahead of the chunk's last step, whose operands are in registers by then.  A block owns 1 / PARTS of a
@@ -303,7 +309,9 @@ __global__ __launch_bounds__(1024 / RPL) void wkv7_seq_kernel(int T, int C, int 
 // heads: VALU issue, four clocks per instruction and SIMD; eight columns per lane put one of a row's four adds over lanes into the
 // lane (24 instead of 28 operations per four elements).  us per call, before / now:
 //   1 x 64 tokens x 12 heads, fp32 tensors 13.4 / 10.6   1 x 512 x 64, fp16 84.8 / 57   3 x 333 x 32 72 / 56
-//   4 x 256 x 64 83.7 / 70   8 x 256 x 64 125 / 113   16 x 256 x 64 223 / 213
+//   4 x 256 x 64 83.7 / 70   8 x 256 x 64 125 / 113   16 x 256 x 64 223 / 213; fp32 tensors 82 / 71, 124 / 108, 238 / 219
+// The fp32 tile for more than 128 heads keeps six wavefronts per SIMD at the price of ten spilled registers: 128 tokens of 1024
+// heads 108 us; five 121, four 135 (512 heads 58.3, 56.9 and 57.2).
 template <typename E, int N>
 struct Loose {  // N elements that are aligned like one
   typedef E type __attribute__((ext_vector_type(N), aligned(sizeof(E))));
@@ -714,15 +722,11 @@ __global__ __launch_bounds__(64 * (NC + NF), WAVES) void wkv7_feed_kernel(int T,
     for (int m = 0; m < G; ++m) __builtin_nontemporal_store(S[i][m], reinterpret_cast<float4_t*>(sblk + i * kHead + 4 * m));
 }
 
-template <typename IO, typename WT, bool FUSED>
+template <typename IO, typename WT, int RPL, int PARTS, bool FUSED, bool STRAIGHT>
 static void launch_seq(hipStream_t st, int B, int T, int C, int H, float* state, const IO* v, IO* y, const TmixSeqArgs& fa,
                        const SeqOperands<IO, WT>& ro) {
-  const int64_t io_bs = static_cast<int64_t>(T) * C;
-  if (T == 1) {
-    hipLaunchKernelGGL((wkv7_seq_kernel<IO, WT, 4, FUSED, false>), dim3(B * H), dim3(256), 0, st, T, C, H, state, v, y, io_bs, fa, ro);
-  } else if constexpr (FUSED) {
-    hipLaunchKernelGGL((wkv7_seq_kernel<IO, WT, 4, FUSED>), dim3(B * H), dim3(256), 0, st, T, C, H, state, v, y, io_bs, fa, ro);
-  }
+  hipLaunchKernelGGL((wkv7_seq_kernel<IO, WT, RPL, PARTS, FUSED, STRAIGHT>), dim3(B * H * PARTS), dim3(1024 / RPL / PARTS), 0, st, T, C, H,
+                     state, v, y, static_cast<int64_t>(T) * C, fa, ro);
 }
 
 template <typename IO, typename WT, int G, int RPL, int NC, int PARTS, int NF, int SETS, int WAVES, bool AHEAD>
@@ -731,7 +735,7 @@ static void launch_feed(hipStream_t st, int B, int T, int C, int H, float* state
                      state, op, y);
 }
 
-// Which tile a call of more than one token takes.  Up to 128 heads the chip has CUs to spare: a head is cut into row ranges of
+// Which tile a call with feeders takes.  Up to 128 heads the chip has CUs to spare: a head is cut into row ranges of
 // four wavefronts each, one state row per lane, and every wavefront is alone on its SIMD.  Up to 512 heads (two per CU) whole
 // heads, 2 x 8 elements per lane, the next step's operands read ahead; with more heads, or fp32 operands (twice the
 // registers), wavefronts are worth more than reading ahead (us per token of 16 x 64 heads, 6 per SIMD / 3 reading ahead: 0.83 /
@@ -744,17 +748,39 @@ constexpr int kSeqAheadHeads = 512;
 // the fused pass cannot: its GroupNorm needs whole heads
 bool tmix_seq_whole_heads(int B, int T, int H) { return !(B * H <= kSeqHalfHeads && T > 1); }
 
+// Whether a call of T tokens on `heads` = B*H heads takes the feeders.  They stage two chunks before the first step where the other
+// kernel stages one, so short calls lose.  us per call, feeders / without: fp16 tensors, 12 heads 2 tokens 3.3 / 2.8, 8 tokens 3.6 /
+// 3.35, 12 4.45 / 4.50; 128 heads 8 tokens 1.11 times, 16 0.99; 256 heads 8 1.12, 17 0.99; 1024 heads 3 tokens 9.9 / 7.5, 17 20.9 / 20.0,
+// 32 32.4 / 32.7; fp32 tensors 256 heads 16 tokens 1.15 times, 40 1.00; 1024 heads 3 tokens 12.6 / 8.2, 32 34.6 / 34.6.  Many more than
+// 1024 heads are more than one round of feeder blocks (four per CU), and the other kernel's rounds, three per CU with longer
+// straight code, are the shorter ones: fp16 tensors, 256 tokens, 1088 heads 262 / 268, 1280 306 / 270, 2048 448 / 418, 4096 833 / 797; fp32
+// tensors, whose staging weighs more, only for shorter calls: 1536 heads 64 tokens 91 / 86, 256 tokens 336 / 333, 2048 heads 424 / 446.
+template <typename IO>
+static bool feeders_pay(int heads, int T) {
+  constexpr bool half = sizeof(IO) == 2;
+  if (heads <= kSeqQuarterHeads) return T >= 12;
+  if (heads <= kSeqHalfHeads) return T >= (half ? 16 : 20);
+  if (heads <= 256) return T >= (half ? 17 : 40);
+  if (heads <= 1152) return T >= (half ? 32 : 40);
+  return !half && T >= 128;
+}
+
 template <typename IO, typename WT>
 static int launch_recurrence(hipStream_t st, int B, int T, int C, int H, float* state, const SeqOperands<IO, WT>& op, IO* y) {
+  const int heads = B * H;
   if (T == 1) {
-    launch_seq<IO, WT, false>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
-  } else if (B * H <= kSeqQuarterHeads) {
+    launch_seq<IO, WT, 4, 1, false, false>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
+  } else if (!feeders_pay<IO>(heads, T)) {
+    if (heads <= kSeqQuarterHeads) launch_seq<IO, WT, 1, 4, false, true>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
+    else if (heads <= kSeqHalfHeads) launch_seq<IO, WT, 2, 2, false, true>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
+    else launch_seq<IO, WT, 4, 1, false, true>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
+  } else if (heads <= kSeqQuarterHeads) {
     launch_feed<IO, WT, 1, 1, 4, 4, 2, 2, 1, true>(st, B, T, C, H, state, op, y);
-  } else if (B * H <= kSeqHalfHeads) {
+  } else if (heads <= kSeqHalfHeads) {
     launch_feed<IO, WT, 2, 1, 4, 2, 2, 4, 1, true>(st, B, T, C, H, state, op, y);
   } else {
     constexpr bool kHalf = sizeof(IO) == 2;
-    if (kHalf && B * H <= kSeqAheadHeads) launch_feed<IO, WT, 2, 2, 4, 1, 2, 2, kHalf ? 4 : 6, kHalf>(st, B, T, C, H, state, op, y);
+    if (kHalf && heads <= kSeqAheadHeads) launch_feed<IO, WT, 2, 2, 4, 1, 2, 2, kHalf ? 4 : 6, kHalf>(st, B, T, C, H, state, op, y);
     else launch_feed<IO, WT, 2, 2, 4, 1, 2, 2, 6, false>(st, B, T, C, H, state, op, y);
   }
   RWKV_LAUNCH_CHECK();
@@ -770,7 +796,9 @@ int tmix_seq_launch(hipStream_t st, int B, int T, int C, int H, float* state, co
                     half_t* y2) {
   RWKV_REQUIRE(fa.r && fa.k && fa.a12 && fa.w12 && fa.g && fa.k_k && fa.a0 && fa.k_a && fa.w0 && fa.r_k && fa.lnx_w && fa.lnx_b,
                "tmix_seq: NULL tensor");
-  launch_seq<half_t, half_t, true>(st, B, T, C, H, state, v, y2, fa, SeqOperands<half_t, half_t>{});
+  const SeqOperands<half_t, half_t> none = {};
+  if (T == 1) launch_seq<half_t, half_t, 4, 1, true, false>(st, B, T, C, H, state, v, y2, fa, none);
+  else launch_seq<half_t, half_t, 4, 1, true, true>(st, B, T, C, H, state, v, y2, fa, none);
   RWKV_LAUNCH_CHECK();
   return RWKV_OK;
 }

@@ -268,6 +268,39 @@ def test_wkv7_call_of_several_tokens_is_bitwise_its_single_tokens(gpu, B, H, io)
     assert t0 == T and same
 
 
+@pytest.mark.parametrize("B,H", [(1, 3), (1, 64), (5, 13), (2, 64), (3, 43), (4, 64), (9, 57), (18, 64), (5, 231)])
+@pytest.mark.parametrize("io", ["f16", "f32"])
+def test_wkv7_call_of_many_chunks_is_bitwise_its_single_tokens(gpu, B, H, io):
+    """75 tokens - ten chunks of eight, the last one of three - in one call and in calls of lengths on either side of where the
+    feeders take over (12, 16, 17, 20, 32, 40 tokens), at heads on either side of every change of tile (64, 128, 256, 512, 1152):
+    the stages and output buffers of the feeders go round several times."""
+    hip = gpu
+    T, C = 75, H * 64
+    dt = np.float16 if io == "f16" else np.float32
+    inp = wkv_inputs(B, T, H, seed=B * H, dtype=dt)
+    names = ["r", "w_raw", "k", "v", "a", "b"]
+    mode = hip.IO_F16 if io == "f16" else hip.IO_F32
+
+    def run(lengths):
+        state = hip.DeviceArray.zeros((B, H, 64, 64), np.float32)
+        rows, t0 = [], 0
+        for n in lengths:
+            d = [dev(hip, np.ascontiguousarray(inp[name][:, t0:t0 + n])) for name in names]
+            y = hip.DeviceArray((B, n, C), dt)
+            hip.wkv7(B, n, C, H, hip.W_RAW_LOGIT, mode, state, *d, y)
+            rows.append(y.numpy())
+            t0 += n
+        assert t0 == T
+        return np.concatenate(rows, axis=1), state.numpy()
+
+    want, want_state = run([1] * T)
+    assert np.isfinite(want_state).all()
+    for lengths in ([75], [11, 12, 15, 16, 21], [19, 20, 17, 19], [31, 32, 12], [39, 36], [35, 40]):
+        got, state = run(lengths)
+        same = np.array_equal(got, want), np.array_equal(state, want_state)
+        assert same == (True, True), lengths
+
+
 # ------------------------------------------------------------------------------- checkpoint tensors
 def test_bf16_to_f16_every_pattern_and_transposes_bit_exact(gpu, orc):
     hip = gpu
