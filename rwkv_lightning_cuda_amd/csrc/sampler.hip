@@ -496,6 +496,7 @@ constexpr int kPartEntries = 4096;
 constexpr int kPartThreads = 256;
 constexpr int kSplitMaxTopK = 256;
 constexpr int kMaxCandidates = 1024;  // one per thread
+constexpr int kFewCandidates = 128;   // up to here the threshold is searched among the candidates in order of value
 constexpr int kMaxSlots = kSampleRegVecs * kSampleThreads * 4 / kSlot;
 static_assert(kMaxSlots == kSampleThreads, "one slot per thread, sixteen per lane of a wavefront");
 
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
   __shared__ __align__(16) unsigned cand_at[kMaxCandidates];
   __shared__ __align__(16) float cand[kMaxCandidates];
   __shared__ unsigned sorted_at[kMaxCandidates];
-  __shared__ float sorted[kMaxCandidates], by_value[kMaxCandidates];
+  __shared__ float sorted[kMaxCandidates], by_value[kFewCandidates];
   const int b = blockIdx.x;
   const int t = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -695,7 +696,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
   if (n > kMaxCandidates) {
     pick = sample_row<true>(a, b, red, s_pick);
   } else {
-    if (t < n) {
+    auto rank_candidates = [&](auto few_c) {
+      constexpr bool kFew = decltype(few_c)::value;
       const unsigned at = cand_at[t];
       const float u = cand[t];
       int rank = 0, larger = 0;
@@ -706,19 +708,25 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           where[q] = *reinterpret_cast<const uint4_t*>(&cand_at[i0 + 4 * q]);
-          value[q] = *reinterpret_cast<const float4_t*>(&cand[i0 + 4 * q]);
+          if constexpr (kFew) value[q] = *reinterpret_cast<const float4_t*>(&cand[i0 + 4 * q]);
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const float x = value[i / 4][i % 4];
           rank += where[i / 4][i % 4] < at ? 1 : 0;
-          larger += x > u || (x == u && i0 + i < t) ? 1 : 0;
+          if constexpr (kFew) {
+            const float x = value[i / 4][i % 4];
+            larger += x > u || (x == u && i0 + i < t) ? 1 : 0;
+          }
         }
       }
       const float prob = exp2f(u - gmax) / den;
       sorted_at[rank] = at;
       sorted[rank] = prob;
-      by_value[larger] = prob;  // (not increasing: the exponential is monotone)
+      if constexpr (kFew) by_value[larger] = prob;  // (not increasing: the exponential is monotone)
+    };
+    if (t < n) {
+      if (n <= kFewCandidates) rank_candidates(std::true_type{});
+      else rank_candidates(std::false_type{});
     }
     __syncthreads();
     if (wave != 0) return;
@@ -726,50 +734,79 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
     auto draw = [&](auto rounds_c) {
       constexpr int kRounds = decltype(rounds_c)::value;
       const int rounds = (n + 63) / 64;
+      constexpr bool kFew = kRounds * 64 <= kFewCandidates;
       float p[kRounds];
-      float pmin = INFINITY, mass = 0.0f;
+      float pmin = INFINITY, pmax = -INFINITY, mass = 0.0f;
 #pragma unroll
       for (int r = 0; r < kRounds; ++r) {
         p[r] = -1.0f;  // past the end: below every threshold
         if (r < rounds && r * 64 + lane < n) {
           p[r] = sorted[r * 64 + lane];
           pmin = fminf(pmin, p[r]);
+          if constexpr (!kFew) pmax = fmaxf(pmax, p[r]);
           mass += p[r];
         }
       }
       pmin = wave_reduce_dpp(pmin, fmin_op);
+      if constexpr (!kFew) pmax = wave_reduce_dpp(pmax, fmax_op);
       mass = wave_reduce_dpp(mass, fadd_op);
       unsigned cnt = zeros_below ? static_cast<unsigned>(V4) * 4u : static_cast<unsigned>(n);
+      // entries at or above v, and their mass
+      auto reach_of = [&](float v, unsigned& c, float& m) {
+        c = 0;
+        m = 0.0f;
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+          if (r < rounds) {
+            c += static_cast<unsigned>(__popcll(__ballot(p[r] >= v)));
+            m += p[r] >= v ? p[r] : 0.0f;
+          }
+        }
+        m = wave_reduce_dpp(m, fadd_op);
+      };
       // The threshold of sample_row's bisection is the largest value that still leaves top_k entries or top_p mass at or above it,
       // and that changes only at an entry: instead of some 25 halvings of the bit pattern (0.3 us each; a row that needs them all
       // held up the launch) the entries in order of value are halved, 6 or 7 times for 50 to 100 of them, with the same sums at each.
+      // More candidates keep sample_row's bisection: ranking them by value, whose pairs grow with their square, costs more than it
+      // saves (us, 64 rows of 65536, ranked / bisected: 125 to 160 candidates of rows as flat as N(0, 9) 30.2 / 27.5, of N(0, 100) 30.0 /
+      // 31.7; top_k 200, top_p 0.8 41.4 / 31.9; top_k 256 48.4 / 32.3).
       float thr = zeros_below ? 0.0f : pmin;
       bool fits = false;  // the kept set has top_k entries or top_p mass as it is
-      if (cnt > top_k || mass > a.top_p) {
-        int low = 0, high = n;  // entries from `high` on leave enough, those before `low` do not
-        while (low < high) {
-          const int mid = (low + high) / 2;
-          const float v = by_value[mid];
-          unsigned c = 0;
-          float m = 0.0f;
-#pragma unroll
-          for (int r = 0; r < kRounds; ++r) {
-            if (r < rounds) {
-              c += static_cast<unsigned>(__popcll(__ballot(p[r] >= v)));
-              m += p[r] >= v ? p[r] : 0.0f;
+      if constexpr (kFew) {
+        if (cnt > top_k || mass > a.top_p) {
+          int low = 0, high = n;  // entries from `high` on leave enough, those before `low` do not
+          while (low < high) {
+            const int mid = (low + high) / 2;
+            unsigned c;
+            float m;
+            reach_of(by_value[mid], c, m);
+            if (c < top_k && m < a.top_p) {
+              low = mid + 1;
+            } else {
+              high = mid;
+              cnt = c;
+              mass = m;
             }
           }
-          m = wave_reduce_dpp(m, fadd_op);
+          if (high < n) thr = by_value[high];
+          fits = cnt <= top_k && mass <= a.top_p;
+        }
+      } else {
+        unsigned left = __float_as_uint(thr), right = __float_as_uint(pmax) + 1u;
+        while ((cnt > top_k || mass > a.top_p) && left < right - 1u) {
+          const unsigned mid = left + (right - left) / 2u;
+          unsigned c;
+          float m;
+          reach_of(__uint_as_float(mid), c, m);
           if (c < top_k && m < a.top_p) {
-            low = mid + 1;
+            right = mid;
           } else {
-            high = mid;
+            left = mid;
             cnt = c;
             mass = m;
           }
         }
-        if (high < n) thr = by_value[high];
-        fits = cnt <= top_k && mass <= a.top_p;
+        thr = __uint_as_float(left);
       }
       unsigned n_eq = 0, n_gt = 0;
       float p_gt = 0.0f;
@@ -820,7 +857,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SampleArgs 
         pick = i * 4 + static_cast<int>(at & 3u);
       }
     };
-    if (n <= 128) draw(std::integral_constant<int, 2>{});
+    if (n <= kFewCandidates) draw(std::integral_constant<int, kFewCandidates / 64>{});
     else draw(std::integral_constant<int, kMaxCandidates / 64>{});
   }
   if (t == 0) a.out[b] = pick;
