@@ -573,6 +573,9 @@ int token_shift_mix_launch(hipStream_t st, const MixArgs& a) {
 // sums six trips through LDS each.  Four channels per lane make requests of 512 bytes and keep the sums in the registers of a DPP row;
 // eight would halve the blocks of a 128-row chunk, which are two per CU.  us, before -> now: 999 rows x 32 heads 12.5 and 9.7
 // -> 9.4 and 5.8; 128 rows x 64 heads 5.2 and 4.6 -> 5.3 and 4.7 (launch and latency).
+// kk / a-gate of fewer than 12 heads per CU keeps one channel per lane: its chain of divisions and exponentials, four times as
+// long with four of them, is then all there is (kk_a_gate_few_kernel; us, back to back, four channels / one: 17 rows x 64 heads 2.24 / 2.05,
+// 64 x 32 2.30 / 2.14, 96 x 32 2.29 / 2.35, 128 x 64 2.84 / 3.26).
 //
 // The sums are those of a wavefront with one channel per lane (wave_sum: channel i adds what i ^ 32, 16, 8, 4, 2, 1 holds), so
 // that the kernels that do this inside a larger one agree bitwise: the first four levels are lane exchanges, the last two lie
@@ -681,10 +684,44 @@ __global__ __launch_bounds__(256) void kk_a_gate_kernel(KkArgs p) {
   if (p.w_sum16) store4<VEC>(p.w_sum16 + idx, ws);
 }
 
+constexpr int kKkFewHeads = 12;  // per CU
+
+// one wavefront per (row, head), lane = channel; few enough heads for 32-bit indices
+__global__ __launch_bounds__(256) void kk_a_gate_few_kernel(KkArgs p) {
+  const int rh = static_cast<int>(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (rh >= static_cast<int>(p.rows_heads)) return;
+  const int lane = threadIdx.x & 63;
+  const int idx = rh * kHead + lane;
+  const int c = rh % p.H * kHead + lane;
+  const float kv = h2f(p.k[idx]);
+  const float u = kv * h2f(p.k_k[c]);
+  const float total = wave_sum(u * u);
+  const float inv = 1.0f / fmaxf(sqrtf(total), kKkEps);
+  const float kk = u * inv;
+  const float av = sigmoid_f(h2f(p.a0[c]) + h2f(p.a12[idx]));
+  const float ka = h2f(p.k_a[c]);
+  const half_t nk = f2h(kv * fmaf(av, ka, 1.0f - ka));
+  const half_t nkk = f2h(-kk);
+  const half_t kka = f2h(kk * av);
+  if (p.new_k) p.new_k[idx] = nk;
+  if (p.neg_kk) p.neg_kk[idx] = nkk;
+  if (p.kka) p.kka[idx] = kka;
+  if (p.d32 || p.w_sum16) {
+    const half_t ws = f2h(h2f(p.w12[idx]) + h2f(p.w0[c]));  // rwkv7_add_vec_launch rounding point
+    if (p.d32) p.d32[idx] = exp2f(-0.8750387749145276f / (1.0f + exp2f(-1.4426950408889634f * h2f(ws))));
+    if (p.w_sum16) p.w_sum16[idx] = ws;
+  }
+}
+
 int kk_a_gate_launch(hipStream_t st, const KkArgs& p) {
   RWKV_REQUIRE(p.rows_heads > 0 && p.H > 0, "kk_a_gate: bad shape");
   RWKV_REQUIRE(p.w_sum16 == nullptr || (p.w12 && p.w0), "kk_a_gate: the rounded decay logit needs w12 and w0");
   RWKV_REQUIRE(reinterpret_cast<uintptr_t>(p.d32) % 16 == 0, "kk_a_gate: the decay must be 16-byte aligned");
+  if (p.rows_heads < kKkFewHeads * device_cu_count()) {
+    hipLaunchKernelGGL(kk_a_gate_few_kernel, dim3(ceil_div(p.rows_heads, 4)), dim3(256), 0, st, p);
+    RWKV_LAUNCH_CHECK();
+    return RWKV_OK;
+  }
   const uintptr_t bits = reinterpret_cast<uintptr_t>(p.k) | reinterpret_cast<uintptr_t>(p.a12) | reinterpret_cast<uintptr_t>(p.k_k) |
                          reinterpret_cast<uintptr_t>(p.a0) | reinterpret_cast<uintptr_t>(p.k_a) | reinterpret_cast<uintptr_t>(p.w12) |
                          reinterpret_cast<uintptr_t>(p.w0) | reinterpret_cast<uintptr_t>(p.new_k) |

@@ -676,6 +676,30 @@ def test_kk_gate_groupnorm_of_tensors_that_are_not_aligned(gpu, rows, H):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("rows,H", [(47, 65), (48, 64), (49, 64), (257, 12)])
+def test_kk_gate_of_few_and_of_many_heads_give_the_same_bits(gpu, rows, H):
+    """One channel per lane below 12 heads per compute unit, four from there on: a call on either side of the line against calls of one
+    and of a few rows, with values as large and as small as fp16 has them and a head of zeros."""
+    hip = gpu
+    rng = np.random.default_rng(rows * H)
+    C = H * 64
+    k, a12 = (rng.standard_normal((rows, C)) * np.exp2(rng.integers(-12, 9, (rows, C)))).astype(np.float16), rng.standard_normal((rows, C)).astype(np.float16)
+    k[0, :64] = 0
+    k_k, a0, k_a = (dev(hip, rng.standard_normal(C).astype(np.float16)) for _ in range(3))
+
+    def run(first, n):
+        assert first + n <= rows
+        outs = [hip.DeviceArray((n, C), np.float16) for _ in range(3)]
+        hip.kk_a_gate(n, C, H, dev(hip, k[first:first + n]), k_k, a0, dev(hip, a12[first:first + n]), k_a, *outs)
+        hip.device_sync()
+        return [o.numpy().view(np.uint16) for o in outs]
+
+    whole = run(0, rows)
+    for first, n in ((0, 1), (rows // 2, 7), (rows - 1, 1)):
+        for got, want in zip(run(first, n), whole):
+            assert np.array_equal(got, want[first:first + n])
+
+
 def test_lora_out_blocks_walk_several_row_tiles(gpu, orc):
     """Ten row tiles, the last one partial; the v-residual epilogue is checked on the same rows."""
     hip = gpu
