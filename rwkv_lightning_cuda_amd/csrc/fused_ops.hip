@@ -448,6 +448,7 @@ __global__ __launch_bounds__(NT) void ln_mix_rows_kernel(LnArgs a, int rows, int
 #pragma unroll
       for (int e = 0; e < 8; ++e) xo[e] = f2h(v[e]);
       *reinterpret_cast<half8_t*>(a.x_out + o) = xo;
+      if (a.y) *reinterpret_cast<half8_t*>(a.y + o) = yv;
       // lerps read the fp16-rounded LN output (rwkv7_v3a_ops.cu:1978-1983)
 #pragma unroll
       for (int s = 0; s < 6; ++s) {

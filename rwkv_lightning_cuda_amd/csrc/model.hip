@@ -737,7 +737,8 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
       TRY_AUX(ln_launch(st, kAddLnMix, rows, a));
     } else if (seq_fused) {
       LnArgs a = {};
-      a.x = b.x; a.res = b.att; a.w = w.t[RWKV_T_LN2_W]; a.b = w.t[RWKV_T_LN2_B]; a.x_out = b.x1; a.y = b.ln2;
+      a.x = b.x; a.res = b.att; a.w = w.t[RWKV_T_LN2_W]; a.b = w.t[RWKV_T_LN2_B]; a.x_out = b.x1;
+      a.y = l + 1 == L ? b.ln2 : nullptr;  // (read by rwkv_hip_session_debug_buffer alone: the last layer's)
       a.shift = shift1; a.shift_next = b.shift_next;
       a.mu[0] = w.t[RWKV_T_FFN_X_K]; a.out[0] = b.mixed; a.n_mix = 1; a.C = C; a.T = T; a.eps = kLnEps;
       take_deferred(a, att_partial);
@@ -807,7 +808,7 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
       } else if (seq_fused) {
         a.shift = shift + static_cast<int64_t>(l + 1) * 2 * B * C;
         a.shift_next = b.shift_next;
-        a.y = b.xx;
+        a.y = l + 2 == L ? b.xx : nullptr;
         a.T = T;
         mix6_args(nx, a);
         TRY_AUX(ln_launch(st, kAddLnMixSeq, rows, a));

@@ -362,6 +362,31 @@ def test_layer_norm_blocks_of_several_rows_match_the_standalone_kernels_bitwise(
     test_fused_launches_match_the_standalone_kernels_bitwise(gpu, 1, B, T)
 
 
+@pytest.mark.parametrize("L", [1, 2, 3])
+@pytest.mark.parametrize("B,T", [(1, 250), (1, 300), (5, 131)])
+def test_debug_buffers_hold_the_last_layers_normalised_rows(gpu, L, B, T):
+    """xx and ln2 of the last layer after a prefill call, up to 256 rows and more: what the stand-alone LayerNorm kernels leave."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=L, C=512, H=8, F=2048, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
+    gmodel = HipModel.from_host_weights(dims, synth_weights(dims, 4), hip.FMT_W8)
+    sess = Session(gmodel)
+    seen = []
+    for tapped in (False, True):
+        rng = np.random.default_rng(9)
+        trace = hip.DeviceArray((L, B * T, dims.C), np.float16)
+        sess.set_trace(trace if tapped else None)
+        lg = hip.DeviceArray((B, dims.V), np.float32)
+        sess.forward(rng.integers(0, dims.V, (B, T)), State(dims, B), lg)   # (other rows in the buffers before the call that counts)
+        sess.forward(rng.integers(0, dims.V, (B, T)), State(dims, B), lg)
+        sess.set_trace(None)
+        seen.append([sess.debug_buffer(name, (B * T, dims.C)).view(np.uint16) for name in ("xx", "ln2")])
+    for name, fused, alone in zip(("xx", "ln2"), *seen):
+        same = np.array_equal(fused, alone)
+        assert same, name
+    sess.close()
+
+
 def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
     """Without set_sparse_ffn a decode step walks the non-zero rows only where the matrix pays for the second launch: a
     small model gives the bits of the dense product, and those of the walk once it is asked for."""
