@@ -125,7 +125,8 @@ struct Arena {
 struct Buffers {
   half_t *x, *xx, *xr, *xw, *xk, *xv, *xa, *xg, *r, *k, *v, *v_first, *w12, *a12, *g, *hw, *ha, *hg, *hv, *k2, *nkk,
       *kka, *y, *y2, *att, *x1, *ln2, *mixed, *act, *cm, *xf, *scratch, *shift_next;
-  float *r32, *d32, *k32, *a32, *b32;
+  float* r32;  // one row: the output projection's input ahead of the gate
+  float* d32;
 };
 
 }  // namespace
@@ -154,6 +155,8 @@ struct rwkv_hip_session {
   size_t gemm_ws_bytes = 0;
   void* sparse_ws = nullptr;  // partial rows of the row-skipping ffn.value product
   size_t sparse_ws_bytes = 0;
+  float* widened[4] = {};     // rwkv_hip_session_debug_buffer: fp32 copies of r, k2, nkk, kka, made when they are asked for
+  size_t widened_cap[4] = {};
   int sparse_ffn_rows = -1;   // decode steps of up to this many rows read only the ffn.value rows with a non-zero activation; -1: where it pays
                               // (2..4 rows share one walk over the rows that are non-zero for any of them)
   bool wkv_fp16 = false;      // the WKV state tensor is fp16 [L,B,H,64,64] (the reference's use_wkv32 == false)
@@ -275,7 +278,8 @@ int ensure_arena(rwkv_hip_session* s, int B, int T) {
   add(static_cast<size_t>(B) * m->C, 2);              // xf
   add(static_cast<size_t>(B) * m->C, 2);              // shift_next
   add(RC, 2);                                         // scratch
-  for (int i = 0; i < 5; ++i) add(RC, 4);             // fp32 WKV operands
+  add(m->C, 4);                                       // r32
+  add(RC, 4);                                         // d32
   if (need > s->arena.cap) {
     // a larger shape invalidates captured graphs (they hold arena addresses)
     for (auto& g : s->graphs) {
@@ -310,11 +314,8 @@ int ensure_arena(rwkv_hip_session* s, int B, int T) {
     b.act = a.take<half_t>(rows * m->F);
     b.xf = a.take<half_t>(static_cast<size_t>(B) * m->C);
     b.shift_next = a.take<half_t>(static_cast<size_t>(B) * m->C);
-    b.r32 = a.take<float>(RC);
+    b.r32 = a.take<float>(m->C);
     b.d32 = a.take<float>(RC);
-    b.k32 = a.take<float>(RC);
-    b.a32 = a.take<float>(RC);
-    b.b32 = a.take<float>(RC);
     s->arena_B = B;
     s->arena_T = T;
   }
@@ -1095,6 +1096,8 @@ int rwkv_hip_session_destroy(rwkv_hip_session* s) {
   if (s->arena.base) (void)hipFree(s->arena.base);
   if (s->gemm_ws) (void)hipFree(s->gemm_ws);
   if (s->sparse_ws) (void)hipFree(s->sparse_ws);
+  for (float* p : s->widened)
+    if (p) (void)hipFree(p);
   if (s->tokens_dev) (void)hipFree(s->tokens_dev);
   if (s->tokens_pinned) (void)hipHostFree(s->tokens_pinned);
   if (s->argmax_dev) (void)hipFree(s->argmax_dev);
@@ -1204,9 +1207,25 @@ int rwkv_hip_session_debug_buffer(rwkv_hip_session* s, int id, void** ptr) {
   const Buffers& b = s->buf;
   void* table[] = {b.x,  b.xx,  b.xr,  b.xw, b.xk, b.xv,  b.xa,  b.xg, b.r,   b.k,     b.v,  b.v_first,
                    b.w12, b.a12, b.g,  b.hw, b.ha, b.hg,  b.hv,  b.k2, b.nkk, b.kka,   b.y,  b.y2,
-                   b.att, b.x1,  b.ln2, b.mixed, b.act, b.cm, b.r32, b.d32, b.k32, b.a32, b.b32};
+                   b.att, b.x1,  b.ln2, b.mixed, b.act, b.cm, b.r32, b.d32, b.k2, b.nkk, b.kka};
   RWKV_REQUIRE(id >= 0 && id < static_cast<int>(sizeof(table) / sizeof(table[0])), "debug_buffer: unknown id %d", id);
   *ptr = table[id];
+  // the recurrence reads its operands in fp16: their fp32 forms are made here
+  constexpr int kR32 = 30, kK32 = 32;
+  const size_t n = static_cast<size_t>(s->arena_B) * s->arena_T * s->model->C;
+  if (!s->arena.base || !(id >= kK32 || (id == kR32 && s->arena_B * s->arena_T > 1))) return RWKV_OK;
+  const int slot = id == kR32 ? 0 : 1 + id - kK32;
+  RWKV_HIP_TRY(hipStreamSynchronize(s->stream));
+  if (n > s->widened_cap[slot]) {
+    if (s->widened[slot]) RWKV_HIP_TRY(hipFree(s->widened[slot]));
+    s->widened[slot] = nullptr;
+    s->widened_cap[slot] = 0;
+    RWKV_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&s->widened[slot]), n * sizeof(float)));
+    s->widened_cap[slot] = n;
+  }
+  TRY(rwkv_hip_f16_to_f32(s->stream, static_cast<int64_t>(n), id == kR32 ? b.r : table[id], s->widened[slot]));
+  RWKV_HIP_TRY(hipStreamSynchronize(s->stream));
+  *ptr = s->widened[slot];
   return RWKV_OK;
 }
 

@@ -387,6 +387,30 @@ def test_debug_buffers_hold_the_last_layers_normalised_rows(gpu, L, B, T):
     sess.close()
 
 
+def test_debug_buffers_of_the_recurrences_fp32_operands(gpu):
+    """r32, k32, a32 and b32 after a prefill call whose recurrence is a launch of its own: the fp16 rows r, k2, nkk and kka, and d32
+    the decay of w12 + w0; a longer and a shorter call after it give theirs."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=2, C=512, H=8, F=2048, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
+    weights = synth_weights(dims, 4)
+    sess = Session(HipModel.from_host_weights(dims, weights, hip.FMT_W8))
+    rng = np.random.default_rng(2)
+    for T in (20, 70, 9):
+        lg = hip.DeviceArray((1, dims.V), np.float32)
+        sess.forward(rng.integers(0, dims.V, (1, T)), State(dims, 1), lg)
+        shape = (T, dims.C)
+        for wide, narrow in (("r32", "r"), ("k32", "k2"), ("a32", "nkk"), ("b32", "kka")):
+            want = sess.debug_buffer(narrow, shape).astype(np.float32)
+            same = np.array_equal(sess.debug_buffer(wide, shape), want)
+            assert same and np.abs(want).max() > 0, (T, wide)
+        # fp16 sums differ by a rounding at most: half an ulp of logits below 8 moves the decay by less than 1e-3
+        logit = sess.debug_buffer("w12", shape).astype(np.float64) + weights["layers"][-1]["w0"].astype(np.float64)
+        decay = np.exp(-np.exp(-0.5) / (1.0 + np.exp(-logit)))
+        assert np.abs(sess.debug_buffer("d32", shape) - decay).max() < 1e-3
+    sess.close()
+
+
 def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
     """Without set_sparse_ffn a decode step walks the non-zero rows only where the matrix pays for the second launch: a
     small model gives the bits of the dense product, and those of the walk once it is asked for."""
