@@ -572,9 +572,9 @@ def main():
     ms_per_step = elapsed * 1e3 / args.steps
     value = args.steps * B / elapsed
 
-    # one-sequence steps over int8 or fp16 weights skip the ffn.value rows with a zero activation (the reference's default
-    # for rows == 1, include/rwkv7_fast_v4_common.hpp:198-211); the dense product is timed beside it below
-    sparse_value = B == 1 and dims.F % 256 == 0 and dims.C % 16 == 0
+    # steps of a few rows skip the ffn.value rows with a zero activation where the matrix is large enough (the reference's
+    # default for rows == 1, include/rwkv7_fast_v4_common.hpp:198-211); the dense product is timed beside it below
+    sparse_value = sess.sparse_ffn_layers(B) == dims.L
     if sparse_value and not args.no_also:
         sess.set_sparse_ffn(0)
         sess.decode_greedy(first, min(args.warmup, 8) or 1, state, logits)
@@ -583,9 +583,9 @@ def main():
         sess.decode_greedy(first, min(args.steps, 64), state, logits)
         hip.device_sync()
         also["decode_dense_ffn_value_tok_s"] = min(args.steps, 64) * B / (time.perf_counter() - td)
-        sess.set_sparse_ffn(4)
+        sess.set_sparse_ffn(None)
         act = sess.debug_buffer("act", (B, dims.F))
-        also["ffn_value_rows_skipped_fraction_last_layer"] = float(np.mean(act == 0))
+        also["ffn_value_rows_skipped_fraction_last_layer"] = float(np.mean((act == 0).all(axis=0)))  # (rows of a step share the walk)
 
     weight_bytes = model.weight_bytes()
     state_bytes = B * (2 * dims.L * dims.H * 64 * 64 * (2 if args.wkv_fp16 else 4) + 2 * dims.L * 2 * dims.C * 2)

@@ -342,15 +342,17 @@ int rwkv_hip_decode_greedy(rwkv_hip_session* s, const int64_t* first_tokens_host
 int rwkv_hip_graph_capture_count(int64_t* count);
 int rwkv_hip_session_set_profile(rwkv_hip_session* s, int mode);
 int rwkv_hip_session_read_profile(rwkv_hip_session* s, int64_t* launches, double* total_ms);
-/* Decode steps of up to max_rows rows (0..12) use the row-skipping ffn.value product (CmixMode::NoFcOne / NoFcRows2
+/* Decode steps of up to max_rows rows (0..12; -1, the default: by matrix size, below) use the row-skipping ffn.value product (CmixMode::NoFcOne / NoFcRows2
  * of the reference, include/rwkv7_fast_v4_common.hpp:198-211, whose default is 12 rows at C = 4096).  Two to four rows
  * share one walk that reads every row that is non-zero for any of them once (with a fraction z of zero activations per row
  * that is 1 - z^rows of the matrix: at the z = 0.5 of random-init weights about what the dense product reads at three and four
- * rows, far less with trained weights).  Without a call steps of up to four rows use it where the matrix is large enough for
+ * rows, far less with trained weights).  By default steps of up to four rows use it where the matrix is large enough for
  * its second launch: from 8 MB on for one and two rows, above 32 MB for three and four (0.1B fp16, one row: 22.0 us per layer
  * dense, 24.3 with the walk).  From five rows on every row walks its own rows, which pays only while rows x (1 - z)
  * stays below 1.  0 selects the dense product. */
 int rwkv_hip_session_set_sparse_ffn(rwkv_hip_session* s, int max_rows);
+/* How many of the model's layers take ffn.value through it in a decode step of `rows` rows, as the session is set. */
+int rwkv_hip_session_sparse_ffn_layers(const rwkv_hip_session* s, int rows, int* layers);
 /* on != 0: the `wkv` tensor of rwkv_hip_forward / rwkv_hip_decode_greedy is the fp16 state, f16 [L,B,H,64,64], and
  * the recurrence runs in fp16 as rwkv_hip_wkv7_f16state does (ModelBackend's use_wkv32 == false, the reference
  * server's default: src/rwkv7_fast_v4.cu:1262-1271; calls of up to 16 tokens add w0 to the decay logit unrounded,

@@ -385,6 +385,13 @@ void take_deferred(LnArgs& a, const DeferredReduce& d) {
   a.res_splits = d.splits;
 }
 
+// Whether a decode step of `rows` rows takes ffn.value through the row-skipping product.
+bool walks_ffn_value(const rwkv_hip_session* s, const Matrix& mv, int rows) {
+  if (!mv.sparse_t) return false;
+  if (s->sparse_ffn_rows >= 0) return rows <= s->sparse_ffn_rows;
+  return rows <= kSparseUnionMaxRows && ffn_sparse_pays(mv.fmt, rows, s->model->C, s->model->F);
+}
+
 #define TRY(expr)                  \
   do {                             \
     const int rc__ = (expr);       \
@@ -475,11 +482,7 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
   const bool gate_split = fused_tmix && rows == 1 && C <= 4096 && !s->trace;
 
   // Decode steps of a few rows read only the ffn.value rows whose relu^2 activation is non-zero.
-  const bool sparse_step = step && s->sparse_ws != nullptr;
-  const auto sparse_value = [&](const Matrix& mv) {
-    if (!sparse_step || !mv.sparse_t) return false;
-    return s->sparse_ffn_rows >= 0 ? rows <= s->sparse_ffn_rows : rows <= kSparseUnionMaxRows && ffn_sparse_pays(mv.fmt, rows, C, F);
-  };
+  const auto sparse_value = [&](const Matrix& mv) { return step && s->sparse_ws != nullptr && walks_ffn_value(s, mv, rows); };
 
   // Prefill calls: residual add + LayerNorm + token shift as one launch per LayerNorm (a block also normalises the row
   // before its first; up to 256 rows a block per row, more in blocks of several rows).  The new shift rows come out in a
@@ -1175,12 +1178,20 @@ int rwkv_hip_session_set_wkv_fp16(rwkv_hip_session* s, int on) {
 
 int rwkv_hip_session_set_sparse_ffn(rwkv_hip_session* s, int max_rows) {
   RWKV_REQUIRE(s, "session is NULL");
-  RWKV_REQUIRE(max_rows >= 0 && max_rows <= kSparseMaxRows, "set_sparse_ffn: max_rows %d out of range (0..%d)", max_rows,
-               kSparseMaxRows);
+  RWKV_REQUIRE(max_rows >= -1 && max_rows <= kSparseMaxRows, "set_sparse_ffn: max_rows %d out of range (0..%d, -1: by matrix size)",
+               max_rows, kSparseMaxRows);
   if (s->sparse_ffn_rows != max_rows) {
     TRY(drop_graphs(s));  // captured decode graphs hold the other kernel
     s->sparse_ffn_rows = max_rows;
   }
+  return RWKV_OK;
+}
+
+int rwkv_hip_session_sparse_ffn_layers(const rwkv_hip_session* s, int rows, int* layers) {
+  RWKV_REQUIRE(s && layers, "sparse_ffn_layers: NULL argument");
+  RWKV_REQUIRE(rows >= 1, "sparse_ffn_layers: rows must be positive, got %d", rows);
+  *layers = 0;
+  for (const Layer& l : s->model->layers) *layers += walks_ffn_value(s, l.m[RWKV_M_FFN_VALUE], rows) ? 1 : 0;
   return RWKV_OK;
 }
 

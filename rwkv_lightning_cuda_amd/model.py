@@ -283,9 +283,15 @@ class Session:
 
     def set_sparse_ffn(self, max_rows):
         """Decode steps of up to max_rows rows (0..12; True = 1, False = 0) read only the ffn.value rows with a
-        non-zero activation (without a call: up to 4 rows, where the matrix is large enough for it to pay; two to four rows
-        share one walk over the rows any of them needs)."""
-        hip.check(hip.load().rwkv_hip_session_set_sparse_ffn(self.handle, ctypes.c_int(int(max_rows))))
+        non-zero activation; None (the default of a new session): up to 4 rows, where the matrix is large enough for it to pay.
+        Two to four rows share one walk over the rows any of them needs."""
+        hip.check(hip.load().rwkv_hip_session_set_sparse_ffn(self.handle, ctypes.c_int(-1 if max_rows is None else int(max_rows))))
+
+    def sparse_ffn_layers(self, rows):
+        """How many layers read ffn.value that way in a decode step of `rows` rows."""
+        n = ctypes.c_int(0)
+        hip.check(hip.load().rwkv_hip_session_sparse_ffn_layers(self.handle, ctypes.c_int(int(rows)), ctypes.byref(n)))
+        return n.value
 
     def set_profile(self, mode):
         """0/False off; 1/True one event pair per linear launch; 2 passes launch the linear kernels only, back to

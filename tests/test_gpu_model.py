@@ -434,6 +434,38 @@ def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
         assert rel_err(out[2], out[1]) <= 2.0 ** -8  # the same products, fp32 sums in another order, rounded to fp16 per layer
 
 
+def test_the_default_of_the_row_skipping_product_can_be_asked_for_again(gpu):
+    """set_sparse_ffn(None) after another setting gives the steps of a new session, and sparse_ffn_layers tells what a step takes:
+    nothing in a small model, all layers of a large one up to its default number of rows."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State
+    hip = gpu
+    for dims, most in ((ModelDims(L=2, C=512, H=8, F=2048, V=512, Rw=32, Ra=32, Rg=64, Rv=32), 0),
+                       (ModelDims(L=2, C=2048, H=32, F=8192, V=512, Rw=32, Ra=32, Rg=64, Rv=32), 2)):
+        model = HipModel.random_on_device(dims, hip.FMT_W8, seed=3)
+        sess = Session(model)
+        layers = lambda: [sess.sparse_ffn_layers(rows) for rows in (1, 2, 3, 4, 5, 12, 13)]
+        default = [dims.L if rows <= most else 0 for rows in (1, 2, 3, 4, 5, 12, 13)]
+        assert layers() == default
+        logits = []
+        for setting in ("new", 0, 4, 12, None):
+            if setting != "new":
+                sess.set_sparse_ffn(setting)
+            assert layers() == (default if setting in ("new", None) else [dims.L if rows <= setting else 0 for rows in (1, 2, 3, 4, 5, 12, 13)])
+            st, lg = State(dims, 1), hip.DeviceArray((1, dims.V), np.float32)
+            for token in (7, 8, 9):
+                sess.forward(np.array([[token]]), st, lg)
+            logits.append(lg.numpy().view(np.uint32).copy())
+        assert np.array_equal(logits[0], logits[-1])
+        assert np.array_equal(logits[1], logits[0]) == (most == 0)
+        for bad in (-2, 13):
+            with pytest.raises(hip.RwkvHipError):
+                sess.set_sparse_ffn(bad)
+        with pytest.raises(hip.RwkvHipError):
+            sess.sparse_ffn_layers(0)
+        sess.close()
+        model.close()
+
+
 def test_chunked_prefill_resume_bitwise_and_chunk_size_invariance(gpu, orc):
     """State carried in HBM across chunks.  (a) Saving the state to the host between chunks and resuming from
     the restored copy is bitwise identical to the uninterrupted run (same chunking).  (b) A different chunking
