@@ -347,8 +347,8 @@ int rwkv_hip_session_read_profile(rwkv_hip_session* s, int64_t* launches, double
  * share one walk that reads every row that is non-zero for any of them once (with a fraction z of zero activations per row
  * that is 1 - z^rows of the matrix: at the z = 0.5 of random-init weights about what the dense product reads at three and four
  * rows, far less with trained weights).  By default steps of up to four rows use it where the matrix is large enough for
- * its second launch: from 8 MB on for one and two rows, above 32 MB for three and four (0.1B fp16, one row: 22.0 us per layer
- * dense, 24.3 with the walk).  From five rows on every row walks its own rows, which pays only while rows x (1 - z)
+ * its second launch: from 8 MB on for one and two rows, from 32 MB on for three and four (smaller ones are faster dense even
+ * where nearly every activation is zero).  From five rows on every row walks its own rows, which pays only while rows x (1 - z)
  * stays below 1.  0 selects the dense product. */
 int rwkv_hip_session_set_sparse_ffn(rwkv_hip_session* s, int max_rows);
 /* How many of the model's layers take ffn.value through it in a decode step of `rows` rows, as the session is set. */

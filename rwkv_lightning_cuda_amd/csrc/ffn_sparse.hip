@@ -438,14 +438,21 @@ static void launch_walk(hipStream_t st, dim3 grid, int tokens, const SparseArgs&
   else hipLaunchKernelGGL((ffn_sparse_kernel<FMT, 4>), grid, block, 0, st, a);
 }
 
-// Bytes of ffn.value from which the walk beats the dense product at the half zeros of random-init weights (walk / dense, us per
-// layer): one and two tokens 1.5B int4 (9 MB) 32.6 / 33.0 and 39.4 / 41.1, int8 32.1 / 34.6, but 0.1B fp16 (5 MB) 24.3 / 22.0 and
-// 27.8 / 25.2 - the second launch costs more than half of the matrix.  Three and four tokens, whose walk reads most of the rows:
-// 1.5B int8 43.4 / 40.8 and 45.2 / 42.6, fp16 (34 MB) 46.9 / 45.2 and 49.2 / 46.6; 7.2B int8 (67 MB) 68.0 / 66.9 and 69.3 / 67.2, int4
-// (35 MB) 62.8 / 61.8 and 65.2 / 61.7: the fewer rows of trained weights decide there.
+// Bytes of ffn.value from which the walk can beat the dense product; below, the dense product is the faster one however many
+// activations are zero, because the walk's second launch and its lists cost more than the whole matrix.  us per layer of a decode
+// step, dense / walk with the given share of the rows needed by any token of the step (1 - z^tokens at a share z of zeros; random-init
+// weights have z = 0.5, and the dense product costs the same at any z):
+//   one token    0.1B fp16 (5 MB) 20.7 / 23.1 at 0.51, 22.2 at 0.04   1.5B int4 (9 MB) 30.5 / 29.9 at 0.49, 29.2 at 0.05
+//   two tokens   0.1B fp16 23.9 / 27.0 at 0.75, 25.7 at 0.07          1.5B int4 38.5 / 37.0 at 0.70, 35.8 at 0.07
+//   three        1.5B int8 (17 MB) 38.9 / 41.1 at 0.82, 40.4 at 0.49, 38.9 at 0.08    1.5B fp16 (32 MB) 43.9 / 44.7, 43.1, 40.7
+//   four         1.5B int8 40.7 / 43.5 at 0.88, 43.0 at 0.54, 41.3 at 0.09            1.5B fp16 45.4 / 46.8, 45.3, 42.8
+//   three, four  7.2B int8 (64 MB) 67.0 / 68.3 at 0.82, 65.3 at 0.49, 60.7 at 0.09 and 67.6 / 69.4 at 0.87, 66.4 at 0.52, 61.7 at 0.09;
+//                7.2B int4 (34 MB) 60.4 / 61.9, 59.5, 55.9 and 60.5 / 64.2, 61.1, 56.6
+// From 32 MB on three and four tokens gain from some 70 to 80 % of zeros per token on and lose 1 to 6 % at one half: the choice counts
+// on weights that are trained (the reference walks for up to 12 tokens by default).
 bool ffn_sparse_pays(int fmt, int rows, int C, int F) {
   const size_t bytes = ffn_sparse_packed_bytes(fmt, C, F);
-  return rows <= 2 ? bytes >= (8u << 20) : rows <= kSparseUnionMaxRows && bytes > (32u << 20);
+  return rows <= 2 ? bytes >= (8u << 20) : rows <= kSparseUnionMaxRows && bytes >= (32u << 20);
 }
 
 int ffn_sparse_launch(hipStream_t st, int fmt, int rows, int C, int F, int activated, const half_t* in, const void* wt,

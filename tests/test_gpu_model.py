@@ -436,12 +436,13 @@ def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
 
 def test_the_default_of_the_row_skipping_product_can_be_asked_for_again(gpu):
     """set_sparse_ffn(None) after another setting gives the steps of a new session, and sparse_ffn_layers tells what a step takes:
-    nothing in a small model, all layers of a large one up to its default number of rows."""
+    nothing in a small model, all layers of a large one up to its default number of rows (16 MB: two; 32 MB: four)."""
     from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State
     hip = gpu
-    for dims, most in ((ModelDims(L=2, C=512, H=8, F=2048, V=512, Rw=32, Ra=32, Rg=64, Rv=32), 0),
-                       (ModelDims(L=2, C=2048, H=32, F=8192, V=512, Rw=32, Ra=32, Rg=64, Rv=32), 2)):
-        model = HipModel.random_on_device(dims, hip.FMT_W8, seed=3)
+    for dims, fmt, most in ((ModelDims(L=2, C=512, H=8, F=2048, V=512, Rw=32, Ra=32, Rg=64, Rv=32), hip.FMT_W8, 0),
+                            (ModelDims(L=2, C=2048, H=32, F=8192, V=512, Rw=32, Ra=32, Rg=64, Rv=32), hip.FMT_W8, 2),
+                            (ModelDims(L=2, C=2048, H=32, F=8192, V=512, Rw=32, Ra=32, Rg=64, Rv=32), hip.FMT_F16, 4)):
+        model = HipModel.random_on_device(dims, fmt, seed=3)
         sess = Session(model)
         layers = lambda: [sess.sparse_ffn_layers(rows) for rows in (1, 2, 3, 4, 5, 12, 13)]
         default = [dims.L if rows <= most else 0 for rows in (1, 2, 3, 4, 5, 12, 13)]
