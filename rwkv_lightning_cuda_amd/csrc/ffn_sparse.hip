@@ -312,6 +312,7 @@ __global__ __launch_bounds__(64 * kSparseWaves) void ffn_sparse_kernel(SparseArg
   const int steps = (n + 2 * G - 1) / (2 * G);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (n > 0 && n + lane < 2 * G * steps) {
     row_s[wave][n + lane] = row_s[wave][0];
 #pragma unroll
@@ -319,6 +320,7 @@ __global__ __launch_bounds__(64 * kSparseWaves) void ffn_sparse_kernel(SparseArg
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
   float acc[TOK][LC];
   float asum[TOK];
