@@ -338,9 +338,10 @@ __global__ __launch_bounds__(NT) void ln_mix_seq_kernel(LnArgs a) {
 // The same for many rows: a block walks several consecutive rows, so that only the row before its first one is normalised a
 // second time, and keeps the LayerNorm output of the row before in registers.  Bound by memory: against a LayerNorm and a
 // token-shift launch the LN rows are neither written nor read again.  The loads of the next row are in flight during the
-// reductions of this one.  Statements and order of ln_mix_seq_kernel: the same bits.  Two rows per block, four from 2048 rows on,
-// us of LN1 + LN2 with 1 / 2 / 4 / 8 rows per block: 2048 rows x 4096 63.9 / 50.4 / 46.8 / 47.8 (two launches each 66.3), 999 x 2048 21.5 /
-// 18.1 / 19.1 / 26.7 (25.4).
+// reductions of this one.  Statements and order of ln_mix_seq_kernel: the same bits.  Two blocks per CU and at least two rows per
+// block, at most four (three from 1536 rows on, four from 2048): us of LN1 + LN2 with 1 / 2 / 4 / 8 rows per block: 2048 rows x 4096 63.9 /
+// 50.4 / 46.8 / 47.8 (two launches each 66.3), 999 x 2048 21.5 / 18.1 / 19.1 / 26.7 (25.4).  us per layer of whole prefill calls, a LayerNorm and a
+// token-shift launch / this: 257 rows x 768 80.8 / 78.8, x 2048 133.2 / 130.3, x 4096 (int8) 287.9 / 285.1; 1536 x 4096 1036 / 1023.
 // PLANES: split-K planes of the residual requested ahead (0: a plain fp16 residual); further ones are read in line.
 template <int NT, int PLANES>
 __global__ __launch_bounds__(NT) void ln_mix_rows_kernel(LnArgs a, int rows, int rows_per_block) {

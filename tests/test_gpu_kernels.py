@@ -700,7 +700,7 @@ def test_kk_gate_of_few_and_of_many_heads_give_the_same_bits(gpu, rows, H):
             assert np.array_equal(got, want[first:first + n])
 
 
-def test_lora_out_blocks_walk_several_row_tiles(gpu, orc):
+def test_lora_out_of_several_row_tiles(gpu, orc):
     """Ten row tiles, the last one partial; the v-residual epilogue is checked on the same rows."""
     hip = gpu
     rng = np.random.default_rng(77)
@@ -811,13 +811,7 @@ def _sparse_w4_pack(hip, orc, w):
     return q, s, z, wt
 
 
-@pytest.mark.parametrize("fmt_name", ["w8", "f16", "w4"])
-@pytest.mark.parametrize("C,F", [(768, 3072), (2560, 10240), (4096, 16384)])
-def test_cmix_sparse_down_matches_dense_product_and_oracle(gpu, orc, C, F, fmt_name):
-    """ffn.value of one token over the transposed copy, skipping rows with a zero activation: against the
-    oracle's dense product of the same weights and against the dense GEMV on the GPU; edge patterns of the
-    activation (none, one, all non-zero; a wavefront's 32 rows all zero); repeat calls bitwise equal."""
-    hip = gpu
+def _one_token_walk_matches_dense_product_and_oracle(hip, orc, C, F, fmt_name):
     rng = np.random.default_rng(C + F)
     w = (rng.standard_normal((C, F)) * 0.02).astype(np.float16)
     z, zd = None, None
@@ -878,6 +872,15 @@ def test_cmix_sparse_down_matches_dense_product_and_oracle(gpu, orc, C, F, fmt_n
 
 
 @pytest.mark.parametrize("fmt_name", ["w8", "f16", "w4"])
+@pytest.mark.parametrize("C,F", [(768, 3072), (2560, 10240), (4096, 16384)])
+def test_cmix_sparse_down_matches_dense_product_and_oracle(gpu, orc, C, F, fmt_name):
+    """ffn.value of one token over the transposed copy, skipping rows with a zero activation: against the
+    oracle's dense product of the same weights and against the dense GEMV on the GPU; edge patterns of the
+    activation (none, one, all non-zero; a wavefront's 32 rows all zero); repeat calls bitwise equal."""
+    _one_token_walk_matches_dense_product_and_oracle(gpu, orc, C, F, fmt_name)
+
+
+@pytest.mark.parametrize("fmt_name", ["w8", "f16", "w4"])
 def test_cmix_sparse_down_rows_matches_the_one_row_product(gpu, orc, fmt_name):
     """Several tokens per call: each row of the output is bitwise what the one-row call gives for that token, and
     matches the oracle's dense product."""
@@ -925,14 +928,7 @@ def test_cmix_sparse_down_rows_matches_the_one_row_product(gpu, orc, fmt_name):
         hip.cmix_sparse_down_relu_rows(fmt, rows, C, F, dev(hip, pre), wt, sd, ws1, out)  # workspace of one row
 
 
-@pytest.mark.parametrize("fmt_name", ["w8", "f16", "w4"])
-@pytest.mark.parametrize("C,F,rows", [(768, 3072, 2), (2048, 8192, 3), (4096, 16384, 4)])
-def test_cmix_sparse_down_shared_walk_matches_oracle_and_per_token_walks(gpu, orc, fmt_name, C, F, rows):
-    """2..4 tokens in one walk over the union of their non-zero rows, at the three benchmark widths: against the
-    oracle's dense product (the bar of the fp16 paths) and against one walk per token (equal up to the last bits of
-    the fp32 sums: within an fp16 ulp of the output's scale after rounding, mostly identical); a token without any active row comes
-    out as zeros; two calls give the same bits."""
-    hip = gpu
+def _shared_walk_matches_oracle_and_per_token_walks(hip, orc, fmt_name, C, F, rows):
     rng = np.random.default_rng(C + rows)
     w = (rng.standard_normal((C, F)) * 0.02).astype(np.float16)
     z = None
@@ -981,13 +977,23 @@ def test_cmix_sparse_down_shared_walk_matches_oracle_and_per_token_walks(gpu, or
 
 
 @pytest.mark.parametrize("fmt_name", ["w8", "f16", "w4"])
+@pytest.mark.parametrize("C,F,rows", [(768, 3072, 2), (2048, 8192, 3), (4096, 16384, 4)])
+def test_cmix_sparse_down_shared_walk_matches_oracle_and_per_token_walks(gpu, orc, fmt_name, C, F, rows):
+    """2..4 tokens in one walk over the union of their non-zero rows, at the three benchmark widths: against the
+    oracle's dense product (the bar of the fp16 paths) and against one walk per token (equal up to the last bits of
+    the fp32 sums: within an fp16 ulp of the output's scale after rounding, mostly identical); a token without any active row comes
+    out as zeros; two calls give the same bits."""
+    _shared_walk_matches_oracle_and_per_token_walks(gpu, orc, fmt_name, C, F, rows)
+
+
+@pytest.mark.parametrize("fmt_name", ["w8", "f16", "w4"])
 @pytest.mark.parametrize("C,F", [(16, 256), (272, 768), (400, 5120), (4112, 8192)])
 def test_cmix_sparse_down_at_the_edges_of_chunks_and_lists(gpu, orc, C, F, fmt_name):
     """A last column chunk of 16 columns, wavefronts of 32, 64 and 128 rows, lists from empty to full: one token, and walks of two
     and four that share it."""
-    test_cmix_sparse_down_matches_dense_product_and_oracle(gpu, orc, C, F, fmt_name)
+    _one_token_walk_matches_dense_product_and_oracle(gpu, orc, C, F, fmt_name)
     for rows in (2, 4):
-        test_cmix_sparse_down_shared_walk_matches_oracle_and_per_token_walks(gpu, orc, fmt_name, C, F, rows)
+        _shared_walk_matches_oracle_and_per_token_walks(gpu, orc, fmt_name, C, F, rows)
 
 
 def test_cmix_sparse_rejects_bad_arguments(gpu):

@@ -316,22 +316,10 @@ def test_decode_with_row_skipping_ffn_value(gpu, orc, fmt, B):
     assert err <= 1e-3
 
 
-@pytest.mark.parametrize("fmt", [1, 2])
-@pytest.mark.parametrize("B,T", [(2, 16), (12, 21), (20, 21), (36, 11), (40, 1), (12, 1)])
-def test_fused_launches_match_the_standalone_kernels_bitwise(gpu, fmt, B, T):
-    """Three fusions of the row-tiled path are switched off while the residual-stream tap is on.  (0) Prefill calls of
-    up to 256 rows run residual add + LayerNorm + token shift as one kernel per LayerNorm, whose blocks normalise the
-    previous row a second time and leave the new shift rows to the next GEMM launch; tapped, the LayerNorm and the
-    token-shift kernel run one after the other.  (1) The LayerNorm
-    kernels after the output projection and after ffn.value sum the fp32 split-K partials of the streaming GEMM
-    themselves; tapped, the reduce kernel runs instead.  (2) kk normalise / a-gate / decay, the WKV recurrence and
-    GroupNorm / bonus / gate run as one launch; tapped, as the three stand-alone kernels.  Same arithmetic in the
-    same order: logits, shift rows and WKV state are bit-identical (prefill chunks with and without a ragged tail,
-    at each of the sequence kernel's three wavefronts-per-head variants, and a batched decode step)."""
-    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
-    hip = gpu
-    dims = ModelDims(L=2, C=512, H=8, F=2048, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
-    gmodel = HipModel.from_host_weights(dims, synth_weights(dims, 4), fmt)
+def _fused_launches_agree_with_the_standalone_kernels(hip, gmodel, B, T):
+    """Logits, shift rows and WKV state of one call with the residual-stream tap off and on, bitwise."""
+    from rwkv_lightning_cuda_amd.model import Session, State
+    dims = gmodel.dims
     rng = np.random.default_rng(B + T)
     tokens = rng.integers(0, dims.V, (B, T))
     sess = Session(gmodel)
@@ -355,11 +343,43 @@ def test_fused_launches_match_the_standalone_kernels_bitwise(gpu, fmt, B, T):
     sess.close()
 
 
+@pytest.mark.parametrize("fmt", [1, 2])
+@pytest.mark.parametrize("B,T", [(2, 16), (12, 21), (20, 21), (36, 11), (40, 1), (12, 1)])
+def test_fused_launches_match_the_standalone_kernels_bitwise(gpu, fmt, B, T):
+    """Three fusions of the row-tiled path are switched off while the residual-stream tap is on.  (0) Prefill calls of
+    up to 256 rows run residual add + LayerNorm + token shift as one kernel per LayerNorm, whose blocks normalise the
+    previous row a second time and leave the new shift rows to the next GEMM launch; tapped, the LayerNorm and the
+    token-shift kernel run one after the other.  (1) The LayerNorm
+    kernels after the output projection and after ffn.value sum the fp32 split-K partials of the streaming GEMM
+    themselves; tapped, the reduce kernel runs instead.  (2) kk normalise / a-gate / decay, the WKV recurrence and
+    GroupNorm / bonus / gate run as one launch; tapped, as the three stand-alone kernels.  Same arithmetic in the
+    same order: logits, shift rows and WKV state are bit-identical (prefill chunks with and without a ragged tail,
+    at each of the sequence kernel's three wavefronts-per-head variants, and a batched decode step)."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, synth_weights
+    dims = ModelDims(L=2, C=512, H=8, F=2048, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
+    _fused_launches_agree_with_the_standalone_kernels(gpu, HipModel.from_host_weights(dims, synth_weights(dims, 4), fmt), B, T)
+
+
 @pytest.mark.parametrize("B,T", [(1, 300), (600, 2), (40, 31), (5, 411), (16, 130)])
 def test_layer_norm_blocks_of_several_rows_match_the_standalone_kernels_bitwise(gpu, B, T):
-    """More than 256 rows: a LayerNorm block walks 1, 2 or 4 rows, with the first row of a sequence at its start, inside it or
+    """More than 256 rows: a LayerNorm block walks 2 or 4 rows, with the first row of a sequence at its start, inside it or
     nowhere, and a last block that is partial."""
-    test_fused_launches_match_the_standalone_kernels_bitwise(gpu, 1, B, T)
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, synth_weights
+    dims = ModelDims(L=2, C=512, H=8, F=2048, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
+    _fused_launches_agree_with_the_standalone_kernels(gpu, HipModel.from_host_weights(dims, synth_weights(dims, 4), 1), B, T)
+
+
+@pytest.mark.parametrize("C,F,B,T", [(512, 8192, 1, 333), (2048, 8192, 1, 300), (2048, 8192, 3, 333), (2048, 2048, 1, 1700), (2560, 10240, 1, 257),
+                                     (2560, 10240, 5, 80), (2560, 2560, 5, 331), (4096, 16384, 2, 151), (4096, 4096, 5, 331),
+                                     (4096, 4096, 3, 687)])
+def test_layer_norm_blocks_of_several_rows_at_other_widths(gpu, C, F, B, T):
+    """Both block sizes with all threads live and with idle ones, 2, 3 and 4 rows per block, and a residual that is plain or still lies in
+    2, 4 or 8 split-K planes (the last four of eight are read in line)."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims
+    dims = ModelDims(L=2, C=C, H=C // 64, F=F, V=512, Rw=32, Ra=32, Rg=64, Rv=32)
+    gmodel = HipModel.random_on_device(dims, gpu.FMT_W8, seed=5)
+    _fused_launches_agree_with_the_standalone_kernels(gpu, gmodel, B, T)
+    gmodel.close()
 
 
 @pytest.mark.parametrize("L", [1, 2, 3])
