@@ -175,7 +175,8 @@ int rwkv_hip_linear_packed(rwkv_stream_t s, int fmt, int M, int N, int K, const 
  *   out[c] = f16(scale[c] * sum over f with vec[f] != 0 of vec[f] * q[c][f]).
  * preact [rows,F], out [rows,C], rows 1..12.  The reference accumulates in half2 with atomicAdd; this one
  * accumulates exact products in fp32 in a fixed order, so it equals the dense product up to fp32 summation order
- * and repeats bitwise.
+ * and repeats bitwise.  How the sums are split goes by the shape and the number of rows: a row of a call of several may
+ * differ from its own call in the last bits of the fp32 sums.
  * cmix_sparse_pack turns the [C,F] matrix (fp16 values, or the codes of rwkv_hip_quantize_w8) into the [F,C]
  * copy `wt` (same size) that the product reads - the layout the reference keeps ffn.value in
  * (include/rwkv7_fast_v4_common.hpp:313-321); `scale` is the per-output-channel tensor of the codes (unused

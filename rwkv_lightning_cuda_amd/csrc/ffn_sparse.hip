@@ -472,13 +472,20 @@ int ffn_sparse_launch(hipStream_t st, int fmt, int rows, int C, int F, int activ
   }
   // 2 .. 4 tokens share one walk over the rows that are non-zero for any of them; otherwise a walk per token
   const int tokens = one_walk && rows >= 2 && rows <= kSparseUnionMaxRows ? rows : 1;
-  // rows per wavefront: as many as leave a block per CU (fewer partial rows; twice the blocks 1-3 % of the step slower)
+  // Rows per wavefront: as many as leave three blocks to four CUs, or more than three to two CUs where every token has its own walk -
+  // what a wavefront does besides its rows, lists and sums, is most of its instructions when few of 32 rows are needed.  us per
+  // call with 32 / 64 / 128 rows, half of the activations zero (a tenth not zero): one token, 2048 x 8192 int8 6.6 / 6.9 / 8.4 (5.5 / 5.3 /
+  // 6.0), 2560 x 10240 int8 7.9 / 7.5 / 8.4 (6.2 / 5.7 / 6.1), fp16 9.9 / 9.9 / 9.3 (7.1 / 6.1 / 6.2), three that share a walk 13.9 / 13.9 / 13.1; 12 tokens, 2048 x
+  // 8192 int8 20.8 / 17.6 / 15.8 (14.6 / 9.9 / 8.5), 2560 x 10240 int4 29.8 / 23.1 / 21.4 (22.3 / 14.3 / 11.5); 3 tokens, 2048 x 8192 fp16 13.3 / 11.8 /
+  // 13.1 (8.5 / 6.7 / 6.7).
+  const int walks = rows / tokens;
   const int chunks = ceil_div(C, 64 / kSparseGroups * sparse_lane_cols(fmt));
+  const int64_t least = walks > 1 ? device_cu_count() * 3 / 2 + 1 : device_cu_count() * 3 / 4;
   int rpw = 128;
-  while (rpw > 32 && (F % (kSparseWaves * rpw) != 0 || static_cast<int64_t>(chunks) * (F / (kSparseWaves * rpw)) < device_cu_count())) rpw /= 2;
+  while (rpw > 32 && (F % (kSparseWaves * rpw) != 0 || static_cast<int64_t>(chunks) * (F / (kSparseWaves * rpw)) * walks < least)) rpw /= 2;
   const SparseArgs a = {C, F, rpw, activated, in, static_cast<const uint8_t*>(wt), static_cast<float*>(workspace)};
   const int n_partial = F / (kSparseWaves * rpw);
-  const dim3 grid(n_partial, chunks, rows / tokens);
+  const dim3 grid(n_partial, chunks, walks);
   if (fmt == RWKV_FMT_W4) launch_walk<RWKV_FMT_W4>(st, grid, tokens, a);
   else if (fmt == RWKV_FMT_W8) launch_walk<RWKV_FMT_W8>(st, grid, tokens, a);
   else launch_walk<RWKV_FMT_F16>(st, grid, tokens, a);

@@ -996,6 +996,74 @@ def test_cmix_sparse_down_at_the_edges_of_chunks_and_lists(gpu, orc, C, F, fmt_n
         _shared_walk_matches_oracle_and_per_token_walks(gpu, orc, fmt_name, C, F, rows)
 
 
+def _sparse_codes_and_copy(hip, orc, w, fmt_name):
+    """(format, transposed copy, scale on the device, exact weights, magnitudes that the sums pass through) of a [C,F] matrix."""
+    C, F = w.shape
+    if fmt_name == "w4":
+        q, s, z, wt = _sparse_w4_pack(hip, orc, w)
+        nib = np.empty((C, F))
+        nib[:, 0::2], nib[:, 1::2] = q & 15, q >> 4
+        s, z = np.repeat(s.reshape(C, F // 128).astype(np.float64), 128, 1), np.repeat(z.reshape(C, F // 128).astype(np.float64), 128, 1)
+        return hip.FMT_W4, wt, None, (nib - z) * s, (nib + z) * s
+    if fmt_name == "w8":
+        q, s = orc.quantize_w8(w)
+        wt, sd, exact = hip.DeviceArray((F, C), np.uint8), dev(hip, s), q * s.astype(np.float64)[:, None]
+    else:
+        q, wt, sd, exact = w, hip.DeviceArray((F, C), np.float16), None, w.astype(np.float64)
+    fmt = hip.FMT_W8 if fmt_name == "w8" else hip.FMT_F16
+    hip.cmix_sparse_pack(fmt, C, F, dev(hip, q), wt)
+    return fmt, wt, sd, exact, np.abs(exact)
+
+
+@pytest.mark.parametrize("fmt_name", ["w8", "f16", "w4"])
+@pytest.mark.parametrize("C,F,counts", [(1536, 6144, (2, 3, 8, 12)), (2048, 8192, (3, 5, 8)), (2560, 10240, (1, 2, 4, 12))])
+def test_cmix_sparse_down_a_walk_per_token_at_every_split(gpu, orc, C, F, counts, fmt_name):
+    """Token counts on either side of where a wavefront takes 32, 64 and 128 rows, against 64-bit sums of the same codes.  A product
+    passes at most 64 fp32 additions (32 in a lane, 2 between lanes, 8 wavefronts, 3 + 16 of the partial rows) and a scale, and
+    the result rounds once to fp16."""
+    hip = gpu
+    rng = np.random.default_rng(C)
+    fmt, wt, sd, exact, passed = _sparse_codes_and_copy(hip, orc, (rng.standard_normal((C, F)) * 0.02).astype(np.float16), fmt_name)
+    for rows in counts:
+        pre = (rng.standard_normal((rows, F)) - rng.choice([0.0, 1.3, 3.0], (rows, 1))).astype(np.float16)
+        pre[rows // 2] = -np.abs(pre[rows // 2])  # a token with no active row
+        act = orc.relu_square(pre).astype(np.float64)
+        want, most = act @ exact.T, act @ passed.T
+        bound = np.spacing(np.abs(want).astype(np.float16)).astype(np.float64) * 0.51 + 65 * 2.0 ** -24 * most
+        ws = hip.DeviceArray((hip.cmix_sparse_workspace(C, F, rows),), np.uint8)
+        out = hip.DeviceArray((rows, C), np.float16)
+        hip.cmix_sparse_down_relu_rows(fmt, rows, C, F, dev(hip, pre), wt, sd, ws, out)
+        hip.device_sync()
+        worst = (np.abs(out.numpy() - want) / bound).max()
+        assert worst <= 1.0, rows
+
+
+def test_cmix_sparse_down_twelve_walks_take_little_longer_than_one(gpu, orc):
+    """int4, 2560 x 10240, a tenth of the activations not zero: 11.5 us a call against 6 to 8, which launching it costs (22.3 with 32
+    rows per wavefront)."""
+    hip = gpu
+    C, F = 2560, 10240
+    rng = np.random.default_rng(3)
+    fmt, wt, sd, _, _ = _sparse_codes_and_copy(hip, orc, (rng.standard_normal((C, F)) * 0.02).astype(np.float16), "w4")
+    best = []
+    for rows in (1, 12):
+        pre = dev(hip, (rng.standard_normal((rows, F)) - 1.3).astype(np.float16))
+        ws = hip.DeviceArray((hip.cmix_sparse_workspace(C, F, rows),), np.uint8)
+        out = hip.DeviceArray((rows, C), np.float16)
+        start, stop = hip.Event(), hip.Event()
+        us = []
+        for _ in range(8):
+            start.record()
+            for _ in range(40):
+                hip.cmix_sparse_down_relu_rows(fmt, rows, C, F, pre, wt, sd, ws, out)
+            stop.record()
+            hip.device_sync()
+            us.append(start.elapsed_ms(stop) * 25)
+        best.append(min(us))
+    print("1 token %.1f us, 12 %.1f us" % tuple(best))
+    assert best[1] <= 2.1 * best[0]
+
+
 def test_cmix_sparse_rejects_bad_arguments(gpu):
     hip = gpu
     with pytest.raises(hip.RwkvHipError):
