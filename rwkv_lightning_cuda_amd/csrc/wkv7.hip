@@ -32,9 +32,9 @@ struct SeqOperands {
 // ---- sequence kernel -------------------------------------------------------------------------
 // grid = B*H*PARTS, block = 1024/RPL/PARTS threads: 16/RPL wavefronts per head, RPL state rows per lane.  Lane (g, c) = (lane / 16,
 // lane % 16) of wavefront q owns rows 4*RPL*q + RPL*g .. +RPL-1 and columns 4c .. 4c+3, so the 16 lanes of one DPP row hold
-// complete state rows and the wavefronts never exchange data.  v,y have `io_bs` elements between batch rows.  The block stages
-// the operands kSeqChunk tokens at a time, double-buffered; a step costs each lane six LDS reads (its four columns of the five
-// operands and its v values) against 28*RPL VALU operations.  y goes back through LDS so that the global stores are coalesced.
+// complete state rows and the wavefronts never exchange data.  The block stages the operands kSeqChunk tokens at a time,
+// double-buffered; a step costs each lane six LDS reads (its four columns of the five operands and its v values) against
+// 28*RPL VALU operations.  y goes back through LDS so that the global stores are coalesced.
 constexpr int kSeqChunk = 8;
 
 // FUSED (the model's row-tiled time-mix path, fp16 io): the operands are not read as fp32 tensors but derived
@@ -52,7 +52,7 @@ constexpr int kSeqChunk = 8;
 template <typename IO, typename WT, int RPL, int PARTS, bool FUSED, bool STRAIGHT = true>
 __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int C, int H, float* __restrict__ state,
                                                               const IO* __restrict__ v, IO* __restrict__ y,
-                                                              int64_t io_bs, TmixSeqArgs fa, SeqOperands<IO, WT> ro) {
+                                                              TmixSeqArgs fa, SeqOperands<IO, WT> ro) {
   constexpr bool RAW = !FUSED;
   static_assert(PARTS == 1 || !FUSED, "the fused pass needs whole heads");
   constexpr int NT = 1024 / RPL / PARTS;
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
 #pragma unroll
   for (int i = 0; i < RPL; ++i) S[i] = __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(sblk + i * kHead));
 
-  const int64_t iob = static_cast<int64_t>(bi) * io_bs + h * kHead;
+  const int64_t iob = static_cast<int64_t>(bi) * T * C + h * kHead;
   // Two sets of staging registers: a chunk is requested two chunks before it is needed - eight steps are shorter
   // than a trip to memory.
   float v_stage[2][kVSlots];
@@ -726,7 +726,7 @@ template <typename IO, typename WT, int RPL, int PARTS, bool FUSED, bool STRAIGH
 static void launch_seq(hipStream_t st, int B, int T, int C, int H, float* state, const IO* v, IO* y, const TmixSeqArgs& fa,
                        const SeqOperands<IO, WT>& ro) {
   hipLaunchKernelGGL((wkv7_seq_kernel<IO, WT, RPL, PARTS, FUSED, STRAIGHT>), dim3(B * H * PARTS), dim3(1024 / RPL / PARTS), 0, st, T, C, H,
-                     state, v, y, static_cast<int64_t>(T) * C, fa, ro);
+                     state, v, y, fa, ro);
 }
 
 template <typename IO, typename WT, int G, int RPL, int NC, int PARTS, int NF, int SETS, int WAVES, bool AHEAD>
