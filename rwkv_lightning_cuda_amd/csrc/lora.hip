@@ -395,12 +395,20 @@ int lora_out_multi(hipStream_t st, const LoraOutMultiArgs& a) {
   // 192 (384) 9.4 / 7.3, 256 (512) 9.8 / 8.2; 768 channels, 256 rows (192) 4.6 / 6.3.
   const int row_tiles = ceil_div(a.M, kLoraRows);
   const int64_t cus = device_cu_count();
-  if (static_cast<int64_t>(ceil_div(a.C, kLoraCols)) * row_tiles * a.n * 2 > 3 * cus) {
+  const int64_t small = static_cast<int64_t>(ceil_div(a.C, kLoraCols)) * row_tiles * a.n;
+  // A problem on its own, whose blocks all take as long, runs in rounds of a block per CU, and from rank 128 on a round of the 32 x
+  // 256 tile is as long as two of the small one: it is taken where it needs no more than half as many.  us, small tile / 32 x 256, rank
+  // 128 without activation: 4096 channels, 500 rows (2 rounds / 1) 6.3 / 6.7, 700 (3 / 2) 8.5 / 10.7, 1000 (4 / 2) 10.5 / 11.1, 1200 (5 / 3)
+  // 12.2 / 15.1; rank 480 with one 11.6 / 11.7, 15.5 / 16.7, 19.6 / 19.3, 23.2 / 24.9; rank 96 with one, 700 rows 8.5 / 7.5.
+  const int64_t wide8 = static_cast<int64_t>(ceil_div(a.C, 256)) * row_tiles;
+  const bool uneven = a.n == 1 && a.p[0].R >= 128 && 2 * ((wide8 + cus - 1) / cus) > (small + cus - 1) / cus;
+  if (small * 2 > 3 * cus) {
     // twice as many channels per block where that still leaves two blocks per CU and no channel of a block unused: 32 x 256 / 32 x
     // 512 at 4096 channels and 500 rows 21.4 / 19.2, 1000 39.0 / 37.4, 2048 68.4 / 57.9; 2048 channels and 999 rows 17.9 / 13.1, 2048
     // 29.2 / 28.7 (before, with the small tile's blocks walking several row tiles: 33.7, 60.5, 107.6; 26.5, 50.1)
     const bool wide = a.C % 512 == 0 && static_cast<int64_t>(a.C / 512) * row_tiles * a.n >= 2 * cus;
-    return wide ? lora_out_wide_launch<16>(st, a) : lora_out_wide_launch<8>(st, a);
+    if (wide) return lora_out_wide_launch<16>(st, a);
+    if (!uneven) return lora_out_wide_launch<8>(st, a);
   }
   hipLaunchKernelGGL(lora_out_kernel, dim3(ceil_div(a.C, kLoraCols), row_tiles, a.n), dim3(kLoraThreads), 0, st, a);
   RWKV_LAUNCH_CHECK();

@@ -722,7 +722,7 @@ def test_lora_out_of_several_row_tiles(gpu, orc):
 
 
 @pytest.mark.parametrize("C,R,rows", [(4064, 24, 417), (4096, 480, 1025), (4096, 40, 2050), (96, 8, 12321), (2048, 512, 4097),
-                                      (352, 136, 4100)])
+                                      (352, 136, 4100), (2080, 136, 825), (2080, 24, 802), (4096, 480, 993), (4096, 128, 700)])
 def test_lora_out_blocks_of_many_channels(gpu, C, R, rows):
     """Both widths of the many-row rank-out: channels that leave wavefronts of the last block idle, a last row tile of one, two
     or four rows, ranks that end in a half step, and the v-residual epilogue.  The result is within half an fp16 ulp (plus the
@@ -759,6 +759,30 @@ def test_lora_out_blocks_of_many_channels(gpu, C, R, rows):
         mags = np.abs(hf).astype(np.float64) @ np.abs(w2).astype(np.float64).T + (2.0 if vres else 0.0)
         bound = 0.5 * np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64) + 1e-6 * mags
         assert np.all(np.abs(got.astype(np.float64) - exact) <= bound)
+
+
+def test_lora_out_of_three_rounds_of_blocks_takes_little_longer_than_of_two(gpu):
+    """4096 channels, rank 128, no activation: 700 rows 8.5 us and 512 rows 6.7 (10.7 with blocks of 256 channels, the second round of
+    which is a third full)."""
+    hip = gpu
+    C, R = 4096, 128
+    w2 = dev(hip, (np.random.default_rng(1).standard_normal((C, R)) * 0.1).astype(np.float16))
+    best = []
+    for rows in (512, 700):
+        h = dev(hip, np.random.default_rng(2).standard_normal((rows, R)).astype(np.float16))
+        o = hip.DeviceArray((rows, C), np.float16)
+        start, stop = hip.Event(), hip.Event()
+        us = []
+        for _ in range(8):
+            start.record()
+            for _ in range(60):
+                hip.lora_out(rows, C, R, hip.ACT_NONE, h, w2, o)
+            stop.record()
+            hip.device_sync()
+            us.append(start.elapsed_ms(stop) * 1000 / 60)
+        best.append(min(us))
+    print("512 rows %.1f us, 700 rows %.1f us" % tuple(best))
+    assert best[1] <= 1.42 * best[0]
 
 
 @pytest.mark.parametrize("rows,C,R", [(1, 96, 8), (33, 256, 136), (70, 768, 480), (128, 4096, 512), (64, 4096, 96),
