@@ -487,9 +487,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
 //                        row in (13.3 of the 23.5 us of 64 rows of 65536, top-k 50, top-p 0.6; 20.8 with sample_row's bisection).  A row with more than kMaxCandidates of them (equal logits) goes through sample_row itself;
 //   sample_decay_kernel  the penalty rows, by the whole chip again.
 // Against the one-block kernel the sum of the exponentials and the masses are added in another order (fp32 both), no more.
-// Rows of 65536, penalties, top-k 50, top-p 0.6, one block per row / this: 1 row 53.4 / 18.0 us, 64 rows 66-70 / 23.6,
-// 128 rows 70.9 / 40.4; 8 rows, top-k 200, top-p 0.8: 64.5 / 27.7.  The same rows masked down to 20 entries: 64 rows 75.1 /
-// 28.8.  Rows of equal logits, which pay for the launches on top of sample_row, lose: 1 row 87 / 95, 256 rows 112 / 144.
+// Rows of 65536, penalties, top-k 50, top-p 0.6, one block per row / this: 1 row 53.4 / 17.6 us, 64 rows 66-70 / 23.7,
+// 128 rows 70.9 / 36.3; 8 rows, top-k 200, top-p 0.8: 64.5 / 24.1.  The same rows masked down to 20 entries: 64 rows 75.1 /
+// 20.4.  Rows of equal logits, which pay for the launches on top of sample_row, lose: 1 row 87 / 95, 256 rows 112 / 143.
 // The slot maxima and the parts' sums lie in `probs`.
 constexpr int kSlot = 64;
 constexpr int kPartEntries = 4096;

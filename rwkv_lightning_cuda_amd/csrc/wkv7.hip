@@ -308,8 +308,8 @@ __global__ __launch_bounds__(1024 / RPL / PARTS) void wkv7_seq_kernel(int T, int
 // a step's 350 clocks; fp16 operands now stay fp16 in LDS (the mixed-precision multiply-add takes them as they are): 104.  Many
 // heads: VALU issue, four clocks per instruction and SIMD; eight columns per lane put one of a row's four adds over lanes into the
 // lane (24 instead of 28 operations per four elements).  us per call, before / now:
-//   1 x 64 tokens x 12 heads, fp32 tensors 13.4 / 10.6   1 x 512 x 64, fp16 84.8 / 57   3 x 333 x 32 72 / 56
-//   4 x 256 x 64 83.7 / 70   8 x 256 x 64 125 / 113   16 x 256 x 64 223 / 213; fp32 tensors 82 / 71, 124 / 108, 238 / 219
+//   1 x 64 tokens x 12 heads, fp32 tensors 12.8 / 9.8   1 x 512 x 64, fp16 84 / 56   3 x 333 x 32 72 / 55
+//   4 x 256 x 64 83.7 / 70   8 x 256 x 64 125 / 113   16 x 256 x 64 221 / 210; fp32 tensors 82 / 71, 124 / 108, 238 / 219
 // The fp32 tile for more than 128 heads keeps six wavefronts per SIMD at the price of ten spilled registers: 128 tokens of 1024
 // heads 108 us; five 121, four 135 (512 heads 58.3, 56.9 and 57.2).
 template <typename E, int N>
