@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "head_ops.h"
 #include "ops.h"
 
 namespace rwkv {
@@ -578,68 +579,6 @@ int token_shift_mix_launch(hipStream_t st, const MixArgs& a) {
 // kk / a-gate of fewer than 12 heads per CU keeps one channel per lane: its chain of divisions and exponentials, four times as
 // long with four of them, is then all there is (kk_a_gate_few_kernel; us, back to back, four channels / one: 17 rows x 64 heads 2.24 / 2.05,
 // 64 x 32 2.30 / 2.14, 96 x 32 2.29 / 2.35, 128 x 64 2.84 / 3.26).
-//
-// The sums are those of a wavefront with one channel per lane (wave_sum: channel i adds what i ^ 32, 16, 8, 4, 2, 1 holds), so
-// that the kernels that do this inside a larger one agree bitwise: the first four levels are lane exchanges, the last two lie
-// within a lane.
-__device__ __forceinline__ float head_sum_tail(float (&t)[4]) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    t[e] += __builtin_bit_cast(float, lane_xor_dpp<4>(__builtin_bit_cast(int, t[e])));
-    t[e] = dpp_add<0x4E>(t[e]);  // lane ^ 2
-    t[e] = dpp_add<0xB1>(t[e]);  // lane ^ 1
-  }
-  return (t[0] + t[2]) + (t[1] + t[3]);
-}
-__device__ __forceinline__ float head_sum(const float (&v)[4]) {
-  float t[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) t[e] = dpp_add<0x128>(v[e]);  // lane ^ 8
-  return head_sum_tail(t);
-}
-// sum of a * b with a fused first level (wave_sum_dpp_of_product)
-__device__ __forceinline__ float head_sum_of_product(const float (&a)[4], const float (&b)[4]) {
-  float t[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float p;
-    {
-#pragma clang fp contract(off)
-      p = a[e] * b[e];
-    }
-    t[e] = fmaf(a[e], b[e], __builtin_bit_cast(float, lane_xor_dpp<8>(__builtin_bit_cast(int, p))));
-  }
-  return head_sum_tail(t);
-}
-// f16(a * b) of four values with one rounding each, what the compiler makes of a product that is only converted
-// (v_fma_mixlo_f16) where a lane has one channel; with four it would convert pairs, which rounds twice.
-__device__ __forceinline__ half4_t mul_f16(const float (&a)[4], const float (&b)[4]) {
-  uint2_t r;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    uint32_t d;
-    asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\tv_fma_mixhi_f16 %0, %3, %4, 0"
-        : "=&v"(d)
-        : "v"(a[2 * i]), "v"(b[2 * i]), "v"(a[2 * i + 1]), "v"(b[2 * i + 1]));
-    r[i] = d;
-  }
-  return __builtin_bit_cast(half4_t, r);
-}
-// four values at p; VEC: p is aligned to them
-template <bool VEC>
-__device__ __forceinline__ half4_t load4(const half_t* p) {
-  if constexpr (VEC) return *reinterpret_cast<const half4_t*>(p);
-  return half4_t{p[0], p[1], p[2], p[3]};
-}
-template <bool VEC>
-__device__ __forceinline__ void store4(half_t* p, half4_t v) {
-  if constexpr (VEC) {
-    *reinterpret_cast<half4_t*>(p) = v;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) p[e] = v[e];
-  }
-}
 
 template <bool VEC>
 __global__ __launch_bounds__(256) void kk_a_gate_kernel(KkArgs p) {
@@ -655,35 +594,17 @@ __global__ __launch_bounds__(256) void kk_a_gate_kernel(KkArgs p) {
     w4 = load4<VEC>(p.w12 + idx);
     w04 = load4<VEC>(p.w0 + c);
   }
-  float u[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) u[e] = h2f(k4[e]) * h2f(kk4[e]);
-  const float total = head_sum_of_product(u, u);
-  const float inv = 1.0f / fmaxf(sqrtf(total), kKkEps);
-  half4_t pkk, ws;
-  float4_t d;
-  float kv[4], kf[4], kk[4], av[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    kk[e] = u[e] * inv;
-    av[e] = sigmoid_f(h2f(a04[e]) + h2f(a4[e]));
-    const float ka = h2f(ka4[e]);
-    kv[e] = h2f(k4[e]);
-    kf[e] = fmaf(av[e], ka, 1.0f - ka);
-    pkk[e] = f2h(kk[e]);
-    ws[e] = f2h(h2f(w4[e]) + h2f(w04[e]));  // rwkv7_add_vec_launch rounding point
-  }
-  if (p.new_k) store4<VEC>(p.new_k + idx, mul_f16(kv, kf));
-  // (negated as halves: the compiler does not get a vector of negated floats through without packed fp32)
-  const uint2_t flipped = __builtin_bit_cast(uint2_t, pkk) ^ uint2_t{0x80008000u, 0x80008000u};
-  if (p.neg_kk) store4<VEC>(p.neg_kk + idx, __builtin_bit_cast(half4_t, flipped));
-  if (p.kka) store4<VEC>(p.kka + idx, mul_f16(kk, av));
+  const HeadGate o = head_gate(k4, a4, w4, kk4, a04, ka4, w04);
+  if (p.new_k) store4<VEC>(p.new_k + idx, o.new_k);
+  if (p.neg_kk) store4<VEC>(p.neg_kk + idx, o.neg_kk);
+  if (p.kka) store4<VEC>(p.kka + idx, o.kka);
   if (p.d32) {
+    float4_t d;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) d[e] = exp2f(-0.8750387749145276f / (1.0f + exp2f(-1.4426950408889634f * h2f(ws[e]))));
+    for (int e = 0; e < 4; ++e) d[e] = head_decay(o.w_sum[e]);
     *reinterpret_cast<float4_t*>(p.d32 + idx) = d;
   }
-  if (p.w_sum16) store4<VEC>(p.w_sum16 + idx, ws);
+  if (p.w_sum16) store4<VEC>(p.w_sum16 + idx, o.w_sum);
 }
 
 constexpr int kKkFewHeads = 12;  // per CU
@@ -750,26 +671,10 @@ __global__ __launch_bounds__(256) void lnx_rkvres_xg_kernel(int64_t rows_heads, 
   const half4_t y4 = load4<VEC>(y + idx), r4 = load4<VEC>(r + idx), k4 = load4<VEC>(k + idx), v4 = load4<VEC>(v + idx),
                 g4 = load4<VEC>(g + idx);
   const half4_t rk4 = load4<VEC>(r_k + c), lw4 = load4<VEC>(lnw + c), lb4 = load4<VEC>(lnb + c);
-  float yv[4], d[4], rk[4], w[4];
+  float yv[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) yv[e] = h2f(y4[e]);
-  const float mean = head_sum(yv) * (1.0f / 64.0f);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    d[e] = yv[e] - mean;
-    rk[e] = mul_f32(h2f(r4[e]), h2f(k4[e]));
-    w[e] = h2f(rk4[e]);
-  }
-  const float var = head_sum_of_product(d, d) * (1.0f / 64.0f);
-  const float rstd = rsqrtf(var + kLnxEps);
-  const float rkv = head_sum_of_product(rk, w);
-  float o[4], gate[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    o[e] = d[e] * rstd * h2f(lw4[e]) + h2f(lb4[e]) + rkv * h2f(v4[e]);
-    gate[e] = h2f(g4[e]);
-  }
-  store4<VEC>(out + idx, mul_f16(o, gate));
+  store4<VEC>(out + idx, head_output(yv, r4, k4, v4, g4, rk4, lw4, lb4));
 }
 
 // ---- small element-wise kernels ---------------------------------------------------------------------

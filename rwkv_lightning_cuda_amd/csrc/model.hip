@@ -127,6 +127,7 @@ struct Buffers {
       *kka, *y, *y2, *att, *x1, *ln2, *mixed, *act, *cm, *xf, *scratch, *shift_next;
   float* r32;  // one row: the output projection's input ahead of the gate
   float* d32;
+  unsigned char* chunk_ws;  // chunked recurrence: the chunks' operands
 };
 
 }  // namespace
@@ -157,6 +158,7 @@ struct rwkv_hip_session {
   size_t sparse_ws_bytes = 0;
   float* widened[4] = {};     // rwkv_hip_session_debug_buffer: fp32 copies of r, k2, nkk, kka, made when they are asked for
   size_t widened_cap[4] = {};
+  bool gate_missing = false;  // the last pass kept k2, nkk, kka and d32 to itself: debug_buffer makes them
   int sparse_ffn_rows = -1;   // decode steps of up to this many rows read only the ffn.value rows with a non-zero activation; -1: where it pays
                               // (2..4 rows share one walk over the rows that are non-zero for any of them)
   bool wkv_fp16 = false;      // the WKV state tensor is fp16 [L,B,H,64,64] (the reference's use_wkv32 == false)
@@ -264,6 +266,7 @@ size_t packed_workspace_bytes(const rwkv_hip_model* m, int B, int rows) {
 
 int ensure_arena(rwkv_hip_session* s, int B, int T) {
   const rwkv_hip_model* m = s->model;
+  s->gate_missing = false;
   const size_t rows = static_cast<size_t>(B) * T;
   if (s->arena.base && B <= s->arena_B && T <= s->arena_T && B * T <= s->arena_B * s->arena_T) {
     // shapes are laid out per call below, so only capacity matters
@@ -280,6 +283,7 @@ int ensure_arena(rwkv_hip_session* s, int B, int T) {
   add(RC, 2);                                         // scratch
   add(m->C, 4);                                       // r32
   add(RC, 4);                                         // d32
+  if (!s->wkv_fp16) add(tmix_chunk_workspace_bytes(B, T, m->H), 1);
   if (need > s->arena.cap) {
     // a larger shape invalidates captured graphs (they hold arena addresses)
     for (auto& g : s->graphs) {
@@ -316,6 +320,7 @@ int ensure_arena(rwkv_hip_session* s, int B, int T) {
     b.shift_next = a.take<half_t>(static_cast<size_t>(B) * m->C);
     b.r32 = a.take<float>(m->C);
     b.d32 = a.take<float>(RC);
+    b.chunk_ws = a.take<unsigned char>(0);  // the rest
     s->arena_B = B;
     s->arena_T = T;
   }
@@ -665,6 +670,10 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
         TRY_AUX(lora_out_multi(st, a));
       }
 
+      TmixSeqArgs fa;  // fp32 state
+      fa.r = b.r; fa.k = b.k; fa.a12 = b.a12; fa.w12 = b.w12; fa.g = b.g;
+      fa.k_k = w.t[RWKV_T_K_K]; fa.a0 = w.t[RWKV_T_A0]; fa.k_a = w.t[RWKV_T_K_A]; fa.w0 = w.t[RWKV_T_W0];
+      fa.r_k = w.t[RWKV_T_R_K]; fa.lnx_w = w.t[RWKV_T_LNX_W]; fa.lnx_b = w.t[RWKV_T_LNX_B];
       if (s->wkv_fp16) {
         // fp16 state (src/rwkv7_fast_v4.cu:1262-1271): kk / a-gate in fp16, the fp16 recurrence, GroupNorm / bonus / gate.
         // Calls of up to 16 tokens add w0 to the decay logit inside the recurrence, unrounded; longer ones round
@@ -694,12 +703,12 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
         TRY_AUX(lnx_launch(st, static_cast<int64_t>(rows) * H, H, b.y, b.r, b.k2, v_cur, w.t[RWKV_T_R_K], w.t[RWKV_T_LNX_W],
                            w.t[RWKV_T_LNX_B], b.g, b.y2));
         }
+      } else if (tmix_chunk_pays(B, T, H, fa)) {
+        // more than a few tokens: the same in chunks of 16 tokens on the matrix cores
+        TRY_AUX(tmix_chunk_launch(st, B, T, C, H, S, fa, v_cur, b.chunk_ws, b.k2, b.y, s->trace || B * H <= 128, b.y2));
+        s->gate_missing = true;
       } else if (!s->trace && tmix_seq_whole_heads(B, T, H)) {
         // kk normalise / a-gate / decay, the WKV recurrence and GroupNorm / bonus / gate in one launch
-        TmixSeqArgs fa;
-        fa.r = b.r; fa.k = b.k; fa.a12 = b.a12; fa.w12 = b.w12; fa.g = b.g;
-        fa.k_k = w.t[RWKV_T_K_K]; fa.a0 = w.t[RWKV_T_A0]; fa.k_a = w.t[RWKV_T_K_A]; fa.w0 = w.t[RWKV_T_W0];
-        fa.r_k = w.t[RWKV_T_R_K]; fa.lnx_w = w.t[RWKV_T_LNX_W]; fa.lnx_b = w.t[RWKV_T_LNX_B];
         TRY_AUX(tmix_seq_launch(st, B, T, C, H, S, fa, v_cur, b.y2));
       } else {
         // with the residual-stream tap on, or few heads in flight: the three stand-alone kernels (same arithmetic,
@@ -1221,6 +1230,19 @@ int rwkv_hip_session_debug_buffer(rwkv_hip_session* s, int id, void** ptr) {
                    b.att, b.x1,  b.ln2, b.mixed, b.act, b.cm, b.r32, b.d32, b.k2, b.nkk, b.kka};
   RWKV_REQUIRE(id >= 0 && id < static_cast<int>(sizeof(table) / sizeof(table[0])), "debug_buffer: unknown id %d", id);
   *ptr = table[id];
+  constexpr int kK2 = 19, kKka = 21, kD32 = 31;
+  if (s->gate_missing && (id >= kD32 || (id >= kK2 && id <= kKka))) {
+    // the chunked recurrence derives them as it goes
+    const Layer& w = s->model->layers.back();
+    KkArgs p = {};
+    p.k = b.k; p.k_k = w.t[RWKV_T_K_K]; p.a0 = w.t[RWKV_T_A0]; p.a12 = b.a12; p.k_a = w.t[RWKV_T_K_A];
+    p.new_k = b.k2; p.neg_kk = b.nkk; p.kka = b.kka;
+    p.w12 = b.w12; p.w0 = w.t[RWKV_T_W0]; p.d32 = b.d32;
+    p.rows_heads = static_cast<int64_t>(s->arena_B) * s->arena_T * s->model->H; p.H = s->model->H;
+    TRY(kk_a_gate_launch(s->stream, p));
+    RWKV_HIP_TRY(hipStreamSynchronize(s->stream));
+    s->gate_missing = false;
+  }
   // the recurrence reads its operands in fp16: their fp32 forms are made here
   constexpr int kR32 = 30, kK32 = 32;
   const size_t n = static_cast<size_t>(s->arena_B) * s->arena_T * s->model->C;

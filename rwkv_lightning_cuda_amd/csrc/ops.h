@@ -243,6 +243,13 @@ bool tmix_seq_whole_heads(int B, int T, int H);
 int wkv7_seq_f16_launch(hipStream_t st, int B, int T, int C, int H, float* state, const half_t* r, const float* d,
                         const half_t* k, const half_t* a, const half_t* b, const half_t* v, half_t* y);
 
+// ---- wkv7_chunk.hip: the same pass (fp32 state) in chunks of 16 tokens on the matrix cores, for calls of more than a few tokens ----
+bool tmix_chunk_pays(int B, int T, int H, const TmixSeqArgs& fa);
+size_t tmix_chunk_workspace_bytes(int B, int T, int H);  // (0 where none is needed)
+// new_k, y: written (y: if asked for) by calls of few heads or tokens on the way to y2; may be scratch
+int tmix_chunk_launch(hipStream_t st, int B, int T, int C, int H, float* state, const TmixSeqArgs& fa, const half_t* v, void* workspace,
+                      half_t* new_k, half_t* y, bool want_y, half_t* y2);
+
 // ---- wkv7_f16state.hip: the recurrence with an fp16 state (w raw decay logits, w0 [C] or NULL added unrounded) ----
 int wkv7_f16state_launch(hipStream_t st, int B, int T, int C, int H, half_t* state, const half_t* r, const half_t* w,
                          const half_t* w0, const half_t* k, const half_t* v, const half_t* a, const half_t* b, half_t* y,

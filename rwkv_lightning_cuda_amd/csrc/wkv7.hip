@@ -9,6 +9,7 @@
 // the lanes that share a row with DPP adds.  The staging converts what the caller has (raw decay logits or decays, or the
 // model's own fp16 rows) on the way into LDS.  Long calls: wkv7_feed_kernel; single tokens, short calls, very many heads and the
 // model's fused pass: wkv7_seq_kernel.  Every variant and every split of T over several calls gives bitwise the same result.
+// (A model's calls of more than a few tokens go in chunks of 16 instead: wkv7_chunk.hip.)
 #include <type_traits>
 #include "ops.h"
 

@@ -1,0 +1,730 @@
+// WKV7 time-mix recurrence of a model's prefill calls in chunks of 16 tokens on the matrix cores, fp32 state.
+//
+// Reference semantics: cuda/rwkv7_wkv_fp32_v2.cu:100-126, with the operands of cuda/rwkv7_fast_ops_fp16.cu (kk normalise, a-gate,
+// decay) and the per-head GroupNorm, bonus and gate behind it.  Per token (state S [value row i][key column j]):
+//   u = S a;  S = S diag(d) + u b^T + v k^T;  y = S r
+// Over a chunk with the running products P_t = d_1 .. d_t (per column) and
+//   A_t = a_t P_{t-1},  R_t = r_t P_t,  B_s = b_s / P_s,  K_s = k_s / P_s
+// the same sums are matrix products:
+//   U = S A^T + U [A B^T]_{s<t} + V [A K^T]_{s<t}        (u of every token; the middle term is a triangular solve)
+//   Y = S R^T + U [R B^T]_{s<=t} + V [R K^T]_{s<=t}
+//   S = (S + U^T B + V^T K) diag(P_16)
+// The solve is taken to the left side once per chunk, without the state: A' = (I - [A B^T])^-1 A and K' the same of [A K^T], so
+// that U = S A'^T + V K'.  The decay map keeps every d above 0.545, so 1 / P_16 stays below 2e4.
+//
+// Precision: nothing is held in less than fp32.  The products of decays and [A B^T], [A K^T] are summed in fp64 (v_mfma_f64_16x16x4),
+// U and Y in fp32 (v_mfma_f32_16x16x4, twice the rate of the vector unit), the update of the state as products of bf16 pieces that
+// add up to the fp32 operands exactly, summed in fp32.  Error of the state against 64-bit sums, 2-norm, chunks / token by token (operands
+// of independent channels and tokens, logits uniform over [-6, 2], state N(0, 1)): 128 tokens x 1024 heads 5.7e-8 / 5.7e-8, 512 x 64
+// 5.7e-8 / 5.7e-8, 2048 x 64 5.8e-8 / 5.7e-8, 333 x 96 5.9e-8 / 6.0e-8.
+//
+// A chunk is one unit: results depend on where a call begins (as those of a prefill call's products do, through their tiles), and a
+// value that is not finite reaches the other tokens of its chunk as well as, from then on, the state.  The operator rwkv_hip_wkv7
+// promises the same bits for every split of a sequence and steps token by token (wkv7.hip).
+//
+// us per layer from the rank-outs to the output projection's input, token by token -> in chunks: 16 x 128 tokens x 64 heads 166 ->
+// 93, 3 x 333 x 32 72 -> 51, 1 x 128 x 64 26.1 -> 22.7, 1 x 512 x 64 73 -> 49.  What bounds them: many heads, the issue of VALU
+// instructions (some 800 per wavefront and chunk) and the matrix core (2700 clocks), which add up although four wavefronts share a
+// SIMD; few heads, launches (three), the latency of one chunk's preparation (6 us) and 0.65 us per link of the chain, most of it LDS
+// and the requests for 31 KB per chunk and CU.
+#include <algorithm>
+
+#include "head_ops.h"
+#include "ops.h"
+
+namespace rwkv {
+
+namespace {
+
+constexpr int kTok = 16;     // tokens of a chunk
+constexpr int kRow = 68;     // floats from row to row of a [16][64] tile in LDS: 16-byte reads down a column touch every bank once
+constexpr int kSquare = 20;  // the same for [16][16]
+
+typedef double double4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
+
+// (LDS alone is exchanged over these barriers: requests to memory stay in flight)
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Lane (g, n) = (lane / 16, lane % 16) gives column g of A's row n and row g of B's column n (eight of each to the bf16 product); the
+// result's register i is row 4 g + i (fp64: 4 i + g) of column n.
+__device__ __forceinline__ float4_t mfma4(float a, float b, float4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ double4_t mfma4(double a, double b, double4_t c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ float4_t mfma32(uint4_t a, uint4_t b, float4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// x as the sum of three bf16 numbers (its 24 bits exactly), four values to two dwords per piece
+struct Pieces {
+  uint2_t p[3];
+};
+__device__ __forceinline__ Pieces split(const float4_t& x) {
+  Pieces o;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    float lo = x[2 * h], hi = x[2 * h + 1];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{lo, hi}, bf16x2_t));
+      o.p[i][h] = w;
+      if (i < 2) {
+        lo -= __builtin_bit_cast(float, w << 16);
+        hi -= __builtin_bit_cast(float, w & 0xffff0000u);
+      }
+    }
+  }
+  return o;
+}
+
+// Register e of the 16-lane row g <-> register g of row e, four sets at once.  (Two idle slots between a register's write and the swap
+// that reads it.)
+__device__ __forceinline__ void transpose4x4(uint4_t (&x)[4]) {
+#define RWKV_SWAPS(OP, I, J) OP " %" #I ", %" #J "\n\t"
+  asm volatile("s_nop 1\n\t"
+               RWKV_SWAPS("v_permlane32_swap_b32", 0, 2) RWKV_SWAPS("v_permlane32_swap_b32", 1, 3)
+               RWKV_SWAPS("v_permlane32_swap_b32", 4, 6) RWKV_SWAPS("v_permlane32_swap_b32", 5, 7)
+               RWKV_SWAPS("v_permlane32_swap_b32", 8, 10) RWKV_SWAPS("v_permlane32_swap_b32", 9, 11)
+               RWKV_SWAPS("v_permlane32_swap_b32", 12, 14) RWKV_SWAPS("v_permlane32_swap_b32", 13, 15)
+               "s_nop 1\n\t"
+               RWKV_SWAPS("v_permlane16_swap_b32", 0, 1) RWKV_SWAPS("v_permlane16_swap_b32", 2, 3)
+               RWKV_SWAPS("v_permlane16_swap_b32", 4, 5) RWKV_SWAPS("v_permlane16_swap_b32", 6, 7)
+               RWKV_SWAPS("v_permlane16_swap_b32", 8, 9) RWKV_SWAPS("v_permlane16_swap_b32", 10, 11)
+               RWKV_SWAPS("v_permlane16_swap_b32", 12, 13) RWKV_SWAPS("v_permlane16_swap_b32", 14, 15)
+               "s_nop 1"
+               : "+v"(x[0][0]), "+v"(x[0][1]), "+v"(x[0][2]), "+v"(x[0][3]), "+v"(x[1][0]), "+v"(x[1][1]), "+v"(x[1][2]), "+v"(x[1][3]),
+                 "+v"(x[2][0]), "+v"(x[2][1]), "+v"(x[2][2]), "+v"(x[2][3]), "+v"(x[3][0]), "+v"(x[3][1]), "+v"(x[3][2]), "+v"(x[3][3]));
+#undef RWKV_SWAPS
+}
+
+// num / den of normal numbers, rounded as the division is (but for its last step's scaling)
+__device__ __forceinline__ float quotient(float num, float den) {
+  float r = rcp_f(den);
+  r = fmaf(fmaf(-den, r, 1.0f), r, r);
+  const float q = num * r;
+  return fmaf(fmaf(-den, q, num), r, q);
+}
+__device__ __forceinline__ float decay_of(float w) {
+  const float e = __builtin_amdgcn_exp2f(-1.4426950408889634f * w);
+  return __builtin_amdgcn_exp2f(quotient(-0.8750387749145276f, 1.0f + (e > 1e30f ? 1e30f : e)));
+}
+
+struct ChannelConstants {
+  half4_t k_k, a0, k_a, w0;
+  __device__ __forceinline__ void load(const TmixSeqArgs& fa, int ch) {
+    k_k = *reinterpret_cast<const half4_t*>(fa.k_k + ch);
+    a0 = *reinterpret_cast<const half4_t*>(fa.a0 + ch);
+    k_a = *reinterpret_cast<const half4_t*>(fa.k_a + ch);
+    w0 = *reinterpret_cast<const half4_t*>(fa.w0 + ch);
+  }
+};
+struct ChunkRows {  // this lane's four channels of one token
+  half4_t r, k, a12, w12, v;
+  __device__ __forceinline__ void load(const TmixSeqArgs& fa, const half_t* v_in, int64_t at) {
+    r = *reinterpret_cast<const half4_t*>(fa.r + at);
+    k = *reinterpret_cast<const half4_t*>(fa.k + at);
+    a12 = *reinterpret_cast<const half4_t*>(fa.a12 + at);
+    w12 = *reinterpret_cast<const half4_t*>(fa.w12 + at);
+    v = *reinterpret_cast<const half4_t*>(v_in + at);
+  }
+};
+
+struct ChunkTiles {
+  float a[kTok][kRow];  // A, then A'
+  float r[kTok][kRow];
+  union {
+    float b[kTok][kRow];
+    float y[kTok][kRow];  // (the kernel for whole heads, when b has been used)
+  };
+  float k[kTok][kRow];
+  union {
+    struct {
+      float ab[kTok][kSquare];  // [s][t]
+      float ak[kTok][kSquare];  // [t][s], then K'
+    };
+    double part[4][kHead];      // products of the four decays of a wavefront: before ab is made
+  };
+  float rb[kTok][kSquare], rk[kTok][kSquare];  // [t][s]
+  float decay[kHead];                          // P_16
+};
+
+// Operands of the state update and V, as the matrix core reads them: lane (g, n) of tile q holds column 16 q + n of the tokens
+// 4 g .. 4 g + 3.
+struct UpdateOperands {
+  uint4_t kb[3][4][kWave];  // pieces of K P_16 (two dwords) and of B P_16
+  uint4_t v[4][kWave];      // V in two pieces (fp16 needs no more)
+};
+
+// kk normalise, a-gate, new k and decay of token 4 wave + g, channels 4 n .. 4 n + 3 (the formulas and rounding points of
+// kk_a_gate_kernel), then the rows of A, R, B, K and the operands of the update.  `live`: the token exists; one past the end of
+// the call leaves the state as it is.  Returns the new k.
+// The products of decays are in fp64, where every A, R, B, K is rounded once.  One barrier inside.
+__device__ __forceinline__ half4_t stage_operands(ChunkTiles& t, UpdateOperands& uo, const ChunkRows& q, const ChannelConstants& c, bool live,
+                                                  int wave, int lane) {
+  const int g = lane >> 4, n = lane & 15;
+  float u[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) u[e] = h2f(q.k[e]) * h2f(c.k_k[e]);
+  const float total = row16_sum((u[0] * u[0] + u[1] * u[1]) + (u[2] * u[2] + u[3] * u[3]));
+  const float inv = quotient(1.0f, fmaxf(sqrtf(total), kKkEps));
+  half4_t nk;
+  uint4_t x[4];  // this token's (new k, -kk), (kk a, r), (v, v), decay of four channels; then this channel's of four tokens
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float kk = u[e] * inv;
+    const float av = sigmoid_f(h2f(c.a0[e]) + h2f(q.a12[e]));
+    const float ka = h2f(c.k_a[e]);
+    nk[e] = f2h(h2f(q.k[e]) * fmaf(av, ka, 1.0f - ka));
+    x[0][e] = live ? __builtin_bit_cast(uint32_t, half2_t{nk[e], f2h(-kk)}) : 0u;
+    x[1][e] = live ? __builtin_bit_cast(uint32_t, half2_t{f2h(kk * av), q.r[e]}) : 0u;
+    x[2][e] = live ? __builtin_bit_cast(uint32_t, half2_t{q.v[e], q.v[e]}) : 0u;
+    x[3][e] = __builtin_bit_cast(uint32_t, live ? decay_of(round_h(h2f(q.w12[e]) + h2f(c.w0[e]))) : 1.0f);
+  }
+  transpose4x4(x);
+  const int col = 4 * n + g;  // tokens 4 wave .. 4 wave + 3 of it
+  double d[4], p[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    d[i] = static_cast<double>(__builtin_bit_cast(float, static_cast<uint32_t>(x[3][i])));
+    p[i] = i == 0 ? d[0] : p[i - 1] * d[i];
+  }
+  t.part[wave][col] = p[3];
+  lds_barrier();
+  double first = 1.0, after = 1.0;  // products over the wavefronts before and behind this one
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {  // (wave-uniform)
+    if (w < wave) first *= t.part[w][col];
+    if (w > wave) after *= t.part[w][col];
+  }
+  const double last = first * p[3];
+  if (wave == 3) t.decay[col] = static_cast<float>(last);
+  double over = __builtin_amdgcn_rcp(last);  // 1 / P_s, from the last token on down
+  over = fma(over, fma(-last, over, 1.0), over);
+  float4_t ub, uk, tv;
+#pragma unroll
+  for (int i = 3; i >= 0; --i) {
+    const half2_t k_a = as_half2(x[0][i]), b_r = as_half2(x[1][i]);
+    const double k = static_cast<double>(h2f(k_a[0])), a = static_cast<double>(h2f(k_a[1]));
+    const double b = static_cast<double>(h2f(b_r[0])), r = static_cast<double>(h2f(b_r[1]));
+    const int tok = 4 * wave + i;
+    t.r[tok][col] = static_cast<float>(r * (first * p[i]));
+    t.a[tok][col] = static_cast<float>(a * (i == 0 ? first : first * p[i - 1]));
+    t.b[tok][col] = static_cast<float>(b * over);
+    t.k[tok][col] = static_cast<float>(k * over);
+    ub[i] = static_cast<float>(b * after);  // P_16 / P_s
+    uk[i] = static_cast<float>(k * after);
+    tv[i] = h2f(as_half2(x[2][i])[0]);
+    over *= d[i];
+    after *= d[i];
+  }
+  const Pieces sk = split(uk), sb = split(ub), sv = split(tv);
+  const int tile = n >> 2, at = 16 * wave + 4 * (n & 3) + g;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) uo.kb[i][tile][at] = uint4_t{sk.p[i][0], sk.p[i][1], sb.p[i][0], sb.p[i][1]};
+  uo.v[tile][at] = uint4_t{sv.p[0][0], sv.p[0][1], sv.p[1][0], sv.p[1][1]};
+  return nk;
+}
+
+// The four products of tokens with tokens, one per wavefront: A B^T, A K^T (s < t), R B^T, R K^T (s <= t).  The first two go through
+// the solve into the state and are summed in fp64.
+__device__ __forceinline__ void token_products(ChunkTiles& t, int wave, int lane) {
+  const int g = lane >> 4, n = lane & 15;
+  if (wave < 2) {
+    const float(&y)[kTok][kRow] = wave ? t.k : t.b;
+    double4_t acc = {};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4_t xs = *reinterpret_cast<const float4_t*>(&t.a[n][16 * q + 4 * g]);
+      const float4_t ys = *reinterpret_cast<const float4_t*>(&y[n][16 * q + 4 * g]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc = mfma4(static_cast<double>(xs[i]), static_cast<double>(ys[i]), acc);
+    }
+    // lane (g, n), register i: token t = 4 i + g, token s = n
+    float* dst = wave == 0 ? &t.ab[n][g] : &t.ak[g][n];
+    const int step = wave == 0 ? 4 : 4 * kSquare;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dst[i * step] = 4 * i + g > n ? static_cast<float>(acc[i]) : 0.0f;
+  } else {
+    const float(&y)[kTok][kRow] = wave == 2 ? t.b : t.k;
+    float4_t acc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4_t xs = *reinterpret_cast<const float4_t*>(&t.r[n][16 * q + 4 * g]);
+      const float4_t ys = *reinterpret_cast<const float4_t*>(&y[n][16 * q + 4 * g]);
+      acc[q] = float4_t{};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[q] = mfma4(xs[i], ys[i], acc[q]);
+    }
+    float(&dst)[kTok][kSquare] = wave == 2 ? t.rb : t.rk;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)  // register i: token t = 4 g + i
+      dst[4 * g + i][n] = 4 * g + i >= n ? (acc[0][i] + acc[1][i]) + (acc[2][i] + acc[3][i]) : 0.0f;
+  }
+}
+
+// x[t] += m[s] of lane t of the row * x[s], for every t > s, s = S0 .. : the factor is read across the row by the multiply-add itself.
+// (The compiler makes a move and an add of this.  Two idle slots between a register's write and a read across lanes.)
+#define RWKV_STEP(T, S) "v_fmac_f32_dpp %[x" #T "], %[m" #S "], %[x" #S "] row_newbcast:" #T " row_mask:0xf bank_mask:0xf\n\t"
+#define RWKV_X(I) [x##I] "+v"(x[I])
+#define RWKV_M(I) [m##I] "v"(m[I])
+__device__ __forceinline__ void substitute(const float (&m)[kTok - 1], float (&x)[kTok]) {
+  asm volatile("s_nop 1\n\t"
+               RWKV_STEP(1, 0) RWKV_STEP(2, 0) RWKV_STEP(3, 0) RWKV_STEP(4, 0) RWKV_STEP(5, 0) RWKV_STEP(6, 0) RWKV_STEP(7, 0) RWKV_STEP(8, 0) RWKV_STEP(9, 0) RWKV_STEP(10, 0) RWKV_STEP(11, 0) RWKV_STEP(12, 0) RWKV_STEP(13, 0) RWKV_STEP(14, 0) RWKV_STEP(15, 0)
+               RWKV_STEP(2, 1) RWKV_STEP(3, 1) RWKV_STEP(4, 1) RWKV_STEP(5, 1) RWKV_STEP(6, 1) RWKV_STEP(7, 1) RWKV_STEP(8, 1) RWKV_STEP(9, 1) RWKV_STEP(10, 1) RWKV_STEP(11, 1) RWKV_STEP(12, 1) RWKV_STEP(13, 1) RWKV_STEP(14, 1) RWKV_STEP(15, 1)
+               RWKV_STEP(3, 2) RWKV_STEP(4, 2) RWKV_STEP(5, 2) RWKV_STEP(6, 2) RWKV_STEP(7, 2) RWKV_STEP(8, 2) RWKV_STEP(9, 2) RWKV_STEP(10, 2) RWKV_STEP(11, 2) RWKV_STEP(12, 2) RWKV_STEP(13, 2) RWKV_STEP(14, 2) RWKV_STEP(15, 2)
+               RWKV_STEP(4, 3) RWKV_STEP(5, 3) RWKV_STEP(6, 3) RWKV_STEP(7, 3) RWKV_STEP(8, 3) RWKV_STEP(9, 3) RWKV_STEP(10, 3) RWKV_STEP(11, 3) RWKV_STEP(12, 3) RWKV_STEP(13, 3) RWKV_STEP(14, 3) RWKV_STEP(15, 3)
+               RWKV_STEP(5, 4) RWKV_STEP(6, 4) RWKV_STEP(7, 4) RWKV_STEP(8, 4) RWKV_STEP(9, 4) RWKV_STEP(10, 4) RWKV_STEP(11, 4) RWKV_STEP(12, 4) RWKV_STEP(13, 4) RWKV_STEP(14, 4) RWKV_STEP(15, 4)
+               : RWKV_X(0), RWKV_X(1), RWKV_X(2), RWKV_X(3), RWKV_X(4), RWKV_X(5), RWKV_X(6), RWKV_X(7), RWKV_X(8), RWKV_X(9), RWKV_X(10), RWKV_X(11),
+                 RWKV_X(12), RWKV_X(13), RWKV_X(14), RWKV_X(15)
+               : RWKV_M(0), RWKV_M(1), RWKV_M(2), RWKV_M(3), RWKV_M(4));
+  asm volatile("s_nop 1\n\t"
+               RWKV_STEP(6, 5) RWKV_STEP(7, 5) RWKV_STEP(8, 5) RWKV_STEP(9, 5) RWKV_STEP(10, 5) RWKV_STEP(11, 5) RWKV_STEP(12, 5) RWKV_STEP(13, 5) RWKV_STEP(14, 5) RWKV_STEP(15, 5)
+               RWKV_STEP(7, 6) RWKV_STEP(8, 6) RWKV_STEP(9, 6) RWKV_STEP(10, 6) RWKV_STEP(11, 6) RWKV_STEP(12, 6) RWKV_STEP(13, 6) RWKV_STEP(14, 6) RWKV_STEP(15, 6)
+               RWKV_STEP(8, 7) RWKV_STEP(9, 7) RWKV_STEP(10, 7) RWKV_STEP(11, 7) RWKV_STEP(12, 7) RWKV_STEP(13, 7) RWKV_STEP(14, 7) RWKV_STEP(15, 7)
+               RWKV_STEP(9, 8) RWKV_STEP(10, 8) RWKV_STEP(11, 8) RWKV_STEP(12, 8) RWKV_STEP(13, 8) RWKV_STEP(14, 8) RWKV_STEP(15, 8)
+               RWKV_STEP(10, 9) RWKV_STEP(11, 9) RWKV_STEP(12, 9) RWKV_STEP(13, 9) RWKV_STEP(14, 9) RWKV_STEP(15, 9)
+               RWKV_STEP(11, 10) RWKV_STEP(12, 10) RWKV_STEP(13, 10) RWKV_STEP(14, 10) RWKV_STEP(15, 10)
+               RWKV_STEP(12, 11) RWKV_STEP(13, 11) RWKV_STEP(14, 11) RWKV_STEP(15, 11)
+               RWKV_STEP(13, 12) RWKV_STEP(14, 12) RWKV_STEP(15, 12)
+               RWKV_STEP(14, 13) RWKV_STEP(15, 13)
+               RWKV_STEP(15, 14)
+               : RWKV_X(5), RWKV_X(6), RWKV_X(7), RWKV_X(8), RWKV_X(9), RWKV_X(10), RWKV_X(11),
+                 RWKV_X(12), RWKV_X(13), RWKV_X(14), RWKV_X(15)
+               : RWKV_M(5), RWKV_M(6), RWKV_M(7), RWKV_M(8), RWKV_M(9), RWKV_M(10), RWKV_M(11), RWKV_M(12), RWKV_M(13), RWKV_M(14));
+}
+#undef RWKV_STEP
+#undef RWKV_X
+#undef RWKV_M
+// (I - [A B^T])^-1 from the left on A (wavefront 0, a column per lane) and on [A K^T] (wavefront 1, 16 of them): forward
+// substitution, the factors out of a row's lanes.
+__device__ __forceinline__ void solve(ChunkTiles& t, int wave, int lane) {
+  if (wave > 1) return;
+  float* col = wave == 0 ? &t.a[0][lane] : &t.ak[0][lane & 15];
+  const int stride = wave == 0 ? kRow : kSquare;
+  float m[kTok - 1], x[kTok];
+#pragma unroll
+  for (int s = 0; s < kTok - 1; ++s) m[s] = t.ab[s][lane & 15];
+#pragma unroll
+  for (int i = 0; i < kTok; ++i) x[i] = col[i * stride];
+  substitute(m, x);
+  if (wave == 0 || lane < 16) {
+#pragma unroll
+    for (int i = 1; i < kTok; ++i) col[i * stride] = x[i];
+  }
+}
+
+// S diag(P_16) + (K^T V + B^T U) P_16 of a tile of 16 columns: six products of the operands' bf16 pieces, all that are not below
+// the last bit of a fp32 product; the five small ones are summed apart.  (In fp64 the error is 4.6e-8 instead of 5.7e-8 and the
+// products take 540 clocks instead of 100.)
+__device__ __forceinline__ float4_t updated(const float4_t& S, const float4_t& p, const uint4_t (&kb)[3], const uint4_t& v, const Pieces& u) {
+  const uint4_t b0 = {v[0], v[1], u.p[0][0], u.p[0][1]};
+  const uint4_t b1 = {v[2], v[3], u.p[1][0], u.p[1][1]};
+  const uint4_t b2 = {0, 0, u.p[2][0], u.p[2][1]};
+  const float4_t big = mfma32(kb[0], b0, float4_t{});
+  float4_t small = mfma32(kb[2], b0, float4_t{});
+  small = mfma32(kb[0], b2, small);
+  small = mfma32(kb[1], b1, small);
+  small = mfma32(kb[1], b0, small);
+  small = mfma32(kb[0], b1, small);
+  float4_t r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = fmaf(S[i], p[i], big[i] + small[i]);
+  return r;
+}
+// V of four tokens out of its pieces (exact)
+__device__ __forceinline__ float4_t whole(const uint4_t& v) {
+  float4_t r;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    r[2 * h] = __builtin_bit_cast(float, v[h] << 16) + __builtin_bit_cast(float, v[2 + h] << 16);
+    r[2 * h + 1] = __builtin_bit_cast(float, v[h] & 0xffff0000u) + __builtin_bit_cast(float, v[2 + h] & 0xffff0000u);
+  }
+  return r;
+}
+__device__ __forceinline__ float4_t sum4(const float4_t& a, const float4_t& b, const float4_t& c, const float4_t& d) {
+  float4_t r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = (a[i] + b[i]) + (c[i] + d[i]);
+  return r;
+}
+
+// GroupNorm, bonus and gate (the formulas and rounding points of lnx_rkvres_xg_kernel)
+__device__ __forceinline__ half4_t normalised_output(const float (&y)[4], half4_t r, half4_t k, half4_t v, half4_t gate, half4_t r_k, half4_t w,
+                                                     half4_t b) {
+  const float mean = row16_sum((y[0] + y[1]) + (y[2] + y[3])) * (1.0f / 64.0f);
+  float d[4], rk[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    d[e] = y[e] - mean;
+    rk[e] = h2f(r[e]) * h2f(k[e]);
+  }
+  const float var = row16_sum((d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3])) * (1.0f / 64.0f);
+  const float rkv = row16_sum((rk[0] * h2f(r_k[0]) + rk[1] * h2f(r_k[1])) + (rk[2] * h2f(r_k[2]) + rk[3] * h2f(r_k[3])));
+  const float rstd = rsqrtf(var + kLnxEps);
+  half4_t o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = f2h((d[e] * rstd * h2f(w[e]) + h2f(b[e]) + rkv * h2f(v[e])) * h2f(gate[e]));
+  return o;
+}
+
+// ---- many heads: whole ones ----------------------------------------------------------------------------------------
+// One block per (sequence, head): wavefront w keeps the value rows 16 w .. 16 w + 15 of the state for the whole call, transposed,
+// as four 16 x 16 tiles (lane (g, n), tile q, register i: column j = 16 q + 4 g + i, row 16 w + n) - which is also how the matrix
+// core wants them as the right operand of S A'^T and S R^T, and how U leaves it and goes back in: the chain from chunk to chunk
+// touches no LDS.  Four blocks per CU (40 KB of LDS, 128 registers, a few spilled); the raised priority around the products is worth 4 %.
+__global__ __launch_bounds__(256, 4) void wkv7_chunk_kernel(int T, int C, int H, float* __restrict__ state, TmixSeqArgs fa,
+                                                            const half_t* __restrict__ v, half_t* __restrict__ y_tap,
+                                                            half_t* __restrict__ out) {
+  __shared__ __align__(16) ChunkTiles t;
+  __shared__ __align__(16) UpdateOperands uo;
+  __shared__ __align__(8) half4_t constants[7][16];  // of the head's channels: registers are what this kernel is short of
+  const int bh = blockIdx.x;
+  const int bi = bh / H, h = bh - bi * H;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const int tok = 4 * wave + g;
+  const int ch = h * kHead + 4 * n;
+  const int64_t base = static_cast<int64_t>(bi) * T * C + ch;
+
+  float* srow = state + (static_cast<int64_t>(bh) * kHead + 16 * wave + n) * kHead + 4 * g;
+  float4_t S[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) S[q] = __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(srow + 16 * q));
+
+  if (wave == 0 && g == 0) {
+    const half_t* const from[7] = {fa.k_k, fa.a0, fa.k_a, fa.w0, fa.r_k, fa.lnx_w, fa.lnx_b};
+#pragma unroll
+    for (int i = 0; i < 7; ++i) constants[i][n] = *reinterpret_cast<const half4_t*>(from[i] + ch);
+  }
+  lds_barrier();
+
+  ChunkRows next;
+  half4_t gate_next;
+  auto request = [&](int t0) {
+    const int64_t at = base + static_cast<int64_t>(min(t0 + tok, T - 1)) * C;
+    next.load(fa, v, at);
+    gate_next = *reinterpret_cast<const half4_t*>(fa.g + at);
+  };
+  request(0);
+  for (int t0 = 0; t0 < T; t0 += kTok) {
+    const half4_t r4 = next.r, v4 = next.v, gate4 = gate_next;
+    const bool live = t0 + tok < T;
+    const half4_t nk = stage_operands(t, uo, next, ChannelConstants{constants[0][n], constants[1][n], constants[2][n], constants[3][n]}, live, wave, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    request(t0 + kTok);
+    lds_barrier();
+    __builtin_amdgcn_s_setprio(1);
+    token_products(t, wave, lane);
+    __builtin_amdgcn_s_setprio(0);
+    lds_barrier();
+    solve(t, wave, lane);
+    lds_barrier();
+    __builtin_amdgcn_s_setprio(1);
+
+    // U, Y and the new state of this wavefront's 16 rows
+    const uint4_t vp = uo.v[wave][lane];
+    const float4_t V = whole(vp);
+    float4_t part[4];
+    {
+      const float4_t kp = *reinterpret_cast<const float4_t*>(&t.ak[n][4 * g]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4_t x = *reinterpret_cast<const float4_t*>(&t.a[n][16 * j + 4 * g]);
+        part[j] = mfma4(kp[j], V[j], float4_t{});
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[j] = mfma4(x[i], S[j][i], part[j]);
+      }
+    }
+    const float4_t U = sum4(part[0], part[1], part[2], part[3]);
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      const float4_t rb = *reinterpret_cast<const float4_t*>(&t.rb[n][4 * g]);
+      const float4_t rk = *reinterpret_cast<const float4_t*>(&t.rk[n][4 * g]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4_t x = *reinterpret_cast<const float4_t*>(&t.r[n][16 * j + 4 * g]);
+        part[j] = mfma4(rk[j], V[j], float4_t{});
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[j] = mfma4(x[i], S[j][i], part[j]);
+        part[j] = mfma4(rb[j], U[j], part[j]);
+      }
+      const float4_t y = sum4(part[0], part[1], part[2], part[3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) t.y[4 * g + i][16 * wave + n] = y[i];
+    }
+    const Pieces up = split(U);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      __builtin_amdgcn_sched_barrier(0);
+      const uint4_t kb[3] = {uo.kb[0][j][lane], uo.kb[1][j][lane], uo.kb[2][j][lane]};
+      S[j] = updated(S[j], *reinterpret_cast<const float4_t*>(&t.decay[16 * j + 4 * g]), kb, vp, up);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    lds_barrier();
+    const float4_t y4 = *reinterpret_cast<const float4_t*>(&t.y[tok][4 * n]);
+    const float yv[4] = {round_h(y4[0]), round_h(y4[1]), round_h(y4[2]), round_h(y4[3])};
+    const half4_t o4 = normalised_output(yv, r4, nk, v4, gate4, constants[4][n], constants[5][n], constants[6][n]);
+    if (live) {
+      const int64_t at = base + static_cast<int64_t>(t0 + tok) * C;
+      *reinterpret_cast<half4_t*>(out + at) = o4;
+      if (y_tap) *reinterpret_cast<half4_t*>(y_tap + at) = half4_t{f2h(yv[0]), f2h(yv[1]), f2h(yv[2]), f2h(yv[3])};
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) __builtin_nontemporal_store(S[q], reinterpret_cast<float4_t*>(srow + 16 * q));
+}
+
+// ---- few heads: the chunks first, all at once, then the chain over them ---------------------------------------------
+// What the chain needs of a chunk, in the order in which its lanes read it (lane (g, n), tile q of 16 columns).
+struct ChunkOperands {
+  UpdateOperands u;
+  float4_t a[4][kWave];  // A'[n][16 q + 4 g ..]
+  float4_t r[4][kWave];  // R[n][16 q + 4 g ..]
+  float kp[4][kWave];    // K'[n][4 g + q]
+  float rb[4][kWave];
+  float rk[4][kWave];
+  float decay[kHead];
+};
+
+// One block per (sequence, head, chunk).  Tokens t_begin .. t_end - 1 of a call of T.
+__global__ __launch_bounds__(256) void wkv7_chunk_prepare_kernel(int T, int C, int H, int t_begin, int t_end, int chunks, TmixSeqArgs fa,
+                                                                 const half_t* __restrict__ v, half_t* __restrict__ new_k,
+                                                                 ChunkOperands* __restrict__ ws) {
+  __shared__ __align__(16) ChunkTiles t;
+  const int bh = blockIdx.x / chunks, chunk = blockIdx.x - bh * chunks;
+  const int bi = bh / H, h = bh - bi * H;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const int ch = h * kHead + 4 * n;
+  const int token = t_begin + chunk * kTok + 4 * wave + g;
+  const bool live = token < t_end;
+  const int64_t at = (static_cast<int64_t>(bi) * T + min(token, t_end - 1)) * C + ch;
+  ChunkOperands& o = ws[blockIdx.x];
+  ChunkRows q;
+  q.load(fa, v, at);
+  ChannelConstants c;
+  c.load(fa, ch);
+  const half4_t nk = stage_operands(t, o.u, q, c, live, wave, lane);
+  if (live) *reinterpret_cast<half4_t*>(new_k + at) = nk;
+  lds_barrier();
+  token_products(t, wave, lane);
+  lds_barrier();
+  solve(t, wave, lane);
+  // what the solve leaves alone
+  o.r[wave][lane] = *reinterpret_cast<const float4_t*>(&t.r[n][16 * wave + 4 * g]);
+  o.rb[wave][lane] = t.rb[n][4 * g + wave];
+  o.rk[wave][lane] = t.rk[n][4 * g + wave];
+  if (wave == 3) o.decay[lane] = t.decay[lane];
+  lds_barrier();
+  o.a[wave][lane] = *reinterpret_cast<const float4_t*>(&t.a[n][16 * wave + 4 * g]);
+  o.kp[wave][lane] = t.ak[n][4 * g + wave];
+}
+
+// One block per (sequence, head, 16 RT value rows); the blocks of a head are eight apart, which puts them on one XCD and their
+// operands into its L2 once.  Wavefronts 0 .. 3 carry the state, a tile of 16 columns each: their shares of U meet in LDS, one
+// barrier per chunk.  Wavefronts 4 .. 7 make Y out of the states that those leave in LDS, a chunk behind.
+template <int RT>
+__global__ __launch_bounds__(512) void wkv7_chunk_chain_kernel(int heads, int T, int C, int H, int t_begin, int t_end, int chunks,
+                                                               float* __restrict__ state, const ChunkOperands* __restrict__ ws,
+                                                               const half_t* __restrict__ v, half_t* __restrict__ y) {
+  __shared__ float4_t u_part[2][RT][4][kWave], y_part[2][RT][4][kWave], s_tile[2][RT][4][kWave];
+  constexpr int kBlocks = 4 / RT;  // per head
+  const int bh = static_cast<int>(blockIdx.x / (8 * kBlocks) * 8 + (blockIdx.x & 7)), row0 = blockIdx.x / 8 % kBlocks * RT;
+  if (bh >= heads) return;
+  const int bi = bh / H, h = bh - bi * H;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int q = wave & 3;  // tile of columns
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const ChunkOperands* op = ws + static_cast<int64_t>(bh) * chunks;
+  auto pick = [&](const float4_t& x) { return q == 0 ? x[0] : (q == 1 ? x[1] : (q == 2 ? x[2] : x[3])); };
+  constexpr int kSets = 3;
+
+  if (wave < 4) {
+    float* srow = state + (static_cast<int64_t>(bh) * kHead + 16 * row0 + n) * kHead + 16 * q + 4 * g;
+    float4_t S[RT];
+#pragma unroll
+    for (int m = 0; m < RT; ++m) S[m] = *reinterpret_cast<const float4_t*>(srow + 16 * m * kHead);
+    struct Set {
+      float4_t a, p;
+      float kp;
+      uint4_t v[RT], kb[3];
+    };
+    Set set[kSets];
+    auto request = [&](Set& s, int c) {  // (chunks past the end repeat the last one)
+      const ChunkOperands& o = op[min(c, chunks - 1)];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) s.kb[i] = o.u.kb[i][q][lane];
+#pragma unroll
+      for (int m = 0; m < RT; ++m) s.v[m] = o.u.v[row0 + m][lane];
+      s.a = o.a[q][lane];
+      s.kp = o.kp[q][lane];
+      s.p = *reinterpret_cast<const float4_t*>(&o.decay[16 * q + 4 * g]);
+    };
+    // this tile's share of a chunk's U, and the state that the chunk begins with
+    auto begin = [&](const Set& s, int c) {
+      float4_t part[RT];
+#pragma unroll
+      for (int m = 0; m < RT; ++m) {
+        s_tile[c & 1][m][q][lane] = S[m];
+        part[m] = mfma4(s.kp, pick(whole(s.v[m])), float4_t{});
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int m = 0; m < RT; ++m) part[m] = mfma4(s.a[i], S[m][i], part[m]);
+#pragma unroll
+      for (int m = 0; m < RT; ++m) u_part[c & 1][m][q][lane] = part[m];
+      lds_barrier();
+    };
+    auto turn = [&](Set& s, const Set& next, int c) {
+      const int buf = c & 1;
+#pragma unroll
+      for (int m = 0; m < RT; ++m) {
+        const float4_t U = sum4(u_part[buf][m][0][lane], u_part[buf][m][1][lane], u_part[buf][m][2][lane], u_part[buf][m][3][lane]);
+        S[m] = updated(S[m], s.p, s.kb, s.v[m], split(U));
+      }
+      request(s, c + kSets);
+      begin(next, c + 1);  // (past the end: what the last turn leaves is not read)
+    };
+#pragma unroll
+    for (int i = 0; i < kSets; ++i) request(set[i], i);
+    begin(set[0], 0);
+    int c = 0;
+    for (; c + kSets <= chunks; c += kSets) {
+#pragma unroll
+      for (int u = 0; u < kSets; ++u) turn(set[u], set[(u + 1) % kSets], c + u);
+    }
+#pragma unroll
+    for (int u = 0; u < kSets - 1; ++u)
+      if (c + u < chunks) turn(set[u], set[u + 1], c + u);
+#pragma unroll
+    for (int m = 0; m < RT; ++m) *reinterpret_cast<float4_t*>(srow + 16 * m * kHead) = S[m];
+    return;
+  }
+
+  const int64_t base = (static_cast<int64_t>(bi) * T + t_begin) * C + h * kHead + 16 * row0 + n;
+  const int tokens = t_end - t_begin;
+  struct Set {
+    float4_t r;
+    float rb, rk;
+    half_t v[RT];
+  };
+  Set set[kSets];
+  auto request = [&](Set& s, int c) {
+    c = min(c, chunks - 1);
+    const ChunkOperands& o = op[c];
+    s.r = o.r[q][lane];
+    s.rb = o.rb[q][lane];
+    s.rk = o.rk[q][lane];
+#pragma unroll
+    for (int m = 0; m < RT; ++m) s.v[m] = v[base + static_cast<int64_t>(min(c * kTok + 4 * g + q, tokens - 1)) * C + 16 * m];
+  };
+  // wavefront 4 + q writes the tokens 4 g + q
+  auto write_out = [&](int c) {
+    const int token = c * kTok + 4 * g + q;
+#pragma unroll
+    for (int m = 0; m < RT; ++m) {
+      const float4_t(&part)[4][kWave] = y_part[c & 1][m];
+      const float yv = (part[0][lane][q] + part[1][lane][q]) + (part[2][lane][q] + part[3][lane][q]);
+      if (token < tokens) y[base + static_cast<int64_t>(token) * C + 16 * m] = f2h(yv);
+    }
+  };
+  auto turn = [&](Set& s, int c) {
+    const int buf = c & 1;
+#pragma unroll
+    for (int m = 0; m < RT; ++m) {
+      const float4_t(&up)[4][kWave] = u_part[buf][m];
+      const float u = (up[0][lane][q] + up[1][lane][q]) + (up[2][lane][q] + up[3][lane][q]);
+      const float4_t S = s_tile[buf][m][q][lane];
+      float4_t part = mfma4(s.rk, h2f(s.v[m]), float4_t{});
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part = mfma4(s.r[i], S[i], part);
+      y_part[buf][m][q][lane] = mfma4(s.rb, u, part);
+    }
+    request(s, c + kSets);
+    if (c > 0) write_out(c - 1);
+    lds_barrier();
+  };
+#pragma unroll
+  for (int i = 0; i < kSets; ++i) request(set[i], i);
+  lds_barrier();
+  int c = 0;
+  for (; c + kSets <= chunks; c += kSets) {
+#pragma unroll
+    for (int u = 0; u < kSets; ++u) turn(set[u], c + u);
+  }
+#pragma unroll
+  for (int u = 0; u < kSets - 1; ++u)
+    if (c + u < chunks) turn(set[u], c + u);
+  write_out(chunks - 1);
+}
+
+constexpr int kSegment = 512;  // tokens that are prepared at a time: bounds the workspace
+
+enum class ChunkPath { kNone, kWhole, kChain };
+
+// Which calls go in chunks, and how.  us per call with everything from the rank-outs to the output projection's input:
+//   heads x tokens             64 x 12   64 x 33   64 x 64   64 x 128  64 x 512  12 x 512  96 x 64  96 x 333  128 x 128
+//   three kernels (token by token)  9.6      12.7      16.4      26.1      73.4      62.1     21.3      72.2       37.5
+//   whole heads                     7.6      16.2      20.6      37.9     141        140      20.6       -         37.6
+//   chain                          10.3      14.0      15.5      22.7      48.6      36.0     20.4      50.8       30.7
+//   heads x tokens             256 x 8   256 x 16  256 x 17  256 x 128  512 x 64  1024 x 128  2048 x 64
+//   one fused kernel (t. by t.)     7.1      11.4      13.1      67.5       52.0      166        160
+//   whole heads                     8.0       8.1      12.6      39.0       33.0       92.9       95.3
+// A chunk costs the same with one token in it as with sixteen.  The chain needs three launches and pays from a few chunks on, as
+// long as there are CUs for the blocks of a head; with more heads the kernel for whole ones has work for every CU.
+ChunkPath chunk_path(int heads, int T) {
+  if (T < 10) return ChunkPath::kNone;
+  if (heads > 128 || T <= kTok) return ChunkPath::kWhole;
+  if (heads <= 64) return T >= 48 + heads / 4 ? ChunkPath::kChain : ChunkPath::kNone;
+  if (T >= 64) return ChunkPath::kChain;
+  return ceil_div(T, kTok) * kTok - T <= 6 ? ChunkPath::kWhole : ChunkPath::kNone;
+}
+constexpr int kNarrowHeads = 64;  // up to here a head's rows go to four blocks of the chain, which one round of CUs takes; then to two
+
+}  // namespace
+
+bool tmix_chunk_pays(int B, int T, int H, const TmixSeqArgs& fa) {
+  uintptr_t bits = 0;  // rows of four channels are read at once
+  for (const half_t* p : {fa.r, fa.k, fa.a12, fa.w12, fa.g, fa.k_k, fa.a0, fa.k_a, fa.w0, fa.r_k, fa.lnx_w, fa.lnx_b})
+    bits |= reinterpret_cast<uintptr_t>(p);
+  return bits % sizeof(half4_t) == 0 && chunk_path(B * H, T) != ChunkPath::kNone;
+}
+
+size_t tmix_chunk_workspace_bytes(int B, int T, int H) {
+  if (chunk_path(B * H, T) != ChunkPath::kChain) return 0;
+  return sizeof(ChunkOperands) * B * H * ceil_div(std::min(T, kSegment), kTok);
+}
+
+int tmix_chunk_launch(hipStream_t st, int B, int T, int C, int H, float* state, const TmixSeqArgs& fa, const half_t* v, void* workspace,
+                      half_t* new_k, half_t* y, bool want_y, half_t* y2) {
+  const int heads = B * H;
+  if (chunk_path(heads, T) == ChunkPath::kWhole) {
+    hipLaunchKernelGGL(wkv7_chunk_kernel, dim3(heads), dim3(256), 0, st, T, C, H, state, fa, v, want_y ? y : nullptr, y2);
+    RWKV_LAUNCH_CHECK();
+    return RWKV_OK;
+  }
+  RWKV_REQUIRE(workspace, "tmix_chunk: no workspace");
+  ChunkOperands* ws = static_cast<ChunkOperands*>(workspace);
+  for (int t0 = 0; t0 < T; t0 += kSegment) {
+    const int t1 = std::min(T, t0 + kSegment);
+    const int chunks = ceil_div(t1 - t0, kTok);
+    hipLaunchKernelGGL(wkv7_chunk_prepare_kernel, dim3(heads * chunks), dim3(256), 0, st, T, C, H, t0, t1, chunks, fa, v, new_k, ws);
+    RWKV_LAUNCH_CHECK();
+    const int eights = ceil_div(heads, 8) * 8;
+    if (heads <= kNarrowHeads)
+      hipLaunchKernelGGL(wkv7_chunk_chain_kernel<1>, dim3(eights * 4), dim3(512), 0, st, heads, T, C, H, t0, t1, chunks, state, ws, v, y);
+    else
+      hipLaunchKernelGGL(wkv7_chunk_chain_kernel<2>, dim3(eights * 2), dim3(512), 0, st, heads, T, C, H, t0, t1, chunks, state, ws, v, y);
+    RWKV_LAUNCH_CHECK();
+  }
+  return lnx_launch(st, static_cast<int64_t>(B) * T * H, H, y, fa.r, new_k, v, fa.r_k, fa.lnx_w, fa.lnx_b, fa.g, y2);
+}
+
+}  // namespace rwkv

@@ -431,6 +431,51 @@ def test_debug_buffers_of_the_recurrences_fp32_operands(gpu):
     sess.close()
 
 
+@pytest.mark.parametrize("H,B,T", [(8, 1, 10), (8, 1, 16), (8, 1, 50), (8, 1, 64), (8, 1, 65), (8, 1, 530), (5, 1, 97), (5, 15, 66),
+                                   (8, 9, 32), (8, 9, 79), (5, 26, 11), (8, 17, 33), (8, 17, 130), (8, 40, 17)])
+@pytest.mark.parametrize("slow", [False, True])
+def test_chunked_recurrence_matches_the_token_by_token_operator(gpu, H, B, T, slow):
+    """Prefill calls of more than a few tokens run the fp32-state recurrence in chunks of 16 tokens: few heads as a chain over prepared
+    chunks (up to 64 heads, up to 128, more than the 512 tokens that are prepared at once, heads that are no multiple of eight), many
+    heads or one chunk in a block per head, with whole and partial last chunks.  Against rwkv_hip_wkv7, which steps token by token, on
+    the operands that the call derived, from the same state.  fp32 sums in another order differ by some 1e-7; the operands may differ
+    where another order of the sum over a head's k moves one of them (4096 values and more) to the neighbouring fp16 number: 5e-4 of
+    one value, 1e-5 of a state that forgets slowly (`slow`: decays of 0.9 and more)."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    C = 64 * H
+    dims = ModelDims(L=1, C=C, H=H, F=4 * C, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
+    weights = synth_weights(dims, 6)
+    if slow:
+        weights["layers"][0]["w0"] = (weights["layers"][0]["w0"].astype(np.float32) - 4.0).astype(np.float16)
+    sess = Session(HipModel.from_host_weights(dims, weights, hip.FMT_W8))
+    rng = np.random.default_rng(B * T + H)
+    before = rng.standard_normal((1, B, H, 64, 64)).astype(np.float32)
+    st = State(dims, B)
+    st.wkv.upload(before)
+    sess.forward(rng.integers(0, dims.V, (B, T)), st, hip.DeviceArray((B, dims.V), np.float32))
+    shape = (B, T, C)
+    tap = {name: sess.debug_buffer(name, shape).astype(np.float32) for name in ("r", "k2", "nkk", "kka", "d32", "v_first", "g", "y2")}
+    state = hip.DeviceArray.from_numpy(before)
+    y = hip.DeviceArray(shape, np.float32)
+    hip.wkv7(B, T, C, H, hip.W_DECAY, hip.IO_F32, state,
+             *[hip.DeviceArray.from_numpy(tap[name]) for name in ("r", "d32", "k2", "v_first", "nkk", "kka")], y)
+    want = state.numpy().astype(np.float64)
+    got = st.wkv.numpy().astype(np.float64)
+    assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+    assert np.abs(got - want).max() <= 1e-3 * np.abs(want).max()
+    # GroupNorm, bonus and gate on the fp16-rounded y: a rounding of y that differs moves the output by some fp16 ulps
+    head = lambda x: x.reshape(B, T, H, 64).astype(np.float64)
+    layer = {n: weights["layers"][0][n].astype(np.float64).reshape(H, 64) for n in ("r_k", "lnx_w", "lnx_b")}
+    yh = head(y.numpy().astype(np.float16))
+    norm = (yh - yh.mean(-1, keepdims=True)) / np.sqrt(yh.var(-1, keepdims=True) + 64e-5) * layer["lnx_w"] + layer["lnx_b"]
+    bonus = (head(tap["r"]) * head(tap["k2"]) * layer["r_k"]).sum(-1, keepdims=True) * head(tap["v_first"])
+    out = ((norm + bonus) * head(tap["g"])).reshape(shape)
+    assert np.linalg.norm(tap["y2"] - out) <= 1e-3 * np.linalg.norm(out)
+    assert np.abs(tap["y2"] - out).max() <= 1e-2 * np.abs(out).max()
+    sess.close()
+
+
 def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
     """Without set_sparse_ffn a decode step walks the non-zero rows only where the matrix pays for the second launch: a
     small model gives the bits of the dense product, and those of the walk once it is asked for."""
