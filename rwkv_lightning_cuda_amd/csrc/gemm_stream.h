@@ -1,5 +1,6 @@
 // What the two files of the packed-weight GEMM share: the launch arguments and the exact expansion of int8 / int4 codes
-// to fp16 (gemm_stream.hip: packing, dispatch, split-K reduce and the wide tiles; gemm_ring.hip: the LDS-ring tiles).
+// to fp16 (gemm_stream.hip: packing, dispatch, split-K reduce and the 64 x 256 tile; gemm_ring.hip: the LDS-ring tiles; gemm_tile.hip: the
+// tiles of many rows).
 #pragma once
 
 #include "ops.h"
@@ -53,15 +54,20 @@ __device__ __forceinline__ half8_t make_half8(half2_t a, half2_t b, half2_t c, h
   return r;
 }
 
-// 8 int8 codes (two dwords) -> 8 fp16, exact: byte^0x80 under exponent 0x64 is 1024 + (code + 128).
+// 8 int8 codes (two dwords) -> 8 fp16, exact: a conversion per code that reads the byte and writes the half in place.  (Bytes under the exponent of
+// 1024, less the bias, take ten instructions; many rows of these products are bound by the chip's power: 16384 x 4096, 2048 rows, blocks of 256
+// x 256 252 us so, 245 with eight conversions.)
 __device__ __forceinline__ half8_t expand_w8(uint32_t d0, uint32_t d1) {
-  const half2_t bias = {static_cast<half_t>(1152.0f), static_cast<half_t>(1152.0f)};
-  d0 ^= 0x80808080u;
-  d1 ^= 0x80808080u;
-  return make_half8(as_half2(__builtin_amdgcn_perm(0x64646464u, d0, 0x04010400u)) - bias,
-                    as_half2(__builtin_amdgcn_perm(0x64646464u, d0, 0x04030402u)) - bias,
-                    as_half2(__builtin_amdgcn_perm(0x64646464u, d1, 0x04010400u)) - bias,
-                    as_half2(__builtin_amdgcn_perm(0x64646464u, d1, 0x04030402u)) - bias);
+  uint4_t r;
+#define RWKV_LOW(R, D, BYTE) "v_cvt_f16_i16_sdwa " R ", sext(" D ") dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:" BYTE "\n\t"
+#define RWKV_HIGH(R, D, BYTE) "v_cvt_f16_i16_sdwa " R ", sext(" D ") dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:" BYTE "\n\t"
+  asm(RWKV_LOW("%0", "%4", "BYTE_0") RWKV_LOW("%1", "%4", "BYTE_2") RWKV_LOW("%2", "%5", "BYTE_0") RWKV_LOW("%3", "%5", "BYTE_2")
+      RWKV_HIGH("%0", "%4", "BYTE_1") RWKV_HIGH("%1", "%4", "BYTE_3") RWKV_HIGH("%2", "%5", "BYTE_1") RWKV_HIGH("%3", "%5", "BYTE_3")
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+      : "v"(d0), "v"(d1));
+#undef RWKV_LOW
+#undef RWKV_HIGH
+  return __builtin_bit_cast(half8_t, r);
 }
 
 // 8 int4 codes (one dword, element 2i in the low nibble of byte i) minus the zero point -> 8 fp16, exact.
@@ -91,5 +97,7 @@ constexpr RingShape kRingShapes[] = {{1, 1, 2, 128}, {1, 1, 2, 256}, {2, 1, 2, 2
 // fmt: the format of the launch's problems; mixed: fp16 problems among them, with half as many columns per block
 bool gemm_ring_has(const RingShape& shape, int fmt, bool mixed);
 int gemm_ring_launch(hipStream_t st, const RingShape& shape, int fmt, bool mixed, const StreamArgs& g);
+// gemm_tile.hip: blocks of 128 or 256 rows x 256 columns for many rows; int8 and fp16 problems
+int gemm_tile_launch(hipStream_t st, int rows, const StreamArgs& g);
 
 }  // namespace rwkv

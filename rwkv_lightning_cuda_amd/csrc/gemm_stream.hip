@@ -14,9 +14,9 @@
 // to the matrix core after an exact in-register expansion of the codes, without any transpose or LDS
 // traffic for the weights; every weight byte leaves HBM once per 32*MT rows of X.
 //
-// Two kernels stream that order.  gemm_ring.hip: up to a few hundred rows (all rows for int4 codes), where the product is
-// bound by the weights' and X's way into the CUs.  Here: the wide tiles for more rows, bound by LDS and issue.  With more
-// than one K split each block writes an fp32 partial tile and a second small kernel sums the partials in split order (a
+// Three kernels stream that order.  gemm_ring.hip: up to a few hundred rows (all rows for int4 codes), where the product is
+// bound by the weights' and X's way into the CUs.  gemm_tile.hip: many rows, bound by the matrix core and the chip's power.  Here: a
+// 64 x 256 tile of int8 codes between the two.  With more than one K split each block writes an fp32 partial tile and a second small kernel sums the partials in split order (a
 // fixed order: results do not depend on scheduling) and applies scale and epilogue - or the LayerNorm kernel that consumes
 // the result does (DeferredReduce).
 #include <algorithm>
@@ -82,7 +82,7 @@ int pack_weights_launch(hipStream_t st, int fmt, int N, int K, const void* w, vo
 
 // ---- the GEMM ---------------------------------------------------------------------------------------------------------
 
-// The wide tile: 32 * MT rows, chunks of KC k, four wavefronts.
+// The 64 x 256 tile: 32 * MT rows, chunks of KC k, four wavefronts.
 template <int FMT, int MT, int KC>
 struct Tile {
   using P = PackTraits<FMT>;
@@ -147,30 +147,19 @@ struct WRegs {
   }
 };
 
-// ---- many rows: 128 rows x 256 columns per block, two bands per wavefront -------------------------------------------
-// From a few hundred rows on the product is bound by the matrix core and by LDS, not by the weights: with one band
-// per wavefront every MFMA needs its own 1 KiB X fragment from LDS, and LDS delivers 128 bytes per clock against
-// 32 clocks per MFMA and SIMD - four wavefronts saturate both at once.  Here a wavefront keeps two 32-column bands
-// (wave w: bands w and w + 4 of the block), so each X fragment feeds two MFMAs and a block reads X from L2 half as
-// often.  One group of four wavefronts, one wavefront per SIMD (128 accumulator registers per lane); int8 and
-// fp16 weights (the int4 path would double the accumulators once more and stays on the narrower tile).
-//
-// ROLL (int8 weights only): the variant that fits two wavefronts per SIMD (at most 256 registers).  Alone on its
-// SIMD a wavefront overlaps nothing - measured per 128-k chunk: 1.18 us of MFMAs, and on top of them, one after the
-// other, 0.2 us for the weight requests, 0.2 for the X requests and stores, 0.18 for the code expansion, 0.1 for
-// the LDS reads - so a second wavefront, whose MFMAs fill those gaps, is worth more than deep prefetch.  The
-// registers come from the weights: one set per band instead of a ring of sets, each piece requested again for the
-// next chunk right after its last use (six MFMA steps ahead), and from X: one set, requested during the first
-// half of a chunk's steps and stored during the second.
-template <int FMT, bool ROLL, int MT>
+// ---- some hundred rows of int8 weights: 64 rows x 256 columns per block, two bands per wavefront ----------------------
+// A wavefront keeps two 32-column bands (wave w: bands w and w + 4 of the block), so each X fragment it reads from LDS feeds two
+// MFMAs.  One weight set per band, each piece requested again for the next chunk right after its last use (six MFMA steps ahead),
+// and one set of X, requested during the first half of a chunk's steps and stored during the second: 166 registers, three
+// wavefronts per SIMD, whose MFMAs fill each other's gaps.
+template <int FMT, int MT>
 __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const StreamProblem& pr, int row_tile, int col_block,
                                                   int split, half_t* xs) {
-  static_assert(!ROLL || FMT == RWKV_FMT_W8, "the rolling weight set is laid out for int8 pieces (two MFMA steps each)");
+  static_assert(FMT == RWKV_FMT_W8, "the rolling weight set is laid out for int8 pieces (two MFMA steps each)");
   constexpr int KC = 128, NB = 2;
   using T = Tile<FMT, MT, KC>;
   using P = typename T::P;
   constexpr int BM = T::BM;
-  static_assert(FMT != RWKV_FMT_W4, "the wide tile takes int8 and fp16 weights");
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
@@ -208,7 +197,7 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
       for (int v = 0; v < 16; ++v) acc[nb][mt][v] = 0.0f;
 
   constexpr int NK = T::GROUPS * T::STEPS;        // MFMA steps of a chunk
-  if constexpr (ROLL) {
+  {
     WRegs<FMT, MT, KC> w[NB];
     XRegs<FMT, MT, KC> xq;
     const int last = nchunks - 1;
@@ -268,88 +257,7 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
       chunk(1, c0 + 1);
     }
     if (c0 < nchunks) chunk(0, c0);
-  } else {
-  constexpr int D = FMT == RWKV_FMT_F16 ? 2 : 3;  // weight register sets per band
-  constexpr int WPS = NB * T::NW / NK;            // weight pieces requested per MFMA step (1 int8, 2 fp16)
-  static_assert(T::XV == NK && NB * T::NW % NK == 0, "one X vector and a whole number of weight pieces per MFMA step");
-  static_assert(MT == 4, "the ring variant is the 128-row tile");
-  WRegs<FMT, MT, KC> wr[D][NB];
-  XRegs<FMT, MT, KC> xr[2];
-  const int last = nchunks - 1;
-  xr[0].request(g, pr, tid, m0, kbeg);
-  xr[1].request(g, pr, tid, m0, kbeg + min(1, last) * KC);
-#pragma unroll
-  for (int i = 0; i < D - 1; ++i)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) wr[i][nb].request(kbeg + min(i, last) * KC, wband[nb]);
-  xr[0].store_x(tid, xs);
-  __syncthreads();
-
-  // Chunk c out of LDS tile u & 1 with the weights of ring set u % D.  A wavefront is alone on its SIMD (its 128
-  // accumulator registers leave no room for a second one), so whatever it issues besides MFMAs leaves the matrix
-  // core idle: the memory work of a chunk is spread over its MFMA steps instead of standing in a block at its
-  // head - each step stores one vector of the next chunk's X (requested during the previous chunk) into the other
-  // tile, requests one vector of the X of the chunk after that into the register set just freed and WPS pieces of
-  // the weights D - 1 chunks ahead.  (Issued in one block, the 16 requests of a chunk took a wavefront 0.5 us of a
-  // 2.2 us chunk: four wavefronts queue for the one address unit of the CU.)
-  auto chunk = [&](int u, int c) {
-    const half_t* tile = xs + (u & 1) * T::kTileHalfs;
-    half_t* tile_next = xs + ((u + 1) & 1) * T::kTileHalfs;
-    const int kx = kbeg + (c + 2 <= last ? c + 2 : c) * KC;
-    const int kw = kbeg + (c + D - 1 <= last ? c + D - 1 : c) * KC;
-    const WRegs<FMT, MT, KC> (&w)[NB] = wr[u % D];
-    const half_t* xlane = tile + j * T::XSTRIDE + h * P::KR;
-    half8_t a[2][MT];
-    auto load_a = [&](int ks, half8_t (&dst)[MT]) {
-      const half_t* xa = xlane + (ks / T::STEPS) * T::G + 8 * (ks % T::STEPS);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) dst[mt] = *reinterpret_cast<const half8_t*>(xa + mt * 32 * T::XSTRIDE);
-    };
-    load_a(0, a[0]);
-#pragma unroll
-    for (int ks = 0; ks < NK; ++ks) {
-      const int gi = ks / T::STEPS;
-      const int st = ks % T::STEPS;
-      if (ks + 1 < NK) load_a(ks + 1, a[(ks + 1) & 1]);
-      xr[(u + 1) & 1].store_one(ks, tid, tile_next);
-      xr[u & 1].request_one(ks, g, pr, tid, m0, kx);
-#pragma unroll
-      for (int q = ks * WPS; q < (ks + 1) * WPS; ++q) wr[(u + D - 1) % D][q / T::NW].request_piece(q % T::NW, kw, wband[q / T::NW]);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        half8_t b;
-        if constexpr (FMT == RWKV_FMT_F16) {
-          b = __builtin_bit_cast(half8_t, w[nb].w[gi * 2 + st]);
-        } else {
-          const uint4_t piece = w[nb].w[gi];
-          b = st == 0 ? expand_w8(piece[0], piece[1]) : expand_w8(piece[2], piece[3]);
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[nb][mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks & 1][mt], b, acc[nb][mt], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __syncthreads();
-  };
-
-  constexpr int U = (D % 2 == 0) ? D : 2 * D;
-  // whole rounds of U chunks as one basic block (with exits between them the compiler waits for every load in flight at the
-  // head of each round), the chunks left over with exits
-  const int whole = nchunks - nchunks % U;
-  int c0 = 0;
-  for (; c0 < whole; c0 += U) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) chunk(u, c0 + u);
   }
-  if (c0 < nchunks) {
-#pragma unroll
-    for (int u = 0; u < U - 1; ++u) {
-      if (c0 + u >= nchunks) break;
-      chunk(u, c0 + u);
-    }
-  }
-  }  // !ROLL
 
   // output: one 128-column half of the tile at a time through LDS (the X tiles are free), written in 16/32-byte
   // pieces along the rows
@@ -397,10 +305,8 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
   }
 }
 
-// MIXED: the problems of the launch may be int8 or fp16 (one wavefront per SIMD); otherwise all are int8 and two
-// blocks share a CU.
-template <bool MIXED, int MT>
-__global__ __launch_bounds__(256, MIXED ? 1 : 2) void gemm_stream_wide_kernel(StreamArgs g) {
+__global__ __launch_bounds__(256, 2) void gemm_stream_wide_kernel(StreamArgs g) {
+  constexpr int MT = 2;
   __shared__ __align__(16) half_t xs[2 * 32 * MT * (128 + 8)];
   ride_along_copy(g.copy, gridDim.x, blockDim.x);
   const int id = blockIdx.x;
@@ -412,14 +318,7 @@ __global__ __launch_bounds__(256, MIXED ? 1 : 2) void gemm_stream_wide_kernel(St
   int pi = 0;
   while (pi + 1 < g.n_problems && col_all >= g.block_end[pi]) ++pi;
   const int col_block = col_all - (pi > 0 ? g.block_end[pi - 1] : 0);
-  const StreamProblem& pr = g.p[pi];
-  if constexpr (!MIXED) {
-    stream_block_wide<RWKV_FMT_W8, true, MT>(g, pr, row_tile, col_block, split, xs);
-  } else if (pr.fmt == RWKV_FMT_W8) {
-    stream_block_wide<RWKV_FMT_W8, false, MT>(g, pr, row_tile, col_block, split, xs);
-  } else {
-    stream_block_wide<RWKV_FMT_F16, false, MT>(g, pr, row_tile, col_block, split, xs);
-  }
+  stream_block_wide<RWKV_FMT_W8, MT>(g, g.p[pi], row_tile, col_block, split, xs);
 }
 
 // int4 scales and zero points by group: the 32 columns of a band then lie in one piece of 64 (32) bytes, where the rows of
@@ -500,14 +399,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(ReduceArgs g) {
 }
 
 struct StreamConfig {
-  RingShape ring = {0, 0, 0, 0};  // mt == 0: the wide tile
-  int wide_mt = 0;                // wide tile: 2 (64 x 256, int8 only) or 4 (128 x 256)
+  RingShape ring = {0, 0, 0, 0};  // mt == 0: another tile
+  int wide_rows = 0;              // of 256 columns: 64 (int8 only), 128 or 256 rows
   int fmt = RWKV_FMT_F16;         // ring: the launch's format
   bool mixed = false;             // ring: fp16 problems beside it
   int splits = 1;
   float us = 1e30f;               // estimate
   bool is_ring() const { return ring.mt > 0; }
-  int rows() const { return 32 * (is_ring() ? ring.mt : wide_mt); }
+  int rows() const { return is_ring() ? 32 * ring.mt : wide_rows; }
   int cols(int problem_fmt) const {
     if (!is_ring()) return 256;
     const int bn = 32 * ring.nb * ring.wp;
@@ -528,21 +427,25 @@ static int count_col_blocks(const StreamConfig& c, int n_problems, const int* Ns
 //   ring: a fixed part (launch, first stage, epilogue); the bytes of the busiest CU at what a CU takes in while all of them
 //   stream (94 GB/s; 130 while half of the chip idles); what of the HBM stream of the weights does not hide behind that; the
 //   products; per further round of blocks its start and end, which a second block hides where two fit a CU.
-//   wide: bound by the matrix core (1 PFLOP/s with the shader clock these products run at).
+//   wide (64 x 256; 128 x 256 without `tiles`): bound by the matrix core.
 //   K splits: their fp32 planes and, where no consumer sums them, the reduce launch; a consumer's block waits longer the more
 //   planes it asks for (0.15 us each; with 0 / 0.4 decode steps of 5 .. 16 rows are 1-4 % slower, 7.2B and 1.5B int8).
 //   int4 scales and zero points as [N][K/128] (group_rows): a cache line each per column and stage, of which the stage uses a few
 //   bytes.  Two bytes per code of what a CU takes in, 1.5 with stages of 256 k; up to 2048 k a column's lie in 48 bytes.
+//   tiles of 128 and 256 rows: a fixed part, then per stage of 64 k and round of blocks a time that grows with the blocks that run - the clock the chip
+//   holds goes down with them (190 launches of the presets' matrices at 256 .. 2048 rows, int8 and fp16: the pick takes 1.03 times the best one's
+//   time in geometric mean).  tiles == false keeps the estimate of the register-staged 128 x 256 tile that it replaced.
 static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred,
-                         bool group_rows) {
+                         bool group_rows, bool tiles) {
   constexpr int kCus = 256;
   const int bm = c.rows();
   int blocks = 0, bn_max = 0;
-  float block_bytes = 0.0f, w_bytes = 0.0f, n_total = 0.0f;
+  float block_bytes = 0.0f, w_bytes = 0.0f, n_total = 0.0f, f16_blocks = 0.0f;
   for (int i = 0; i < n_problems; ++i) {
     const int bn = c.cols(fmts[i]);
     const float per = fmts[i] == RWKV_FMT_F16 ? 2.0f : (fmts[i] == RWKV_FMT_W8 ? 1.0f : 0.55f);
     blocks += ceil_div(Ns[i], bn);
+    if (fmts[i] == RWKV_FMT_F16) f16_blocks += ceil_div(Ns[i], bn);
     const float lines = group_rows && K > 2048 && fmts[i] == RWKV_FMT_W4 ? (c.k_step() == 128 ? 2.0f : 1.5f) : 0.0f;
     block_bytes = std::max(block_bytes, bn * (per + lines) + bm * 2.0f);
     bn_max = std::max(bn_max, bn);
@@ -550,6 +453,7 @@ static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, co
     n_total += Ns[i];
   }
   const float k_block = static_cast<float>(K) / c.splits;
+  const float f16_share = f16_blocks / blocks;
   blocks *= c.splits;
   // (each eighth pair of column block and split goes to the same XCD, whose 32 CUs run all its row tiles: twelve pairs of 18
   // row tiles leave four XCDs with 36 blocks.  Launches of several problems have too many pairs for it to matter.)
@@ -569,8 +473,16 @@ static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, co
     const bool wide_ring = c.ring.mt == 4 || c.ring.wp == 4;
     us += rounds * gflop * (c.fmt == RWKV_FMT_W4 ? (wide_ring ? 0.73f : 0.57f) : (c.ring.mt == 4 && c.fmt == RWKV_FMT_W8 ? 0.55f : (c.ring.nb == 2 ? 0.37f : (c.ring.mt == 1 && c.ring.wp == 4 ? 0.30f : 0.28f))));
     us += (two_per_cu ? 1.5f : 4.5f) * (rounds - 1);
-  } else if (c.wide_mt == 2) {
+  } else if (c.wide_rows > 64 && tiles) {
+    auto round_us = [&](int running) {
+      const float stage = c.wide_rows == 256 ? 1.08f + 0.0027f * running + f16_share * (0.22f - 0.0006f * running) : 0.58f + 0.0013f * running;
+      return stage * k_block / 64.0f;
+    };
+    us = (c.wide_rows == 256 ? 10.0f : 11.0f) + full * round_us(kCus) + (rest > 0 ? round_us(rest) : 0.0f) +
+         (c.wide_rows == 256 ? 0.0f : 6.0f * (rounds - 1));
+  } else if (c.wide_rows == 64) {
     us = 7.0f + 34.0f * std::max(1.0f, blocks * 1.05f / kCus) * k_block / 4096.0f;
+    if (tiles) us *= 1.09f;  // (measured beside the tiles: 256 .. 1000 rows 5 to 13 % over the line above)
   } else {
     us = 6.0f + (full + (rest > 0 ? (full > 0 ? 0.75f + 0.25f * rest / kCus : 1.0f) : 0.0f)) * (11.0f + 58.0f * k_block / 4096.0f);
   }
@@ -587,17 +499,19 @@ static bool sums_at_consumer(int n_problems, int epilogue, int out_f32) {
 
 // Blocks that occupy the 256 CUs well enough without a K split.
 constexpr int kFilledBlocks = 200;
-// Rows from which the wide tiles, whose wavefronts feed two MFMAs from every X fragment they read from LDS, are looked at.
+// Rows from which the tiles of 256 columns, whose wavefronts feed two MFMAs from every X fragment they read from LDS, are looked at.
 constexpr int kWideMinRows = 160;
 
+// tiles: the blocks of 128 and 256 rows go by their own estimate.  Without, the choice - and with it the workspace that a call needs -
+// is what it was before them: the operator's for up to 512 rows, whose callers may rely on a product that needs no workspace.
 static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, bool group_rows,
-                                  int max_splits) {
+                                  int max_splits, bool tiles) {
   bool any[3] = {false, false, false};
   for (int i = 0; i < n_problems; ++i) any[fmts[i]] = true;
   StreamConfig best;
   auto consider = [&](StreamConfig c) {
     for (c.splits = 1; c.splits == 1 || (c.splits <= max_splits && K % (c.splits * c.k_step()) == 0); c.splits *= 2) {
-      c.us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred, group_rows);
+      c.us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred, group_rows, tiles);
       if (c.us < best.us) best = c;
     }
   };
@@ -611,12 +525,16 @@ static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, c
   }
   if (M >= kWideMinRows && !any[RWKV_FMT_W4]) {
     c.ring = RingShape{0, 0, 0, 0};
-    c.wide_mt = 4;
-    // (from 1025 rows on, with most of the chip busy, the wide tile is the faster one whatever the estimates' last percent)
-    if (M > 1024 && ceil_div(M, 128) * count_col_blocks(c, n_problems, Ns, fmts) >= kFilledBlocks) best.us = 1e30f;
+    c.wide_rows = 128;
+    // (from 1025 rows on, with most of the chip busy, the register-staged tile was the faster one whatever the estimates' last percent)
+    if (!tiles && M > 1024 && ceil_div(M, 128) * count_col_blocks(c, n_problems, Ns, fmts) >= kFilledBlocks) best.us = 1e30f;
     consider(c);
+    if (tiles) {
+      c.wide_rows = 256;
+      consider(c);
+    }
     if (!any[RWKV_FMT_F16] && K <= 4096 && M <= 1024) {
-      c.wide_mt = 2;
+      c.wide_rows = 64;
       consider(c);
     }
   }
@@ -627,7 +545,7 @@ static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, c
 // launch: each thread keeps the latest by all that they depend on (us per step, searching / kept: 1.5B shape fp16 4 rows
 // 1270 / 1236, int8 13 rows 1189 / 1158; 7.2B shape int8 8 rows 2239 / 2198; 0.1B shape fp16 8 rows 460 / 447).
 static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, bool group_rows,
-                                  int max_splits) {
+                                  int max_splits, bool tiles) {
   struct Entry {
     int key[5 + 2 * kMaxProblems];
     bool used;
@@ -636,7 +554,7 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
   constexpr unsigned kSets = 32, kWays = 4;
   static thread_local Entry table[kSets][kWays];
   static thread_local unsigned oldest[kSets];
-  int key[5 + 2 * kMaxProblems] = {M, K, n_problems, (deferred ? 1 : 0) + (group_rows ? 2 : 0), max_splits};
+  int key[5 + 2 * kMaxProblems] = {M, K, n_problems, (deferred ? 1 : 0) + (group_rows ? 2 : 0) + (tiles ? 4 : 0), max_splits};
   for (int i = 0; i < n_problems; ++i) {
     key[5 + 2 * i] = Ns[i];
     key[6 + 2 * i] = fmts[i];
@@ -648,17 +566,21 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
     if (e.used && memcmp(e.key, key, sizeof key) == 0) return e.config;
   Entry& e = table[set][oldest[set]];
   oldest[set] = (oldest[set] + 1) % kWays;
-  e.config = search_config(M, K, n_problems, Ns, fmts, deferred, group_rows, max_splits);
+  e.config = search_config(M, K, n_problems, Ns, fmts, deferred, group_rows, max_splits, tiles);
   memcpy(e.key, key, sizeof key);
   e.used = true;
   return e.config;
 }
 
-// The format is not known here: the largest that any of the choices would need.
+constexpr int kOperatorTileRows = 512;  // the operator goes by the tiles' estimate above them, where a K split is an offer (packed_launch)
+
+// The format is not known here: the largest that any of the choices would need, and never less than before the tiles had an estimate
+// of their own.
 size_t linear_packed_workspace_bytes(int M, int N, int K) {
   int splits = 1;
   for (const int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16})
-    splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, false, fmt == RWKV_FMT_W4, 32).splits);
+    for (const bool tiles : {false, M > kOperatorTileRows})
+      splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, false, fmt == RWKV_FMT_W4, 32, tiles).splits);
   return splits > 1 ? static_cast<size_t>(splits) * M * N * sizeof(float) : 0;
 }
 
@@ -690,7 +612,7 @@ size_t linear_packed_multi_workspace_bytes(int M, int K, int n_problems, const P
       fmts[i] = part[i].fmt;
       group_rows = group_rows || (fmts[i] == RWKV_FMT_W4 && !part[i].groups_first);
     }
-    const int splits = choose_config(M, K, n, Ns, fmts, sums_at_consumer(n, epilogue, out_f32), group_rows, 32).splits;
+    const int splits = choose_config(M, K, n, Ns, fmts, sums_at_consumer(n, epilogue, out_f32), group_rows, 32, true).splits;
     if (splits > 1) bytes = std::max(bytes, static_cast<size_t>(splits) * M * n_total * sizeof(float));
     return RWKV_OK;
   });
@@ -706,14 +628,14 @@ bool linear_packed_apart(int M, int K, int n_first, int n_problems, const Packed
     fmts[i] = problems[i].fmt;
     if (i < n_first && fmts[i] != RWKV_FMT_W8) return false;
   }
-  const float together = choose_config(M, K, n_problems, Ns, fmts, false, false, 32).us;
-  const float apart = choose_config(M, K, n_first, Ns, fmts, false, false, 32).us +
-                      choose_config(M, K, n_problems - n_first, Ns + n_first, fmts + n_first, false, false, 32).us;
+  const float together = choose_config(M, K, n_problems, Ns, fmts, false, false, 32, true).us;
+  const float apart = choose_config(M, K, n_first, Ns, fmts, false, false, 32, true).us +
+                      choose_config(M, K, n_problems - n_first, Ns + n_first, fmts + n_first, false, false, 32, true).us;
   return apart < 0.9f * together;
 }
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
-                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer,
+                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, bool tiles,
                          DeferredReduce* defer, const RowCopy* copy);
 
 static int require_supported(int M, int K, int n_problems, const PackedProblem* problems) {
@@ -731,14 +653,14 @@ int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const Pack
   return for_each_launch(n_problems, problems, [&](int n, const PackedProblem* part) {
     // (several problems take no more K splits than fit the workspace)
     const int rc = packed_launch(st, M, K, n, part, epilogue, out_f32, workspace, workspace_bytes, n_problems > 1,
-                                 sums_at_consumer(n, epilogue, out_f32), n == n_problems ? defer : nullptr, copy);
+                                 sums_at_consumer(n, epilogue, out_f32), true, n == n_problems ? defer : nullptr, copy);
     copy = nullptr;  // the rows ride on the first launch
     return rc;
   });
 }
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
-                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, DeferredReduce* defer,
+                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, bool tiles, DeferredReduce* defer,
                          const RowCopy* copy) {
   StreamArgs g;
   ReduceArgs r;
@@ -766,7 +688,7 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
   fit_splits = fit_splits || fmts[0] == RWKV_FMT_W4 || M > 512 || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 ||
                static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
   const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace ? workspace_bytes / plane : 0)) : 32;
-  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, max_splits);
+  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, max_splits, tiles);
   int col_blocks = 0;
   for (int i = 0; i < n_problems; ++i) {
     const PackedProblem& q = problems[i];
@@ -806,10 +728,11 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
   if (cfg.is_ring()) {
     const int rc = gemm_ring_launch(st, cfg.ring, cfg.fmt, cfg.mixed, g);
     if (rc != RWKV_OK) return rc;
+  } else if (cfg.wide_rows > 64) {
+    const int rc = gemm_tile_launch(st, cfg.wide_rows, g);
+    if (rc != RWKV_OK) return rc;
   } else {
-    const dim3 grid(g.row_tiles * ceil_div(col_blocks * g.splits, 8) * 8);
-    if (cfg.wide_mt == 2) hipLaunchKernelGGL((gemm_stream_wide_kernel<false, 2>), grid, dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((gemm_stream_wide_kernel<true, 4>), grid, dim3(256), 0, st, g);
+    hipLaunchKernelGGL(gemm_stream_wide_kernel, dim3(g.row_tiles * ceil_div(col_blocks * g.splits, 8) * 8), dim3(256), 0, st, g);
     RWKV_LAUNCH_CHECK();
   }
   if (defer) *defer = DeferredReduce{};
@@ -832,7 +755,8 @@ int linear_packed(hipStream_t st, int fmt, int M, int N, int K, const half_t* x,
                   const uint8_t* zp, int epilogue, int out_f32, void* y, void* workspace, size_t workspace_bytes) {
   const PackedProblem q = {packed, scale, zp, x, y, N, fmt};
   if (const int rc = require_supported(M, K, 1, &q)) return rc;
-  return packed_launch(st, M, K, 1, &q, epilogue, out_f32, workspace, workspace_bytes, false, false, nullptr, nullptr);
+  return packed_launch(st, M, K, 1, &q, epilogue, out_f32, workspace, workspace_bytes, false, false, M > kOperatorTileRows,
+                       nullptr, nullptr);
 }
 
 }  // namespace rwkv

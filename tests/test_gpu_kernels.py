@@ -1276,6 +1276,45 @@ def test_linear_packed_wide_tiles_with_a_k_split(gpu, orc, fmt_name, M, N, K):
     assert err <= F16_TOL
 
 
+@pytest.mark.parametrize("fmt_name,M,N,K", [("w8", 2049, 1696, 256), ("f16", 2049, 1696, 256), ("w8", 2049, 3136, 256), ("f16", 2049, 3136, 256),
+                                            ("w8", 1900, 3104, 768), ("f16", 2300, 3104, 768), ("w8", 2049, 832, 8192), ("w8", 2049, 1120, 4096),
+                                            ("w8", 2049, 544, 8192), ("f16", 1024, 8224, 512)])
+def test_linear_packed_tiles_of_many_rows(gpu, orc, fmt_name, M, N, K):
+    """Blocks of 128 and of 256 rows x 256 columns: as few stages as there are, a last row tile of one row and others, a last block of two
+    and more bands, two, four and eight splits of K; both epilogues and output types, rows on both sides of the tiles' edges against
+    the oracle."""
+    hip = gpu
+    rng = np.random.default_rng(M + N + K)
+    fmt = {"f16": hip.FMT_F16, "w8": hip.FMT_W8}[fmt_name]
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    parts = _quant_parts(orc, hip, fmt, (rng.standard_normal((N, K)) * 0.02).astype(np.float16))
+    dparts = [dev(hip, p) if p is not None else None for p in parts]
+    packed = hip.DeviceArray(parts[0].shape, parts[0].dtype)
+    hip.pack_weights(fmt, N, K, dparts[0], packed)
+    ws = hip.DeviceArray((max(hip.linear_packed_workspace(M, N, K), 16),), np.uint8)
+    rows = sorted({0, 1, 31, 32, 63, 64, 127, 128, 191, 255, 256, 511, M // 256 * 256 - 1, M - 2, M - 1})
+    want = orc.gemv(fmt, x[rows], parts[0], parts[1], parts[2]).astype(np.float32)
+    dx = dev(hip, x)
+    y = hip.DeviceArray((M + 1, N), np.float16)   # one row more: nothing may be stored past the last row
+    y.fill0()
+    hip.linear_packed(fmt, M, N, K, dx, packed, dparts[1], dparts[2], y, ws)
+    got = y.numpy()
+    err = rel_err(got[rows].astype(np.float32), want)
+    assert err <= F16_TOL
+    untouched = not got[M].any()
+    assert untouched
+    every = np.abs(got[:M].astype(np.float32)).max(axis=1)     # every row has been written
+    assert (every > 0).all()
+    y32 = hip.DeviceArray((M, N), np.float32)
+    hip.linear_packed(fmt, M, N, K, dx, packed, dparts[1], dparts[2], y32, ws, out_f32=1)
+    same = np.array_equal(y32.numpy().astype(np.float16), got[:M])
+    assert same
+    hip.linear_packed(fmt, M, N, K, dx, packed, dparts[1], dparts[2], y, ws, epilogue=hip.EPI_RELU_SQUARE)
+    relu = np.maximum(got[:M].astype(np.float32), 0)
+    same = np.array_equal(y.numpy()[:M], (relu * relu).astype(np.float16))
+    assert same
+
+
 @pytest.mark.parametrize("fmt_name", ["f16", "w8", "w4"])
 @pytest.mark.parametrize("M,N,K", [(8, 2048, 2048), (13, 4096, 4096), (33, 768, 3072), (129, 4096, 4096)])
 def test_linear_packed_gives_one_product_for_both_output_types(gpu, orc, fmt_name, M, N, K):
