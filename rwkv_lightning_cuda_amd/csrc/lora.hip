@@ -17,6 +17,7 @@
 // act(h) of a row tile staged in LDS; many rows take wider blocks (lora_out_wide_kernel).
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "ops.h"
 
@@ -182,6 +183,38 @@ __global__ __launch_bounds__(kLoraThreads) void lora_out_kernel(LoraOutMultiArgs
   if (orow < mn && ocol_ok) *reinterpret_cast<half8_t*>(p.out + o) = res;
 }
 
+// Eight values of the hidden, activated, as two fp16 terms; exact zeros where `live` is not set.
+template <int ACT>
+__device__ __forceinline__ void activate8(const uint4_t& raw, bool live, uint4_t& hi, uint4_t& lo) {
+  const half8_t x = __builtin_bit_cast(half8_t, raw);
+  half8_t h, l;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float f = h2f(x[e]);
+    if constexpr (ACT == RWKV_ACT_TANH) f = tanh_f(f);
+    if constexpr (ACT == RWKV_ACT_SIGMOID) f = sigmoid_f(f);
+    h[e] = f2h(f);
+    l[e] = f2h(f - h2f(h[e]));
+  }
+  hi = __builtin_bit_cast(uint4_t, h);
+  lo = __builtin_bit_cast(uint4_t, l);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    hi[e] = live ? hi[e] : 0u;
+    lo[e] = live ? lo[e] : 0u;
+  }
+}
+// The choice of the activation stands around a block's whole share of the hidden: asked per value it kept the exponentials and
+// reciprocals of a thread in line one behind the other (us of the four problems of a layer, weights out of HBM, per value / around: 4096
+// channels, 250 rows 11.5 / 10.9, 2048 rows 56.3 / 54.5; 2048 channels, 333 rows 8.5 / 8.0.  The small tile, whose threads hold 30 values
+// at most, gains nothing by it).
+template <typename Stage>
+__device__ __forceinline__ void with_activation(int act, Stage stage) {
+  if (act == RWKV_ACT_TANH) stage(std::integral_constant<int, RWKV_ACT_TANH>{});
+  else if (act == RWKV_ACT_SIGMOID) stage(std::integral_constant<int, RWKV_ACT_SIGMOID>{});
+  else stage(std::integral_constant<int, RWKV_ACT_NONE>{});
+}
+
 // The same products for many rows.  The kernel above evaluates the activation of a hidden value once per 128 output channels
 // and takes the sums through LDS and two barriers; this one takes 32 rows x 32*NW channels per block.  The weights are the
 // A operand: accumulator v of lane (j, h) is row j of the tile, and the channels are dealt to A's rows so that a lane's 16
@@ -237,28 +270,21 @@ __global__ __launch_bounds__(NW * 64) void lora_out_wide_kernel(LoraOutMultiArgs
     }
 #pragma unroll
     for (int u = 0; u < kDepth; ++u) w[u] = request(min(u, steps - 1));
+    with_activation(p.act, [&](auto act_c) {
+      constexpr int kAct = decltype(act_c)::value;
 #pragma unroll
-    for (int i = 0; i < kStage; ++i) {
-      if (i * kTpr * 8 <= R) {
-        const int ks = ks0 + i * kTpr * 8;
-        const bool live = row < mn && ks < R;  // rows past M and the pad hold exact zeros
-        const half8_t raw = __builtin_bit_cast(half8_t, hv[i]);
-        half8_t hi, lo;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          float f = h2f(raw[e]);
-          if (p.act == RWKV_ACT_TANH) f = tanh_f(f);
-          if (p.act == RWKV_ACT_SIGMOID) f = sigmoid_f(f);
-          if (!live) f = 0.0f;
-          hi[e] = f2h(f);
-          lo[e] = f2h(f - h2f(hi[e]));
-        }
-        if (ks <= R) {
-          *reinterpret_cast<half8_t*>(&hi_s[row * ld + ks]) = hi;
-          if (split) *reinterpret_cast<half8_t*>(&lo_s[row * ld + ks]) = lo;
+      for (int i = 0; i < kStage; ++i) {
+        if (i * kTpr * 8 <= R) {
+          const int ks = ks0 + i * kTpr * 8;
+          uint4_t hi, lo;
+          activate8<kAct>(hv[i], row < mn && ks < R, hi, lo);  // rows past M and the pad hold exact zeros
+          if (ks <= R) {
+            *reinterpret_cast<uint4_t*>(&hi_s[row * ld + ks]) = hi;
+            if constexpr (kAct != RWKV_ACT_NONE) *reinterpret_cast<uint4_t*>(&lo_s[row * ld + ks]) = lo;
+          }
         }
       }
-    }
+    });
   }
   __syncthreads();
   if (!busy) return;
@@ -307,12 +333,17 @@ __global__ __launch_bounds__(NW * 64) void lora_out_wide_kernel(LoraOutMultiArgs
   }
 }
 
-template <int NW>
-int lora_out_wide_launch(hipStream_t st, const LoraOutMultiArgs& a) {
-  // the longest problem first: its blocks would be the launch's tail otherwise
+// the longest problem first: its blocks would be the launch's tail otherwise
+static LoraOutMultiArgs longest_first(const LoraOutMultiArgs& a) {
   LoraOutMultiArgs o = a;
   const auto cost = [](const LoraOutProblem& p) { return p.R * (p.act != RWKV_ACT_NONE ? 2 : 1); };
   std::stable_sort(o.p, o.p + o.n, [&](const LoraOutProblem& x, const LoraOutProblem& y) { return cost(x) > cost(y); });
+  return o;
+}
+
+template <int NW>
+int lora_out_wide_launch(hipStream_t st, const LoraOutMultiArgs& a) {
+  const LoraOutMultiArgs o = longest_first(a);
   size_t lds = 0;
   for (int i = 0; i < o.n; ++i)
     lds = std::max(lds, static_cast<size_t>(kLoraRows) * (o.p[i].R + 8) * (o.p[i].act != RWKV_ACT_NONE ? 4 : 2));
@@ -389,10 +420,11 @@ int lora_out_multi(hipStream_t st, const LoraOutMultiArgs& a) {
     }
     return RWKV_OK;
   }
-  // Up to one and a half blocks per CU the small tile is the faster one (its rank is walked by two groups of wavefronts); past
-  // that, what the blocks repeat counts.  us of the four problems of a layer, small tile / 32 x 256: 4096 channels, 64 rows
-  // (256 blocks) 8.3 / 11.1, 128 (512) 12.0 / 10.7, 160 15.0 / 12.3, 256 20.0 / 13.2; 2048 channels, 128 rows (256) 6.9 / 7.2,
-  // 192 (384) 9.4 / 7.3, 256 (512) 9.8 / 8.2; 768 channels, 256 rows (192) 4.6 / 6.3.
+  // As long as all blocks of the small tile are on the chip at once, two per CU, it is the faster one (its rank is walked by two groups
+  // of wavefronts, all weights of which are requested at once); past that, what the blocks repeat counts.  us of the four problems of a
+  // layer, weights out of HBM, small tile / 32 x 256: 4096 channels, 64 rows (256 blocks) 8.0 / 11.2, 96 (384) 8.7 / 11.3, 125 (512) 9.0 /
+  // 11.3, 192 (768) 12.1 / 11.9; 2560 channels, 190 rows (480) 6.9 / 8.3; 2048 channels, 256 rows (512) 6.3 / 7.4, 333 (704) 9.3 / 8.0; 768
+  // channels, 512 rows (384) 5.5 / 5.8, 768 (576) 7.3 / 6.9.
   const int row_tiles = ceil_div(a.M, kLoraRows);
   const int64_t cus = device_cu_count();
   const int64_t small = static_cast<int64_t>(ceil_div(a.C, kLoraCols)) * row_tiles * a.n;
@@ -402,7 +434,7 @@ int lora_out_multi(hipStream_t st, const LoraOutMultiArgs& a) {
   // 12.2 / 15.1; rank 480 with one 11.6 / 11.7, 15.5 / 16.7, 19.6 / 19.3, 23.2 / 24.9; rank 96 with one, 700 rows 8.5 / 7.5.
   const int64_t wide8 = static_cast<int64_t>(ceil_div(a.C, 256)) * row_tiles;
   const bool uneven = a.n == 1 && a.p[0].R >= 128 && 2 * ((wide8 + cus - 1) / cus) > (small + cus - 1) / cus;
-  if (small * 2 > 3 * cus) {
+  if (a.n == 1 ? small * 2 > 3 * cus : small > 2 * cus) {
     // twice as many channels per block where that still leaves two blocks per CU and no channel of a block unused: 32 x 256 / 32 x
     // 512 at 4096 channels and 500 rows 21.4 / 19.2, 1000 39.0 / 37.4, 2048 68.4 / 57.9; 2048 channels and 999 rows 17.9 / 13.1, 2048
     // 29.2 / 28.7 (before, with the small tile's blocks walking several row tiles: 33.7, 60.5, 107.6; 26.5, 50.1)
@@ -410,7 +442,9 @@ int lora_out_multi(hipStream_t st, const LoraOutMultiArgs& a) {
     if (wide) return lora_out_wide_launch<16>(st, a);
     if (!uneven) return lora_out_wide_launch<8>(st, a);
   }
-  hipLaunchKernelGGL(lora_out_kernel, dim3(ceil_div(a.C, kLoraCols), row_tiles, a.n), dim3(kLoraThreads), 0, st, a);
+  // (with fewer blocks the last ones would share a CU with the first, the longest)
+  const LoraOutMultiArgs o = 2 * small >= 3 * cus ? longest_first(a) : a;
+  hipLaunchKernelGGL(lora_out_kernel, dim3(ceil_div(o.C, kLoraCols), row_tiles, o.n), dim3(kLoraThreads), 0, st, o);
   RWKV_LAUNCH_CHECK();
   return RWKV_OK;
 }
