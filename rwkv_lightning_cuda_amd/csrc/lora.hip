@@ -32,6 +32,37 @@ constexpr int kLoraKG = 2;       // wavefront groups that split the rank between
 constexpr int kLoraThreads = 2 * kLoraCols * kLoraKG;
 constexpr int kLoraStage = (kLoraRows * (kLoraMaxR / 8 + 1) + kLoraThreads - 1) / kLoraThreads;  // pieces per thread
 
+// Eight values of the hidden, activated, as two fp16 terms; exact zeros where `live` is not set.
+template <int ACT>
+__device__ __forceinline__ void activate8(const uint4_t& raw, bool live, uint4_t& hi, uint4_t& lo) {
+  const half8_t x = __builtin_bit_cast(half8_t, raw);
+  half8_t h, l;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float f = h2f(x[e]);
+    if constexpr (ACT == RWKV_ACT_TANH) f = tanh_f(f);
+    if constexpr (ACT == RWKV_ACT_SIGMOID) f = sigmoid_f(f);
+    h[e] = f2h(f);
+    l[e] = f2h(f - h2f(h[e]));
+  }
+  hi = __builtin_bit_cast(uint4_t, h);
+  lo = __builtin_bit_cast(uint4_t, l);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    hi[e] = live ? hi[e] : 0u;
+    lo[e] = live ? lo[e] : 0u;
+  }
+}
+// The choice of the activation stands around eight values or more: asked per value it kept the exponentials and reciprocals of a thread
+// in line one behind the other (us of the four problems of a layer, weights out of HBM, per value / around: 4096 channels, 250 rows 11.5 /
+// 10.9, 2048 rows 56.3 / 54.5; 2048 channels, 333 rows 8.5 / 8.0, 192 rows 6.0 / 5.5).
+template <typename Stage>
+__device__ __forceinline__ void with_activation(int act, Stage stage) {
+  if (act == RWKV_ACT_TANH) stage(std::integral_constant<int, RWKV_ACT_TANH>{});
+  else if (act == RWKV_ACT_SIGMOID) stage(std::integral_constant<int, RWKV_ACT_SIGMOID>{});
+  else stage(std::integral_constant<int, RWKV_ACT_NONE>{});
+}
+
 // Every lane requests its whole weight row (up to 16 pieces of 8), its pieces of the 32 x R hidden slice and its
 // piece of the epilogue operands (v, v_first) in one go; the block turns the hidden slice into hi / lo fp16 in LDS (one barrier), each
 // wavefront runs its MFMA steps, both groups lay their 32 x 128 sums out in LDS (over the hi / lo tiles, free by
@@ -88,17 +119,23 @@ __global__ __launch_bounds__(kLoraThreads) void lora_out_kernel(LoraOutMultiArgs
   // without a bias any readable address does (C values of W2); the values are dropped in the epilogue
   uint4_t bias_raw = *reinterpret_cast<const uint4_t*>((p.bias ? p.bias : p.w2) + (ocol_ok ? ocol : 0));
 
-  const int pieces = (R >> 3) + 1;  // R/8 pieces of 8 per row + the zeroed pad
   const int m0 = blockIdx.y * kLoraRows;
   const int mn = min(kLoraRows, a.M - m0);
-  uint4_t hv[kLoraStage];  // all of them loaded, whatever the rank: a value left undefined costs more than the load
+  // As many threads per row as the rows (their power of two) leave, so that few rows take one turn of the threads and none is spent on
+  // the pad.  Rows that do not exist are not staged: what lies there meets rows of the product that are not stored.  (us of the four
+  // problems, all 32 rows staged piece by piece / this: 4096 channels, 8 rows 7.5 / 6.2, 64 rows 7.9 / 7.8, 125 rows 8.8 / 8.4; 2048
+  // channels, 13 rows 5.0 / 4.2, 128 rows 5.4 / 5.0; 768 channels, 50 rows 4.3 / 3.8.  Of the 6.5 us of a rank-480 gate alone at 32 rows
+  // two are activations, which every 128 channels make again.)
+  const int tpr_log = 9 - (mn > 1 ? 32 - __builtin_clz(mn - 1) : 0);
+  static_assert(kLoraThreads == 512, "threads per row");
+  const int hrow = threadIdx.x >> tpr_log;
+  const int ks0 = (threadIdx.x & ((1 << tpr_log) - 1)) * 8;
+  const half_t* hsrc = p.h + static_cast<int64_t>(m0 + (hrow < mn ? hrow : mn - 1)) * R;
+  uint4_t hv[kLoraStage];
 #pragma unroll
   for (int i = 0; i < kLoraStage; ++i) {
-    const int idx = threadIdx.x + i * kLoraThreads;
-    const int m = idx / pieces;
-    const int ks = (idx - m * pieces) * 8;
-    hv[i] = *reinterpret_cast<const uint4_t*>(p.h + static_cast<int64_t>(m0 + (m < mn ? m : mn - 1)) * R +
-                                              (ks < R ? ks : R - 8));
+    const int ks = ks0 + ((i * 8) << tpr_log);
+    if ((i * 8) << tpr_log < R) hv[i] = *reinterpret_cast<const uint4_t*>(hsrc + (ks < R ? ks : R - 8));
   }
   const int64_t o = static_cast<int64_t>(m0 + (orow < mn ? orow : mn - 1)) * a.C + (ocol_ok ? ocol : 0);
   // without the v-residual gate: the output row itself, readable and unused
@@ -112,27 +149,19 @@ __global__ __launch_bounds__(kLoraThreads) void lora_out_kernel(LoraOutMultiArgs
 
 #pragma unroll
   for (int i = 0; i < kLoraStage; ++i) {
-    if (i * kLoraThreads < kLoraRows * pieces) {
-      const int idx = threadIdx.x + i * kLoraThreads;
-      const int m = idx / pieces;
-      const int ks = (idx - m * pieces) * 8;
-      if (m < kLoraRows) {
-        const bool live = m < mn && ks < R;  // rows past M and the pad hold exact zeros
-        const half8_t raw = __builtin_bit_cast(half8_t, hv[i]);
-        half8_t hi, lo;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          float f = h2f(raw[e]);
-          if (p.act == RWKV_ACT_TANH) f = tanh_f(f);
-          if (p.act == RWKV_ACT_SIGMOID) f = sigmoid_f(f);
-          if (!live) f = 0.0f;
-          hi[e] = f2h(f);
-          lo[e] = f2h(f - h2f(hi[e]));
-        }
-        *reinterpret_cast<half8_t*>(&hi_s[m * ld + ks]) = hi;
-        if (split) *reinterpret_cast<half8_t*>(&lo_s[m * ld + ks]) = lo;
+    if ((i * 8) << tpr_log < R) {
+      const int ks = ks0 + ((i * 8) << tpr_log);
+      uint4_t hi, lo;
+      with_activation(p.act, [&](auto act_c) { activate8<decltype(act_c)::value>(hv[i], true, hi, lo); });
+      if (ks < R) {
+        *reinterpret_cast<uint4_t*>(&hi_s[hrow * ld + ks]) = hi;
+        if (split) *reinterpret_cast<uint4_t*>(&lo_s[hrow * ld + ks]) = lo;
       }
     }
+  }
+  if (ks0 == 0) {  // the pad holds exact zeros
+    *reinterpret_cast<half8_t*>(&hi_s[hrow * ld + R]) = half8_t{};
+    if (split) *reinterpret_cast<half8_t*>(&lo_s[hrow * ld + R]) = half8_t{};
   }
   __syncthreads();
 
@@ -181,38 +210,6 @@ __global__ __launch_bounds__(kLoraThreads) void lora_out_kernel(LoraOutMultiArgs
     }
   }
   if (orow < mn && ocol_ok) *reinterpret_cast<half8_t*>(p.out + o) = res;
-}
-
-// Eight values of the hidden, activated, as two fp16 terms; exact zeros where `live` is not set.
-template <int ACT>
-__device__ __forceinline__ void activate8(const uint4_t& raw, bool live, uint4_t& hi, uint4_t& lo) {
-  const half8_t x = __builtin_bit_cast(half8_t, raw);
-  half8_t h, l;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    float f = h2f(x[e]);
-    if constexpr (ACT == RWKV_ACT_TANH) f = tanh_f(f);
-    if constexpr (ACT == RWKV_ACT_SIGMOID) f = sigmoid_f(f);
-    h[e] = f2h(f);
-    l[e] = f2h(f - h2f(h[e]));
-  }
-  hi = __builtin_bit_cast(uint4_t, h);
-  lo = __builtin_bit_cast(uint4_t, l);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    hi[e] = live ? hi[e] : 0u;
-    lo[e] = live ? lo[e] : 0u;
-  }
-}
-// The choice of the activation stands around a block's whole share of the hidden: asked per value it kept the exponentials and
-// reciprocals of a thread in line one behind the other (us of the four problems of a layer, weights out of HBM, per value / around: 4096
-// channels, 250 rows 11.5 / 10.9, 2048 rows 56.3 / 54.5; 2048 channels, 333 rows 8.5 / 8.0.  The small tile, whose threads hold 30 values
-// at most, gains nothing by it).
-template <typename Stage>
-__device__ __forceinline__ void with_activation(int act, Stage stage) {
-  if (act == RWKV_ACT_TANH) stage(std::integral_constant<int, RWKV_ACT_TANH>{});
-  else if (act == RWKV_ACT_SIGMOID) stage(std::integral_constant<int, RWKV_ACT_SIGMOID>{});
-  else stage(std::integral_constant<int, RWKV_ACT_NONE>{});
 }
 
 // The same products for many rows.  The kernel above evaluates the activation of a hidden value once per 128 output channels
@@ -422,9 +419,9 @@ int lora_out_multi(hipStream_t st, const LoraOutMultiArgs& a) {
   }
   // As long as all blocks of the small tile are on the chip at once, two per CU, it is the faster one (its rank is walked by two groups
   // of wavefronts, all weights of which are requested at once); past that, what the blocks repeat counts.  us of the four problems of a
-  // layer, weights out of HBM, small tile / 32 x 256: 4096 channels, 64 rows (256 blocks) 8.0 / 11.2, 96 (384) 8.7 / 11.3, 125 (512) 9.0 /
-  // 11.3, 192 (768) 12.1 / 11.9; 2560 channels, 190 rows (480) 6.9 / 8.3; 2048 channels, 256 rows (512) 6.3 / 7.4, 333 (704) 9.3 / 8.0; 768
-  // channels, 512 rows (384) 5.5 / 5.8, 768 (576) 7.3 / 6.9.
+  // layer, weights out of HBM, small tile / 32 x 256: 4096 channels, 64 rows (256 blocks) 7.8 / 11.2, 96 (384) 8.7 / 11.3, 125 (512) 8.4 /
+  // 11.3, 192 (768) 12.1 / 11.9; 2560 channels, 190 rows (480) 7.0 / 8.3; 2048 channels, 256 rows (512) 6.3 / 7.4, 333 (704) 9.3 / 8.0; 768
+  // channels, 512 rows (384) 4.9 / 5.8, 768 (576) 7.3 / 6.9.
   const int row_tiles = ceil_div(a.M, kLoraRows);
   const int64_t cus = device_cu_count();
   const int64_t small = static_cast<int64_t>(ceil_div(a.C, kLoraCols)) * row_tiles * a.n;

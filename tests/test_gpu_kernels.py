@@ -721,6 +721,35 @@ def test_lora_out_of_several_row_tiles(gpu, orc):
     assert rel_err(og.numpy().astype(np.float32), ref.astype(np.float32)) <= F16_TOL
 
 
+@pytest.mark.parametrize("R", [8, 120, 128, 136, 480, 512])
+@pytest.mark.parametrize("rows", [1, 2, 3, 16, 17, 33])
+def test_lora_out_of_few_rows_stages_the_rows_that_exist(gpu, rows, R):
+    """The threads of a block are shared out among the rows of its tile: one row, powers of two and one more, a second tile of one row;
+    ranks that end in a half step, at a round of the threads, and the largest.  The rows past the last one are whatever LDS holds - a call
+    of large values runs before - and reach nothing.  Half an fp16 ulp and the fp32 sums' own error."""
+    hip = gpu
+    rng = np.random.default_rng(rows * 1000 + R)
+    C = 160  # a second column block of one band
+    h = (rng.standard_normal((rows, R)) * 2).astype(np.float16)
+    w2 = (rng.standard_normal((C, R)) * 0.1).astype(np.float16)
+    dh, dw = dev(hip, h), dev(hip, w2)
+    huge = dev(hip, np.full((64, 512), 60000, np.float16))
+    waste = hip.DeviceArray((64, C), np.float16)
+    for act in (hip.ACT_NONE, hip.ACT_TANH, hip.ACT_SIGMOID):
+        hip.lora_out(64, C, 512, hip.ACT_NONE, huge, huge, waste)
+        o = hip.DeviceArray((rows, C), np.float16)
+        hip.lora_out(rows, C, R, act, dh, dw, o)
+        hip.device_sync()
+        hf = h.astype(np.float64)
+        if act == hip.ACT_TANH:
+            hf = np.tanh(hf)
+        elif act == hip.ACT_SIGMOID:
+            hf = 1.0 / (1.0 + np.exp(-hf))
+        exact = hf @ w2.astype(np.float64).T
+        bound = 0.5 * np.spacing(np.abs(exact).astype(np.float16)).astype(np.float64) + 1e-6 * (np.abs(hf) @ np.abs(w2).astype(np.float64).T)
+        assert np.all(np.abs(o.numpy().astype(np.float64) - exact) <= bound)
+
+
 @pytest.mark.parametrize("C,R,rows", [(4064, 24, 417), (4096, 480, 1025), (4096, 40, 2050), (96, 8, 12321), (2048, 512, 4097),
                                       (352, 136, 4100), (2080, 136, 825), (2080, 24, 802), (4096, 480, 993), (4096, 128, 700)])
 def test_lora_out_blocks_of_many_channels(gpu, C, R, rows):
