@@ -14,9 +14,11 @@
 //
 // Precision: nothing is held in less than fp32.  The products of decays and [A B^T], [A K^T] are summed in fp64 (v_mfma_f64_16x16x4),
 // U and Y in fp32 (v_mfma_f32_16x16x4, twice the rate of the vector unit), the update of the state as products of bf16 pieces that
-// add up to the fp32 operands exactly, summed in fp32.  Error of the state against 64-bit sums, 2-norm, chunks / token by token (operands
-// of independent channels and tokens, logits uniform over [-6, 2], state N(0, 1)): 128 tokens x 1024 heads 5.7e-8 / 5.7e-8, 512 x 64
-// 5.7e-8 / 5.7e-8, 2048 x 64 5.8e-8 / 5.7e-8, 333 x 96 5.9e-8 / 6.0e-8.
+// add up to the fp32 operands exactly, summed in fp32.  The operands have the bits that kk_a_gate_kernel gives them.  Error of the state
+// against 64-bit sums, 2-norm, chunks / token by token (operands of independent channels and tokens, logits uniform over [-6, 2], state
+// N(0, 1)): 128 tokens x 1024 heads 5.7e-8 / 5.7e-8, 512 x 64 5.7e-8 / 5.7e-8, 2048 x 64 5.8e-8 / 5.7e-8, 333 x 96 5.9e-8 / 6.0e-8, 64 x 128
+// 5.8e-8 / 5.8e-8; keys that follow one another closely under slow decay, 512 x 24: 2.3e-7 / 3.6e-7; the operands of a layer, 7.2B shape
+// 7.7e-8 / 1.1e-7, 1.5B 7.6e-8 / 1.2e-7 (median over heads).
 //
 // A chunk is one unit: results depend on where a call begins (as those of a prefill call's products do, through their tiles), and a
 // value that is not finite reaches the other tokens of its chunk as well as, from then on, the state.  The operator rwkv_hip_wkv7
@@ -168,7 +170,7 @@ __device__ __forceinline__ half4_t stage_operands(ChunkTiles& t, UpdateOperands&
   float u[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) u[e] = h2f(q.k[e]) * h2f(c.k_k[e]);
-  const float total = row16_sum((u[0] * u[0] + u[1] * u[1]) + (u[2] * u[2] + u[3] * u[3]));
+  const float total = head_sum_of_product(u, u);  // (in any other order -kk of one token in some hundred differs by an fp16 ulp)
   const float inv = quotient(1.0f, fmaxf(sqrtf(total), kKkEps));
   half4_t nk;
   uint4_t x[4];  // this token's (new k, -kk), (kk a, r), (v, v), decay of four channels; then this channel's of four tokens
