@@ -50,7 +50,7 @@ REQUIRED_OCCUPANCY = {"linear_gemv_row1_kernelILi1024ELb1ELi0ELi1ELi1E": 8, "lin
 # heads are ten registers over and measured to be faster so than with fewer wavefronts.
 MOST_SPILLS = {"gemm_tile_kernel": 0, "gemm_ring_kernelILi2ELb1ELi4ELi1ELi4ELi128E": 2, "gemm_ring_kernelI": 0,
                "wkv7_feed_kernelIffLi2ELi2ELi4ELi1ELi2ELi2ELi6ELb0E": 10, "wkv7_feed_kernelI": 0, "wkv7_seq_kernelI": 0,
-               "wkv7_chunk_kernel": 10, "wkv7_chunk_prepare_kernel": 0, "wkv7_chunk_chain_kernelI": 0}
+               "wkv7_chunk_kernel": 10, "wkv7_chunk_prepare_kernel": 0, "wkv7_chunk_chain_kernel": 0}
 
 
 def _check_occupancy(src, stderr_text):

@@ -25,7 +25,7 @@
 // promises the same bits for every split of a sequence and steps token by token (wkv7.hip).
 //
 // us per layer from the rank-outs to the output projection's input, token by token -> in chunks: 16 x 128 tokens x 64 heads 166 ->
-// 93, 3 x 333 x 32 72 -> 51, 1 x 128 x 64 26.1 -> 22.7, 1 x 512 x 64 73 -> 49.  What bounds them: many heads, the issue of VALU
+// 95, 3 x 333 x 32 72 -> 48, 1 x 128 x 64 26.4 -> 22.4, 1 x 512 x 64 75 -> 47.  What bounds them: many heads, the issue of VALU
 // instructions (some 800 per wavefront and chunk) and the matrix core (2700 clocks), which add up although four wavefronts share a
 // SIMD; few heads, launches (three), the latency of one chunk's preparation (6 us) and 0.65 us per link of the chain, most of it LDS
 // and the requests for 31 KB per chunk and CU.
@@ -527,16 +527,17 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prepare_kernel(int T, int C, i
   o.kp[wave][lane] = t.ak[n][4 * g + wave];
 }
 
-// One block per (sequence, head, 16 RT value rows); the blocks of a head are eight apart, which puts them on one XCD and their
+// One block per (sequence, head, 16 value rows), two to a CU; the blocks of a head are eight apart, which puts them on one XCD and their
 // operands into its L2 once.  Wavefronts 0 .. 3 carry the state, a tile of 16 columns each: their shares of U meet in LDS, one
-// barrier per chunk.  Wavefronts 4 .. 7 make Y out of the states that those leave in LDS, a chunk behind.
-template <int RT>
-__global__ __launch_bounds__(512) void wkv7_chunk_chain_kernel(int heads, int T, int C, int H, int t_begin, int t_end, int chunks,
-                                                               float* __restrict__ state, const ChunkOperands* __restrict__ ws,
-                                                               const half_t* __restrict__ v, half_t* __restrict__ y) {
-  __shared__ float4_t u_part[2][RT][4][kWave], y_part[2][RT][4][kWave], s_tile[2][RT][4][kWave];
-  constexpr int kBlocks = 4 / RT;  // per head
-  const int bh = static_cast<int>(blockIdx.x / (8 * kBlocks) * 8 + (blockIdx.x & 7)), row0 = blockIdx.x / 8 % kBlocks * RT;
+// barrier per chunk.  Wavefronts 4 .. 7 make Y out of the states that those leave in LDS, a chunk behind.  Operands are requested two
+// chunks ahead: three need 172 registers, which leaves a CU one block (us per call, one block of 32 rows and three chunks ahead above 64
+// heads / this: 96 heads x 333 tokens 50.4 / 48.4; one of 16 rows and three chunks: 64 x 2048 192 / 187, 24 x 512 38.7 / 37.0).
+constexpr int kChainBlocks = kHead / 16;  // per head
+__global__ __launch_bounds__(512, 4) void wkv7_chunk_chain_kernel(int heads, int T, int C, int H, int t_begin, int t_end, int chunks,
+                                                                  float* __restrict__ state, const ChunkOperands* __restrict__ ws,
+                                                                  const half_t* __restrict__ v, half_t* __restrict__ y) {
+  __shared__ float4_t u_part[2][4][kWave], y_part[2][4][kWave], s_tile[2][4][kWave];
+  const int bh = static_cast<int>(blockIdx.x / (8 * kChainBlocks) * 8 + (blockIdx.x & 7)), rows16 = blockIdx.x / 8 % kChainBlocks;
   if (bh >= heads) return;
   const int bi = bh / H, h = bh - bi * H;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -545,52 +546,38 @@ __global__ __launch_bounds__(512) void wkv7_chunk_chain_kernel(int heads, int T,
   const int g = lane >> 4, n = lane & 15;
   const ChunkOperands* op = ws + static_cast<int64_t>(bh) * chunks;
   auto pick = [&](const float4_t& x) { return q == 0 ? x[0] : (q == 1 ? x[1] : (q == 2 ? x[2] : x[3])); };
-  constexpr int kSets = 3;
+  constexpr int kSets = 2;
 
   if (wave < 4) {
-    float* srow = state + (static_cast<int64_t>(bh) * kHead + 16 * row0 + n) * kHead + 16 * q + 4 * g;
-    float4_t S[RT];
-#pragma unroll
-    for (int m = 0; m < RT; ++m) S[m] = *reinterpret_cast<const float4_t*>(srow + 16 * m * kHead);
+    float* srow = state + (static_cast<int64_t>(bh) * kHead + 16 * rows16 + n) * kHead + 16 * q + 4 * g;
+    float4_t S = *reinterpret_cast<const float4_t*>(srow);
     struct Set {
       float4_t a, p;
       float kp;
-      uint4_t v[RT], kb[3];
+      uint4_t v, kb[3];
     };
     Set set[kSets];
     auto request = [&](Set& s, int c) {  // (chunks past the end repeat the last one)
       const ChunkOperands& o = op[min(c, chunks - 1)];
 #pragma unroll
       for (int i = 0; i < 3; ++i) s.kb[i] = o.u.kb[i][q][lane];
-#pragma unroll
-      for (int m = 0; m < RT; ++m) s.v[m] = o.u.v[row0 + m][lane];
+      s.v = o.u.v[rows16][lane];
       s.a = o.a[q][lane];
       s.kp = o.kp[q][lane];
       s.p = *reinterpret_cast<const float4_t*>(&o.decay[16 * q + 4 * g]);
     };
     // this tile's share of a chunk's U, and the state that the chunk begins with
     auto begin = [&](const Set& s, int c) {
-      float4_t part[RT];
+      s_tile[c & 1][q][lane] = S;
+      float4_t part = mfma4(s.kp, pick(whole(s.v)), float4_t{});
 #pragma unroll
-      for (int m = 0; m < RT; ++m) {
-        s_tile[c & 1][m][q][lane] = S[m];
-        part[m] = mfma4(s.kp, pick(whole(s.v[m])), float4_t{});
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int m = 0; m < RT; ++m) part[m] = mfma4(s.a[i], S[m][i], part[m]);
-#pragma unroll
-      for (int m = 0; m < RT; ++m) u_part[c & 1][m][q][lane] = part[m];
+      for (int i = 0; i < 4; ++i) part = mfma4(s.a[i], S[i], part);
+      u_part[c & 1][q][lane] = part;
       lds_barrier();
     };
     auto turn = [&](Set& s, const Set& next, int c) {
-      const int buf = c & 1;
-#pragma unroll
-      for (int m = 0; m < RT; ++m) {
-        const float4_t U = sum4(u_part[buf][m][0][lane], u_part[buf][m][1][lane], u_part[buf][m][2][lane], u_part[buf][m][3][lane]);
-        S[m] = updated(S[m], s.p, s.kb, s.v[m], split(U));
-      }
+      const float4_t(&up)[4][kWave] = u_part[c & 1];
+      S = updated(S, s.p, s.kb, s.v, split(sum4(up[0][lane], up[1][lane], up[2][lane], up[3][lane])));
       request(s, c + kSets);
       begin(next, c + 1);  // (past the end: what the last turn leaves is not read)
     };
@@ -605,17 +592,16 @@ __global__ __launch_bounds__(512) void wkv7_chunk_chain_kernel(int heads, int T,
 #pragma unroll
     for (int u = 0; u < kSets - 1; ++u)
       if (c + u < chunks) turn(set[u], set[u + 1], c + u);
-#pragma unroll
-    for (int m = 0; m < RT; ++m) *reinterpret_cast<float4_t*>(srow + 16 * m * kHead) = S[m];
+    *reinterpret_cast<float4_t*>(srow) = S;
     return;
   }
 
-  const int64_t base = (static_cast<int64_t>(bi) * T + t_begin) * C + h * kHead + 16 * row0 + n;
+  const int64_t base = (static_cast<int64_t>(bi) * T + t_begin) * C + h * kHead + 16 * rows16 + n;
   const int tokens = t_end - t_begin;
   struct Set {
     float4_t r;
     float rb, rk;
-    half_t v[RT];
+    half_t v;
   };
   Set set[kSets];
   auto request = [&](Set& s, int c) {
@@ -624,31 +610,24 @@ __global__ __launch_bounds__(512) void wkv7_chunk_chain_kernel(int heads, int T,
     s.r = o.r[q][lane];
     s.rb = o.rb[q][lane];
     s.rk = o.rk[q][lane];
-#pragma unroll
-    for (int m = 0; m < RT; ++m) s.v[m] = v[base + static_cast<int64_t>(min(c * kTok + 4 * g + q, tokens - 1)) * C + 16 * m];
+    s.v = v[base + static_cast<int64_t>(min(c * kTok + 4 * g + q, tokens - 1)) * C];
   };
   // wavefront 4 + q writes the tokens 4 g + q
   auto write_out = [&](int c) {
     const int token = c * kTok + 4 * g + q;
-#pragma unroll
-    for (int m = 0; m < RT; ++m) {
-      const float4_t(&part)[4][kWave] = y_part[c & 1][m];
-      const float yv = (part[0][lane][q] + part[1][lane][q]) + (part[2][lane][q] + part[3][lane][q]);
-      if (token < tokens) y[base + static_cast<int64_t>(token) * C + 16 * m] = f2h(yv);
-    }
+    const float4_t(&part)[4][kWave] = y_part[c & 1];
+    const float yv = (part[0][lane][q] + part[1][lane][q]) + (part[2][lane][q] + part[3][lane][q]);
+    if (token < tokens) y[base + static_cast<int64_t>(token) * C] = f2h(yv);
   };
   auto turn = [&](Set& s, int c) {
     const int buf = c & 1;
+    const float4_t(&up)[4][kWave] = u_part[buf];
+    const float u = (up[0][lane][q] + up[1][lane][q]) + (up[2][lane][q] + up[3][lane][q]);
+    const float4_t S = s_tile[buf][q][lane];
+    float4_t part = mfma4(s.rk, h2f(s.v), float4_t{});
 #pragma unroll
-    for (int m = 0; m < RT; ++m) {
-      const float4_t(&up)[4][kWave] = u_part[buf][m];
-      const float u = (up[0][lane][q] + up[1][lane][q]) + (up[2][lane][q] + up[3][lane][q]);
-      const float4_t S = s_tile[buf][m][q][lane];
-      float4_t part = mfma4(s.rk, h2f(s.v[m]), float4_t{});
-#pragma unroll
-      for (int i = 0; i < 4; ++i) part = mfma4(s.r[i], S[i], part);
-      y_part[buf][m][q][lane] = mfma4(s.rb, u, part);
-    }
+    for (int i = 0; i < 4; ++i) part = mfma4(s.r[i], S[i], part);
+    y_part[buf][q][lane] = mfma4(s.rb, u, part);
     request(s, c + kSets);
     if (c > 0) write_out(c - 1);
     lds_barrier();
@@ -672,10 +651,10 @@ constexpr int kSegment = 512;  // tokens that are prepared at a time: bounds the
 enum class ChunkPath { kNone, kWhole, kChain };
 
 // Which calls go in chunks, and how.  us per call with everything from the rank-outs to the output projection's input:
-//   heads x tokens             64 x 12   64 x 33   64 x 64   64 x 128  64 x 512  12 x 512  96 x 64  96 x 333  128 x 128
-//   three kernels (token by token)  9.6      12.7      16.4      26.1      73.4      62.1     21.3      72.2       37.5
-//   whole heads                     7.6      16.2      20.6      37.9     141        140      20.6       -         37.6
-//   chain                          10.3      14.0      15.5      22.7      48.6      36.0     20.4      50.8       30.7
+//   heads x tokens             64 x 12   64 x 33   64 x 48   64 x 128  64 x 512  12 x 512  96 x 64  96 x 333  128 x 128
+//   three kernels (token by token)  9.7      12.6      14.2      26.4      74.7      62.5     21.3      72.6       37.7
+//   whole heads                     7.5      16.1      16.1      37.9     141        140      20.6       -         37.5
+//   chain                          10.3      13.5      13.6      22.4      47.4      34.3     20.0      47.9       29.4
 //   heads x tokens             256 x 8   256 x 16  256 x 17  256 x 128  512 x 64  1024 x 128  2048 x 64
 //   one fused kernel (t. by t.)     7.1      11.4      13.1      67.5       52.0      166        160
 //   whole heads                     8.0       8.1      12.6      39.0       33.0       92.9       95.3
@@ -684,11 +663,10 @@ enum class ChunkPath { kNone, kWhole, kChain };
 ChunkPath chunk_path(int heads, int T) {
   if (T < 10) return ChunkPath::kNone;
   if (heads > 128 || T <= kTok) return ChunkPath::kWhole;
-  if (heads <= 64) return T >= 48 + heads / 4 ? ChunkPath::kChain : ChunkPath::kNone;
+  if (heads <= 64) return T >= 48 ? ChunkPath::kChain : ChunkPath::kNone;
   if (T >= 64) return ChunkPath::kChain;
   return ceil_div(T, kTok) * kTok - T <= 6 ? ChunkPath::kWhole : ChunkPath::kNone;
 }
-constexpr int kNarrowHeads = 64;  // up to here a head's rows go to four blocks of the chain, which one round of CUs takes; then to two
 
 }  // namespace
 
@@ -719,11 +697,8 @@ int tmix_chunk_launch(hipStream_t st, int B, int T, int C, int H, float* state, 
     const int chunks = ceil_div(t1 - t0, kTok);
     hipLaunchKernelGGL(wkv7_chunk_prepare_kernel, dim3(heads * chunks), dim3(256), 0, st, T, C, H, t0, t1, chunks, fa, v, new_k, ws);
     RWKV_LAUNCH_CHECK();
-    const int eights = ceil_div(heads, 8) * 8;
-    if (heads <= kNarrowHeads)
-      hipLaunchKernelGGL(wkv7_chunk_chain_kernel<1>, dim3(eights * 4), dim3(512), 0, st, heads, T, C, H, t0, t1, chunks, state, ws, v, y);
-    else
-      hipLaunchKernelGGL(wkv7_chunk_chain_kernel<2>, dim3(eights * 2), dim3(512), 0, st, heads, T, C, H, t0, t1, chunks, state, ws, v, y);
+    hipLaunchKernelGGL(wkv7_chunk_chain_kernel, dim3(ceil_div(heads, 8) * 8 * kChainBlocks), dim3(512), 0, st, heads, T, C, H, t0, t1, chunks, state,
+                       ws, v, y);
     RWKV_LAUNCH_CHECK();
   }
   return lnx_launch(st, static_cast<int64_t>(B) * T * H, H, y, fa.r, new_k, v, fa.r_k, fa.lnx_w, fa.lnx_b, fa.g, y2);
