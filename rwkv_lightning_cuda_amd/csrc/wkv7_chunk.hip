@@ -655,14 +655,19 @@ enum class ChunkPath { kNone, kWhole, kChain };
 //   three kernels (token by token)  9.7      12.6      14.2      26.4      74.7      62.5     21.3      72.6       37.7
 //   whole heads                     7.5      16.1      16.1      37.9     141        140      20.6       -         37.5
 //   chain                          10.3      13.5      13.6      22.4      47.4      34.3     20.0      47.9       29.4
+//   heads x tokens             160 x 64  160 x 128 160 x 256 192 x 128 192 x 256 192 x 512 224 x 128 224 x 256 320 x 128
+//   whole heads                    20.9      37.5      72.0      38.0      72.3     140.6      38.3      72.2      55.6
+//   chain                          26.6      35.1      57.6      37.9      60.8     126.4      42.2      71.2      52.7
 //   heads x tokens             256 x 8   256 x 16  256 x 17  256 x 128  512 x 64  1024 x 128  2048 x 64
 //   one fused kernel (t. by t.)     7.1      11.4      13.1      67.5       52.0      166        160
 //   whole heads                     8.0       8.1      12.6      39.0       33.0       92.9       95.3
 // A chunk costs the same with one token in it as with sixteen.  The chain needs three launches and pays from a few chunks on, as
-// long as there are CUs for the blocks of a head; with more heads the kernel for whole ones has work for every CU.
+// long as there are CUs for the blocks of a head; with more heads the kernel for whole ones has work for every CU (the few percent
+// around 320 heads, whose blocks are a round and a quarter, are not worth 31 KB per head and chunk).  Three prompts of the 7.2B shape,
+// whole heads / chain, ms a pass: 128 tokens 8.30 / 8.29, 256 14.80 / 14.44, 512 26.2 / 26.2.
 ChunkPath chunk_path(int heads, int T) {
   if (T < 10) return ChunkPath::kNone;
-  if (heads > 128 || T <= kTok) return ChunkPath::kWhole;
+  if (heads > 192 || (heads > 128 && T < 128) || T <= kTok) return ChunkPath::kWhole;
   if (heads <= 64) return T >= 48 ? ChunkPath::kChain : ChunkPath::kNone;
   if (T >= 64) return ChunkPath::kChain;
   return ceil_div(T, kTok) * kTok - T <= 6 ? ChunkPath::kWhole : ChunkPath::kNone;

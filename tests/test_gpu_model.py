@@ -432,12 +432,12 @@ def test_debug_buffers_of_the_recurrences_fp32_operands(gpu):
 
 
 @pytest.mark.parametrize("H,B,T", [(8, 1, 10), (8, 1, 16), (8, 1, 50), (8, 1, 64), (8, 1, 65), (8, 1, 530), (5, 1, 97), (5, 15, 66),
-                                   (8, 9, 32), (8, 9, 79), (5, 26, 11), (8, 17, 33), (8, 17, 130), (8, 40, 17)])
+                                   (8, 9, 32), (8, 9, 79), (5, 26, 11), (8, 17, 33), (8, 17, 130), (8, 25, 130), (8, 40, 17)])
 @pytest.mark.parametrize("slow", [False, True])
 def test_chunked_recurrence_matches_the_token_by_token_operator(gpu, H, B, T, slow):
     """Prefill calls of more than a few tokens run the fp32-state recurrence in chunks of 16 tokens: few heads as a chain over prepared
-    chunks (up to 64 heads, up to 128, more than the 512 tokens that are prepared at once, heads that are no multiple of eight), many
-    heads or one chunk in a block per head, with whole and partial last chunks.  Against rwkv_hip_wkv7, which steps token by token, on
+    chunks (up to 64 heads, up to 128, up to 192 from 128 tokens on, more than the 512 tokens that are prepared at once, heads that are
+    no multiple of eight), many heads or one chunk in a block per head, with whole and partial last chunks.  Against rwkv_hip_wkv7, which steps token by token, on
     the operands that the call derived, bit for bit those that the chunks are made of, from the same state.  Either side is within some
     1e-7 of 64-bit sums (2-norm; a single fp16 rounding that differs in one operand would show as 1e-6 and more), also where the state
     forgets slowly (`slow`: decays of 0.9 and more)."""
