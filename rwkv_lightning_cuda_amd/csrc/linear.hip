@@ -506,26 +506,26 @@ struct LnRow1xV {  // V8 groups of eight values, M rows
   half8_t wv[V8], bv[V8], mv[V8];           // shared by the rows: LN weight and bias, lerp coefficients
 };
 
-// thread t of the computing wavefronts owns the groups t, t + NTL, ... (NTL computing threads).  Every row's
+// thread t of the wavefronts that compute these rows (first .. first + M - 1) owns the groups t, t + NTL, ... (NTL of them).  Every row's
 // operands are requested in one go, so that the rows share one trip to memory.
 template <int V8, int NTL, int M>
-__device__ __forceinline__ LnRow1xV<V8, M> ln_row1_request8(const LnPrologue& ln, const half_t* __restrict__ mu, int K) {
+__device__ __forceinline__ LnRow1xV<V8, M> ln_row1_request8(const LnPrologue& ln, const half_t* __restrict__ mu, int K, int thread, int first) {
   LnRow1xV<V8, M> q;
 #pragma unroll
   for (int g = 0; g < V8; ++g) {
-    const int c = (threadIdx.x + g * NTL) * 8;
+    const int c = (thread + g * NTL) * 8;
     const int cc = c < K ? c : 0;
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-      const int64_t row = static_cast<int64_t>(m) * K;
-      const int64_t xsrc = ln.mode == 2 ? ln.tokens[m] * static_cast<int64_t>(K) : row;
+      const int64_t row = static_cast<int64_t>(first + m) * K;
+      const int64_t xsrc = ln.mode == 2 ? ln.tokens[first + m] * static_cast<int64_t>(K) : row;
       q.xv[m][g] = *reinterpret_cast<const half8_t*>(ln.x + xsrc + cc);
       q.rv[m][g] = *reinterpret_cast<const half8_t*>(ln.mode == 1 ? ln.res + row + cc : ln.x + xsrc + cc);
     }
     q.wv[g] = *reinterpret_cast<const half8_t*>(ln.w + cc);
     q.bv[g] = *reinterpret_cast<const half8_t*>(ln.b + cc);
 #pragma unroll
-    for (int m = 0; m < M; ++m) q.pv[m][g] = *reinterpret_cast<const half8_t*>(ln.shift + static_cast<int64_t>(m) * K + cc);
+    for (int m = 0; m < M; ++m) q.pv[m][g] = *reinterpret_cast<const half8_t*>(ln.shift + static_cast<int64_t>(first + m) * K + cc);
     q.mv[g] = *reinterpret_cast<const half8_t*>(mu + cc);
   }
   return q;
@@ -576,16 +576,16 @@ __device__ __forceinline__ float front_waves_sum(float v, int wave, float* scrat
 
 // (W4: xs in nibble-pair order, the slice sums to xsum - see w4_pair_order)
 template <int NT, int V8, int NTL, int M, bool W4, bool FLAGS>
-__device__ __forceinline__ void ln_row1_finish8(const LnRow1xV<V8, M>& q, const LnPrologue& ln, int K, int m, half_t* xs,
+__device__ __forceinline__ void ln_row1_finish8(const LnRow1xV<V8, M>& q, const LnPrologue& ln, int K, int m, int first, half_t* xs,
                                                 float* xsum, float* stash, float* red, LnFlags* flags, bool store,
-                                                int wave) {
-  const int64_t row = static_cast<int64_t>(m) * K;
+                                                int wave, int thread) {
+  const int64_t row = static_cast<int64_t>(first + m) * K;
   constexpr int NWL = NTL / 64;  // wavefronts that compute
   half_t* hstash = reinterpret_cast<half_t*>(stash + NT * 4);
   float sum = 0.0f;
 #pragma unroll
   for (int g = 0; g < V8; ++g) {
-    const int c = (threadIdx.x + g * NTL) * 8;
+    const int c = (thread + g * NTL) * 8;
     float v[8];
     if (ln.mode == 1) {
 #pragma unroll
@@ -603,12 +603,12 @@ __device__ __forceinline__ void ln_row1_finish8(const LnRow1xV<V8, M>& q, const 
     *reinterpret_cast<half8_t*>(hstash + c + NT * 12) = q.mv[g];
   }
   __builtin_amdgcn_sched_barrier(0);
-  sum = front_waves_sum<NWL, FLAGS>(sum, wave, red, &flags->count[2 * m]);
+  sum = front_waves_sum<NWL, FLAGS>(sum, wave, red, &flags->count[2 * (first + m)]);
   const float mean = sum / static_cast<float>(K);
   float sv = 0.0f;
 #pragma unroll
   for (int g = 0; g < V8; ++g) {
-    const int c = (threadIdx.x + g * NTL) * 8;
+    const int c = (thread + g * NTL) * 8;
     if (c < K) {
       const float4_t v0 = *reinterpret_cast<const float4_t*>(stash + c);
       const float4_t v1 = *reinterpret_cast<const float4_t*>(stash + c + 4);
@@ -624,11 +624,11 @@ __device__ __forceinline__ void ln_row1_finish8(const LnRow1xV<V8, M>& q, const 
       }
     }
   }
-  sv = front_waves_sum<NWL, FLAGS>(sv, wave, red + NT / 64, &flags->count[2 * m + 1]);
+  sv = front_waves_sum<NWL, FLAGS>(sv, wave, red + NT / 64, &flags->count[2 * (first + m) + 1]);
   const float rstd = rsqrtf(sv / static_cast<float>(K) + ln.eps);
 #pragma unroll
   for (int g = 0; g < V8; ++g) {
-    const int c = (threadIdx.x + g * NTL) * 8;
+    const int c = (thread + g * NTL) * 8;
     half8_t ov;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ov[e] = static_cast<half_t>(0.0f);
@@ -658,7 +658,7 @@ __device__ __forceinline__ void ln_row1_finish8(const LnRow1xV<V8, M>& q, const 
       const uint4_t raw = __builtin_bit_cast(uint4_t, ov);
       const float s32 = w4_slice_sum(raw);
       *reinterpret_cast<uint4_t*>(xs + c) = w4_pair_order(raw);
-      if ((threadIdx.x & 3) == 0) xsum[c >> 5] = s32;
+      if ((thread & 3) == 0) xsum[c >> 5] = s32;
     } else {
       *reinterpret_cast<half8_t*>(xs + c) = ov;
     }
@@ -805,6 +805,13 @@ __device__ __forceinline__ void ln_one_finish8(const LnRowOne<V8>& q, const LnPr
 // launch, while a prologue before them leaves HBM idle for its 1.5 us.  So the wavefronts share the work: some
 // compute the prologue and request their weights afterwards, the others request theirs at once and meet the first
 // at the barrier (7.2B shape, int8: 1.79 -> 1.72 ms per step against the prologue in every wavefront first).
+// Two rows of int4 codes: their prologues side by side, a quarter of the wavefronts for each, instead of one after the other in the same
+// ones - twice the meetings were the launch's head.  The same bits.  us per decode step of two rows, one after the other / side by side:
+// 1.5B shape 919 / 849, 0.1B 368 / 346; 7.2B, whose prologue hides behind twice the codes, 1755 / 1749.  (int8 and fp16 rows have half of the wavefronts for a row: a quarter each
+// adds the sums up in another order, for 3 % of a step at 1.5B int8, and costs fp16 weights the early requests of a quarter of the block,
+// 1008 / 1065 us.)
+constexpr bool ln_rows_apart(int fmt, bool ln, int m) { return ln && m == 2 && fmt == RWKV_FMT_W4; }
+
 template <int FMT, int NT, bool LN, int M, int RX>
 __device__ __forceinline__ void gemv_row1_block(const LinearArgs& args, const LinearProblem& prob, int blk, half_t* xs,
                                                float* red, LnFlags* flags) {
@@ -832,9 +839,10 @@ __device__ __forceinline__ void gemv_row1_block(const LinearArgs& args, const Li
   // LDS: M rows of x, then (used by int4 blocks) the sums of every 32 values of each row, then the prologue's stash
   float* xsum = reinterpret_cast<float*>(xs + M * KCAP);
   float* stash = xsum + M * (KCAP / 32);
-  constexpr int NTL = NT / (FMT == RWKV_FMT_W4 ? 4 : 2);  // threads that compute the prologue
+  constexpr bool kApart = ln_rows_apart(FMT, LN, M);
+  constexpr int NTL = NT / (kW4 ? 4 : 2);  // threads that compute the prologue (apart: of each row)
   constexpr int V8 = NT * 4 / (NTL * 8);  // groups of eight values per computing thread
-  const bool ln_wave = LN && wave < NTL / 64;
+  const bool ln_wave = LN && wave < (kApart ? 2 : 1) * (NTL / 64);
   uint4_t xq[M];
 #pragma unroll
   for (int m = 0; m < M; ++m) xq[m] = uint4_t{0u, 0u, 0u, 0u};
@@ -997,7 +1005,10 @@ __device__ __forceinline__ void gemv_row1_block(const LinearArgs& args, const Li
         ln_one_finish8<NT, V8, NTL, kW4, kFlags>(lnq, args.ln, K, xs, xsum, stash, red, flags, blockIdx.x == 0, wave);
         __builtin_amdgcn_sched_barrier(0);
       } else {
-        const LnRow1xV<V8, M> lnq = ln_row1_request8<V8, NTL, M>(args.ln, prob.mu, K);
+        constexpr int kTogether = kApart ? 1 : M;  // rows of this wavefront's
+        const int first = kApart ? wave / static_cast<int>(NWL) : 0;
+        const int thread = static_cast<int>(threadIdx.x) - first * NTL;
+        const LnRow1xV<V8, kTogether> lnq = ln_row1_request8<V8, NTL, kTogether>(args.ln, prob.mu, K, thread, first);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (kFlags) {
           if (threadIdx.x <= kLnFlagX) flags->count[threadIdx.x] = 0u;
@@ -1005,11 +1016,12 @@ __device__ __forceinline__ void gemv_row1_block(const LinearArgs& args, const Li
           __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
+        for (int m = 0; m < kTogether; ++m) {
           // (the stash of row m is rewritten by row m + 1 only after every wavefront has passed row m's second
-          // meeting, i.e. has read what it needs of it: each thread reads only what it wrote)
-          ln_row1_finish8<NT, V8, NTL, M, kW4, kFlags>(lnq, args.ln, K, m, xs + m * KCAP, xsum + m * (KCAP / 32), stash,
-                                                       red, flags, blockIdx.x == 0, wave);
+          // meeting, i.e. has read what it needs of it: each thread reads only what it wrote.  Rows side by side have one each.)
+          ln_row1_finish8<NT, V8, NTL, kTogether, kW4, kFlags>(lnq, args.ln, K, m, first, xs + (first + m) * KCAP,
+                                                               xsum + (first + m) * (KCAP / 32), stash + first * (NT * 4 * 3), red + first * NWL,
+                                                               flags, blockIdx.x == 0, wave - first * static_cast<int>(NWL), thread);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -1020,7 +1032,7 @@ __device__ __forceinline__ void gemv_row1_block(const LinearArgs& args, const Li
       // conservatively), and the arithmetic - microseconds of it per launch - ran after the stream, not under it.
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (kFlags) {
-        ln_flag_wait(&flags->count[kLnFlagX], NWL);
+        ln_flag_wait(&flags->count[kLnFlagX], kApart ? 2 * NWL : NWL);
       } else {
         __syncthreads();
       }
@@ -1031,10 +1043,10 @@ __device__ __forceinline__ void gemv_row1_block(const LinearArgs& args, const Li
       request_all();
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (kFlags) {
-        ln_flag_wait(&flags->count[kLnFlagX], NWL);
+        ln_flag_wait(&flags->count[kLnFlagX], kApart ? 2 * NWL : NWL);
       } else {
 #pragma unroll 1
-        for (int m = 0; m < M; ++m) {
+        for (int m = 0; m < (kApart ? 1 : M); ++m) {
           __syncthreads();
           __syncthreads();
         }
@@ -1114,7 +1126,7 @@ static int row1_format(const LinearArgs& args) {
 
 // Rows of x the whole-rows-in-flight kernel takes: up to 4 (each more row costs every weight vector another eight
 // v_dot2 and two LDS reads; beyond 4 the matrix core is the better tool), up to 2 with the LayerNorm prologue (each
-// row's prologue runs before the computing wavefronts request their weights, and the stash shares the LDS).
+// row's prologue runs before the wavefronts that compute it request their weights, and the stash shares the LDS).
 constexpr int kRow1MaxRows = 4;
 constexpr int kRow1MaxRowsLn = 2;
 static_assert(2 * kRow1MaxRowsLn <= kLnFlagX, "two counters per prologue row");
@@ -1136,7 +1148,8 @@ static int launch_row1(hipStream_t st, LinearArgs& args) {
   }
   args.KT = LN ? NT * 4 : NT * 8;
   // x rows, the slice sums of int4 blocks (4 bytes per 32 values and row), with the prologue also its stash
-  const size_t lds = static_cast<size_t>(args.KT) * (2 * M + (LN ? 4 + 4 * 2 : 0)) + static_cast<size_t>(M) * (args.KT / 32) * 4;
+  constexpr int kStashes = !LN ? 0 : (ln_rows_apart(DF, LN, M) ? 2 : 1);
+  const size_t lds = static_cast<size_t>(args.KT) * (2 * M + kStashes * (4 + 4 * 2)) + static_cast<size_t>(M) * (args.KT / 32) * 4;
   if (lds > 48 * 1024) {  // beyond the default limit of dynamic LDS: raised once per instantiation
     static bool raised = false;
     if (!raised) {

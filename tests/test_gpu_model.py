@@ -1088,6 +1088,32 @@ def test_decode_step_with_layernorm_folded_into_linear_matches_the_unfused_step(
     sess.close()
 
 
+@pytest.mark.parametrize("C", [128, 1024, 1152, 2048, 2176])
+def test_prologues_of_two_rows_of_int4_codes(gpu, C):
+    """The prologues of two rows run side by side in a quarter of the wavefronts each, beside the fp16 rank-ins of the launch, which take
+    them one after the other: rows that fill each size of block and rows that do not.  Against the stand-alone LayerNorm launches, the
+    bar of the test above: formulas and rounding points are the same, sums associate differently, which moves single values by an
+    fp16 step."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=2, C=C, H=C // 64, F=2 * C, V=512, Rw=32, Ra=32, Rg=64, Rv=32)
+    sess = Session(HipModel.from_host_weights(dims, synth_weights(dims, 3), hip.FMT_W4))
+    sess.set_graph(False)
+    rng = np.random.default_rng(C)
+    states = [State(dims, 2) for _ in range(2)]
+    logits = [hip.DeviceArray((2, dims.V), np.float32) for _ in range(2)]
+    for step in range(3):
+        tok = rng.integers(0, dims.V, (2, 1))
+        for fused, st, lg in zip((True, False), states, logits):
+            sess.set_fused_ln(fused)
+            sess.forward(tok, st, lg)
+        assert rel_err(logits[0].numpy(), logits[1].numpy()) <= 2e-3
+        assert rel_err(states[0].shift.numpy().astype(np.float32), states[1].shift.numpy().astype(np.float32)) <= 2e-3
+        assert rel_err(states[0].wkv.numpy(), states[1].wkv.numpy()) <= 1e-3
+    assert logits[0].numpy()[0].tobytes() != logits[0].numpy()[1].tobytes()
+    sess.close()
+
+
 @pytest.mark.parametrize("B,C", [(5, 1024), (8, 1024), (7, 2048), (8, 4096), (12, 1024)])
 def test_decode_step_of_five_to_eight_rows_folds_layernorm_into_the_few_row_launch(gpu, B, C):
     """Models whose rank-ins have no packed copy (a rank that is no multiple of 32) run the int8 and fp16 products of decode
