@@ -56,13 +56,14 @@ __device__ __forceinline__ half8_t make_half8(half2_t a, half2_t b, half2_t c, h
 
 // 8 int8 codes (two dwords) -> 8 fp16, exact: a conversion per code that reads the byte and writes the half in place.  (Bytes under the exponent of
 // 1024, less the bias, take ten instructions; many rows of these products are bound by the chip's power: 16384 x 4096, 2048 rows, blocks of 256
-// x 256 252 us so, 245 with eight conversions.)
+// x 256 252 us so, 245 with eight conversions.  It ends in the two wait states that a product which reads the last of them needs: the compiler does
+// not see these writes.)
 __device__ __forceinline__ half8_t expand_w8(uint32_t d0, uint32_t d1) {
   uint4_t r;
 #define RWKV_LOW(R, D, BYTE) "v_cvt_f16_i16_sdwa " R ", sext(" D ") dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:" BYTE "\n\t"
 #define RWKV_HIGH(R, D, BYTE) "v_cvt_f16_i16_sdwa " R ", sext(" D ") dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:" BYTE "\n\t"
   asm(RWKV_LOW("%0", "%4", "BYTE_0") RWKV_LOW("%1", "%4", "BYTE_2") RWKV_LOW("%2", "%5", "BYTE_0") RWKV_LOW("%3", "%5", "BYTE_2")
-      RWKV_HIGH("%0", "%4", "BYTE_1") RWKV_HIGH("%1", "%4", "BYTE_3") RWKV_HIGH("%2", "%5", "BYTE_1") RWKV_HIGH("%3", "%5", "BYTE_3")
+      RWKV_HIGH("%0", "%4", "BYTE_1") RWKV_HIGH("%1", "%4", "BYTE_3") RWKV_HIGH("%2", "%5", "BYTE_1") RWKV_HIGH("%3", "%5", "BYTE_3") "s_nop 1"
       : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
       : "v"(d0), "v"(d1));
 #undef RWKV_LOW
