@@ -20,9 +20,14 @@
 // 5.8e-8 / 5.8e-8; keys that follow one another closely under slow decay, 512 x 24: 2.3e-7 / 3.6e-7; the operands of a layer, 7.2B shape
 // 7.7e-8 / 1.1e-7, 1.5B 7.6e-8 / 1.2e-7 (median over heads).
 //
-// A chunk is one unit: results depend on where a call begins (as those of a prefill call's products do, through their tiles), and a
-// value that is not finite reaches the other tokens of its chunk as well as, from then on, the state.  The operator rwkv_hip_wkv7
-// promises the same bits for every split of a sequence and steps token by token (wkv7.hip).
+// A chunk is one unit: results depend on where a call begins (as those of a prefill call's products do, through their tiles).  The
+// operator rwkv_hip_wkv7 promises the same bits for every split of a sequence and steps token by token (wkv7.hip).
+//
+// Operands that are not finite: a product takes zero times such a value to the tokens ahead of it, so they are taken out before the products
+// (without_spoilt_tokens).  A token whose k, v, decay or gate is not finite makes its head's outputs from there on and the state NaN - token
+// by token it is the outputs, by GroupNorm, and the rows or columns of the state that it reaches first - one whose r is not finite its own
+// output.  (us per launch without / with the look at every operand: whole heads, 1024 x 128 tokens 100.0 / 102.0; 96 heads x 333 tokens,
+// preparation 19.0 / 19.5, chain 23.9 / 24.0.)
 //
 // us per layer from the rank-outs to the output projection's input, token by token -> in chunks: 16 x 128 tokens x 64 heads 166 ->
 // 95, 3 x 333 x 32 72 -> 48, 1 x 128 x 64 26.4 -> 22.4, 1 x 512 x 64 75 -> 47.  What bounds them: many heads, the issue of VALU
@@ -151,6 +156,7 @@ struct ChunkTiles {
   };
   float rb[kTok][kSquare], rk[kTok][kSquare];  // [t][s]
   float decay[kHead];                          // P_16
+  uint4_t spoilt;                              // of each wavefront's tokens (without_spoilt_tokens)
 };
 
 // Operands of the state update and V, as the matrix core reads them: lane (g, n) of tile q holds column 16 q + n of the tokens
@@ -160,11 +166,38 @@ struct UpdateOperands {
   uint4_t v[4][kWave];      // V in two pieces (fp16 needs no more)
 };
 
+__device__ __forceinline__ bool not_finite(half_t x) { return (__builtin_bit_cast(uint16_t, x) & 0x7c00) == 0x7c00; }
+
+// Takes tokens with operands that are not finite out of this lane's column of four tokens (stage_operands): bit i of the result, those that
+// leave nothing of the state, bit 4 + i, those that have lost r alone.
+__device__ __forceinline__ uint32_t without_spoilt_tokens(uint4_t (&x)[4]) {
+  uint32_t spoilt = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const half2_t k_a = as_half2(x[0][i]), b_r = as_half2(x[1][i]);
+    const float d = __builtin_bit_cast(float, static_cast<uint32_t>(x[3][i]));
+    if (__ballot(not_finite(k_a[0]) || not_finite(k_a[1]) || not_finite(b_r[0]) || not_finite(as_half2(x[2][i])[0]) || d != d)) {
+      x[0][i] = x[1][i] = x[2][i] = 0u;
+      x[3][i] = __builtin_bit_cast(uint32_t, 1.0f);
+      spoilt |= 1u << i;
+    } else if (__ballot(not_finite(b_r[1]))) {
+      x[1][i] &= 0xffffu;
+      spoilt |= 16u << i;
+    }
+  }
+  return spoilt;
+}
+
+struct Staged {
+  half4_t new_k;
+  uint32_t lost;  // tokens whose y is NaN, a bit each (the same in all wavefronts)
+};
+
 // kk normalise, a-gate, new k and decay of token 4 wave + g, channels 4 n .. 4 n + 3 (the formulas and rounding points of
 // kk_a_gate_kernel), then the rows of A, R, B, K and the operands of the update.  `live`: the token exists; one past the end of
-// the call leaves the state as it is.  Returns the new k.
+// the call leaves the state as it is.
 // The products of decays are in fp64, where every A, R, B, K is rounded once.  One barrier inside.
-__device__ __forceinline__ half4_t stage_operands(ChunkTiles& t, UpdateOperands& uo, const ChunkRows& q, const ChannelConstants& c, bool live,
+__device__ __forceinline__ Staged stage_operands(ChunkTiles& t, UpdateOperands& uo, const ChunkRows& q, const ChannelConstants& c, bool live,
                                                   int wave, int lane) {
   const int g = lane >> 4, n = lane & 15;
   float u[4];
@@ -185,14 +218,32 @@ __device__ __forceinline__ half4_t stage_operands(ChunkTiles& t, UpdateOperands&
     x[2][e] = live ? __builtin_bit_cast(uint32_t, half2_t{q.v[e], q.v[e]}) : 0u;
     x[3][e] = __builtin_bit_cast(uint32_t, live ? decay_of(round_h(h2f(q.w12[e]) + h2f(c.w0[e]))) : 1.0f);
   }
+  // NaN where something is not finite (kk a and the decay, which is never infinite: below)
+  float spoil = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) spoil = __builtin_amdgcn_fdot2(as_half2(x[0][e]), half2_t{}, spoil, false);
+#pragma unroll
+  for (int e = 0; e < 4; e += 2) {
+    spoil = __builtin_amdgcn_fdot2(half2_t{q.r[e], q.r[e + 1]}, half2_t{}, spoil, false);
+    spoil = __builtin_amdgcn_fdot2(half2_t{q.v[e], q.v[e + 1]}, half2_t{}, spoil, false);
+  }
   transpose4x4(x);
   const int col = 4 * n + g;  // tokens 4 wave .. 4 wave + 3 of it
   double d[4], p[4];
+  auto multiply_decays = [&]() {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    d[i] = static_cast<double>(__builtin_bit_cast(float, static_cast<uint32_t>(x[3][i])));
-    p[i] = i == 0 ? d[0] : p[i - 1] * d[i];
+    for (int i = 0; i < 4; ++i) {
+      d[i] = static_cast<double>(__builtin_bit_cast(float, static_cast<uint32_t>(x[3][i])));
+      p[i] = i == 0 ? d[0] : p[i - 1] * d[i];
+    }
+  };
+  multiply_decays();
+  uint32_t spoilt_here = 0;
+  if (__builtin_expect(__ballot(spoil != spoil || p[3] != p[3]) != 0, 0)) {  // (a gate that is not a number has made new k one)
+    spoilt_here = without_spoilt_tokens(x);
+    multiply_decays();
   }
+  if (lane == 0) reinterpret_cast<uint32_t*>(&t.spoilt)[wave] = spoilt_here;
   t.part[wave][col] = p[3];
   lds_barrier();
   double first = 1.0, after = 1.0;  // products over the wavefronts before and behind this one
@@ -202,7 +253,20 @@ __device__ __forceinline__ half4_t stage_operands(ChunkTiles& t, UpdateOperands&
     if (w > wave) after *= t.part[w][col];
   }
   const double last = first * p[3];
-  if (wave == 3) t.decay[col] = static_cast<float>(last);
+  const uint4_t spoilt = t.spoilt;
+  uint32_t lost = 0;
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(spoilt[0] | spoilt[1] | spoilt[2] | spoilt[3]) != 0, 0)) {
+    uint32_t all = 0, r = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t m = __builtin_amdgcn_readfirstlane(spoilt[w]);
+      all |= (m & 15u) << (4 * w);
+      r |= (m >> 4) << (4 * w);
+    }
+    lost = (0u - (all & (0u - all))) | r;  // from the first one on
+  }
+  const bool state_lost = lost >> 31;  // (that of r alone has no bits past the tokens)
+  if (wave == 3) t.decay[col] = state_lost ? __builtin_nanf("") : static_cast<float>(last);
   double over = __builtin_amdgcn_rcp(last);  // 1 / P_s, from the last token on down
   over = fma(over, fma(-last, over, 1.0), over);
   float4_t ub, uk, tv;
@@ -227,12 +291,12 @@ __device__ __forceinline__ half4_t stage_operands(ChunkTiles& t, UpdateOperands&
 #pragma unroll
   for (int i = 0; i < 3; ++i) uo.kb[i][tile][at] = uint4_t{sk.p[i][0], sk.p[i][1], sb.p[i][0], sb.p[i][1]};
   uo.v[tile][at] = uint4_t{sv.p[0][0], sv.p[0][1], sv.p[1][0], sv.p[1][1]};
-  return nk;
+  return Staged{nk, lost};
 }
 
 // The four products of tokens with tokens, one per wavefront: A B^T, A K^T (s < t), R B^T, R K^T (s <= t).  The first two go through
 // the solve into the state and are summed in fp64.
-__device__ __forceinline__ void token_products(ChunkTiles& t, int wave, int lane) {
+__device__ __forceinline__ void token_products(ChunkTiles& t, uint32_t lost, int wave, int lane) {
   const int g = lane >> 4, n = lane & 15;
   if (wave < 2) {
     const float(&y)[kTok][kRow] = wave ? t.k : t.b;
@@ -264,6 +328,11 @@ __device__ __forceinline__ void token_products(ChunkTiles& t, int wave, int lane
 #pragma unroll
     for (int i = 0; i < 4; ++i)  // register i: token t = 4 g + i
       dst[4 * g + i][n] = 4 * g + i >= n ? (acc[0][i] + acc[1][i]) + (acc[2][i] + acc[3][i]) : 0.0f;
+    if (__builtin_expect(lost != 0, 0)) {  // the rows that make y NaN
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (lost >> (4 * g + i) & 1u) dst[4 * g + i][n] = __builtin_nanf("");
+    }
   }
 }
 
@@ -415,12 +484,12 @@ __global__ __launch_bounds__(256, 4) void wkv7_chunk_kernel(int T, int C, int H,
   for (int t0 = 0; t0 < T; t0 += kTok) {
     const half4_t r4 = next.r, v4 = next.v, gate4 = gate_next;
     const bool live = t0 + tok < T;
-    const half4_t nk = stage_operands(t, uo, next, ChannelConstants{constants[0][n], constants[1][n], constants[2][n], constants[3][n]}, live, wave, lane);
+    const Staged staged = stage_operands(t, uo, next, ChannelConstants{constants[0][n], constants[1][n], constants[2][n], constants[3][n]}, live, wave, lane);
     __builtin_amdgcn_sched_barrier(0);
     request(t0 + kTok);
     lds_barrier();
     __builtin_amdgcn_s_setprio(1);
-    token_products(t, wave, lane);
+    token_products(t, staged.lost, wave, lane);
     __builtin_amdgcn_s_setprio(0);
     lds_barrier();
     solve(t, wave, lane);
@@ -469,7 +538,7 @@ __global__ __launch_bounds__(256, 4) void wkv7_chunk_kernel(int T, int C, int H,
     lds_barrier();
     const float4_t y4 = *reinterpret_cast<const float4_t*>(&t.y[tok][4 * n]);
     const float yv[4] = {round_h(y4[0]), round_h(y4[1]), round_h(y4[2]), round_h(y4[3])};
-    const half4_t o4 = normalised_output(yv, r4, nk, v4, gate4, constants[4][n], constants[5][n], constants[6][n]);
+    const half4_t o4 = normalised_output(yv, r4, staged.new_k, v4, gate4, constants[4][n], constants[5][n], constants[6][n]);
     if (live) {
       const int64_t at = base + static_cast<int64_t>(t0 + tok) * C;
       *reinterpret_cast<half4_t*>(out + at) = o4;
@@ -491,6 +560,7 @@ struct ChunkOperands {
   float rk[4][kWave];
   float decay[kHead];
 };
+static_assert(sizeof(ChunkOperands) == 27904, "the figures at the head of this file, at chunk_path and in the documents");
 
 // One block per (sequence, head, chunk).  Tokens t_begin .. t_end - 1 of a call of T.
 __global__ __launch_bounds__(256) void wkv7_chunk_prepare_kernel(int T, int C, int H, int t_begin, int t_end, int chunks, TmixSeqArgs fa,
@@ -511,10 +581,10 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prepare_kernel(int T, int C, i
   q.load(fa, v, at);
   ChannelConstants c;
   c.load(fa, ch);
-  const half4_t nk = stage_operands(t, o.u, q, c, live, wave, lane);
-  if (live) *reinterpret_cast<half4_t*>(new_k + at) = nk;
+  const Staged staged = stage_operands(t, o.u, q, c, live, wave, lane);
+  if (live) *reinterpret_cast<half4_t*>(new_k + at) = staged.new_k;
   lds_barrier();
-  token_products(t, wave, lane);
+  token_products(t, staged.lost, wave, lane);
   lds_barrier();
   solve(t, wave, lane);
   // what the solve leaves alone
@@ -624,7 +694,7 @@ __global__ __launch_bounds__(512, 4) void wkv7_chunk_chain_kernel(int heads, int
     const float4_t(&up)[4][kWave] = u_part[buf];
     const float u = (up[0][lane][q] + up[1][lane][q]) + (up[2][lane][q] + up[3][lane][q]);
     const float4_t S = s_tile[buf][q][lane];
-    float4_t part = mfma4(s.rk, h2f(s.v), float4_t{});
+    float4_t part = mfma4(s.rk, not_finite(s.v) ? 0.0f : h2f(s.v), float4_t{});
 #pragma unroll
     for (int i = 0; i < 4; ++i) part = mfma4(s.r[i], S[i], part);
     y_part[buf][q][lane] = mfma4(s.rb, u, part);

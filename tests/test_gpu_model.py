@@ -476,6 +476,92 @@ def test_chunked_recurrence_matches_the_token_by_token_operator(gpu, H, B, T, sl
     sess.close()
 
 
+@pytest.mark.parametrize("H,B,T,at", [(8, 1, 50, 20), (8, 1, 50, 16), (8, 1, 50, 49), (8, 1, 16, 5), (8, 17, 33, 15), (8, 17, 33, 32)])
+@pytest.mark.parametrize("kind", ["r", "k", "v", "w", "a"])
+def test_chunked_recurrence_keeps_what_is_not_finite_from_earlier_tokens(gpu, H, B, T, at, kind):
+    """One token of one sequence has one channel of r, k or v that overflows, or a decay or gate that is not a number (both paths; first, middle and
+    last tokens of a chunk and of the call).  The tokens before it, the other heads and the other sequences keep their bits; its head is NaN
+    from there on, for r in that token alone, whose later tokens and state are those of the token-by-token operator."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    C, head, channel, row = 64 * H, 3, 3 * 64 + 17, B // 2
+    dims = ModelDims(L=1, C=C, H=H, F=4 * C, V=256, Rw=32, Ra=32, Rg=64, Rv=32)
+    weights = synth_weights(dims, 6)
+    layer = weights["layers"][0]
+    # token 0 lies along s, the others across it: a row of weights along s overflows for token 0 alone (C = 512 channels of 300)
+    rng = np.random.default_rng(at)
+    s = rng.permutation(np.repeat([1.0, -1.0], C // 2))
+    emb = rng.standard_normal((dims.V, C))
+    emb -= emb.mean(axis=1, keepdims=True)
+    emb -= np.outer(emb @ s, s) / C
+    emb[0] = s
+    weights["emb_ln0"] = emb.astype(np.float16)
+    layer["ln1_w"][:], layer["ln1_b"][:] = 1, 0
+    for name in ("x_r", "x_w", "x_k", "x_v", "x_a", "x_g"):
+        layer[name][:] = 0  # no token shift: the next token sees nothing of it
+    if kind in ("r", "k", "v"):
+        layer["att_" + kind][channel] = 300 * s
+    else:  # minus infinity, and plus infinity for token 0
+        layer[kind + "0"][channel] = -np.inf
+        layer[kind + "1"][:2] = 20 * s
+        layer[kind + "2"][channel] = 0
+        layer[kind + "2"][channel, :2] = 65504 if kind == "w" else 10
+    model = HipModel.from_host_weights(dims, weights, hip.FMT_F16)
+    tokens = rng.integers(1, dims.V, (B, T))
+    before = (0.1 * rng.standard_normal((1, B, H, 64, 64))).astype(np.float32)
+    shape = (B, T, H, 64)
+    seen = []
+    for spoilt in (False, True):
+        sess, st = Session(model), State(dims, B)
+        st.wkv.upload(before)
+        tok = tokens.copy()
+        if spoilt:
+            tok[row, at] = 0
+        sess.forward(tok, st, hip.DeviceArray((B, dims.V), np.float32))
+        tap = {n: sess.debug_buffer(n, (B, T, C)) for n in ("y2", "r", "d32", "k2", "v_first", "nkk", "kka", "g")}
+        seen.append((tap, tap["y2"].reshape(shape), st.wkv.numpy()[0]))
+        sess.close()
+    clean, (tap, y2, state) = seen[0], seen[1]
+    assert np.isfinite(clean[1]).all() and np.isfinite(clean[2]).all()
+    name = {"r": "r", "k": "k2", "v": "v_first", "w": "d32", "a": "kka"}[kind]
+    assert not np.isfinite(tap[name][row, at, channel]) and np.isfinite(np.delete(tap[name][row], at, axis=0)).all()
+    same = np.ones(shape[:3], bool)  # what sees nothing of the token
+    same[row, at] = False
+    same[row, at:] = False
+    assert np.array_equal(y2[same], clean[1][same])
+    others = np.arange(H) != head
+    assert np.isfinite(y2[row, at:][:, others]).all()
+    # the operator on the same operands
+    want = hip.DeviceArray.from_numpy(before)
+    y = hip.DeviceArray((B, T, C), np.float32)
+    hip.wkv7(B, T, C, H, hip.W_DECAY, hip.IO_F32, want,
+             *[hip.DeviceArray.from_numpy(tap[n].astype(np.float32)) for n in ("r", "d32", "k2", "v_first", "nkk", "kka")], y)
+    want, y = want.numpy()[0].astype(np.float64), y.numpy().reshape(shape)
+    finite = np.isfinite(want) & np.isfinite(state)
+    assert np.linalg.norm((state - want)[finite]) <= 6e-7 * np.linalg.norm(want[finite])
+    lost = np.zeros(shape[:3], bool)
+    lost[row, at:, head] = True
+    if kind == "r":
+        lost[row, at + 1:, head] = False
+        assert finite.all()
+    else:
+        kept = np.ones((B, H), bool)
+        kept[row, head] = False
+        assert finite[kept].all() and not np.isfinite(state[row, head]).any()
+        assert not np.isfinite(want[row, head]).all()
+    assert np.isnan(y2[lost]).all() and np.isfinite(y2[~lost]).all()
+    # the operator's outputs behind GroupNorm: a row that is not finite takes its head with it
+    yh = y.astype(np.float16).astype(np.float64)
+    with np.errstate(all="ignore"):
+        normed = (yh - yh.mean(-1, keepdims=True)) / np.sqrt(yh.var(-1, keepdims=True) + 64e-5)
+    assert np.array_equal(np.isnan(normed).any(-1), lost)
+    heads = lambda n: tap[n].reshape(shape).astype(np.float64)
+    per = {n: layer[n].astype(np.float64).reshape(H, 64) for n in ("r_k", "lnx_w", "lnx_b")}
+    out = (normed * per["lnx_w"] + per["lnx_b"] + (heads("r") * heads("k2") * per["r_k"]).sum(-1, keepdims=True) * heads("v_first")) * heads("g")
+    ok = ~lost
+    assert np.linalg.norm(y2[ok] - out[ok]) <= 1e-3 * np.linalg.norm(out[ok])
+
+
 def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
     """Without set_sparse_ffn a decode step walks the non-zero rows only where the matrix pays for the second launch: a
     small model gives the bits of the dense product, and those of the walk once it is asked for."""
