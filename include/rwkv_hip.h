@@ -384,7 +384,9 @@ int rwkv_hip_session_set_tmix_rows(rwkv_hip_session* s, int rows);
  * r32, d32, k32, a32, b32 (f32).  Which of them a pass writes depends on its shape (decode steps fuse most
  * of them away).  r32 (calls of more than one row), k32, a32 and b32 are copies of r, k2, nkk and kka widened by this
  * call, which waits for the stream; they live until the next such call for the same id.  A one-row step leaves the output
- * projection's input ahead of the gate in r32.  No counterpart in the reference. */
+ * projection's input ahead of the gate in r32.  Prefill calls with the fp32 state that keep nkk, kka, d32 and k2 to themselves have them
+ * made by this call, which then waits for the stream; y is RWKV_E_STATE where the last call kept it to itself (more than 128 heads of all
+ * sequences, without the residual-stream tap below).  No counterpart in the reference. */
 int rwkv_hip_session_debug_buffer(rwkv_hip_session* s, int id, void** ptr);
 /* debugging/parity tap: residual stream after every layer of the last rwkv_hip_forward call,
  * f16 [L, B*T, C], valid only if enabled before the call */

@@ -107,6 +107,10 @@ inline int packed_min_rows(const rwkv_hip_model* m) {
 // this launch / the row-tiled kernels: 16 rows 14 / 17, 32 rows 25 / 24)
 inline int tmix_step_max_blocks() { return device_cu_count(); }
 
+// Heads (of all sequences) up to which every prefill call leaves y behind for rwkv_hip_session_debug_buffer: there its stores are a few per
+// cent of the recurrence, beyond them only a call with the residual-stream tap on writes it.
+constexpr int kTapHeads = 128;
+
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 struct Arena {
@@ -158,7 +162,8 @@ struct rwkv_hip_session {
   size_t sparse_ws_bytes = 0;
   float* widened[4] = {};     // rwkv_hip_session_debug_buffer: fp32 copies of r, k2, nkk, kka, made when they are asked for
   size_t widened_cap[4] = {};
-  bool gate_missing = false;  // the last pass kept k2, nkk, kka and d32 to itself: debug_buffer makes them
+  // what the last prefill pass kept to itself: debug_buffer makes k2, nkk, kka and d32, and refuses y
+  bool gate_missing = false, y_missing = false;
   int sparse_ffn_rows = -1;   // decode steps of up to this many rows read only the ffn.value rows with a non-zero activation; -1: where it pays
                               // (2..4 rows share one walk over the rows that are non-zero for any of them)
   bool wkv_fp16 = false;      // the WKV state tensor is fp16 [L,B,H,64,64] (the reference's use_wkv32 == false)
@@ -266,7 +271,7 @@ size_t packed_workspace_bytes(const rwkv_hip_model* m, int B, int rows) {
 
 int ensure_arena(rwkv_hip_session* s, int B, int T) {
   const rwkv_hip_model* m = s->model;
-  s->gate_missing = false;
+  s->gate_missing = s->y_missing = false;
   const size_t rows = static_cast<size_t>(B) * T;
   if (s->arena.base && B <= s->arena_B && T <= s->arena_T && B * T <= s->arena_B * s->arena_T) {
     // shapes are laid out per call below, so only capacity matters
@@ -705,11 +710,14 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
         }
       } else if (tmix_chunk_pays(B, T, H, fa)) {
         // more than a few tokens: the same in chunks of 16 tokens on the matrix cores
-        TRY_AUX(tmix_chunk_launch(st, B, T, C, H, S, fa, v_cur, b.chunk_ws, b.k2, b.y, s->trace || B * H <= 128, b.y2));
+        const bool tap_y = s->trace || B * H <= kTapHeads;
+        TRY_AUX(tmix_chunk_launch(st, B, T, C, H, S, fa, v_cur, b.chunk_ws, b.k2, b.y, tap_y, b.y2));
         s->gate_missing = true;
+        s->y_missing = !tmix_chunk_chains(B, T, H) && !tap_y;
       } else if (!s->trace && tmix_seq_whole_heads(B, T, H)) {
         // kk normalise / a-gate / decay, the WKV recurrence and GroupNorm / bonus / gate in one launch
         TRY_AUX(tmix_seq_launch(st, B, T, C, H, S, fa, v_cur, b.y2));
+        if (!step) s->gate_missing = s->y_missing = true;
       } else {
         // with the residual-stream tap on, or few heads in flight: the three stand-alone kernels (same arithmetic,
         // bitwise the same)
@@ -1230,9 +1238,13 @@ int rwkv_hip_session_debug_buffer(rwkv_hip_session* s, int id, void** ptr) {
                    b.att, b.x1,  b.ln2, b.mixed, b.act, b.cm, b.r32, b.d32, b.k2, b.nkk, b.kka};
   RWKV_REQUIRE(id >= 0 && id < static_cast<int>(sizeof(table) / sizeof(table[0])), "debug_buffer: unknown id %d", id);
   *ptr = table[id];
-  constexpr int kK2 = 19, kKka = 21, kD32 = 31;
+  constexpr int kK2 = 19, kKka = 21, kY = 22, kD32 = 31;
+  if (id == kY && s->y_missing) {
+    set_error("debug_buffer: the last pass did not write y (calls of more than %d heads write it with the residual-stream tap on)", kTapHeads);
+    return RWKV_E_STATE;
+  }
   if (s->gate_missing && (id >= kD32 || (id >= kK2 && id <= kKka))) {
-    // the chunked recurrence derives them as it goes
+    // the recurrence derives them as it goes
     const Layer& w = s->model->layers.back();
     KkArgs p = {};
     p.k = b.k; p.k_k = w.t[RWKV_T_K_K]; p.a0 = w.t[RWKV_T_A0]; p.a12 = b.a12; p.k_a = w.t[RWKV_T_K_A];

@@ -246,7 +246,8 @@ int wkv7_seq_f16_launch(hipStream_t st, int B, int T, int C, int H, float* state
 // ---- wkv7_chunk.hip: the same pass (fp32 state) in chunks of 16 tokens on the matrix cores, for calls of more than a few tokens ----
 bool tmix_chunk_pays(int B, int T, int H, const TmixSeqArgs& fa);
 size_t tmix_chunk_workspace_bytes(int B, int T, int H);  // (0 where none is needed)
-// new_k, y: written (y: if asked for) by calls of few heads or tokens on the way to y2; may be scratch
+bool tmix_chunk_chains(int B, int T, int H);             // new_k and y are written on the way to y2
+// new_k, y: otherwise y alone is, if it is asked for
 int tmix_chunk_launch(hipStream_t st, int B, int T, int C, int H, float* state, const TmixSeqArgs& fa, const half_t* v, void* workspace,
                       half_t* new_k, half_t* y, bool want_y, half_t* y2);
 

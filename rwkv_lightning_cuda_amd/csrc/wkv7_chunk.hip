@@ -752,8 +752,10 @@ bool tmix_chunk_pays(int B, int T, int H, const TmixSeqArgs& fa) {
   return bits % sizeof(half4_t) == 0 && chunk_path(B * H, T) != ChunkPath::kNone;
 }
 
+bool tmix_chunk_chains(int B, int T, int H) { return chunk_path(B * H, T) == ChunkPath::kChain; }
+
 size_t tmix_chunk_workspace_bytes(int B, int T, int H) {
-  if (chunk_path(B * H, T) != ChunkPath::kChain) return 0;
+  if (!tmix_chunk_chains(B, T, H)) return 0;
   return sizeof(ChunkOperands) * B * H * ceil_div(std::min(T, kSegment), kTok);
 }
 

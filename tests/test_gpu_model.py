@@ -562,6 +562,41 @@ def test_chunked_recurrence_keeps_what_is_not_finite_from_earlier_tokens(gpu, H,
     assert np.linalg.norm(y2[ok] - out[ok]) <= 1e-3 * np.linalg.norm(out[ok])
 
 
+@pytest.mark.parametrize("B,T", [(17, 33), (17, 5)])
+def test_debug_buffers_of_a_pass_that_keeps_its_operands(gpu, B, T):
+    """More than 128 heads of all sequences: y is refused where the call did not write it (instead of what an earlier one left there) and comes
+    with the residual-stream tap, y2 but for roundings behind GroupNorm, bonus and gate; k2, nkk and kka are those of the stand-alone kernel."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=1, C=512, H=8, F=2048, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
+    weights = synth_weights(dims, 4)
+    sess = Session(HipModel.from_host_weights(dims, weights, hip.FMT_W8))
+    rng = np.random.default_rng(2)
+    lg = hip.DeviceArray((B, dims.V), np.float32)
+    shape = (B, T, dims.C)
+    up = lambda n: hip.DeviceArray.from_numpy(weights["layers"][0][n])
+    for tokens in rng.integers(0, dims.V, (2, B, T)):  # the second call behind one that wrote y
+        sess.forward(tokens, State(dims, B), lg)
+        with pytest.raises(hip.RwkvHipError, match="did not write y"):
+            sess.debug_buffer("y", shape)
+        made = {n: sess.debug_buffer(n, shape) for n in ("k2", "nkk", "kka", "y2")}
+        sess.set_trace(hip.DeviceArray((1, B * T, dims.C), np.float16))
+        sess.forward(tokens, State(dims, B), lg)
+        sess.set_trace(None)
+        tap = {n: sess.debug_buffer(n, shape) for n in ("k", "a12", "r", "v_first", "g", "y", "y2")}
+        on = {n: hip.DeviceArray.from_numpy(x) for n, x in tap.items()}
+        k2, nkk, kka, y2 = (hip.DeviceArray(shape, np.float16) for _ in range(4))
+        hip.kk_a_gate(B * T, dims.C, dims.H, on["k"], up("k_k"), up("a0"), on["a12"], up("k_a"), k2, nkk, kka)
+        for name, x in (("k2", k2), ("nkk", nkk), ("kka", kka)):
+            assert made[name].tobytes() == x.numpy().tobytes(), name
+        hip.lnx_rkvres_xg(B * T, dims.C, dims.H, on["y"], on["r"], k2, on["v_first"], up("r_k"), up("lnx_w"), up("lnx_b"), on["g"], y2)
+        assert np.abs(tap["y2"].astype(np.float32) - y2.numpy().astype(np.float32)).max() <= 4e-3 * np.abs(tap["y2"]).max()
+        assert made["y2"].tobytes() == tap["y2"].tobytes()
+    sess.forward(rng.integers(0, dims.V, (1, T)), State(dims, 1), hip.DeviceArray((1, dims.V), np.float32))
+    assert np.isfinite(sess.debug_buffer("y", (1, T, dims.C))).all()
+    sess.close()
+
+
 def test_ffn_value_of_a_small_matrix_is_dense_by_default(gpu):
     """Without set_sparse_ffn a decode step walks the non-zero rows only where the matrix pays for the second launch: a
     small model gives the bits of the dense product, and those of the walk once it is asked for."""
