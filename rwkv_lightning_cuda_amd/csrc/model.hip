@@ -162,8 +162,8 @@ struct rwkv_hip_session {
   size_t sparse_ws_bytes = 0;
   float* widened[4] = {};     // rwkv_hip_session_debug_buffer: fp32 copies of r, k2, nkk, kka, made when they are asked for
   size_t widened_cap[4] = {};
-  // what the last prefill pass kept to itself: debug_buffer makes k2, nkk, kka and d32, and refuses y
-  bool gate_missing = false, y_missing = false;
+  // what the last prefill pass kept to itself: debug_buffer makes k2, and nkk, kka and d32, and refuses y
+  bool k2_missing = false, gate_missing = false, y_missing = false;
   int sparse_ffn_rows = -1;   // decode steps of up to this many rows read only the ffn.value rows with a non-zero activation; -1: where it pays
                               // (2..4 rows share one walk over the rows that are non-zero for any of them)
   bool wkv_fp16 = false;      // the WKV state tensor is fp16 [L,B,H,64,64] (the reference's use_wkv32 == false)
@@ -271,7 +271,7 @@ size_t packed_workspace_bytes(const rwkv_hip_model* m, int B, int rows) {
 
 int ensure_arena(rwkv_hip_session* s, int B, int T) {
   const rwkv_hip_model* m = s->model;
-  s->gate_missing = s->y_missing = false;
+  s->k2_missing = s->gate_missing = s->y_missing = false;
   const size_t rows = static_cast<size_t>(B) * T;
   if (s->arena.base && B <= s->arena_B && T <= s->arena_T && B * T <= s->arena_B * s->arena_T) {
     // shapes are laid out per call below, so only capacity matters
@@ -713,11 +713,12 @@ int enqueue_forward(rwkv_hip_session* s, int B, int T, half_t* shift, void* wkv_
         const bool tap_y = s->trace || B * H <= kTapHeads;
         TRY_AUX(tmix_chunk_launch(st, B, T, C, H, S, fa, v_cur, b.chunk_ws, b.k2, b.y, tap_y, b.y2));
         s->gate_missing = true;
-        s->y_missing = !tmix_chunk_chains(B, T, H) && !tap_y;
+        s->k2_missing = !tmix_chunk_chains(B, T, H);
+        s->y_missing = s->k2_missing && !tap_y;
       } else if (!s->trace && tmix_seq_whole_heads(B, T, H)) {
         // kk normalise / a-gate / decay, the WKV recurrence and GroupNorm / bonus / gate in one launch
         TRY_AUX(tmix_seq_launch(st, B, T, C, H, S, fa, v_cur, b.y2));
-        if (!step) s->gate_missing = s->y_missing = true;
+        if (!step) s->k2_missing = s->gate_missing = s->y_missing = true;
       } else {
         // with the residual-stream tap on, or few heads in flight: the three stand-alone kernels (same arithmetic,
         // bitwise the same)
@@ -1248,12 +1249,13 @@ int rwkv_hip_session_debug_buffer(rwkv_hip_session* s, int id, void** ptr) {
     const Layer& w = s->model->layers.back();
     KkArgs p = {};
     p.k = b.k; p.k_k = w.t[RWKV_T_K_K]; p.a0 = w.t[RWKV_T_A0]; p.a12 = b.a12; p.k_a = w.t[RWKV_T_K_A];
-    p.new_k = b.k2; p.neg_kk = b.nkk; p.kka = b.kka;
+    p.new_k = s->k2_missing ? b.k2 : nullptr;  // (otherwise the pass's own)
+    p.neg_kk = b.nkk; p.kka = b.kka;
     p.w12 = b.w12; p.w0 = w.t[RWKV_T_W0]; p.d32 = b.d32;
     p.rows_heads = static_cast<int64_t>(s->arena_B) * s->arena_T * s->model->H; p.H = s->model->H;
     TRY(kk_a_gate_launch(s->stream, p));
     RWKV_HIP_TRY(hipStreamSynchronize(s->stream));
-    s->gate_missing = false;
+    s->k2_missing = s->gate_missing = false;
   }
   // the recurrence reads its operands in fp16: their fp32 forms are made here
   constexpr int kR32 = 30, kK32 = 32;

@@ -438,9 +438,10 @@ def test_chunked_recurrence_matches_the_token_by_token_operator(gpu, H, B, T, sl
     """Prefill calls of more than a few tokens run the fp32-state recurrence in chunks of 16 tokens: few heads as a chain over prepared
     chunks (up to 64 heads, up to 128, up to 192 from 128 tokens on, more than the 512 tokens that are prepared at once, heads that are
     no multiple of eight), many heads or one chunk in a block per head, with whole and partial last chunks.  Against rwkv_hip_wkv7, which steps token by token, on
-    the operands that the call derived, bit for bit those that the chunks are made of, from the same state.  Either side is within some
+    the operands that the stand-alone kernel makes of the call's projections, from the same state.  Either side is within some
     1e-7 of 64-bit sums (2-norm; a single fp16 rounding that differs in one operand would show as 1e-6 and more), also where the state
-    forgets slowly (`slow`: decays of 0.9 and more)."""
+    forgets slowly (`slow`: decays of 0.9 and more).  A chain's new k, which the preparation of its chunks leaves behind, has the
+    stand-alone kernel's bits."""
     from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
     hip = gpu
     C = 64 * H
@@ -455,6 +456,12 @@ def test_chunked_recurrence_matches_the_token_by_token_operator(gpu, H, B, T, sl
     st.wkv.upload(before)
     sess.forward(rng.integers(0, dims.V, (B, T)), st, hip.DeviceArray((B, dims.V), np.float32))
     shape = (B, T, C)
+    new_k = sess.debug_buffer("k2", shape)
+    k, a12 = (hip.DeviceArray.from_numpy(sess.debug_buffer(name, shape)) for name in ("k", "a12"))
+    alone = [hip.DeviceArray(shape, np.float16) for _ in range(3)]
+    up = lambda n: hip.DeviceArray.from_numpy(weights["layers"][0][n])
+    hip.kk_a_gate(B * T, C, H, k, up("k_k"), up("a0"), a12, up("k_a"), *alone)
+    assert new_k.tobytes() == alone[0].numpy().tobytes()
     tap = {name: sess.debug_buffer(name, shape).astype(np.float32) for name in ("r", "k2", "nkk", "kka", "d32", "v_first", "g", "y2")}
     state = hip.DeviceArray.from_numpy(before)
     y = hip.DeviceArray(shape, np.float32)
