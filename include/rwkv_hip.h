@@ -166,6 +166,12 @@ int rwkv_hip_linear_packed_workspace(int M, int N, int K, size_t* bytes);
 int rwkv_hip_linear_packed(rwkv_stream_t s, int fmt, int M, int N, int K, const void* x, const void* packed,
                            const void* scale, const void* zp, int epilogue, int out_f32, void* y,
                            void* workspace, size_t workspace_bytes);
+/* parity tap, on the host alone: the rows and columns of a block and the K split that rwkv_hip_linear_packed takes with a workspace of
+ * workspace_bytes (one problem), or a model's launch of several int8 and fp16 matrices over the same rows; apart (may be NULL): whether a
+ * model gives the leading int8 ones a launch of their own instead.  Blocks of 256 columns are kernels of their own, so tests can tell
+ * which one they run.  No counterpart in the reference. */
+int rwkv_hip_linear_packed_plan(int M, int K, int n_problems, const int* N, const int* fmt, size_t workspace_bytes, int* tile_rows,
+                                int* tile_cols, int* splits, int* apart);
 
 /* ---- ffn.value of a few tokens, reading per token only the rows with a non-zero activation.  Replaces
  * rwkv7_cmix_sparse_down_relu_one_launch and rwkv7_cmix_sparse_down_relu_rows_launch

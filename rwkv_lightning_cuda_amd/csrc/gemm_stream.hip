@@ -638,6 +638,21 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
                          void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, bool tiles,
                          DeferredReduce* defer, const RowCopy* copy);
 
+// What a launch with this workspace takes.
+// A split is an offer, not a need, for int4 codes, from 513 rows on, where blocks of 32 x 32 alone occupy the chip and where K
+// has no power of two of whole 512s (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a
+// workspace too, with the split that fits.  Elsewhere a workspace too small for the split is an error.
+static StreamConfig launch_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool at_consumer, bool group_rows,
+                                  size_t workspace_bytes, bool fit_splits, bool tiles) {
+  int64_t n_total = 0;
+  for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
+  const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
+  fit_splits = fit_splits || fmts[0] == RWKV_FMT_W4 || M > 512 || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 ||
+               static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
+  const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace_bytes / plane)) : 32;
+  return choose_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, max_splits, tiles);
+}
+
 static int require_supported(int M, int K, int n_problems, const PackedProblem* problems) {
   RWKV_REQUIRE(n_problems >= 1 && n_problems <= kMaxProblems, "linear_packed: %d problems (1..%d allowed)", n_problems,
                kMaxProblems);
@@ -682,13 +697,8 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
     group_rows = group_rows || (fmts[i] == RWKV_FMT_W4 && !problems[i].groups_first);
   }
   const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
-  // A split is an offer, not a need, for int4 codes, from 513 rows on, where blocks of 32 x 32 alone occupy the chip and where K
-  // has no power of two of whole 512s (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a
-  // workspace too, with the split that fits.  Elsewhere a workspace too small for the split is an error.
-  fit_splits = fit_splits || fmts[0] == RWKV_FMT_W4 || M > 512 || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 ||
-               static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
-  const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace ? workspace_bytes / plane : 0)) : 32;
-  const StreamConfig cfg = choose_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, max_splits, tiles);
+  const StreamConfig cfg = launch_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, workspace ? workspace_bytes : 0, fit_splits,
+                                         tiles);
   int col_blocks = 0;
   for (int i = 0; i < n_problems; ++i) {
     const PackedProblem& q = problems[i];
@@ -772,6 +782,32 @@ int rwkv_hip_pack_weights(rwkv_stream_t s, int fmt, int N, int K, const void* w,
 int rwkv_hip_linear_packed_workspace(int M, int N, int K, size_t* bytes) {
   RWKV_REQUIRE(bytes && M > 0 && N > 0 && K > 0, "linear_packed_workspace: bad arguments");
   *bytes = linear_packed_workspace_bytes(M, N, K);
+  return RWKV_OK;
+}
+
+int rwkv_hip_linear_packed_plan(int M, int K, int n_problems, const int* N, const int* fmt, size_t workspace_bytes, int* tile_rows,
+                                int* tile_cols, int* splits, int* apart) {
+  RWKV_REQUIRE(M > 0 && K > 0 && N && fmt && tile_rows && tile_cols && splits, "linear_packed_plan: bad arguments");
+  RWKV_REQUIRE(n_problems >= 1 && n_problems <= kMaxProblems, "linear_packed_plan: %d problems (1..%d allowed)", n_problems, kMaxProblems);
+  for (int i = 0; i < n_problems; ++i)
+    RWKV_REQUIRE(linear_packed_supported(fmt[i], M, N[i], K) && (n_problems == 1 || fmt[i] != RWKV_FMT_W4),
+                 "linear_packed_plan: unsupported shape M=%d N=%d K=%d fmt=%d", M, N[i], K, fmt[i]);
+  const bool several = n_problems > 1;
+  const StreamConfig c = launch_config(M, K, n_problems, N, fmt, false, fmt[0] == RWKV_FMT_W4, workspace_bytes, several,
+                                       several || M > kOperatorTileRows);
+  *tile_rows = c.rows();
+  *tile_cols = c.cols(c.fmt);
+  *splits = c.splits;
+  if (apart) {
+    PackedProblem p[kMaxProblems] = {};
+    int first = 0;  // the leading int8 matrices
+    for (int i = 0; i < n_problems; ++i) {
+      p[i].N = N[i];
+      p[i].fmt = fmt[i];
+      if (first == i && fmt[i] == RWKV_FMT_W8) ++first;
+    }
+    *apart = first > 0 && first < n_problems && linear_packed_apart(M, K, first, n_problems, p) ? 1 : 0;
+  }
   return RWKV_OK;
 }
 

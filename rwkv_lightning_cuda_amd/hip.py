@@ -37,7 +37,7 @@ EXPORTS = [
     "rwkv_hip_event_elapsed_ms", "rwkv_hip_measure_launch_chain", "rwkv_hip_wkv7", "rwkv_hip_wkv7_f16state", "rwkv_hip_quantize_w8", "rwkv_hip_dequant_w8",
     "rwkv_hip_quantize_w4", "rwkv_hip_dequant_w4", "rwkv_hip_bf16_to_f16", "rwkv_hip_bf16_to_f16_transpose",
     "rwkv_hip_emb_ln0_bf16_to_f16", "rwkv_hip_fill_normal_f16", "rwkv_hip_linear",
-    "rwkv_hip_pack_weights", "rwkv_hip_linear_packed_workspace", "rwkv_hip_linear_packed", "rwkv_hip_lora_in", "rwkv_hip_lora_out",
+    "rwkv_hip_pack_weights", "rwkv_hip_linear_packed_workspace", "rwkv_hip_linear_packed_plan", "rwkv_hip_linear_packed", "rwkv_hip_lora_in", "rwkv_hip_lora_out",
     "rwkv_hip_cmix_sparse_pack", "rwkv_hip_cmix_sparse_pack_w4", "rwkv_hip_cmix_sparse_packed_bytes",
     "rwkv_hip_cmix_sparse_workspace", "rwkv_hip_cmix_sparse_down_relu_one",
     "rwkv_hip_cmix_sparse_down_relu_rows", "rwkv_hip_cmix_sparse_down_relu_rows_static",
@@ -252,6 +252,17 @@ def linear_packed_workspace(M, N, K):
     n = ctypes.c_size_t(0)
     check(load().rwkv_hip_linear_packed_workspace(_i(M), _i(N), _i(K), ctypes.byref(n)))
     return n.value
+
+
+def linear_packed_plan(M, K, problems, workspace_bytes):
+    """(rows, columns, K splits) of the tile that the packed product takes, and whether a model splits the launch in two; problems:
+    (format, N) each, several for a model's launch."""
+    Ns = (ctypes.c_int * len(problems))(*[n for _fmt, n in problems])
+    fmts = (ctypes.c_int * len(problems))(*[fmt for fmt, _n in problems])
+    out = [ctypes.c_int(0) for _ in range(4)]
+    check(load().rwkv_hip_linear_packed_plan(_i(M), _i(K), _i(len(problems)), Ns, fmts, ctypes.c_size_t(workspace_bytes),
+                                             *[ctypes.byref(x) for x in out]))
+    return tuple(x.value for x in out[:3]), out[3].value != 0
 
 
 def linear_packed(fmt, M, N, K, x, packed, scale, zp, y, workspace, epilogue=EPI_NONE, out_f32=0, stream=None):

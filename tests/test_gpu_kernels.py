@@ -1283,10 +1283,12 @@ def test_linear_packed_of_33_to_64_rows_without_a_workspace(gpu, orc, fmt_name, 
     assert err <= F16_TOL
 
 
-@pytest.mark.parametrize("fmt_name,M,N,K", [("w8", 330, 5184, 3072), ("w8", 1300, 4704, 2560), ("f16", 1300, 4704, 2560)])
-def test_linear_packed_wide_tiles_with_a_k_split(gpu, orc, fmt_name, M, N, K):
-    """The tiles of 64 x 256 and 128 x 256 where they split K (no other shape here makes them), rows on both sides of the tiles'
-    edges against the oracle."""
+@pytest.mark.parametrize("fmt_name,M,N,K,tile", [("w8", 330, 5184, 3072, (64, 256, 2)), ("w8", 1038, 1056, 10240, (128, 256, 4)),
+                                                 ("f16", 1556, 2400, 11264, (128, 256, 4)), ("w8", 2074, 2080, 4608, (256, 256, 2)),
+                                                 ("f16", 4109, 288, 4096, (256, 256, 4)), ("f16", 4109, 544, 7168, (256, 256, 8))])
+def test_linear_packed_wide_tiles_with_a_k_split(gpu, orc, fmt_name, M, N, K, tile):
+    """The tiles of 64, 128 and 256 rows x 256 columns where they split K, int8 and fp16, rows on both sides of the tiles' edges against
+    the oracle."""
     hip = gpu
     rng = np.random.default_rng(M + N)
     fmt = {"f16": hip.FMT_F16, "w8": hip.FMT_W8}[fmt_name]
@@ -1295,8 +1297,8 @@ def test_linear_packed_wide_tiles_with_a_k_split(gpu, orc, fmt_name, M, N, K):
     dparts = [dev(hip, p) if p is not None else None for p in parts]
     packed = hip.DeviceArray(parts[0].shape, parts[0].dtype)
     hip.pack_weights(fmt, N, K, dparts[0], packed)
-    assert hip.linear_packed_workspace(M, N, K) > 0
     ws = hip.DeviceArray((hip.linear_packed_workspace(M, N, K),), np.uint8)
+    assert hip.linear_packed_plan(M, K, [(fmt, N)], ws.nbytes)[0] == tile
     y = hip.DeviceArray((M, N), np.float16)
     hip.linear_packed(fmt, M, N, K, dev(hip, x), packed, dparts[1], dparts[2], y, ws)
     hip.device_sync()
@@ -1305,10 +1307,12 @@ def test_linear_packed_wide_tiles_with_a_k_split(gpu, orc, fmt_name, M, N, K):
     assert err <= F16_TOL
 
 
-@pytest.mark.parametrize("fmt_name,M,N,K", [("w8", 2049, 1696, 256), ("f16", 2049, 1696, 256), ("w8", 2049, 3136, 256), ("f16", 2049, 3136, 256),
-                                            ("w8", 1900, 3104, 768), ("f16", 2300, 3104, 768), ("w8", 2049, 832, 8192), ("w8", 2049, 1120, 4096),
-                                            ("w8", 2049, 544, 8192), ("f16", 1024, 8224, 512)])
-def test_linear_packed_tiles_of_many_rows(gpu, orc, fmt_name, M, N, K):
+@pytest.mark.parametrize("fmt_name,M,N,K,tile", [("w8", 2049, 1696, 256, (128, 256, 1)), ("f16", 2049, 1696, 256, (128, 256, 1)),
+                                                 ("w8", 2049, 3136, 256, (256, 256, 1)), ("f16", 2049, 3136, 256, (256, 256, 1)),
+                                                 ("w8", 1900, 3104, 768, (128, 256, 1)), ("f16", 2300, 3104, 768, (256, 256, 1)),
+                                                 ("w8", 2049, 832, 8192, (128, 256, 2)), ("w8", 2049, 1120, 4096, (256, 256, 4)),
+                                                 ("w8", 2049, 544, 8192, (256, 256, 8)), ("f16", 1024, 8224, 512, (256, 256, 1))])
+def test_linear_packed_tiles_of_many_rows(gpu, orc, fmt_name, M, N, K, tile):
     """Blocks of 128 and of 256 rows x 256 columns: as few stages as there are, a last row tile of one row and others, a last block of two
     and more bands, two, four and eight splits of K; both epilogues and output types, rows on both sides of the tiles' edges against
     the oracle."""
@@ -1321,6 +1325,7 @@ def test_linear_packed_tiles_of_many_rows(gpu, orc, fmt_name, M, N, K):
     packed = hip.DeviceArray(parts[0].shape, parts[0].dtype)
     hip.pack_weights(fmt, N, K, dparts[0], packed)
     ws = hip.DeviceArray((max(hip.linear_packed_workspace(M, N, K), 16),), np.uint8)
+    assert hip.linear_packed_plan(M, K, [(fmt, N)], ws.nbytes)[0] == tile
     rows = sorted({0, 1, 31, 32, 63, 64, 127, 128, 191, 255, 256, 511, M // 256 * 256 - 1, M - 2, M - 1})
     want = orc.gemv(fmt, x[rows], parts[0], parts[1], parts[2]).astype(np.float32)
     dx = dev(hip, x)

@@ -108,16 +108,20 @@ def test_small_model_prefill_and_decode(gpu, orc, fmt):
     sess.close()
 
 
+@pytest.mark.parametrize("T,tile", [(128, (128, 128)), (180, (128, 256)), (336, (256, 256))])
 @pytest.mark.parametrize("fmt", [0, 1])
-def test_many_row_prefill_chunk_on_the_wide_gemm_tile(gpu, orc, fmt):
-    """13 sequences x 128 tokens = 1664 rows: the r/k/v + rank-in launch (seven problems, int8 or fp16 next to fp16,
-    column counts of 512 and 32..64) has 13 x 10 tiles of 128 x 256 and takes the two-band tile; the other launches
-    stay on the 64- and 128-row tiles."""
+def test_many_row_prefill_chunk_on_the_wide_gemm_tile(gpu, orc, fmt, T, tile):
+    """13 sequences x 128, 180 and 336 tokens: the launch of r, k, v and the rank-ins (six problems, int8 or fp16 next to fp16, 512
+    columns and 32, 32 and 64, whose blocks have one and two bands) on the ring's largest tile and on the blocks of 128 and 256 rows x
+    256 columns.  k and v of every row reach the state, r and the gates of 13 rows, the last of each sequence, the logits."""
     from rwkv_lightning_cuda_amd.model import ModelDims, Session, State
     hip = gpu
-    dims = ModelDims(L=1, C=512, H=8, F=2048, V=256, Rw=32, Ra=32, Rg=64, Rv=32)
+    dims = ModelDims(L=1, C=512, H=8, F=512, V=256, Rw=32, Ra=32, Rg=64, Rv=32)
     omodel, gmodel = build_pair(gpu, orc, dims, fmt, seed=33)
-    B, T = 13, 128
+    B = 13
+    launch = [(fmt, dims.C)] * 3 + [(hip.FMT_F16, rank) for rank in (dims.Rw, dims.Ra, dims.Rg)]
+    plan, apart = hip.linear_packed_plan(B * T, dims.C, launch, 1 << 40)
+    assert plan == (*tile, 1) and not apart
     tokens = np.random.default_rng(8).integers(0, dims.V, (B, T))
     sess = Session(gmodel)
     gstate = State(dims, B)
