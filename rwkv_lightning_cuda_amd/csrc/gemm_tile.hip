@@ -43,7 +43,7 @@ struct WideTile {
 // 64 lanes x 16 bytes from base + off into LDS from `lds` on.  In asm, because the compiler would wait for every such load in flight
 // at the next read of LDS.
 __device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t off, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(off), "s"(base) : "memory");
 }
 
 template <int N>
