@@ -82,15 +82,15 @@ int pack_weights_launch(hipStream_t st, int fmt, int N, int K, const void* w, vo
 
 // ---- the GEMM ---------------------------------------------------------------------------------------------------------
 
-// The 64 x 256 tile: 32 * MT rows, chunks of KC k, four wavefronts.
-template <int FMT, int MT, int KC>
+// The 64 x 256 tile: 32 * MT rows, chunks of KC k, four wavefronts, int8 codes.
 struct Tile {
-  using P = PackTraits<FMT>;
+  using P = PackTraits<RWKV_FMT_W8>;
+  static constexpr int MT = 2, KC = 128;
   static constexpr int BM = 32 * MT;
   static constexpr int G = 2 * P::KR;
   static constexpr int GROUPS = KC / G;
   static constexpr int NW = GROUPS * P::PIECES;     // weight pieces per lane per chunk and band
-  static constexpr int STEPS = P::KR / 8;
+  static constexpr int STEPS = P::KR / 8;           // MFMA steps per group
   static constexpr int XSTRIDE = KC + 8;            // fp16 per staged row: 16-byte pad keeps b128 reads conflict-free
   static constexpr int GT = 256;                    // threads of the block
   static constexpr int XV = BM * (KC / 8) / GT;     // 16-byte vectors of X per thread per chunk
@@ -98,9 +98,9 @@ struct Tile {
 };
 
 // One chunk's slice of X held by a thread between request and its store to LDS.
-template <int FMT, int MT, int KC>
 struct XRegs {
-  using T = Tile<FMT, MT, KC>;
+  using T = Tile;
+  static constexpr int KC = T::KC;
   uint4_t xv[T::XV];
 
   // vector i of the thread's slice
@@ -132,9 +132,8 @@ struct XRegs {
 };
 
 // One chunk's weight pieces held by a lane between request and use.
-template <int FMT, int MT, int KC>
 struct WRegs {
-  using T = Tile<FMT, MT, KC>;
+  using T = Tile;
   uint4_t w[T::NW];
 
   // piece i of the chunk at kc
@@ -152,14 +151,11 @@ struct WRegs {
 // MFMAs.  One weight set per band, each piece requested again for the next chunk right after its last use (six MFMA steps ahead),
 // and one set of X, requested during the first half of a chunk's steps and stored during the second: 166 registers, three
 // wavefronts per SIMD, whose MFMAs fill each other's gaps.
-template <int FMT, int MT>
 __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const StreamProblem& pr, int row_tile, int col_block,
                                                   int split, half_t* xs) {
-  static_assert(FMT == RWKV_FMT_W8, "the rolling weight set is laid out for int8 pieces (two MFMA steps each)");
-  constexpr int KC = 128, NB = 2;
-  using T = Tile<FMT, MT, KC>;
-  using P = typename T::P;
-  constexpr int BM = T::BM;
+  using T = Tile;
+  using P = T::P;
+  constexpr int MT = T::MT, KC = T::KC, BM = T::BM, NB = 2;
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
@@ -183,10 +179,7 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
   }
   half_t scale_h[NB];  // the columns' int8 scales, requested before the main loop (in the epilogue: 1.2 us per launch)
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    scale_h[nb] = static_cast<half_t>(1.0f);
-    if constexpr (FMT == RWKV_FMT_W8) scale_h[nb] = pr.scale[n[nb]];
-  }
+  for (int nb = 0; nb < NB; ++nb) scale_h[nb] = pr.scale[n[nb]];
 
   float16_t acc[NB][MT];
 #pragma unroll
@@ -197,67 +190,65 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
       for (int v = 0; v < 16; ++v) acc[nb][mt][v] = 0.0f;
 
   constexpr int NK = T::GROUPS * T::STEPS;        // MFMA steps of a chunk
-  {
-    WRegs<FMT, MT, KC> w[NB];
-    XRegs<FMT, MT, KC> xq;
-    const int last = nchunks - 1;
-    xq.request(g, pr, tid, m0, kbeg);
+  WRegs w[NB];
+  XRegs xq;
+  const int last = nchunks - 1;
+  xq.request(g, pr, tid, m0, kbeg);
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) w[nb].request(kbeg, wband[nb]);
-    xq.store_x(tid, xs);
-    __syncthreads();
-    static_assert(T::XV % (NK / 2) == 0 && T::STEPS == 2 && T::NW == T::GROUPS,
-                  "a whole number of X vectors per MFMA step, two steps per weight piece");
-    constexpr int XPS = T::XV / (NK / 2);  // X vectors requested (first half of the steps) or stored (second half) per step
-    auto chunk = [&](int u, int c) {
-      const half_t* tile = xs + (u & 1) * T::kTileHalfs;
-      half_t* tile_next = xs + ((u + 1) & 1) * T::kTileHalfs;
-      const int knext = kbeg + (c + 1 <= last ? c + 1 : c) * KC;  // past the end: the current chunk again (in cache)
-      const half_t* xlane = tile + j * T::XSTRIDE + h * P::KR;
-      half8_t a[2][MT];
-      auto load_a = [&](int ks, half8_t (&dst)[MT]) {
-        const half_t* xa = xlane + (ks / T::STEPS) * T::G + 8 * (ks % T::STEPS);
+  for (int nb = 0; nb < NB; ++nb) w[nb].request(kbeg, wband[nb]);
+  xq.store_x(tid, xs);
+  __syncthreads();
+  static_assert(T::XV % (NK / 2) == 0 && T::STEPS == 2 && T::NW == T::GROUPS,
+                "a whole number of X vectors per MFMA step, two steps per weight piece");
+  constexpr int XPS = T::XV / (NK / 2);  // X vectors requested (first half of the steps) or stored (second half) per step
+  auto chunk = [&](int u, int c) {
+    const half_t* tile = xs + (u & 1) * T::kTileHalfs;
+    half_t* tile_next = xs + ((u + 1) & 1) * T::kTileHalfs;
+    const int knext = kbeg + (c + 1 <= last ? c + 1 : c) * KC;  // past the end: the current chunk again (in cache)
+    const half_t* xlane = tile + j * T::XSTRIDE + h * P::KR;
+    half8_t a[2][MT];
+    auto load_a = [&](int ks, half8_t (&dst)[MT]) {
+      const half_t* xa = xlane + (ks / T::STEPS) * T::G + 8 * (ks % T::STEPS);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) dst[mt] = *reinterpret_cast<const half8_t*>(xa + mt * 32 * T::XSTRIDE);
-      };
-      load_a(0, a[0]);
+      for (int mt = 0; mt < MT; ++mt) dst[mt] = *reinterpret_cast<const half8_t*>(xa + mt * 32 * T::XSTRIDE);
+    };
+    load_a(0, a[0]);
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks) {
-        const int gi = ks / T::STEPS;
-        const int st = ks % T::STEPS;
-        if (ks + 1 < NK) load_a(ks + 1, a[(ks + 1) & 1]);
+    for (int ks = 0; ks < NK; ++ks) {
+      const int gi = ks / T::STEPS;
+      const int st = ks % T::STEPS;
+      if (ks + 1 < NK) load_a(ks + 1, a[(ks + 1) & 1]);
 #pragma unroll
-        for (int i = 0; i < XPS; ++i) {
-          if (ks < NK / 2) {
-            xq.request_one(XPS * ks + i, g, pr, tid, m0, knext);
-          } else {
-            xq.store_one(XPS * (ks - NK / 2) + i, tid, tile_next);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const uint4_t piece = w[nb].w[gi];
-          const half8_t b = st == 0 ? expand_w8(piece[0], piece[1]) : expand_w8(piece[2], piece[3]);
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) acc[nb][mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks & 1][mt], b, acc[nb][mt], 0, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (st == T::STEPS - 1) {  // piece gi has been expanded for the last time: the next chunk's takes its place
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) w[nb].request_piece(gi, knext, wband[nb]);
+      for (int i = 0; i < XPS; ++i) {
+        if (ks < NK / 2) {
+          xq.request_one(XPS * ks + i, g, pr, tid, m0, knext);
+        } else {
+          xq.store_one(XPS * (ks - NK / 2) + i, tid, tile_next);
         }
       }
-      __syncthreads();
-    };
-    const int whole = nchunks - nchunks % 2;
-    int c0 = 0;
-    for (; c0 < whole; c0 += 2) {
-      chunk(0, c0);
-      chunk(1, c0 + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const uint4_t piece = w[nb].w[gi];
+        const half8_t b = st == 0 ? expand_w8(piece[0], piece[1]) : expand_w8(piece[2], piece[3]);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nb][mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks & 1][mt], b, acc[nb][mt], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (st == T::STEPS - 1) {  // piece gi has been expanded for the last time: the next chunk's takes its place
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) w[nb].request_piece(gi, knext, wband[nb]);
+      }
     }
-    if (c0 < nchunks) chunk(0, c0);
+    __syncthreads();
+  };
+  const int whole = nchunks - nchunks % 2;
+  int c0 = 0;
+  for (; c0 < whole; c0 += 2) {
+    chunk(0, c0);
+    chunk(1, c0 + 1);
   }
+  if (c0 < nchunks) chunk(0, c0);
 
   // output: one 128-column half of the tile at a time through LDS (the X tiles are free), written in 16/32-byte
   // pieces along the rows
@@ -306,8 +297,7 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
 }
 
 __global__ __launch_bounds__(256, 2) void gemm_stream_wide_kernel(StreamArgs g) {
-  constexpr int MT = 2;
-  __shared__ __align__(16) half_t xs[2 * 32 * MT * (128 + 8)];
+  __shared__ __align__(16) half_t xs[2 * Tile::kTileHalfs];
   ride_along_copy(g.copy, gridDim.x, blockDim.x);
   const int id = blockIdx.x;
   const int row_tile = (id >> 3) % g.row_tiles;
@@ -318,7 +308,7 @@ __global__ __launch_bounds__(256, 2) void gemm_stream_wide_kernel(StreamArgs g) 
   int pi = 0;
   while (pi + 1 < g.n_problems && col_all >= g.block_end[pi]) ++pi;
   const int col_block = col_all - (pi > 0 ? g.block_end[pi - 1] : 0);
-  stream_block_wide<RWKV_FMT_W8, MT>(g, g.p[pi], row_tile, col_block, split, xs);
+  stream_block_wide(g, g.p[pi], row_tile, col_block, split, xs);
 }
 
 // int4 scales and zero points by group: the 32 columns of a band then lie in one piece of 64 (32) bytes, where the rows of
