@@ -404,29 +404,32 @@ struct StreamConfig {
   }
   int k_step() const { return is_ring() ? ring.kc : 128; }
 };
-static int count_col_blocks(const StreamConfig& c, int n_problems, const int* Ns, const int* fmts) {
-  int col_blocks = 0;
-  for (int i = 0; i < n_problems; ++i) col_blocks += ceil_div(Ns[i], c.cols(fmts[i]));
-  return col_blocks;
-}
+
+// Blocks that occupy the 256 CUs well enough without a K split.
+constexpr int kFilledBlocks = 200;
+// Rows from which the tiles of 256 columns, whose wavefronts feed two MFMAs from every X fragment they read from LDS, are looked at.
+constexpr int kWideMinRows = 160;
 
 // Estimated microseconds of a launch: what the choice between tiles and K splits goes by.  Fitted to sweeps of every tile and
 // split over 5 .. 3000 rows x the matrices of the presets (768 .. 65536 columns, 768 .. 16384 k, three formats: 969 launches).
 // Its pick takes the best one's time in half of them; in geometric mean 1.04 (int8), 1.02 (fp16), 1.01 (int4 scales by row)
-// and 1.03 (by group) times, in one of ten more than 1.16 / 1.09 / 1.02 / 1.13 times.
+// and 1.03 (by group) times, in one of ten more than 1.16 / 1.09 / 1.02 / 1.13 times (before the tiles of 128 and 256 rows).
 //   ring: a fixed part (launch, first stage, epilogue); the bytes of the busiest CU at what a CU takes in while all of them
 //   stream (94 GB/s; 130 while half of the chip idles); what of the HBM stream of the weights does not hide behind that; the
 //   products; per further round of blocks its start and end, which a second block hides where two fit a CU.
-//   wide (64 x 256; 128 x 256 without `tiles`): bound by the matrix core.
+//   64 x 256: bound by the matrix core; rounds past the second overlap.
+//   128 and 256 x 256: a fixed part, then per stage of 64 k and round of blocks a time that grows with the blocks that run - the clock the
+//   chip holds goes down with them - but not less than the stage's weights take at 4 TB/s out of HBM, where few row tiles share them
+//   (fp16, 4096 x 16384, 160 .. 255 rows: tiles 56 .. 65 us, ring 46 .. 50); 128 rows: the start and end of every further round, 256
+//   rows of fp16: a clock that goes on falling over full rounds (65536 x 4096, 512 rows 287 us, blocks of 128 rows 260).
 //   K splits: their fp32 planes and, where no consumer sums them, the reduce launch; a consumer's block waits longer the more
 //   planes it asks for (0.15 us each; with 0 / 0.4 decode steps of 5 .. 16 rows are 1-4 % slower, 7.2B and 1.5B int8).
 //   int4 scales and zero points as [N][K/128] (group_rows): a cache line each per column and stage, of which the stage uses a few
 //   bytes.  Two bytes per code of what a CU takes in, 1.5 with stages of 256 k; up to 2048 k a column's lie in 48 bytes.
-//   tiles of 128 and 256 rows: a fixed part, then per stage of 64 k and round of blocks a time that grows with the blocks that run - the clock the chip
-//   holds goes down with them (190 launches of the presets' matrices at 256 .. 2048 rows, int8 and fp16: the pick takes 1.03 times the best one's
-//   time in geometric mean).  tiles == false keeps the estimate of the register-staged 128 x 256 tile that it replaced.
+// From 160 rows on, int8 and fp16, the pick takes 1.010 times the best one's time in geometric mean, in one call of twenty more than
+// 1.08 times (every tile and split measured over 14 matrices of the presets' sizes, 552 launches of 160 .. 2048 rows).
 static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred,
-                         bool group_rows, bool tiles) {
+                         bool group_rows) {
   constexpr int kCus = 256;
   const int bm = c.rows();
   int blocks = 0, bn_max = 0;
@@ -463,18 +466,17 @@ static float estimate_us(const StreamConfig& c, int M, int K, int n_problems, co
     const bool wide_ring = c.ring.mt == 4 || c.ring.wp == 4;
     us += rounds * gflop * (c.fmt == RWKV_FMT_W4 ? (wide_ring ? 0.73f : 0.57f) : (c.ring.mt == 4 && c.fmt == RWKV_FMT_W8 ? 0.55f : (c.ring.nb == 2 ? 0.37f : (c.ring.mt == 1 && c.ring.wp == 4 ? 0.30f : 0.28f))));
     us += (two_per_cu ? 1.5f : 4.5f) * (rounds - 1);
-  } else if (c.wide_rows > 64 && tiles) {
+  } else if (c.wide_rows > 64) {
+    const float stage_bytes = 64.0f * 256.0f * (1.0f + f16_share) / ceil_div(M, bm);  // of weights, per block: the row tiles share them
     auto round_us = [&](int running) {
       const float stage = c.wide_rows == 256 ? 1.08f + 0.0027f * running + f16_share * (0.22f - 0.0006f * running) : 0.58f + 0.0013f * running;
-      return stage * k_block / 64.0f;
+      return std::max(stage, running * stage_bytes / 4.0e6f) * k_block / 64.0f;
     };
     us = (c.wide_rows == 256 ? 10.0f : 11.0f) + full * round_us(kCus) + (rest > 0 ? round_us(rest) : 0.0f) +
-         (c.wide_rows == 256 ? 0.0f : 6.0f * (rounds - 1));
-  } else if (c.wide_rows == 64) {
-    us = 7.0f + 34.0f * std::max(1.0f, blocks * 1.05f / kCus) * k_block / 4096.0f;
-    if (tiles) us *= 1.09f;  // (measured beside the tiles: 256 .. 1000 rows 5 to 13 % over the line above)
+         (c.wide_rows == 256 ? f16_share * 0.3f * k_block / 64.0f * std::max(0, full - 1) : 6.0f * (rounds - 1));
   } else {
-    us = 6.0f + (full + (rest > 0 ? (full > 0 ? 0.75f + 0.25f * rest / kCus : 1.0f) : 0.0f)) * (11.0f + 58.0f * k_block / 4096.0f);
+    const float part = std::max(1.0f, blocks * 1.05f / kCus);
+    us = 1.09f * (7.0f + 34.0f * (part - 0.15f * std::max(0.0f, part - 2.0f)) * k_block / 4096.0f);
   }
   if (c.splits > 1) us += (deferred ? 0.35f + 0.15f * c.splits : 2.6f) + c.splits * M * n_total * (deferred ? 6.0f : 8.0f) / 5e6f;
   return us;
@@ -487,21 +489,15 @@ static bool sums_at_consumer(int n_problems, int epilogue, int out_f32) {
   return n_problems == 1 && epilogue == RWKV_EPI_NONE && !out_f32;
 }
 
-// Blocks that occupy the 256 CUs well enough without a K split.
-constexpr int kFilledBlocks = 200;
-// Rows from which the tiles of 256 columns, whose wavefronts feed two MFMAs from every X fragment they read from LDS, are looked at.
-constexpr int kWideMinRows = 160;
-
-// tiles: the blocks of 128 and 256 rows go by their own estimate.  Without, the choice - and with it the workspace that a call needs -
-// is what it was before them: the operator's for up to 512 rows, whose callers may rely on a product that needs no workspace.
+// wide: tiles of 256 columns are looked at (launch_config)
 static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, bool group_rows,
-                                  int max_splits, bool tiles) {
+                                  int max_splits, bool wide) {
   bool any[3] = {false, false, false};
   for (int i = 0; i < n_problems; ++i) any[fmts[i]] = true;
   StreamConfig best;
   auto consider = [&](StreamConfig c) {
     for (c.splits = 1; c.splits == 1 || (c.splits <= max_splits && K % (c.splits * c.k_step()) == 0); c.splits *= 2) {
-      c.us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred, group_rows, tiles);
+      c.us = estimate_us(c, M, K, n_problems, Ns, fmts, deferred, group_rows);
       if (c.us < best.us) best = c;
     }
   };
@@ -513,16 +509,9 @@ static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, c
     c.ring = shape;
     consider(c);
   }
-  if (M >= kWideMinRows && !any[RWKV_FMT_W4]) {
+  if (wide && M >= kWideMinRows && !any[RWKV_FMT_W4]) {
     c.ring = RingShape{0, 0, 0, 0};
-    c.wide_rows = 128;
-    // (from 1025 rows on, with most of the chip busy, the register-staged tile was the faster one whatever the estimates' last percent)
-    if (!tiles && M > 1024 && ceil_div(M, 128) * count_col_blocks(c, n_problems, Ns, fmts) >= kFilledBlocks) best.us = 1e30f;
-    consider(c);
-    if (tiles) {
-      c.wide_rows = 256;
-      consider(c);
-    }
+    for (c.wide_rows = 128; c.wide_rows <= 256; c.wide_rows *= 2) consider(c);
     if (!any[RWKV_FMT_F16] && K <= 4096 && M <= 1024) {
       c.wide_rows = 64;
       consider(c);
@@ -535,7 +524,7 @@ static StreamConfig search_config(int M, int K, int n_problems, const int* Ns, c
 // launch: each thread keeps the latest by all that they depend on (us per step, searching / kept: 1.5B shape fp16 4 rows
 // 1270 / 1236, int8 13 rows 1189 / 1158; 7.2B shape int8 8 rows 2239 / 2198; 0.1B shape fp16 8 rows 460 / 447).
 static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool deferred, bool group_rows,
-                                  int max_splits, bool tiles) {
+                                  int max_splits, bool wide) {
   struct Entry {
     int key[5 + 2 * kMaxProblems];
     bool used;
@@ -544,7 +533,7 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
   constexpr unsigned kSets = 32, kWays = 4;
   static thread_local Entry table[kSets][kWays];
   static thread_local unsigned oldest[kSets];
-  int key[5 + 2 * kMaxProblems] = {M, K, n_problems, (deferred ? 1 : 0) + (group_rows ? 2 : 0) + (tiles ? 4 : 0), max_splits};
+  int key[5 + 2 * kMaxProblems] = {M, K, n_problems, (deferred ? 1 : 0) + (group_rows ? 2 : 0) + (wide ? 4 : 0), max_splits};
   for (int i = 0; i < n_problems; ++i) {
     key[5 + 2 * i] = Ns[i];
     key[6 + 2 * i] = fmts[i];
@@ -556,21 +545,24 @@ static StreamConfig choose_config(int M, int K, int n_problems, const int* Ns, c
     if (e.used && memcmp(e.key, key, sizeof key) == 0) return e.config;
   Entry& e = table[set][oldest[set]];
   oldest[set] = (oldest[set] + 1) % kWays;
-  e.config = search_config(M, K, n_problems, Ns, fmts, deferred, group_rows, max_splits, tiles);
+  e.config = search_config(M, K, n_problems, Ns, fmts, deferred, group_rows, max_splits, wide);
   memcpy(e.key, key, sizeof key);
   e.used = true;
   return e.config;
 }
 
-constexpr int kOperatorTileRows = 512;  // the operator goes by the tiles' estimate above them, where a K split is an offer (packed_launch)
+// The operator: a K split is an offer, not a need, for int4 codes, from 513 rows on, where blocks of 32 x 32 alone occupy the chip and
+// where K has no power of two of whole 512s (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a
+// workspace too, with the split that fits.  Elsewhere a workspace too small for the split is an error.
+static bool split_is_an_offer(int fmt, int M, int64_t N, int K) {
+  return fmt == RWKV_FMT_W4 || M > 512 || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 || ceil_div(M, 32) * (N / 32) >= kFilledBlocks;
+}
 
-// The format is not known here: the largest that any of the choices would need, and never less than before the tiles had an estimate
-// of their own.
+// The format is not known here: the largest that any of the choices would need.
 size_t linear_packed_workspace_bytes(int M, int N, int K) {
   int splits = 1;
   for (const int fmt : {RWKV_FMT_W8, RWKV_FMT_W4, RWKV_FMT_F16})
-    for (const bool tiles : {false, M > kOperatorTileRows})
-      splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, false, fmt == RWKV_FMT_W4, 32, tiles).splits);
+    splits = std::max(splits, choose_config(M, K, 1, &N, &fmt, false, fmt == RWKV_FMT_W4, 32, split_is_an_offer(fmt, M, N, K)).splits);
   return splits > 1 ? static_cast<size_t>(splits) * M * N * sizeof(float) : 0;
 }
 
@@ -625,22 +617,20 @@ bool linear_packed_apart(int M, int K, int n_first, int n_problems, const Packed
 }
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
-                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, bool tiles,
-                         DeferredReduce* defer, const RowCopy* copy);
+                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, bool op, DeferredReduce* defer,
+                         const RowCopy* copy);
 
-// What a launch with this workspace takes.
-// A split is an offer, not a need, for int4 codes, from 513 rows on, where blocks of 32 x 32 alone occupy the chip and where K
-// has no power of two of whole 512s (1024s up to 32 rows, and up to 64 rows of K up to 2048): such a call runs without a
-// workspace too, with the split that fits.  Elsewhere a workspace too small for the split is an error.
+// What a launch with this workspace takes: no more K splits than fit it where they are an offer or the caller says so (fit_splits).  A
+// model's launches look at every tile, the operator (op) at those of 256 columns only where a split is an offer.  Elsewhere fewer than
+// 200 blocks of 32 x 32 leave them a handful of blocks, which want a split, and a call that runs without a workspace must go on to.
 static StreamConfig launch_config(int M, int K, int n_problems, const int* Ns, const int* fmts, bool at_consumer, bool group_rows,
-                                  size_t workspace_bytes, bool fit_splits, bool tiles) {
+                                  size_t workspace_bytes, bool fit_splits, bool op) {
   int64_t n_total = 0;
   for (int i = 0; i < n_problems; ++i) n_total += Ns[i];
   const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
-  fit_splits = fit_splits || fmts[0] == RWKV_FMT_W4 || M > 512 || K % (M <= 32 || (M <= 64 && K <= 2048) ? 1024 : 512) != 0 ||
-               static_cast<int64_t>(ceil_div(M, 32)) * (n_total / 32) >= kFilledBlocks;
-  const int max_splits = fit_splits ? static_cast<int>(std::min<size_t>(32, workspace_bytes / plane)) : 32;
-  return choose_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, max_splits, tiles);
+  const bool offer = split_is_an_offer(fmts[0], M, n_total, K);
+  const int max_splits = offer || fit_splits ? static_cast<int>(std::min<size_t>(32, workspace_bytes / plane)) : 32;
+  return choose_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, max_splits, !op || offer);
 }
 
 static int require_supported(int M, int K, int n_problems, const PackedProblem* problems) {
@@ -658,14 +648,14 @@ int linear_packed_multi(hipStream_t st, int M, int K, int n_problems, const Pack
   return for_each_launch(n_problems, problems, [&](int n, const PackedProblem* part) {
     // (several problems take no more K splits than fit the workspace)
     const int rc = packed_launch(st, M, K, n, part, epilogue, out_f32, workspace, workspace_bytes, n_problems > 1,
-                                 sums_at_consumer(n, epilogue, out_f32), true, n == n_problems ? defer : nullptr, copy);
+                                 sums_at_consumer(n, epilogue, out_f32), false, n == n_problems ? defer : nullptr, copy);
     copy = nullptr;  // the rows ride on the first launch
     return rc;
   });
 }
 
 static int packed_launch(hipStream_t st, int M, int K, int n_problems, const PackedProblem* problems, int epilogue, int out_f32,
-                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, bool tiles, DeferredReduce* defer,
+                         void* workspace, size_t workspace_bytes, bool fit_splits, bool at_consumer, bool op, DeferredReduce* defer,
                          const RowCopy* copy) {
   StreamArgs g;
   ReduceArgs r;
@@ -688,7 +678,7 @@ static int packed_launch(hipStream_t st, int M, int K, int n_problems, const Pac
   }
   const size_t plane = static_cast<size_t>(M) * n_total * sizeof(float);
   const StreamConfig cfg = launch_config(M, K, n_problems, Ns, fmts, at_consumer, group_rows, workspace ? workspace_bytes : 0, fit_splits,
-                                         tiles);
+                                         op);
   int col_blocks = 0;
   for (int i = 0; i < n_problems; ++i) {
     const PackedProblem& q = problems[i];
@@ -755,8 +745,7 @@ int linear_packed(hipStream_t st, int fmt, int M, int N, int K, const half_t* x,
                   const uint8_t* zp, int epilogue, int out_f32, void* y, void* workspace, size_t workspace_bytes) {
   const PackedProblem q = {packed, scale, zp, x, y, N, fmt};
   if (const int rc = require_supported(M, K, 1, &q)) return rc;
-  return packed_launch(st, M, K, 1, &q, epilogue, out_f32, workspace, workspace_bytes, false, false, M > kOperatorTileRows,
-                       nullptr, nullptr);
+  return packed_launch(st, M, K, 1, &q, epilogue, out_f32, workspace, workspace_bytes, false, false, true, nullptr, nullptr);
 }
 
 }  // namespace rwkv
@@ -783,8 +772,7 @@ int rwkv_hip_linear_packed_plan(int M, int K, int n_problems, const int* N, cons
     RWKV_REQUIRE(linear_packed_supported(fmt[i], M, N[i], K) && (n_problems == 1 || fmt[i] != RWKV_FMT_W4),
                  "linear_packed_plan: unsupported shape M=%d N=%d K=%d fmt=%d", M, N[i], K, fmt[i]);
   const bool several = n_problems > 1;
-  const StreamConfig c = launch_config(M, K, n_problems, N, fmt, false, fmt[0] == RWKV_FMT_W4, workspace_bytes, several,
-                                       several || M > kOperatorTileRows);
+  const StreamConfig c = launch_config(M, K, n_problems, N, fmt, false, fmt[0] == RWKV_FMT_W4, workspace_bytes, several, !several);
   *tile_rows = c.rows();
   *tile_cols = c.cols(c.fmt);
   *splits = c.splits;

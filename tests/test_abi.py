@@ -87,3 +87,28 @@ def test_workspace_queries_that_repeat_cost_no_search():
     for t in threads:
         t.join()
     assert all(row == want for out in got for row in out)
+
+
+@pytest.mark.parametrize("fmt,M,N,K,tile", [("w8", 208, 12288, 4096, (128, 128, 1)), ("w8", 256, 16384, 4096, (128, 128, 1)),
+                                            ("w8", 256, 65536, 4096, (256, 256, 1)), ("f16", 384, 12288, 4096, (128, 256, 1)),
+                                            ("f16", 208, 4096, 16384, (128, 128, 4)), ("f16", 512, 65536, 4096, (128, 256, 1))])
+def test_the_operator_of_some_hundred_rows_takes_the_tile_that_is_fastest(fmt, M, N, K, tile):
+    """Up to 512 rows the operator went by the time of a 128 x 256 tile that is not there any more, and the estimate of the ones that are
+    knew nothing of what few row tiles take out of HBM.  The fastest of every tile and split as measured; the next one takes 1.08 to
+    1.3 times as long.  Without a workspace there is no split, and no other tile where there was none."""
+    from rwkv_lightning_cuda_amd import hip
+    problem = [({"f16": hip.FMT_F16, "w8": hip.FMT_W8}[fmt], N)]
+    assert hip.linear_packed_plan(M, K, problem, hip.linear_packed_workspace(M, N, K))[0] == tile
+    assert hip.linear_packed_plan(M, K, problem, 0)[0][2] == 1
+    if tile[2] == 1:
+        assert hip.linear_packed_plan(M, K, problem, 0)[0] == tile
+
+
+def test_no_workspace_is_asked_for_that_no_launch_takes():
+    """From 513 rows on every launch runs with the splits that fit: the query is what the largest choice of the three formats takes (1300 x
+    4704 x 2560 asked for the two planes of a tile that was not looked at)."""
+    from rwkv_lightning_cuda_amd import hip
+    for M, N, K in ((1300, 4704, 2560), (1030, 3872, 512), (2049, 832, 8192), (1038, 1056, 10240), (600, 768, 3072)):
+        need = hip.linear_packed_workspace(M, N, K)
+        splits = [hip.linear_packed_plan(M, K, [(fmt, N)], 1 << 40)[0][2] for fmt in (hip.FMT_W8, hip.FMT_W4, hip.FMT_F16)]
+        assert need == (max(splits) * M * N * 4 if max(splits) > 1 else 0)

@@ -1283,7 +1283,7 @@ def test_linear_packed_of_33_to_64_rows_without_a_workspace(gpu, orc, fmt_name, 
     assert err <= F16_TOL
 
 
-@pytest.mark.parametrize("fmt_name,M,N,K,tile", [("w8", 330, 5184, 3072, (64, 256, 2)), ("w8", 1038, 1056, 10240, (128, 256, 4)),
+@pytest.mark.parametrize("fmt_name,M,N,K,tile", [("w8", 330, 5184, 4096, (64, 256, 2)), ("w8", 1038, 1056, 10240, (128, 256, 4)),
                                                  ("f16", 1556, 2400, 11264, (128, 256, 4)), ("w8", 2074, 2080, 4608, (256, 256, 2)),
                                                  ("f16", 4109, 288, 4096, (256, 256, 4)), ("f16", 4109, 544, 7168, (256, 256, 8))])
 def test_linear_packed_wide_tiles_with_a_k_split(gpu, orc, fmt_name, M, N, K, tile):
