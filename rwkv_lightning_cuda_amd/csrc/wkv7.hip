@@ -768,10 +768,12 @@ static bool feeders_pay(int heads, int T) {
 
 template <typename IO, typename WT>
 static int launch_recurrence(hipStream_t st, int B, int T, int C, int H, float* state, const SeqOperands<IO, WT>& op, IO* y) {
+  // a model's call: above kSeqHalfHeads such go in chunks or in the fused pass, unless they are tapped and a layer's vectors are off alignment
+  constexpr bool kModel = !std::is_same_v<IO, WT>;
   const int heads = B * H;
   if (T == 1) {
     launch_seq<IO, WT, 4, 1, false, false>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
-  } else if (!feeders_pay<IO>(heads, T)) {
+  } else if (!feeders_pay<IO>(heads, T) || (kModel && heads > kSeqHalfHeads)) {
     if (heads <= kSeqQuarterHeads) launch_seq<IO, WT, 1, 4, false, true>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
     else if (heads <= kSeqHalfHeads) launch_seq<IO, WT, 2, 2, false, true>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
     else launch_seq<IO, WT, 4, 1, false, true>(st, B, T, C, H, state, op.v, y, TmixSeqArgs{}, op);
@@ -779,7 +781,7 @@ static int launch_recurrence(hipStream_t st, int B, int T, int C, int H, float* 
     launch_feed<IO, WT, 1, 1, 4, 4, 2, 2, 1, true>(st, B, T, C, H, state, op, y);
   } else if (heads <= kSeqHalfHeads) {
     launch_feed<IO, WT, 2, 1, 4, 2, 2, 4, 1, true>(st, B, T, C, H, state, op, y);
-  } else {
+  } else if constexpr (!kModel) {
     constexpr bool kHalf = sizeof(IO) == 2;
     if (kHalf && heads <= kSeqAheadHeads) launch_feed<IO, WT, 2, 2, 4, 1, 2, 2, kHalf ? 4 : 6, kHalf>(st, B, T, C, H, state, op, y);
     else launch_feed<IO, WT, 2, 2, 4, 1, 2, 2, 6, false>(st, B, T, C, H, state, op, y);

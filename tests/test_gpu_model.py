@@ -364,6 +364,29 @@ def test_fused_launches_match_the_standalone_kernels_bitwise(gpu, fmt, B, T):
     _fused_launches_agree_with_the_standalone_kernels(gpu, HipModel.from_host_weights(dims, synth_weights(dims, 4), fmt), B, T)
 
 
+@pytest.mark.parametrize("B,T", [(17, 17), (17, 40), (33, 64), (8, 50)])
+def test_layer_vectors_off_alignment_keep_the_token_by_token_recurrence(gpu, B, T):
+    """k_k one half off its alignment: prefill calls that would go in chunks go token by token, above 128 heads in the fused launch or, tapped,
+    through the stand-alone kernels without feeders.  Bitwise the same, and the aligned model's chunks within fp16 roundings."""
+    from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
+    hip = gpu
+    dims = ModelDims(L=2, C=512, H=8, F=2048, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
+    weights = synth_weights(dims, 4)
+    models = [HipModel.from_host_weights(dims, weights, hip.FMT_W8) for _ in range(2)]
+    for l, w in enumerate(weights["layers"]):
+        models[1].set_tensor(l, hip.T_K_K, hip.DeviceArray.from_numpy(np.concatenate([w["k_k"][:1], w["k_k"]])).view(1, (dims.C,)))
+    _fused_launches_agree_with_the_standalone_kernels(hip, models[1], B, T)
+    tokens = np.random.default_rng(B + T).integers(0, dims.V, (B, T))
+    outs = []
+    for m in models:
+        sess, st, lg = Session(m), State(dims, B), hip.DeviceArray((B, dims.V), np.float32)
+        sess.forward(tokens, st, lg)
+        outs.append((lg.numpy(), st.wkv.numpy()))
+        sess.close()
+    assert outs[0][1].tobytes() != outs[1][1].tobytes()  # another route
+    assert rel_err(outs[1][0], outs[0][0]) <= 3e-3 and rel_err(outs[1][1], outs[0][1]) <= 3e-3
+
+
 @pytest.mark.parametrize("B,T", [(1, 300), (600, 2), (40, 31), (5, 411), (16, 130)])
 def test_layer_norm_blocks_of_several_rows_match_the_standalone_kernels_bitwise(gpu, B, T):
     """More than 256 rows: a LayerNorm block walks 2 or 4 rows, with the first row of a sequence at its start, inside it or
