@@ -318,7 +318,9 @@ int rwkv_hip_model_weight_bytes(const rwkv_hip_model* m, uint64_t* bytes);
 
 /* A session owns a stream, the activation arena and captured decode graphs.  One session serves
  * one caller at a time; several sessions may run concurrently against one model (the reference
- * instead allocates a stream + arena per call, src/rwkv7_fast_v4.cu:1087-1096). */
+ * instead allocates a stream + arena per call, src/rwkv7_fast_v4.cu:1087-1096).  The arena grows with the largest call and
+ * is kept: some 30 rows of C halves per token, and with the fp32 state, for prefill calls whose recurrence prepares its chunks
+ * ahead (up to 192 heads of all sequences), 28 KB per head and 16 tokens of up to 512: 171 MB at most. */
 int rwkv_hip_session_create(rwkv_hip_session** out, const rwkv_hip_model* m);
 int rwkv_hip_session_destroy(rwkv_hip_session* s);
 int rwkv_hip_session_stream(rwkv_hip_session* s, rwkv_stream_t* stream);

@@ -33,7 +33,7 @@
 // 95, 3 x 333 x 32 72 -> 48, 1 x 128 x 64 26.4 -> 22.4, 1 x 512 x 64 75 -> 47.  What bounds them: many heads, the issue of VALU
 // instructions (some 800 per wavefront and chunk) and the matrix core (2700 clocks), which add up although four wavefronts share a
 // SIMD; few heads, launches (three), the latency of one chunk's preparation (6 us) and 0.65 us per link of the chain, most of it LDS
-// and the requests for 31 KB per chunk and CU.
+// and the requests for 25 KB per chunk and block, two of which share a CU.
 #include <algorithm>
 
 #include "head_ops.h"
@@ -422,7 +422,8 @@ __device__ __forceinline__ float4_t sum4(const float4_t& a, const float4_t& b, c
   return r;
 }
 
-// GroupNorm, bonus and gate (the formulas and rounding points of lnx_rkvres_xg_kernel)
+// GroupNorm, bonus and gate (the formulas and rounding points of lnx_rkvres_xg_kernel, which the chain ends in; its sums are in the order of a
+// lane per channel, these in that of four: the two paths' outputs differ by roundings)
 __device__ __forceinline__ half4_t normalised_output(const float (&y)[4], half4_t r, half4_t k, half4_t v, half4_t gate, half4_t r_k, half4_t w,
                                                      half4_t b) {
   const float mean = row16_sum((y[0] + y[1]) + (y[2] + y[3])) * (1.0f / 64.0f);
@@ -560,7 +561,8 @@ struct ChunkOperands {
   float rk[4][kWave];
   float decay[kHead];
 };
-static_assert(sizeof(ChunkOperands) == 27904, "the figures at the head of this file, at chunk_path and in the documents");
+static_assert(sizeof(ChunkOperands) == 27904, "28 KB in the figures of this file, of rwkv_hip.h and of the documents; a block of the chain reads V's "
+                                               "rows of its own, 3 KB less");
 
 // One block per (sequence, head, chunk).  Tokens t_begin .. t_end - 1 of a call of T.
 __global__ __launch_bounds__(256) void wkv7_chunk_prepare_kernel(int T, int C, int H, int t_begin, int t_end, int chunks, TmixSeqArgs fa,
@@ -733,7 +735,7 @@ enum class ChunkPath { kNone, kWhole, kChain };
 //   whole heads                     8.0       8.1      12.6      39.0       33.0       92.9       95.3
 // A chunk costs the same with one token in it as with sixteen.  The chain needs three launches and pays from a few chunks on, as
 // long as there are CUs for the blocks of a head; with more heads the kernel for whole ones has work for every CU (the few percent
-// around 320 heads, whose blocks are a round and a quarter, are not worth 31 KB per head and chunk).  Three prompts of the 7.2B shape,
+// around 320 heads, whose blocks are a round and a quarter, are not worth 28 KB per head and chunk).  Three prompts of the 7.2B shape,
 // whole heads / chain, ms a pass: 128 tokens 8.30 / 8.29, 256 14.80 / 14.44, 512 26.2 / 26.2.
 ChunkPath chunk_path(int heads, int T) {
   if (T < 10) return ChunkPath::kNone;
