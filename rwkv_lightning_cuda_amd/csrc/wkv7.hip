@@ -768,7 +768,7 @@ static bool feeders_pay(int heads, int T) {
 
 template <typename IO, typename WT>
 static int launch_recurrence(hipStream_t st, int B, int T, int C, int H, float* state, const SeqOperands<IO, WT>& op, IO* y) {
-  // a model's call: above kSeqHalfHeads such go in chunks or in the fused pass, unless they are tapped and a layer's vectors are off alignment
+  // a model's call: above kSeqHalfHeads such go in chunks or in the fused pass, unless they are tapped and too short for chunks or off alignment
   constexpr bool kModel = !std::is_same_v<IO, WT>;
   const int heads = B * H;
   if (T == 1) {

@@ -737,12 +737,18 @@ enum class ChunkPath { kNone, kWhole, kChain };
 // long as there are CUs for the blocks of a head; with more heads the kernel for whole ones has work for every CU (the few percent
 // around 320 heads, whose blocks are a round and a quarter, are not worth 28 KB per head and chunk).  Three prompts of the 7.2B shape,
 // whole heads / chain, ms a pass: 128 tokens 8.30 / 8.29, 256 14.80 / 14.44, 512 26.2 / 26.2.
+// Whole heads pay for the tokens that a last chunk has not: us per layer of a model, chunks less token by token, 17 / 18 / 20 / 21 tokens: 192
+// heads -0.1 / -0.4 / -1.3 / -, 320 1.6 / 1.1 / 0.7 / -, 384 1.4 / 1.2 / 0.2 / -0.7, 512 1.1 / 1.0 / 0.2 / -, 1024 -0.5 / -1.4 / -3.1 / -, 2048 0.6 / -1.5 /
+// -5.2 / - (up to 512 heads the fused kernel has two of them on a CU); 96 heads 26 / 32 / 42 / 48 / 58 / 63 tokens -1.3 / -1.3 / 2.1 / 1.0 / 3.1 / 1.6,
+// 128 heads -1.1 / -0.6 / 0.1 / -0.1 / 2.8 / 1.9.
 ChunkPath chunk_path(int heads, int T) {
   if (T < 10) return ChunkPath::kNone;
-  if (heads > 192 || (heads > 128 && T < 128) || T <= kTok) return ChunkPath::kWhole;
+  if (T <= kTok) return ChunkPath::kWhole;
+  if (heads > 128 && T <= (heads > 256 && heads <= 512 ? 20 : 17)) return ChunkPath::kNone;
+  if (heads > 192 || (heads > 128 && T < 128)) return ChunkPath::kWhole;
   if (heads <= 64) return T >= 48 ? ChunkPath::kChain : ChunkPath::kNone;
   if (T >= 64) return ChunkPath::kChain;
-  return ceil_div(T, kTok) * kTok - T <= 6 ? ChunkPath::kWhole : ChunkPath::kNone;
+  return T >= 26 && T <= 32 ? ChunkPath::kWhole : ChunkPath::kNone;
 }
 
 }  // namespace

@@ -364,10 +364,13 @@ def test_fused_launches_match_the_standalone_kernels_bitwise(gpu, fmt, B, T):
     _fused_launches_agree_with_the_standalone_kernels(gpu, HipModel.from_host_weights(dims, synth_weights(dims, 4), fmt), B, T)
 
 
-@pytest.mark.parametrize("B,T", [(17, 17), (17, 40), (33, 64), (8, 50)])
-def test_layer_vectors_off_alignment_keep_the_token_by_token_recurrence(gpu, B, T):
+@pytest.mark.parametrize("B,T,chunks", [(17, 17, False), (17, 18, True), (17, 40, True), (33, 20, False), (33, 21, True), (64, 20, False), (65, 18, True),
+                                        (33, 64, True), (8, 50, True), (9, 25, False), (16, 32, True), (9, 33, False), (9, 42, False), (16, 48, False),
+                                        (9, 63, False), (9, 64, True)])
+def test_layer_vectors_off_alignment_keep_the_token_by_token_recurrence(gpu, B, T, chunks):
     """k_k one half off its alignment: prefill calls that would go in chunks go token by token, above 128 heads in the fused launch or, tapped,
-    through the stand-alone kernels without feeders.  Bitwise the same, and the aligned model's chunks within fp16 roundings."""
+    through the stand-alone kernels without feeders.  Bitwise the same, and the aligned model's chunks within fp16 roundings; where the
+    aligned model does not go in chunks (a last chunk of few tokens, and what lies between one chunk and a chain), the same bits."""
     from rwkv_lightning_cuda_amd.model import HipModel, ModelDims, Session, State, synth_weights
     hip = gpu
     dims = ModelDims(L=2, C=512, H=8, F=2048, V=1024, Rw=32, Ra=32, Rg=64, Rv=32)
@@ -383,7 +386,7 @@ def test_layer_vectors_off_alignment_keep_the_token_by_token_recurrence(gpu, B, 
         sess.forward(tokens, st, lg)
         outs.append((lg.numpy(), st.wkv.numpy()))
         sess.close()
-    assert outs[0][1].tobytes() != outs[1][1].tobytes()  # another route
+    assert (outs[0][1].tobytes() != outs[1][1].tobytes()) == chunks
     assert rel_err(outs[1][0], outs[0][0]) <= 3e-3 and rel_err(outs[1][1], outs[0][1]) <= 3e-3
 
 
@@ -459,7 +462,7 @@ def test_debug_buffers_of_the_recurrences_fp32_operands(gpu):
 
 
 @pytest.mark.parametrize("H,B,T", [(8, 1, 10), (8, 1, 16), (8, 1, 50), (8, 1, 64), (8, 1, 65), (8, 1, 530), (5, 1, 97), (5, 15, 66),
-                                   (8, 9, 32), (8, 9, 79), (5, 26, 11), (8, 17, 33), (8, 17, 130), (8, 25, 130), (8, 40, 17)])
+                                   (8, 9, 32), (8, 9, 79), (5, 26, 11), (8, 17, 33), (8, 17, 130), (8, 25, 130), (8, 40, 17), (8, 40, 21)])
 @pytest.mark.parametrize("slow", [False, True])
 def test_chunked_recurrence_matches_the_token_by_token_operator(gpu, H, B, T, slow):
     """Prefill calls of more than a few tokens run the fp32-state recurrence in chunks of 16 tokens: few heads as a chain over prepared
