@@ -42,13 +42,14 @@ HIP_FLAGS = [
 REQUIRED_OCCUPANCY = {"linear_gemv_row1_kernelILi1024ELb1ELi0ELi1ELi1E": 8, "linear_gemv_row1_kernelILi1024ELb1ELi1ELi1ELi1E": 8,
                       "linear_gemv_row1_kernelILi1024ELb1ELi2ELi1ELi1E": 8, "linear_gemv_row1_kernelILi1024ELb1ELi1ELi2ELi1E": 8,
                       "gemm_tile_kernel": 2,  # two wavefronts per SIMD: one block per CU
+                      "gemm_stream_wide_kernel": 3,  # three blocks per CU
                       "wkv7_chunk_kernel": 4,  # four blocks of a head per CU
                       "linear_gemv_row1_kernelILi1024ELb1ELi2ELi1ELi2E": 4, "linear_gemv_row1_kernelILi1024ELb1ELi2ELi2ELi2E": 4}
 # Kernels of 768 threads get three wavefronts per SIMD whatever they need and spill the rest: most spilled registers (the first
 # fragment that matches counts; the int4 tile of 128 x 128 beside fp16 problems is two over its 168).  The WKV feeders' tiles demand
 # their wavefronts in the launch bounds (template arguments: ..., sets, wavefronts per SIMD, reading ahead); fp32 tensors on many
 # heads are ten registers over and measured to be faster so than with fewer wavefronts.
-MOST_SPILLS = {"gemm_tile_kernel": 0, "gemm_ring_kernelILi2ELb1ELi4ELi1ELi4ELi128E": 2, "gemm_ring_kernelI": 0,
+MOST_SPILLS = {"gemm_tile_kernel": 0, "gemm_stream_wide_kernel": 9, "gemm_ring_kernelILi2ELb1ELi4ELi1ELi4ELi128E": 2, "gemm_ring_kernelI": 0,
                "wkv7_feed_kernelIffLi2ELi2ELi4ELi1ELi2ELi2ELi6ELb0E": 10, "wkv7_feed_kernelI": 0, "wkv7_seq_kernelI": 0,
                "wkv7_chunk_kernel": 10, "wkv7_chunk_prepare_kernel": 0, "wkv7_chunk_chain_kernel": 0}
 

@@ -149,8 +149,10 @@ struct WRegs {
 // ---- some hundred rows of int8 weights: 64 rows x 256 columns per block, two bands per wavefront ----------------------
 // A wavefront keeps two 32-column bands (wave w: bands w and w + 4 of the block), so each X fragment it reads from LDS feeds two
 // MFMAs.  One weight set per band, each piece requested again for the next chunk right after its last use (six MFMA steps ahead),
-// and one set of X, requested during the first half of a chunk's steps and stored during the second: 166 registers, three
-// wavefronts per SIMD, whose MFMAs fill each other's gaps.
+// and one set of X, requested during the first half of a chunk's steps and stored during the second: 168 registers and nine spilled,
+// three wavefronts per SIMD, whose MFMAs fill each other's gaps.  (us per launch, 178 registers and two wavefronts / this: 65536 x 768, 160 rows
+// 34.0 / 31.7, 600 rows 90.6 / 85.6; 32768 x 1024, 320 rows 37.7 / 34.1; 65536 x 2048, 192 rows 64.1 / 62.4; 16384 x 4096, 600 rows 102.5 /
+// 96.7, 320 rows, about a block per CU, 60.6 / 62.1.)
 __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const StreamProblem& pr, int row_tile, int col_block,
                                                   int split, half_t* xs) {
   using T = Tile;
@@ -296,7 +298,7 @@ __device__ __forceinline__ void stream_block_wide(const StreamArgs& g, const Str
   }
 }
 
-__global__ __launch_bounds__(256, 2) void gemm_stream_wide_kernel(StreamArgs g) {
+__global__ __launch_bounds__(256, 3) void gemm_stream_wide_kernel(StreamArgs g) {
   __shared__ __align__(16) half_t xs[2 * Tile::kTileHalfs];
   ride_along_copy(g.copy, gridDim.x, blockDim.x);
   const int id = blockIdx.x;
