@@ -740,15 +740,16 @@ enum class ChunkPath { kNone, kWhole, kChain };
 // Whole heads pay for the tokens that a last chunk has not: us per layer of a model, chunks less token by token, 17 / 18 / 20 / 21 tokens: 192
 // heads -0.1 / -0.4 / -1.3 / -, 320 1.6 / 1.1 / 0.7 / -, 384 1.4 / 1.2 / 0.2 / -0.7, 512 1.1 / 1.0 / 0.2 / -, 1024 -0.5 / -1.4 / -3.1 / -, 2048 0.6 / -1.5 /
 // -5.2 / - (up to 512 heads the fused kernel has two of them on a CU); 96 heads 26 / 32 / 42 / 48 / 58 / 63 tokens -1.3 / -1.3 / 2.1 / 1.0 / 3.1 / 1.6,
-// 128 heads -1.1 / -0.6 / 0.1 / -0.1 / 2.8 / 1.9.
+// 128 heads -1.1 / -0.6 / 0.1 / -0.1 / 2.8 / 1.9.  A chain of four chunks, 48 / 49 / 64 / 65 tokens: 12 heads -0.8 / -0.7 / -1.0 / -0.8, 32 -0.5 / 0.6 / -0.3 /
+// 0.0, 48 0.6 / 0.0 / -1.1 / -0.9, 64 0.6 / 0.8 / -0.6 / -0.1.
 ChunkPath chunk_path(int heads, int T) {
   if (T < 10) return ChunkPath::kNone;
   if (T <= kTok) return ChunkPath::kWhole;
   if (heads > 128 && T <= (heads > 256 && heads <= 512 ? 20 : 17)) return ChunkPath::kNone;
   if (heads > 192 || (heads > 128 && T < 128)) return ChunkPath::kWhole;
-  if (heads <= 64) return T >= 48 ? ChunkPath::kChain : ChunkPath::kNone;
+  if (heads <= 32) return T >= 48 ? ChunkPath::kChain : ChunkPath::kNone;
   if (T >= 64) return ChunkPath::kChain;
-  return T >= 26 && T <= 32 ? ChunkPath::kWhole : ChunkPath::kNone;
+  return heads > 64 && T >= 26 && T <= 32 ? ChunkPath::kWhole : ChunkPath::kNone;
 }
 
 }  // namespace

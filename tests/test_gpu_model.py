@@ -365,7 +365,7 @@ def test_fused_launches_match_the_standalone_kernels_bitwise(gpu, fmt, B, T):
 
 
 @pytest.mark.parametrize("B,T,chunks", [(17, 17, False), (17, 18, True), (17, 40, True), (33, 20, False), (33, 21, True), (64, 20, False), (65, 18, True),
-                                        (33, 64, True), (8, 50, True), (9, 25, False), (16, 32, True), (9, 33, False), (9, 42, False), (16, 48, False),
+                                        (33, 64, True), (4, 47, False), (4, 48, True), (8, 30, False), (8, 63, False), (8, 64, True), (9, 25, False), (16, 32, True), (9, 33, False), (9, 42, False), (16, 48, False),
                                         (9, 63, False), (9, 64, True)])
 def test_layer_vectors_off_alignment_keep_the_token_by_token_recurrence(gpu, B, T, chunks):
     """k_k one half off its alignment: prefill calls that would go in chunks go token by token, above 128 heads in the fused launch or, tapped,
